@@ -1,12 +1,26 @@
-// Causal attention over paged rows for any head widths, one workgroup per (token, query head), f32 arithmetic throughout:
-// 32-bit models, and head widths that the MFMA kernels do not take.
+// Causal attention over paged rows for any head widths in f32 arithmetic throughout (f32 MFMA): 32-bit models, and head widths that
+// the bf16 MFMA kernels do not take.
+//
+// Workgroup = 16 rows of one key head, its waves split the keys 16 at a time and meet in LDS. The rows are the query heads of one
+// token (up to 16 of them), or, where several tokens of a launch belong to one sequence, of 16 / heads tokens, so that a prompt's
+// keys are read once for them; a group whose tokens belong to several sequences walks each one's keys.
+// Per 16 keys and wave, with v_mfma_f32_16x16x4_f32:
+//   S^T = K Q^T: lane 16 g + r loads 16 bytes of key r at column 16 s + 4 g, the operands of four MFMAs, and meets the same columns of
+//   row r, which wait in LDS; it ends with the scores of keys 4 g .. 4 g + 3 and row r, so that maximum and rescale are two lane
+//   exchanges and lane-local;
+//   O^T += V^T P^T: those registers are the second operand as they stand; 16 bytes of value row 4 g + j at column 64 q + 4 r are
+//   the first operand of the four tiles of columns 64 q + 4 m + e.
+// Loads run one chunk of key columns and two of value columns ahead; nothing goes through LDS but the queries and the merge.
+// What bounds it: the matrix pipe on prompts (32 cycles per MFMA, rows past a run's last token included), the walk over a row's keys on
+// small grids. Three prompts of 300 tokens, 16 heads of 128 over 4: 823 us (one workgroup per row and head, a serial walk) -> 43 us;
+// four decoded tokens behind 300 keys: 136 -> 16 us.
 #pragma once
 #include "../kernels/common.h"
 
 namespace nls_plain {
 
-constexpr int NC = 4;         // output columns per thread: values of up to 256 * NC columns
-constexpr int MAXK = 2048;    // key columns
+constexpr int MAXV = 1024, MAXK = 2048;     // value and key columns
+constexpr int VB = 512;                     // value columns of a workgroup (its accumulators; wider values score twice)
 
 struct PA {
   const void *q, *k, *v;
@@ -23,6 +37,7 @@ struct PA {
   int Dk, Dv;                 // columns (Dk a multiple of 4)
   float scale;
   int window, keep, sink;     // window > 0: the newest `window` keys and the first `keep`; sink: one more in the denominator
+  int T, tb, sub;             // tokens; tokens of a workgroup; workgroups that share a key head's query heads
 };
 
 template <typename T> DEVI f32x4 ld4(const T* p) {
@@ -31,74 +46,227 @@ template <typename T> DEVI f32x4 ld4(const T* p) {
   return f32x4{(float)a[0], (float)a[1], (float)a[2], (float)a[3]};
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void attn_plain_kernel(PA p) {
-  __shared__ __attribute__((aligned(16))) float q[MAXK], sc[64];
-  const int t = blockIdx.x, h = blockIdx.y;
-  const int ctx = p.ctx_len[t];
-  const int* bt = p.bt + (size_t)p.tok_seq[t] * p.bts;
-  const T* kc = reinterpret_cast<const T*>(p.k) + (size_t)(h / p.gs) * p.khs;
-  const T* vc = reinterpret_cast<const T*>(p.v) + (size_t)(h / p.gs) * p.khs;
-  const T* qr = reinterpret_cast<const T*>(p.q) + (size_t)t * p.ldq + (size_t)h * p.qhs;
-  for (int i = threadIdx.x; i < p.Dk; i += 256) q[i] = (float)qr[i];
-  __syncthreads();
-  const int key = threadIdx.x >> 2, part = threadIdx.x & 3;
-  float m = p.sink ? 0.f : -INFINITY, l = p.sink ? 1.f : 0.f, acc[NC] = {0.f, 0.f, 0.f, 0.f};
-  const int low = p.window > 0 ? ctx - p.window : 0;                  // first key of the window
-  for (int k0 = 0; k0 < ctx; k0 += 64) {
-    if (k0 >= p.keep && k0 + 64 <= low) k0 = low & ~63;               // (none of the tiles between is seen)
-    const int k = k0 + key;
-    const bool see = k < ctx && (k >= low || k < p.keep);
-    float s = 0.f;
-    if (k < ctx) {
-      const T* c = kc + ((size_t)bt[k / p.bs] * p.bs + k % p.bs) * p.ldkv;
-      for (int d = part * 4; d < p.Dk; d += 16) {
-        const f32x4 a = ld4(c + d), b = *reinterpret_cast<const f32x4*>(q + d);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s = fmaf(a[e], b[e], s);
-      }
+// NQ: 64-column blocks of the values; NW: waves
+template <typename T, int NQ, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
+  constexpr int KC = NQ > 2 ? 4 : 8;               // 16-column steps of a key chunk
+  constexpr int ML = NW * 32;                      // floats of the waves' maxima and sums
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nks = (p.Dk + 15) >> 4, nc = (nks + KC - 1) / KC, ldl = nc * KC * 16 + 4;
+  float *mls = sm, *ob = sm + ML, *qs = ob;        // (the merge takes the queries' place)
+  const int kh = blockIdx.y / p.sub, h0 = (blockIdx.y % p.sub) * 16;          // key head, first of its query heads
+  const int gr = min(p.gs - h0, 16);                                          // query heads of this workgroup
+  const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * p.tb, tn = min(p.tb, p.T - t0);      // (later tokens see more keys)
+  const int nrow = tn * gr;
+  const int v0 = blockIdx.z * VB, dv = min(p.Dv - v0, VB);                    // this workgroup's value columns
+  const T* kc = reinterpret_cast<const T*>(p.k) + (size_t)kh * p.khs;
+  const T* vc = reinterpret_cast<const T*>(p.v) + (size_t)kh * p.khs + v0;
+  auto head = [&](int row) { return (size_t)kh * p.gs + h0 + row % gr; };
+  for (int i = threadIdx.x; i < 4 * ldl; i += 64 * NW) {
+    const int row = i / (ldl / 4), c = (i - row * (ldl / 4)) * 4;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (row < nrow && c < p.Dk) {
+      const T* x = reinterpret_cast<const T*>(p.q) + (size_t)(t0 + row / gr) * p.ldq + head(row) * p.qhs + c;
+      v = f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
     }
-    s += __shfl_xor(s, 1, 64);
-    s += __shfl_xor(s, 2, 64);
-    if (part == 0) sc[key] = see ? s * p.scale : -INFINITY;
-    __syncthreads();
-    float mn = m;
-    for (int i = 0; i < 64; ++i) mn = fmaxf(mn, sc[i]);
-    const float alpha = m == -INFINITY ? 0.f : expf(m - mn), base = mn == -INFINITY ? 0.f : mn;
-    l *= alpha;
-#pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] *= alpha;
-    m = mn;
-    const int n = min(64, ctx - k0);
-    for (int i = 0; i < n; ++i) {
-      const float e = expf(sc[i] - base);
-      l += e;
-      const int kk = k0 + i;
-      const T* c = vc + ((size_t)bt[kk / p.bs] * p.bs + kk % p.bs) * p.ldkv;
-#pragma unroll
-      for (int q4 = 0; q4 < NC; ++q4) {
-        const int col = threadIdx.x + 256 * q4;
-        if (col < p.Dv) acc[q4] = fmaf(e, (float)c[col], acc[q4]);
-      }
-    }
-    __syncthreads();
+    *reinterpret_cast<f32x4*>(qs + row * ldl + c) = v;
   }
-  const float inv = (l > 0.f ? 1.f / l : 0.f) * (p.gate ? p.gate[(size_t)t * p.ldg + h] : 1.f);
-  T* y = reinterpret_cast<T*>(p.out) + (size_t)t * p.ldo + (size_t)h * p.ohs;
+  __syncthreads();
+
+  f32x4 o[NQ][4];
 #pragma unroll
-  for (int q4 = 0; q4 < NC; ++q4) {
-    const int col = threadIdx.x + 256 * q4;
-    if (col < p.Dv) y[col] = (T)(acc[q4] * inv);
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[q][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = p.sink && wave == 0 ? 0.f : -INFINITY, l = p.sink && wave == 0 && g == 0 ? 1.f : 0.f;      // (l: four lanes' shares)
+  for (int a = 0; a < tn;) {
+    // tokens a .. b - 1 of the group belong to one sequence
+    const int seq = p.tok_seq[t0 + a];
+    int b = a, ctx = 0, low = 1 << 30;
+    for (; b < tn && p.tok_seq[t0 + b] == seq; ++b) {
+      const int c = p.ctx_len[t0 + b];
+      ctx = max(ctx, c);
+      if (c > 0) low = min(low, p.window > 0 ? max(c - p.window, 0) : 0);
+    }
+    const int tok = r / gr;
+    const int rctx = r < nrow && tok >= a && tok < b ? p.ctx_len[t0 + tok] : 0, rlow = p.window > 0 ? rctx - p.window : 0;
+    a = b;
+    if (ctx <= 0) continue;
+    const int* bt = p.bt + (size_t)seq * p.bts;
+    // tiles that no row sees are left out: `skip` of them behind the kept keys' `nkt`
+    const int lowt = low >> 4, nkt = min((p.keep + 15) >> 4, lowt), skip = lowt - nkt, ntile = ((ctx + 15) >> 4) - skip;
+    auto key0 = [&](int t) { return (t < nkt ? t : t + skip) * 16; };
+    auto slot = [&](int t) { return [&](int k) { return bt[k / p.bs] * p.bs + k % p.bs; }(min(key0(t) + r, ctx - 1)); };
+    auto load_k = [&](f32x4 (&f)[KC], int s, int c) __attribute__((always_inline)) {
+      const T* row = kc + (size_t)s * p.ldkv;
+      const int c0 = c * (KC * 16) + 4 * g;
+      if ((c + 1) * (KC * 16) <= p.Dk) {
+#pragma unroll
+        for (int i = 0; i < KC; ++i) f[i] = ld4(row + c0 + 16 * i);
+      } else {
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {             // (zeros past the last column: what is loaded there may not be finite)
+          f[i] = ld4(row + min(c0 + 16 * i, p.Dk - 4));
+          if (c0 + 16 * i >= p.Dk) f[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    };
+    auto load_v = [&](f32x4 (&f)[4], const int (&s)[4], int q) __attribute__((always_inline)) {
+      const int c0 = 64 * q + 4 * r;               // (columns past the last one are computed and not stored)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const T* row = vc + (size_t)s[j] * p.ldkv;
+        if (!(dv & 3)) f[j] = ld4(row + min(c0, dv - 4));
+        else
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f[j][e] = (float)row[min(c0 + e, dv - 1)];
+      }
+    };
+    if (wave >= ntile) continue;
+    int sk = slot(wave);
+    f32x4 kf[KC], kn[KC], vf[2][4];
+    load_k(kf, sk, 0);
+    for (int t = wave; t < ntile; t += NW) {
+      const int sn = slot(min(t + NW, ntile - 1));
+      int sv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sv[j] = __shfl(sk, 4 * g + j, 64);
+      load_v(vf[0], sv, 0);
+      if (NQ > 1) load_v(vf[1], sv, 1);
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+      for (int c = 0; c < nc; ++c) {
+        if (c + 1 < nc) load_k(kn, sk, c + 1);
+        else load_k(kn, sn, 0);
+        const float* qr = qs + r * ldl + c * (KC * 16) + 4 * g;
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(qr + 16 * i);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][j], x[j], s, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < KC; ++i) kf[i] = kn[i];
+      }
+      const int k0 = key0(t) + 4 * g;
+      float mx = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int k = k0 + j;
+        s[j] = k < rctx && (k >= rlow || k < p.keep) ? s[j] * p.scale : -INFINITY;
+        mx = fmaxf(mx, s[j]);
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(m, mx), base = mn == -INFINITY ? 0.f : mn;
+      if (!__all(mn == m)) {
+        const float alpha = m == -INFINITY ? 0.f : expf(m - base);
+        l *= alpha;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[q][e] *= alpha;
+        m = mn;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s[j] = expf(s[j] - base);
+        l += s[j];
+      }
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[q][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[q & 1][j][e], s[j], o[q][e], 0, 0, 0);
+        if (q + 2 < NQ) load_v(vf[q & 1], sv, q + 2);
+      }
+      sk = sn;
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (g == 0) {
+    mls[wave * 32 + r] = m;
+    mls[wave * 32 + 16 + r] = l;
+  }
+  __syncthreads();                                 // (the queries have been read, too)
+  float M = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) M = fmaxf(M, mls[w * 32 + r]);
+  const float f = m == -INFINITY ? 0.f : expf(m - M);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (64 * q >= dv) break;
+    if (q) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)                    // columns 64 q + 16 g + 4 i .. of row r
+      *reinterpret_cast<f32x4*>(ob + (wave * 16 + r) * 68 + 16 * g + 4 * i) =
+          f32x4{o[q][0][i] * f, o[q][1][i] * f, o[q][2][i] * f, o[q][3][i] * f};
+    __syncthreads();
+    for (int i = threadIdx.x; i < nrow * 16; i += 64 * NW) {
+      const int row = i >> 4, c = (i & 15) * 4;
+      if (64 * q + c >= dv) continue;
+      float mm = -INFINITY, ll = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) mm = fmaxf(mm, mls[w * 32 + row]);
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float mw = mls[w * 32 + row];
+        if (mw != -INFINITY) ll += mls[w * 32 + 16 + row] * expf(mw - mm);
+        v += *reinterpret_cast<const f32x4*>(ob + (w * 16 + row) * 68 + c);
+      }
+      const size_t tk = t0 + row / gr;
+      v *= (ll > 0.f ? 1.f / ll : 0.f) * (p.gate ? p.gate[tk * p.ldg + head(row)] : 1.f);
+      T* y = reinterpret_cast<T*>(p.out) + tk * p.ldo + head(row) * p.ohs + v0 + 64 * q + c;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (64 * q + c + e < dv) y[e] = (T)v[e];
+    }
   }
 }
 
-template <typename T>
-int launch(const PA& p, int T_, int H, hipStream_t st) {
-  if (T_ < 1 || H < 1 || H > 65535 || p.gs < 1 || p.Dk > MAXK || (p.Dk & 3) || (p.ldkv & 3) || (p.khs & 3) || p.Dv > 256 * NC ||
-      p.bs < 1)
-    return -1;
-  hipLaunchKernelGGL(attn_plain_kernel<T>, dim3(T_, H), dim3(256), 0, st, p);
+template <typename T, int NQ, int NW>
+int launch_w(const PA& p, dim3 grid, hipStream_t st) {
+  constexpr int KC = NQ > 2 ? 4 : 8;
+  const int nc = ((p.Dk + 15) / 16 + KC - 1) / KC;
+  const size_t lds = sizeof(float) * (NW * 32 + max(16 * (nc * KC * 16 + 4), NW * 16 * 68));
+  if (lds > 64 * 1024) {
+    static bool attr = false;
+    if (!attr && hipFuncSetAttribute((const void*)attn_plain_kernel<T, NQ, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     160 * 1024) != hipSuccess)
+      return -1;
+    attr = true;
+  }
+  hipLaunchKernelGGL((attn_plain_kernel<T, NQ, NW>), grid, dim3(64 * NW), lds, st, p);
   return (int)hipGetLastError();
+}
+
+template <typename T, int NQ>
+int launch_q(const PA& p, dim3 grid, hipStream_t st) {
+  // four waves once they fill the chip, eight (which halve the walk over a row's keys) on smaller grids
+  if (NQ <= 4 && (long)grid.x * grid.y <= 512) return launch_w<T, NQ, NQ <= 4 ? 8 : 4>(p, grid, st);
+  return launch_w<T, NQ, 4>(p, grid, st);
+}
+
+template <typename T>
+int launch(PA p, int T_, int H, hipStream_t st) {
+  if (T_ < 1 || H < 1 || H > 65535 || p.gs < 1 || H % p.gs || p.Dk < 4 || p.Dk > MAXK || (p.Dk & 3) || p.Dv < 1 || (p.ldkv & 3) ||
+      (p.khs & 3) || p.Dv > MAXV || p.bs < 1)
+    return -1;
+  p.T = T_;
+  // A few tokens are mostly of several sequences, which a group would walk one after another; with many, that costs nothing.
+  p.tb = T_ <= 64 ? 1 : max(1, 16 / p.gs);
+  p.sub = (p.gs + 15) / 16;
+  const dim3 grid((T_ + p.tb - 1) / p.tb, H / p.gs * p.sub, (p.Dv + VB - 1) / VB);
+  switch ((p.Dv + 63) / 64) {
+    case 1: return launch_q<T, 1>(p, grid, st);
+    case 2: return launch_q<T, 2>(p, grid, st);
+    case 3: case 4: return launch_q<T, 4>(p, grid, st);
+    default: return launch_q<T, 8>(p, grid, st);
+  }
 }
 
 }  // namespace nls_plain

@@ -9,7 +9,7 @@
 // registers), the four waves of a block exchange row maxima and the bf16 weights through LDS, and each owns a quarter of
 // the output columns: O^T += C^T P^T with C^T fragments from transposed LDS reads of the same tile. Softmax in base 2, all
 // of it f32.
-// 32-bit models: one workgroup per (token, head) (attn_plain.h).
+// 32-bit models: attn_plain.h.
 #include "../kernels/lds_dma.h"
 #include "attn_plain.h"
 
