@@ -92,8 +92,9 @@ struct LinTile {
   const int* rows;      // routed: entries of this tile
 };
 
-// tile id -> tile (BN weight rows x BM rows); false: past the routed list
-template <int BN, int BM>
+// tile id -> tile (BN weight rows x BM rows); false: past the routed list. DENSE: the ids of a routed segment are those of its list's
+// tiles, the list walked LIN_GM tiles at a time like rows (an expert's tiles follow each other in it).
+template <int BN, int BM, bool DENSE = false>
 DEVI bool lin_tile(const LinArgs& a, int id, LinTile& t) {
   int s = 0;
 #pragma unroll
@@ -101,10 +102,10 @@ DEVI bool lin_tile(const LinArgs& a, int id, LinTile& t) {
     if (i < a.nseg && id >= a.begin[i]) s = i;
   const LinSeg& S = a.s[s];
   int q = id - a.begin[s];
-  const int nmt = a.nmt[s];
+  const int nmt = DENSE && S.rows ? max(*a.ntiles, 1) : a.nmt[s];
   const int nnt = (S.N + BN - 1) / BN;
   int mi = q % nmt, ni = q / nmt;
-  if (nmt > LIN_GM && !S.rows && S.ng == 1 && S.ks == 1) {
+  if (nmt > LIN_GM && (S.rows ? DENSE : S.ng == 1 && S.ks == 1)) {
     // LIN_GM row tiles at a time: the workgroups that an XCD runs together share weight tiles and row tiles in its L2
     const int first = q / (LIN_GM * nnt) * LIN_GM, gm = min(LIN_GM, nmt - first), r = q - first * nnt;
     mi = first + r % gm;
@@ -267,6 +268,9 @@ DEVI void lin_store4(const LinSeg& S, int grp, int ks, int n, int yr, f32x4 v) {
         if (n + e < S.N) y[e] = v[e];
   }
 }
+
+// swizzle of a row's four 16-byte chunks in an activation sub-tile of the LDS
+DEVI int lin_swz(int r) { return (0x1320 >> (4 * ((r >> 2) & 3))) & 3; }
 
 // Tile ids of a launch with BN x BM tiles; returns the tile count, or -1 for a descriptor the kernels do not take.
 inline int lin_count(LinArgs& a, int BN, int BM) {

@@ -15,7 +15,7 @@ using nls_dma::glds16;
 using nls_dma::lds_addr;
 using nls_dma::wait_vm_lgkm0;
 
-DEVI int lin_swz(int r) { return (0x1320 >> (4 * ((r >> 2) & 3))) & 3; }
+int lin_phased(LinArgs& a, hipStream_t st);      // lin_phased.hip
 
 template <int BN, int BM, int WN, int WM, int NST>
 struct LG {
@@ -158,9 +158,11 @@ int gemm_d(LinArgs& a, int cfg, hipStream_t st) {
 extern "C" {
 
 // cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256,
-// 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU), 6 = 192 x 128
+// 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU), 6 = 192 x 128,
+// 7 = 256 x 256 in phases (bf16)
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
+  if (cfg == 7) return f32 ? -1 : nls_lin::lin_phased(a, (hipStream_t)stream);
   return f32 ? nls_lin::gemm_d<float>(a, cfg, (hipStream_t)stream)
              : nls_lin::gemm_d<__bf16>(a, cfg, (hipStream_t)stream);
 }

@@ -1,0 +1,300 @@
+// The large prompt GEMM on packed bf16 weights: 256 weight rows x 256 activation rows per workgroup, in four phases per 64-deep step.
+//
+// What bounds the 256 x 128 tile of lin_gemm.hip: a wave's 64 x 64 block reads 16 KB of fragments from LDS per step for 32 MFMAs, so
+// the eight waves' reads (128 KB, 1024 cycles) last as long as their MFMAs (1024 cycles per SIMD), and its one barrier per step puts all
+// waves into the same section at once. Here a wave owns 128 x 64 (24 KB for 64 MFMAs) and
+//   * 8 waves = 2 groups (wr: 128 weight rows each) x 4 (wc: 64 rows each); group 1 runs one barrier behind group 0, so that on every
+//     SIMD (a wave of each) one wave's MFMAs overlap the other's LDS reads and DMA;
+//   * a step is 4 phases of 16 MFMAs: (weights 0, rows 0), (0, 1), (1, 1), (1, 0) of the halves of the wave's block; each phase reads
+//     the fragments that it lacks and starts one 16 KB DMA unit: U0 = weight halves 0, U1 = row halves 0, U2 = row halves 1,
+//     U3 = weight halves 1, each restaged as soon as both groups have read it (two phases later): U2 and U3 of the next step in phases
+//     0 and 1, U0 and U1 of the one after it in phases 2 and 3. The last three units stay in flight (vmcnt(6));
+//   * two 64 KB buffers, one workgroup per CU, which stays for several tiles: the DMA of the next tile's first steps takes the place of
+//     the last steps' successors, so that it is under way during the epilogue.
+// Weight sub-tiles are packed in fragment order and arrive verbatim; activation sub-tiles are swizzled as in lin_gemm.hip.
+// 2000 x 35888 x 4096 (rows x weights x K): 743 us on 256 x 128 -> 490 us (1.20 PFLOP/s), 4096 x 35888 x 4096: 1311 -> 886 us (1.36), 4096 x 4096 x
+// 17408, a single round of tiles: 521 -> 407 us (1.44); a workgroup for each tile instead: 644, 1165 and 422 us. What is left: 16 KB of
+// LDS reads per 43 MFMAs, and rounds of tiles that the shape does not fill.
+#include "../kernels/lds_dma.h"
+#include "lin.h"
+
+namespace nls_lin {
+using nls_dma::glds16;
+using nls_dma::lds_addr;
+
+constexpr int PB = 256;                                  // weight and activation rows of a tile
+constexpr int PHALF = PB * 128, PSTG = 2 * PHALF;        // bytes of an operand's half, of a step's buffer
+
+template <int N>
+DEVI void ph_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+DEVI void ph_barrier() {
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <typename P>
+DEVI P* uniform(P* p) {                                  // (a value that the compiler does not see to be the wave's)
+  const uint64_t v = (uint64_t)p;
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)), lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+  return (P*)((uint64_t)hi << 32 | lo);
+}
+
+// where a tile's operands start: weights by wave, rows by lane
+struct PhTile {
+  LinTile t;
+  const uint8_t* w[2];
+  const __bf16* x[2];
+  int nst;                                               // steps
+};
+
+// The epilogue of a lane's 8 x 4 blocks. Rows, column offsets and the choice of the epilogue are taken out of the blocks where whole
+// 4-column groups are written; the rest goes through lin_store4. (Row lists and positions are loads: with one of them in each block,
+// a tile of experts took 35 us longer.)
+template <int E>
+DEVI void ph_store(const LinSeg& S, const LinTile& t, const f32x4 (&acc)[8][4], int n, int row0, const int (&yr)[4]) {
+  typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  constexpr bool GLU = E == LE_GEGLU || E == LE_SWIGLU || E == LE_SILUGLU;
+  int col[8], nr[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = n + 16 * i, nb = S.cb < S.N ? c / S.cb : 0;
+    nr[i] = c - nb * S.cb;
+    col[i] = GLU ? c >> 1 : nb * S.cstep + nr[i];
+  }
+  const float* cs[4];
+  if constexpr (E == LE_ROPE)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cs[j] = S.cs + (size_t)S.pos[yr[j]] * S.half * 2;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (row0 + 16 * j >= t.cnt) break;
+    const size_t o = (size_t)yr[j] * S.ldy + (size_t)t.grp * S.ygs + (size_t)t.ks * S.yks;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (n + 16 * i >= S.N) break;
+      f32x4 v = acc[i][j];
+      if constexpr (GLU) {
+        float u[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          u[e] = E == LE_SWIGLU ? lin_swiglu(v[2 * e], v[2 * e + 1], S.alpha)
+                                : (E == LE_SILUGLU ? v[2 * e] * lin_sigmoid(v[2 * e]) : lin_gelu(v[2 * e])) * v[2 * e + 1];
+        *reinterpret_cast<bf2*>(reinterpret_cast<__bf16*>(S.y) + o + col[i]) = bf2{(__bf16)u[0], (__bf16)u[1]};
+        continue;
+      }
+      if constexpr (E == LE_ROPE) {
+        if (nr[i] < 2 * S.half) {                        // (half is even: both pairs turn or none)
+          const f32x4 w = *reinterpret_cast<const f32x4*>(cs[j] + nr[i]);
+          v = f32x4{v[0] * w[0] - v[1] * w[1], v[1] * w[0] + v[0] * w[1], v[2] * w[2] - v[3] * w[3], v[3] * w[2] + v[2] * w[3]};
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (E == LE_SILU) v[e] = v[e] * lin_sigmoid(v[e]);
+        if constexpr (E == LE_SIGMOID) v[e] = S.alpha * lin_sigmoid(v[e]);
+        if constexpr (E == LE_RELU2) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
+      }
+      if (S.yact) *reinterpret_cast<bf4*>(reinterpret_cast<__bf16*>(S.y) + o + col[i]) = bf4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+      else *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(S.y) + o + col[i]) = v;
+    }
+  }
+}
+
+DEVI void ph_epilogue(const LinSeg& S, const LinTile& t, f32x4 (&acc)[8][4], int n, int row0) {
+  const bool glu = S.epi == LE_GEGLU || S.epi == LE_SWIGLU || S.epi == LE_SILUGLU;
+  const bool whole = !(S.N & 3) && !((S.ldy | S.ygs | S.yks | S.cstep) & 3) && (!glu || S.yact);
+  int yr[4], xr;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) lin_row(S, t, row0 + 16 * j, xr, yr[j]);
+  switch (whole ? S.epi : -1) {
+    case LE_NONE: ph_store<LE_NONE>(S, t, acc, n, row0, yr); break;
+    case LE_SILU: ph_store<LE_SILU>(S, t, acc, n, row0, yr); break;
+    case LE_SIGMOID: ph_store<LE_SIGMOID>(S, t, acc, n, row0, yr); break;
+    case LE_RELU2: ph_store<LE_RELU2>(S, t, acc, n, row0, yr); break;
+    case LE_GEGLU: ph_store<LE_GEGLU>(S, t, acc, n, row0, yr); break;
+    case LE_SWIGLU: ph_store<LE_SWIGLU>(S, t, acc, n, row0, yr); break;
+    case LE_SILUGLU: ph_store<LE_SILUGLU>(S, t, acc, n, row0, yr); break;
+    case LE_ROPE:
+      if (!(S.half & 1)) {
+        ph_store<LE_ROPE>(S, t, acc, n, row0, yr);
+        break;
+      }
+    default:
+      // (a loop over the blocks of 16 columns that moves them up: the general epilogue unrolled 32 times is more code than the loop)
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (row0 + 16 * j < t.cnt) lin_store4<__bf16>(S, t.grp, t.ks, n + 16 * i, yr[j], acc[0][j]);
+#pragma unroll
+          for (int k = 0; k < 7; ++k) acc[k][j] = acc[k + 1][j];
+        }
+      }
+  }
+}
+
+__global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t phlds[];
+  typedef LT<__bf16> L;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int wr = wave >> 2, wc = wave & 3;
+  // tile ids are dealt to the XCDs in contiguous ranges, which an XCD's workgroups walk together
+  const int xcd = blockIdx.x & 7, nx = gridDim.x >> 3;
+  const LinSeg& R = a.s[0];                              // (only the first segment may be routed)
+  const int listed = R.rows ? ((R.N + PB - 1) / PB) * __builtin_amdgcn_readfirstlane(*a.ntiles) : a.begin[1];
+  const int gap = a.begin[1] - listed;                   // ids that a full list would have
+  ntot -= gap;
+  const int per = (ntot + 7) >> 3, last = min(ntot, (xcd + 1) * per);
+
+  // DMA: in every unit a wave brings both sub-tiles (k halves) of one 16-row tile. Tiles 0 .. 3 and 8 .. 11 of the weights are U0, the
+  // others U3; tiles with (tile & 2) == 0 of the rows are U1, the others U2.
+  const int ta = (wave & 3) + 8 * (wave >> 2), tb = (wave & 1) + 4 * (wave >> 1);
+  auto open = [&](int id, PhTile& p) __attribute__((always_inline)) -> int {      // tile id, if there is one; else -1
+    if (id >= last || !lin_tile<PB, PB, true>(a, id < listed ? id : id + gap, p.t)) return -1;
+    p.t.grp = __builtin_amdgcn_readfirstlane(p.t.grp);
+    p.t.cnt = __builtin_amdgcn_readfirstlane(p.t.cnt);
+    p.t.rows = uniform(p.t.rows);
+    const LinSeg& S = a.s[p.t.seg];
+    const int nsub = S.nsub, nwt = (S.N + 15) >> 4;
+    const int jb = (nsub >> 1) * p.t.ks / S.ks;
+    p.nst = (nsub >> 1) * (p.t.ks + 1) / S.ks - jb;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      p.w[h] = uniform((const uint8_t*)S.w + (size_t)p.t.grp * S.wstride +
+                       ((size_t)min((p.t.n0 >> 4) + ta + 4 * h, nwt - 1) * nsub + 2 * jb) * 1024);
+      int xr, yr;
+      lin_row(S, p.t, 16 * (tb + 2 * h) + (lane >> 2), xr, yr);
+      p.x[h] = (const __bf16*)S.x + (size_t)xr * S.ldx + (size_t)p.t.grp * S.xgs + ((lane & 3) ^ lin_swz(lane >> 2)) * L::EL +
+               (size_t)jb * 2 * L::KS;
+    }
+    return id;
+  };
+  const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(phlds));
+  auto dma_w = [&](int h, const uint8_t* s, uint32_t buf) __attribute__((always_inline)) {      // U0 / U3
+    const uint32_t d = base + buf + (uint32_t)(ta + 4 * h) * 2048u;
+    glds16(s, lane * 16, d);
+    glds16(s, lane * 16 + 1024, d + 1024u);
+  };
+  auto dma_x = [&](int h, const __bf16* s, uint32_t buf) __attribute__((always_inline)) {       // U1 / U2
+    const uint32_t d = base + buf + PHALF + (uint32_t)(tb + 2 * h) * 2048u;
+    glds16(s, d);
+    glds16(s + L::KS, d + 1024u);
+  };
+
+  u32x4 A[4][2], B0[2][2], B1[2][2];
+  const int xfo = r * 64 + ((g ^ lin_swz(r)) << 4);
+  auto rd_w = [&](int h, uint32_t buf) __attribute__((always_inline)) {
+    const uint8_t* p = phlds + buf + (8 * wr + 4 * h) * 2048 + lane * 16;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) A[i][s] = *reinterpret_cast<const u32x4*>(p + (2 * i + s) * 1024);
+  };
+  auto rd_x = [&](u32x4 (&B)[2][2], int h, uint32_t buf) __attribute__((always_inline)) {
+    const uint8_t* p = phlds + buf + PHALF + (4 * wc + 2 * h) * 2048 + xfo;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) B[i][s] = *reinterpret_cast<const u32x4*>(p + (2 * i + s) * 1024);
+  };
+  f32x4 acc[8][4];
+  auto mma = [&](int nh, int mh, const u32x4 (&B)[2][2]) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[4 * nh + i][2 * mh + j] = L::mma(A[i][s], B[j][s], acc[4 * nh + i][2 * mh + j]);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto reads_done = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+
+  PhTile nxt;
+  int id = open(xcd * per + (blockIdx.x >> 3), nxt);
+  if (id < 0) return;
+  // the four streams' next sources: halves 0 run two steps ahead of the multiplications, halves 1 one step
+  const uint8_t *w0 = nxt.w[0], *w1 = nxt.w[1];
+  const __bf16 *x0 = nxt.x[0], *x1 = nxt.x[1];
+  uint32_t buf = 0;                                      // byte offset of the step's buffer
+  dma_w(0, w0, 0);
+  dma_x(0, x0, 0);
+  dma_x(1, x1, 0);
+  dma_w(1, w1, 0);
+  dma_w(0, w0 += 2048, PSTG);
+  dma_x(0, x0 += 2 * L::KS, PSTG);
+  ph_wait<4>();                                          // step 0 has landed
+  ph_barrier();
+  if (wr == 1) ph_barrier();
+  for (;;) {
+    const LinTile t = nxt.t;
+    const int nst = nxt.nst, nid = open(id + nx, nxt);
+    if (nid < 0) nxt.w[0] = w0, nxt.w[1] = w1, nxt.x[0] = x0, nxt.x[1] = x1;       // (staged, not used)
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < nst; ++j, buf ^= PSTG) {
+      rd_w(0, buf);
+      rd_x(B0, 0, buf);
+      x1 = j + 1 == nst ? nxt.x[1] : x1 + 2 * L::KS;
+      dma_x(1, x1, buf ^ PSTG);
+      ph_barrier();
+      reads_done();
+      mma(0, 0, B0);
+      ph_wait<6>();
+      ph_barrier();
+
+      rd_x(B1, 1, buf);
+      w1 = j + 1 == nst ? nxt.w[1] : w1 + 2048;
+      dma_w(1, w1, buf ^ PSTG);
+      ph_barrier();
+      reads_done();
+      mma(0, 1, B1);
+      ph_wait<6>();
+      ph_barrier();
+
+      rd_w(1, buf);
+      w0 = j + 2 == nst ? nxt.w[0] : w0 + 2048;
+      dma_w(0, w0, buf);
+      ph_barrier();
+      reads_done();
+      mma(1, 1, B1);
+      ph_wait<6>();
+      ph_barrier();
+
+      x0 = j + 2 == nst ? nxt.x[0] : x0 + 2 * L::KS;
+      dma_x(0, x0, buf);
+      ph_barrier();
+      mma(1, 0, B0);
+      ph_wait<6>();
+      ph_barrier();
+    }
+    ph_epilogue(a.s[t.seg], t, acc, t.n0 + 128 * wr + 4 * g, 64 * wc + r);
+    if (nid < 0) break;
+    id = nid;
+  }
+  if (wr == 0) ph_barrier();                             // both groups have met the same number of barriers
+  ph_wait<0>();                                          // the staged tail lands before the workgroup's LDS is freed
+}
+
+int lin_phased(LinArgs& a, hipStream_t st) {
+  const int n = lin_count(a, PB, PB);
+  if (n < 1) return -1;
+  for (int i = 0; i < a.nseg; ++i)
+    if ((i && a.s[i].rows) || a.s[i].nsub / 2 / a.s[i].ks < 3) return -1;      // (the streams run two steps ahead, and a last tile's tail restages steps 1 and 2)
+  static bool attr = false;
+  if (!attr) {
+    if (hipFuncSetAttribute((const void*)lin_phased_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * PSTG) != hipSuccess)
+      return -1;
+    attr = true;
+  }
+  hipLaunchKernelGGL(lin_phased_kernel, dim3(min((n + 7) / 8 * 8, 256)), dim3(512), 2 * PSTG, st, a, n);
+  return (int)hipGetLastError();
+}
+
+}  // namespace nls_lin

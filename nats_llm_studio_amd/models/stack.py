@@ -291,11 +291,12 @@ class MoeFeedForward(_Part):
         k = c.top
         design = self.m.cfg.design
         act = self.EPI[design.expert_act]
-        key = ("plan", c.experts, k, c.groups, c.keep, c.scale)
+        tall = K.MoePlan.takes_tall(self.m.f32, self.m.cfg.d_model, c.ff, c.shared_ff or c.ff)
+        key = ("plan", c.experts, k, c.groups, c.keep, c.scale, tall)
         plan = b.launches.get(key)
         if plan is None:
             plan = b.launches[key] = K.MoePlan(P, c.experts, k, c.groups, c.keep, c.scale, self.m.device, design.router_score,
-                                               {"top2": 2, "max": 1}[design.router_group])
+                                               {"top2": 2, "max": 1}[design.router_group], tall=tall)
         z = self.scratch(b, "moe.z", P, c.experts, torch.float32)
         h = self.scratch(b, "moe.h", P * k, K.act_ld(c.ff))
         ye = self.scratch(b, "moe.y", P * (k + 1), self.m.cfg.d_model, torch.float32)

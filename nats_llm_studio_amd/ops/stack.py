@@ -185,12 +185,18 @@ class Seg:
 
 
 # (weight rows, rows) of lin_gemm's configs
-GEMM_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (256, 256), (64, 64), (192, 128))
+GEMM_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (256, 256), (64, 64), (192, 128), (256, 256))
 
 
-# relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU
-GEMM_RATE = {4: (0, 0.96, 0.96), 3: (0, 1.0, 1.0), 6: (0, 0.96, 0.96), 2: (256, 0.47, 0.72),
+# Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
+# phased 256 x 256 tile: a round of 256 workgroups took 88 us at K = 4096 (1.24 PFLOP/s, 1.36 over many rounds), one of 3 (256 x 128)
+# 70 us, one of 6 (192 x 128) 54 us, so it wins where rounds fill: 2000 x 35888 490 us against 743 (3) and 652 (6), 512 x 24576 92
+# against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 298 against 262 (3).
+GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 0.47, 0.72),
              1: (512, 0.5, 0.63), 0: (1024, 0.45, 0.55)}
+# 32-bit operands: f32 MFMAs leave LDS and waits behind, the small tile loses little and wastes least (900 x 2048 x 7680: 280 us against
+# 488 on 128 x 64 and 703 on 192 x 128; 1500 x 35888 x 4096: 3573 against 3584 on 256 x 128 and 3415 on 192 x 128)
+GEMM_RATE_F32 = {6: (0, 1.0, 1.0), 0: (0, 0.9, 0.9)}
 
 
 class LinLaunch:
@@ -225,6 +231,8 @@ class LinLaunch:
                 return False, 1, (4 if self._tiles(16, 16, M) >= 1536 else 8), 1
             if bm == 64:
                 return True, 0
+            if bm == 256:
+                return True, 7
             return True, (3 if self._tiles(256, 128, M) >= 224 else 2)
         n16, n64 = self._tiles(16, 16, M), self._tiles(64, 64, M)
         ns = max(s.w.nsub for s in self.segs)
@@ -242,16 +250,19 @@ class LinLaunch:
             return True, (0 if M <= 2048 else 1)
         if n64 < 96 and n16 <= 1024:
             return False, 1, 16, 1
-        if M > 512:
-            cand = GEMM_RATE
+        rate = GEMM_RATE_F32 if self.f32 else GEMM_RATE
+        if self.f32 or M > 512:
+            cand = list(rate)
         elif self._tiles(256, 128, M) >= 120:
-            cand = (3, 6)
+            cand = [3, 6, 7]
         else:
             return True, (5 if n64 <= 256 else 0)
+        if 7 in cand and min(s.w.nsub for s in self.segs) < 6:      # (its DMA runs two steps ahead)
+            cand.remove(7)
 
         # rounds of 256 workgroups times a tile's cost
         def cost(c):
-            n, (few, lo, hi) = self._tiles(*GEMM_TILES[c], M), GEMM_RATE[c]
+            n, (few, lo, hi) = self._tiles(*GEMM_TILES[c], M), rate[c]
             return -(-n // 256) * GEMM_TILES[c][0] * GEMM_TILES[c][1] / (lo if n <= few else hi)
         return True, min(cand, key=cost)
 
@@ -299,10 +310,11 @@ class LinLaunch:
 class MoePlan:
     """Expert choice and routed-entry lists of one step (csrc/stack/stack_ops.hip moe_plan_kernel), shared by the layers
     of a step. Scores: sigmoid of the router logits, or their softmax; the `keep` groups with the largest score (the sum of
-    their `group_best` best) of `groups` stay eligible; a chosen expert's weight is score * scale."""
+    their `group_best` best) of `groups` stay eligible; a chosen expert's weight is score * scale. tall: the products' tiles may have 256 rows (lin_gemm config 7)."""
 
     def __init__(self, cap: int, experts: int, top: int, groups: int, keep: int, scale: float, device, score: str = "sigmoid",
-                 group_best: int = 2):
+                 group_best: int = 2, tall: bool = False):
+        self.tall = tall
         self.softmax, self.group_best = {"sigmoid": 0, "softmax": 1}[score], group_best
         self.experts, self.top, self.groups, self.keep, self.scale = experts, top, groups, keep, scale
         i32 = dict(dtype=torch.int32, device=device)
@@ -315,7 +327,14 @@ class MoePlan:
     def bm(self, T: int) -> int:
         """Rows per tile of the expert products at T tokens."""
         avg = T * self.top / self.experts
-        return 16 if avg <= 6 else (64 if avg <= 96 else 128)
+        # 256 rows: eight experts of 875 rows took 251 -> 175 us at N = 6144, K = 2048 and 204 -> 149 us at N = 2048, K = 6144; from about
+        # 160 rows on an expert's last tile wastes less than the phased kernel gains
+        return 16 if avg <= 6 else 64 if avg <= 96 else 256 if self.tall and avg >= 160 else 128
+
+    @staticmethod
+    def takes_tall(f32: bool, *inputs: int) -> bool:
+        """Whether products of these input widths run on 256-row tiles."""
+        return not f32 and all(act_ld(k) >= 192 for k in inputs)
 
     def max_tiles(self, T: int, bm: Optional[int] = None) -> int:
         bm = bm or self.bm(T)

@@ -27,6 +27,76 @@ def relerr(got, want):
     return float((got.double().cpu() - want).norm() / want.norm())
 
 
+def act(x, ld):
+    out = torch.zeros(x.shape[0], ld, dtype=torch.bfloat16)
+    out[:, :x.shape[1]] = x.to(torch.bfloat16)
+    return out.cuda()
+
+
+@pytest.mark.parametrize("M", [1, 255, 256, 257, 513, 1300])
+@pytest.mark.parametrize("Kd", [150, 192, 530])
+def test_phased_gemm(K, M, Kd):
+    """256 x 256 tiles: rows and columns around a tile's edge, three to nine steps of K, more tiles than a pass of an XCD takes, every
+    kind of epilogue, whole and ragged columns, outputs of both types, segments beside each other."""
+    bf = torch.bfloat16
+    x = rnd(M, Kd, seed=1).to(bf)
+    xd, X = x.double(), act(x, K.act_ld(Kd))
+    ws = {n: (rnd(N, Kd, seed=10 + i) * Kd ** -0.5).to(bf) for i, (n, N) in enumerate(
+        [("none", 515), ("silu", 260), ("tanh", 64), ("geglu", 512), ("f32", 2304), ("rope", 96)])}
+    z = {n: xd @ w.double().T for n, w in ws.items()}
+    y = {n: torch.full((M + 1, {"geglu": 256, "rope": 200}.get(n, w.shape[0])), 7.0, dtype=torch.float32 if n in ("f32", "none") else bf,
+                       device="cuda") for n, w in ws.items()}
+    P = {n: K.PackedLinear(w, False, "cuda") for n, w in ws.items()}
+    pos = torch.arange(M, dtype=torch.int32).flip(0) % 50
+    ang = rnd(50, 10, seed=5)
+    cs = torch.stack([torch.cos(ang), torch.sin(ang)], -1).float()
+    turn = dict(block=(32, 64), rope=(cs.cuda(), pos.cuda(), 10))          # 20 of a block's 32 columns turn
+    L = K.LinLaunch([K.Seg(P[n], X, y[n][:M], "none" if n == "f32" else n, **(turn if n == "rope" else {})) for n in ws])
+    L._cfg[M] = (True, 7), 1
+    L.run(M, st())
+    gelu = torch.nn.functional.gelu
+    want = {"none": z["none"], "silu": z["silu"] * torch.sigmoid(z["silu"]), "tanh": torch.tanh(z["tanh"]),
+            "geglu": gelu(z["geglu"][:, 0::2], approximate="tanh") * z["geglu"][:, 1::2], "f32": z["f32"]}
+    for n, w in want.items():
+        # f32 sums of Kd products; bf16 outputs round to 2^-9
+        assert relerr(y[n][:M], w) < (2e-6 if y[n].dtype == torch.float32 else 3e-3), n
+    o = y["rope"][:M].cpu()
+    u = z["rope"].view(M, 3, 16, 2)
+    c, s = (torch.cat([v[pos.long()].double()[:, None], torch.full((M, 1, 6), one, dtype=torch.float64)], 2)
+            for v, one in ((cs[..., 0], 1.0), (cs[..., 1], 0.0)))
+    w = torch.stack([u[..., 0] * c - u[..., 1] * s, u[..., 1] * c + u[..., 0] * s], -1).view(M, 96)
+    assert relerr(torch.cat([o[:, 64 * i:64 * i + 32] for i in range(3)], 1), w) < 3e-3
+    assert (o[:, 32:64] == 7).all() and all((t[M] == 7).all() for t in y.values())
+
+
+@pytest.mark.parametrize("T,E", [(700, 3), (1100, 8)])
+def test_phased_gemm_of_experts(K, T, E):
+    """Experts' row lists in tiles of 256 rows: several tiles, part tiles, an expert without rows; both products and the choice."""
+    bf, d, ff = torch.bfloat16, 192, 300
+    x = rnd(T, d, seed=1).to(bf)
+    z = rnd(T, E, seed=2).float()
+    z[:, 1] = -9.0
+    up, down = (rnd(E, ff, d, seed=3) * d ** -0.5).to(bf), (rnd(E, d, ff, seed=4) * ff ** -0.5).to(bf)
+    plan = K.MoePlan(T, E, 2, 1, 1, 1.0, "cuda", tall=K.MoePlan.takes_tall(False, d, ff))
+    assert plan.bm(T) == 256
+    h, ye = torch.zeros(2 * T, K.act_ld(ff), dtype=bf, device="cuda"), torch.zeros(2 * T, d, device="cuda")
+    U, D = K.PackedLinear(up, False, "cuda"), K.PackedLinear(down, False, "cuda")
+    plan.run(z.cuda(), T, st())
+    K.LinLaunch([K.Seg(U, act(x, K.act_ld(d)), h, "relu2", routed=(plan.rows, 2))], plan).run(T, st())
+    K.LinLaunch([K.Seg(D, h, ye, routed=(plan.rows, 1))], plan).run(T, st())
+    sel = plan.sel.view(T, 2).long().cpu()
+    assert (z.topk(2, 1).indices.sort(1).values == sel.sort(1).values).all()
+    for j in range(2):
+        e = sel[:, j]
+        hid = torch.zeros(T, ff, dtype=torch.float64)
+        for k in range(E):
+            hid[e == k] = torch.relu(x[e == k].double() @ up[k].double().T) ** 2
+        assert relerr(h[j::2, :ff], hid) < 3e-3
+        got = h[j::2, :ff].double().cpu()
+        want = torch.stack([got[t] @ down[e[t]].double().T for t in range(T)])
+        assert relerr(ye[j::2], want) < 2e-6
+
+
 # heads, key heads, key and value columns: groups that do and do not divide 16, single heads, widths with a part of a block
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
 @pytest.mark.parametrize("H,G,D", [(8, 2, 128), (6, 2, 20), (3, 3, 64), (20, 1, 32), (2, 1, 300), (1, 1, 600)])
