@@ -763,7 +763,7 @@ class SharedNormLayer:
             c0 += w
         b.launches[key, "parts"] = e
         b.launches[key, "in"] = [K.LinLaunch(segs[o:o + K.SEGS]) for o in range(0, len(segs), K.SEGS)]
-        # small steps may split K: slabs of up to 512 rows, added by the residual's launch
+        # the product may split K: slabs that the residual's launch adds
         b.launches[key, "out"] = K.LinLaunch([K.Seg(self.o, cat, self.m.slabs(b), slabs=_SLABS, slab_rows=b.slab_rows)])
 
     def new_caches(self, slots):
@@ -776,9 +776,10 @@ class SharedNormLayer:
         caches = kc.get(step.layer, {})
         for j, (q, e) in enumerate(zip(self.parts, b.launches[key, "parts"])):
             q.run(b, e, caches.get(j), state, step)
-        n = b.launches[key, "out"].run(step.T, step.st)
+        out = b.launches[key, "out"]
+        n = out.run(step.T, step.st)
         K.norm_add(self.m.slabs(b), None, b.x, fin.pop("copy", None), step.T, cfg.eps, step.st, rms=cfg.design.norm == "rms",
-                   slabs=n, slab_rows=b.slab_rows, **fin)
+                   slabs=n, slab_rows=out.slab_rows, **fin)
 
 
 class SandwichNormLayer:
@@ -827,7 +828,7 @@ class SandwichNormLayer:
                 for launch in inputs:
                     launch.run(T, st)
                 q.run(b, e, kc.get(step.layer), state, step)
-                y = dict(y=self.m.slabs(b), slabs=out.run(T, st), slab_rows=b.slab_rows)
+                y = dict(y=self.m.slabs(b), slabs=out.run(T, st), slab_rows=out.slab_rows)
             nxt = fin if j == len(self.parts) - 1 else dict(out_norm=self.norm_ff, out=b.h)
             K.norm_add(w=self.after[j], x=b.x, xb=None, T=T, eps=cfg.eps, st=st, rms=cfg.design.norm == "rms", groups=cfg.norm_groups,
                        **y, **nxt)
@@ -1067,7 +1068,7 @@ class StackModel:
         return {} if qb is None else dict(qblocks=torch.from_numpy(qb).to(self.device), nqb=len(qb), row_info=info)
 
     def slabs(self, b: StackBuffers) -> torch.Tensor:
-        """f32 outputs of a product into the residual, in up to _SLABS blocks of slab_rows rows where K is split."""
+        """f32 outputs of a product into the residual, in blocks of a step's rows (at least slab_rows) where K is split."""
         if "slabs" not in b.shared:
             rows = max(b.pad, _SLABS * b.slab_rows)
             b.shared["slabs"] = torch.zeros(rows, self.cfg.d_model, dtype=torch.float32, device=self.device)
@@ -1137,7 +1138,7 @@ class StackModel:
         for i, layer in enumerate(self.layers):
             if self.passes[i] is not None and steps[i] is None:
                 n = b.launches["pass"].run(T, st)
-                K.norm_add(self.slabs(b), None, b.x, None, T, cfg.eps, st, rms=rms, slabs=n, slab_rows=b.slab_rows, keep=False,
+                K.norm_add(self.slabs(b), None, b.x, None, T, cfg.eps, st, rms=rms, slabs=n, slab_rows=b.launches["pass"].slab_rows, keep=False,
                            add=self.loop_step[self.passes[i]], **self._norms(b, i))
             if i == last:
                 fin = dict(out_norm=self.final_norm, out=b.hn) if direct else {}

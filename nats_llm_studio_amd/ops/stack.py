@@ -142,8 +142,8 @@ class Seg:
     routed = (entry list, xdiv): the rows are routed entries (x row = entry / xdiv, y row = entry).
     rope = (table, pos, pairs). alpha: constant of the epilogue (sigmoid, sigpow, softcap, swiglu); sigpow: `gate`,
     a vector, gives an exponent per column instead. geglu, swiglu, siluglu: the rows of w alternate gate and up, y has half as many
-    columns. slabs: K splits that launches of up to slab_rows rows may use; y holds that many slabs of slab_rows rows, added by
-    the caller (LinLaunch.run returns how many were written)."""
+    columns. slabs: K splits that a launch may use; y holds that many slabs of slab_rows rows, or as many of a larger launch's rows as
+    fit, added by the caller (LinLaunch.run returns how many were written)."""
 
     def __init__(self, w: PackedLinear, x: torch.Tensor, y: torch.Tensor, epi: str = "none", ycol: int = 0,
                  xcol: int = 0, xgs: int = 0, ygs: int = 0, block=None, bias=None, gate=None, routed=None, rope=None,
@@ -199,6 +199,10 @@ GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 
 GEMM_RATE_F32 = {6: (0, 1.0, 1.0), 0: (0, 0.9, 0.9)}
 
 
+# Microseconds of a round of 256 workgroups of a tile: fixed + per input column (from rounds at K = 1024 .. 17408)
+ROUND_US = {7: (8.0, 0.0215), 3: (8.0, 0.0151), 6: (8.0, 0.0112)}
+
+
 class LinLaunch:
     """A launch of up to SEGS independent linear layers, bound to its buffers once (only the row count and the launch
     config change from step to step)."""
@@ -213,6 +217,7 @@ class LinLaunch:
         if plan is not None:
             self.a.tiles, self.a.ntiles = plan.tiles.data_ptr(), plan.ntiles.data_ptr()
         self._cfg = {}
+        self.slab_rows = segs[0].slab_rows       # rows from slab to slab of the last run
 
     def _tiles(self, bn: int, bm: int, M: int) -> int:
         """Workgroups of a launch with bn x bm tiles."""
@@ -279,8 +284,22 @@ class LinLaunch:
             return (True, 3), -(-256 // big)
         return (True, 0), -(-512 // small)
 
+    def tall_split(self, M: int):
+        """(config, K splits) of more rows than slab_rows: as many slabs of M rows as y holds. A narrow product has fewer tiles than
+        there are CUs, or lasts two rounds for a few more; each further slab is written and read again (about 4 TB/s). 2000 x 4096 x
+        17408: 286 us in one round of 256 x 128 -> 222 in two splits of 256 x 256; the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
+        s = self.segs[0]
+        most = min(s.slabs, s.y.shape[0] // M, s.w.nsub // 16)
+
+        def us(c, ks):
+            fixed, per = ROUND_US[c]
+            rounds = -(-self._tiles(*GEMM_TILES[c], M) * ks // 256)
+            return rounds * (fixed + per * s.w.K / ks) + (ks - 1) * M * s.w.N * 2e-6
+        c, ks = min(((c, ks) for c in ROUND_US for ks in range(1, most + 1)), key=lambda v: us(*v))
+        return ((True, c), ks) if ks > 1 else (self.config(M), 1)
+
     def run(self, M: int, st: int) -> int:
-        """Returns the slabs of output rows that were written (1 unless a segment may split K)."""
+        """Returns the slabs of output rows that were written (1 unless a segment may split K), `slab_rows` rows apart."""
         if self.plan is not None:
             self.a.maxtiles = self.plan.max_tiles(M)
         for i, s in enumerate(self.segs):
@@ -292,14 +311,21 @@ class LinLaunch:
             if len(self._cfg) > 4096:
                 self._cfg.clear()
             s = self.segs[0]
-            if s.slabs > 1 and len(self.segs) == 1 and M <= s.slab_rows and s.w.nsub >= 64:
+            splits = s.slabs > 1 and len(self.segs) == 1 and s.w.nsub >= 64
+            if splits and M <= s.slab_rows:
                 cfg, ks = self.split_config(M)
                 cfg = cfg, max(1, min(ks, s.slabs, s.w.nsub // 16))
+            elif splits and not self.f32:
+                cfg = self.tall_split(M)
             else:
                 cfg = self.config(M), 1
             self._cfg[M] = cfg
         cfg, ks = cfg
         self.a.s[0].ks = ks
+        if ks > 1:
+            s = self.segs[0]
+            self.slab_rows = max(M, s.slab_rows)
+            self.a.s[0].yks = self.slab_rows * s.y.stride(0)
         if cfg[0]:
             _check(lib().nls_lin_gemm(ctypes.byref(self.a), self.f32, cfg[1], st), "nls_lin_gemm")
         else:

@@ -69,6 +69,22 @@ def test_phased_gemm(K, M, Kd):
     assert (o[:, 32:64] == 7).all() and all((t[M] == 7).all() for t in y.values())
 
 
+@pytest.mark.parametrize("M,N,rows", [(300, 160, 1500), (600, 512, 1200), (700, 160, 1399)])
+def test_tall_split(K, M, N, rows):
+    """More rows than a slab was bound for: as many slabs as the buffer holds (4, 2, 1), apart by the launch's rows."""
+    bf, Kd = torch.bfloat16, 4160
+    x, w = rnd(M, Kd, seed=1).to(bf), (rnd(N, Kd, seed=2) * Kd ** -0.5).to(bf)
+    y = torch.full((rows, N), 7.0, device="cuda")
+    L = K.LinLaunch([K.Seg(K.PackedLinear(w, False, "cuda"), act(x, K.act_ld(Kd)), y, slabs=4, slab_rows=128)])
+    n = L.run(M, st())
+    assert n == min(4, rows // M) and (n == 1 or L.slab_rows == M)
+    assert relerr(sum(y[i * M:(i + 1) * M].double() for i in range(n)), x.double() @ w.double().T) < 2e-6
+    assert (y[n * M:] == 7).all()
+    z = torch.zeros(M, N, device="cuda")
+    K.norm_add(y, None, z, None, M, 1e-5, st(), slabs=n, slab_rows=L.slab_rows)
+    assert relerr(z, x.double() @ w.double().T) < 2e-6
+
+
 @pytest.mark.parametrize("T,E", [(700, 3), (1100, 8)])
 def test_phased_gemm_of_experts(K, T, E):
     """Experts' row lists in tiles of 256 rows: several tiles, part tiles, an expert without rows; both products and the choice."""
