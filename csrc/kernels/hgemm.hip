@@ -215,6 +215,47 @@ DEVI void hg_epi(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, 
     }
     return;
   }
+  if (a.epi == EPI_ROPE) {
+    // RoPE pair (row, row ^ 1) = lanes r, r ^ 1 (same b). An activation row's slot and position are loaded once, its head
+    // and column once for a weight row (rope_store1 does both for each value: 384 x 6144 x 4096 52 -> 46 us)
+    int sl[MTW][4];
+    const float* cs[MTW][4];
+#pragma unroll
+    for (int i = 0; i < MTW; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int b = a.m0 + min(mbase + 16 * i + 4 * g + e, M - 1);
+        sl[i][e] = a.slot[b];
+        cs[i][e] = a.cs + (size_t)a.pos[b] * a.D;
+      }
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) {
+      const int row = rbase + 16 * j + r, col = S.ycol + min(row, S.rows - 1);
+      const bool odd = col & 1;
+      const int h = col / a.D, dd = col - h * a.D, kh = h - a.Hq;       // (kh: key head, value heads behind them)
+      const float own = a.bias ? a.bias[col] : 0.f, pair = a.bias ? a.bias[col ^ 1] : 0.f;
+      const bool kv = kh >= 0, value = kh >= a.Hkv;
+      __bf16* const base = !kv ? a.q_out + col : (value ? a.vc + (kh - a.Hkv) * a.D : a.kc + kh * a.D) + dd;
+      const long step = kv ? (long)a.Hkv * a.D : a.ldq;
+#pragma unroll
+      for (int i = 0; i < MTW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int b = mbase + 16 * i + 4 * g + e;
+          float v = acc[i][j][e] * a.alpha;
+          const float p = __shfl_xor(v, 1, 64) + pair;
+          v += own;
+          const long at = kv ? sl[i][e] : a.m0 + b;
+          if (b >= M || row >= S.rows || at < 0) continue;
+          if (!value) {
+            const float2 c = *reinterpret_cast<const float2*>(cs[i][e] + (dd & ~1));
+            v = odd ? p * c.y + v * c.x : v * c.x - p * c.y;
+          }
+          base[at * step] = (__bf16)v;
+        }
+    }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < NTW; ++j) {
     const int row = rbase + 16 * j + r;
@@ -224,12 +265,6 @@ DEVI void hg_epi(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, 
       for (int e = 0; e < 4; ++e) {
         const int b = mbase + 16 * i + 4 * g + e;
         const float v = acc[i][j][e] * a.alpha;
-        if (a.epi == EPI_ROPE) {
-          // RoPE pair (row, row ^ 1) = lanes r, r ^ 1 (same b)
-          const float pv = __shfl_xor(v, 1, 64);
-          if (b < M && row < S.rows) rope_store1(a, S.ycol + row, a.m0 + b, v, pv);
-          continue;
-        }
         if (a.epi == EPI_SWIGLU) {
           // interleaved [g0..g7, u0..u7] per 16 weight rows: the partner row is lane ^ 8 (same b)
           const float u = __shfl_xor(v, 8, 64);

@@ -38,21 +38,24 @@ using nls_dma::lds_addr;
 // weight half of a K-tile buffer and each wave's weight rows halve; the activation half, the phase schedule
 // and the unit order stay, only the DMA instruction counts of the two weight units (and so the counted
 // vmcnt of each phase) change.
-constexpr int BM = 256;
+// Row blocks of 64 MT rows: 256 (MT 4), or 192 (MT 3: the second half of a wave's rows is one tile), which 257 .. 384 rows and many
+// larger counts fill better (launch_dense10).
 constexpr int KT = 64;                       // K per tile
-template <int BN>
+template <int BN, int MT>
 struct H10 {
+  static constexpr int BM = 64 * MT;
   static constexpr int AB = BN * KT * 2;     // weight half of a K-tile buffer (32 or 16 KiB)
   static constexpr int TB = AB + BM * KT * 2;
   static constexpr int LDS = 2 * TB;
   static constexpr int RTG = BN / 32;        // 16-row weight tiles per wave group (wr)
   static constexpr int NQH = RTG / 2;        // ... per quadrant half (nq)
-  static constexpr int NA = BN / 128;        // DMA instructions per lane of a weight unit (B units: 2)
-  // counted waits: the last three units issued stay in flight (units U0/U3 carry NA, U1/U2 two)
-  static constexpr int VM_PRO = NA + 2;      // after the prologue: U0(1) U1(1)
-  static constexpr int VM_Q0 = NA + 4;       // U0(T+1) U1(T+1) U2(T+1)
-  static constexpr int VM_Q1 = NA + 4;       // U1(T+1) U2(T+1) U3(T+1)
-  static constexpr int VM_Q2 = 2 * NA + 2;   // U2(T+1) U3(T+1) U0(T+2)
+  static constexpr int NA = BN / 128;        // DMA instructions per lane of a weight unit (U1: 2)
+  static constexpr int NB2 = MT - 2;         // ... of U2
+  // counted waits: the last three units issued stay in flight (units U0/U3 carry NA, U1 two, U2 NB2)
+  static constexpr int VM_PRO = NA + 2;            // after the prologue: U0(1) U1(1)
+  static constexpr int VM_Q0 = NA + 2 + NB2;       // U0(T+1) U1(T+1) U2(T+1)
+  static constexpr int VM_Q1 = NA + 2 + NB2;       // U1(T+1) U2(T+1) U3(T+1)
+  static constexpr int VM_Q2 = 2 * NA + NB2;       // U2(T+1) U3(T+1) U0(T+2)
   static constexpr int VM_Q3 = 2 * NA + 2;   // U3(T+1) U0(T+2) U1(T+2)
 };
 
@@ -65,36 +68,39 @@ DEVI void wait_vm() {
 
 // unit u's (row-tile, k-step) subtiles; a subtile = 16 rows x 32 k = 1 KiB at (rt * 2 + ks) * 1 KiB of
 // its operand region. A units (0, 3): weight row-tiles; B units (1, 2): activation row-tiles.
-template <int BN>
+template <int BN, int MT>
 DEVI int unit_rt(int u, int idx) {           // idx: row-tile slot of the unit
   // BN 256: U0: A {0-3, 8-11}; U3: A {4-7, 12-15}. BN 128: U0: A {0-1, 4-5}; U3: A {2-3, 6-7}.
-  // U1: B {0,1,4,5,8,9,12,13}; U2: B {2,3,6,7,10,11,14,15}
-  constexpr int NQH = H10<BN>::NQH, RTG = H10<BN>::RTG;
+  // U1: B {0,1,4,5,8,9,12,13}; U2: B {2,3,6,7,10,11,14,15}. MT 3: U1: B {0,1,3,4,6,7,9,10}; U2: B {2,5,8,11}
+  constexpr int NQH = H10<BN, MT>::NQH, RTG = H10<BN, MT>::RTG;
   if (u == 0) return (idx % NQH) + RTG * (idx / NQH);
   if (u == 3) return NQH + (idx % NQH) + RTG * (idx / NQH);
-  if (u == 1) return (idx & 1) + 4 * (idx >> 1);
-  return 2 + (idx & 1) + 4 * (idx >> 1);
+  if (u == 1) return (idx & 1) + MT * (idx >> 1);
+  return MT == 4 ? 2 + (idx & 1) + 4 * (idx >> 1) : 2 + MT * idx;
 }
 
 // ---- epilogue (mode 8's; shared by modes 10 and 11): lane holds weight rows nb + 16i + 4(l >> 4) + e, activation
 // row mb + 16j + (l & 15)
-template <int BN>
-DEVI void h10_epilogue(const f32x4 (&acc)[2 * H10<BN>::NQH][4], const Seg& S, int row0, int kslice, int ks,
+template <int BN, int MT>
+using H10Acc = f32x4[2 * H10<BN, MT>::NQH][MT];
+
+template <int BN, int MT>
+DEVI void h10_epilogue(H10Acc<BN, MT>& acc, const Seg& S, int row0, int kslice, int ks,
                        const GemvArgs& a, float* ws) {
-  constexpr int NQH = H10<BN>::NQH;
+  constexpr int NQH = H10<BN, MT>::NQH;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 2, wc = wave & 3;
   const int M = a.M;
   const int g4 = 4 * (lane >> 4), r16 = lane & 15;
-  const int nb = row0 + wr * (BN / 2), mb = wc * 64;
+  const int nb = row0 + wr * (BN / 2), mb = wc * 16 * MT;
   if (ks > 1 || a.epi == EPI_SLABS) {
 #pragma unroll
     for (int i = 0; i < 2 * NQH; ++i) {
       const int n = nb + 16 * i + g4;
       if (n >= S.rows) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         const int m = mb + 16 * j + r16;
         if (m >= M) continue;
         *reinterpret_cast<f32x4*>(ws + ((size_t)kslice * a.mtot + a.m0 + m) * a.pad + S.tile_begin_col + n) = acc[i][j];
@@ -105,19 +111,58 @@ DEVI void h10_epilogue(const f32x4 (&acc)[2 * H10<BN>::NQH][4], const Seg& S, in
   const float al = a.alpha;
   if (a.epi == EPI_ROPE) {
     // RoPE pairs (e, e + 1) of the lane's 4 consecutive weight rows: no cross-lane traffic
+    if ((a.D & 3) || (a.ldq & 3)) {
+      for (int i = 0; i < 2 * NQH; ++i) {               // (moved up instead of unrolled: the general form is long)
+        const int n = nb + 16 * i + g4;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          const int m = mb + 16 * j + r16;
+          const f32x4 v = acc[0][j] * al;
+          if (m < M && n < S.rows) {
+            rope_store1(a, S.ycol + n, a.m0 + m, v[0], v[1]);
+            rope_store1(a, S.ycol + n + 1, a.m0 + m, v[1], v[0]);
+            rope_store1(a, S.ycol + n + 2, a.m0 + m, v[2], v[3]);
+            rope_store1(a, S.ycol + n + 3, a.m0 + m, v[3], v[2]);
+          }
+#pragma unroll
+          for (int k = 0; k + 1 < 2 * NQH; ++k) acc[k][j] = acc[k + 1][j];
+        }
+      }
+      return;
+    }
+    // 4 columns of one head: a row's slot and position once, 8-byte stores (one value at a time, with its own loads,
+    // 3000 x 6144 x 4096 took 307 us, 181 this way)
+    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+    long sl[MT];
+    const float* cs[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const int m = a.m0 + min(mb + 16 * j + r16, M - 1);
+      sl[j] = a.slot[m];
+      cs[j] = a.cs + (size_t)a.pos[m] * a.D;
+    }
 #pragma unroll
     for (int i = 0; i < 2 * NQH; ++i) {
       const int n = nb + 16 * i + g4;
       if (n >= S.rows) continue;
+      const int col = S.ycol + n, h = col / a.D, dd = col - h * a.D;
+      f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+      if (a.bias) bias = f32x4{a.bias[col], a.bias[col + 1], a.bias[col + 2], a.bias[col + 3]};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         const int m = mb + 16 * j + r16;
         if (m >= M) continue;
-        const f32x4 v = acc[i][j] * al;
-        rope_store1(a, S.ycol + n, a.m0 + m, v[0], v[1]);
-        rope_store1(a, S.ycol + n + 1, a.m0 + m, v[1], v[0]);
-        rope_store1(a, S.ycol + n + 2, a.m0 + m, v[2], v[3]);
-        rope_store1(a, S.ycol + n + 3, a.m0 + m, v[3], v[2]);
+        f32x4 v = acc[i][j] * al + bias;
+        __bf16* d = nullptr;
+        if (h < a.Hq + a.Hkv) {
+          const float2 c0 = *reinterpret_cast<const float2*>(cs[j] + dd), c1 = *reinterpret_cast<const float2*>(cs[j] + dd + 2);
+          v = f32x4{v[0] * c0.x - v[1] * c0.y, v[0] * c0.y + v[1] * c0.x, v[2] * c1.x - v[3] * c1.y, v[2] * c1.y + v[3] * c1.x};
+          if (h < a.Hq) d = a.q_out + (size_t)(a.m0 + m) * a.ldq + col;
+          else if (sl[j] >= 0) d = a.kc + ((size_t)sl[j] * a.Hkv + (h - a.Hq)) * a.D + dd;
+        } else if (sl[j] >= 0) {
+          d = a.vc + ((size_t)sl[j] * a.Hkv + (h - a.Hq - a.Hkv)) * a.D + dd;
+        }
+        if (d) *reinterpret_cast<bf4*>(d) = bf4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
       }
     }
     return;
@@ -126,7 +171,7 @@ DEVI void h10_epilogue(const f32x4 (&acc)[2 * H10<BN>::NQH][4], const Seg& S, in
 #pragma unroll
     for (int i = 0; i < 2 * NQH; ++i) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         f32x4 u;
 #pragma unroll
         for (int e = 0; e < 4; ++e) u[e] = __shfl_xor(acc[i][j][e] * al, 32, 64);
@@ -148,7 +193,7 @@ DEVI void h10_epilogue(const f32x4 (&acc)[2 * H10<BN>::NQH][4], const Seg& S, in
       const int n = nb + 16 * i + g4;
       if (n >= S.rows) continue;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < MT; ++j) {
         const int m = mb + 16 * j + r16;
         if (m >= M) continue;
         const f32x4 v = acc[i][j] * al;
@@ -165,7 +210,7 @@ DEVI void h10_epilogue(const f32x4 (&acc)[2 * H10<BN>::NQH][4], const Seg& S, in
   }
   if (a.argmax) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < MT; ++j) {
       unsigned long long k = 0ull;
 #pragma unroll
       for (int i = 0; i < 2 * NQH; ++i)
@@ -185,10 +230,10 @@ DEVI void h10_epilogue(const f32x4 (&acc)[2 * H10<BN>::NQH][4], const Seg& S, in
   }
 }
 
-template <int BN>
+template <int BN, int MT>
 DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, uint8_t* lds) {
-  typedef H10<BN> C;
-  constexpr int TB = C::TB, NQH = C::NQH, NA = C::NA;
+  typedef H10<BN, MT> C;
+  constexpr int TB = C::TB, NQH = C::NQH, NA = C::NA, NB2 = C::NB2;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 2, wc = wave & 3;
@@ -207,12 +252,12 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
     const int Tc = t0 + min(T, nkt - 1);       // clamped: past the end re-stages the last tile (same bytes)
     const bool bu = u == 1 || u == 2;
     const uint32_t buf = base + (uint32_t)(T & 1) * TB + (bu ? (uint32_t)C::AB : 0u);
-    const int n = bu ? 2 : NA;
+    const int n = u == 1 ? 2 : u == 2 ? NB2 : NA;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if (j >= n) break;
       const int idx = n * wave + j;
-      const int rt = unit_rt<BN>(u, idx >> 1), kstep = idx & 1;
+      const int rt = unit_rt<BN, MT>(u, idx >> 1), kstep = idx & 1;
       const act_t* src;
       if (u == 1 || u == 2) {
         const int row = min(16 * rt + (lane >> 2), M - 1);
@@ -227,7 +272,7 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
 
   // ---- fragments: lane reads row (l & 15) of a 16-row subtile, logical chunk l >> 4
   const int fro = (lane & 15) * 64 + (((lane >> 4) ^ swz(lane & 15)) << 4);
-  f16x8 FA[NQH][2], FB0[2][2], FB1[2][2];
+  f16x8 FA[NQH][2], FB0[2][2], FB1[NB2][2];
   auto rdA = [&](int T, int nq) __attribute__((always_inline)) {
     const uint8_t* p = lds + (T & 1) * TB + fro;
 #pragma unroll
@@ -236,25 +281,25 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
       for (int s = 0; s < 2; ++s)
         FA[i][s] = *reinterpret_cast<const f16x8*>(p + ((wr * C::RTG + nq * NQH + i) * 2 + s) * 1024);
   };
-  auto rdB = [&](f16x8 (&F)[2][2], int T, int mh) __attribute__((always_inline)) {
+  auto rdB = [&](auto& F, int T, int mh) __attribute__((always_inline)) {
     const uint8_t* p = lds + (T & 1) * TB + C::AB + fro;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < (mh ? NB2 : 2); ++i)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) F[i][s] = *reinterpret_cast<const f16x8*>(p + ((wc * 4 + mh * 2 + i) * 2 + s) * 1024);
+      for (int s = 0; s < 2; ++s) F[i][s] = *reinterpret_cast<const f16x8*>(p + ((wc * MT + mh * 2 + i) * 2 + s) * 1024);
   };
-  f32x4 acc[2 * NQH][4];
+  f32x4 acc[2 * NQH][MT];
 #pragma unroll
   for (int i = 0; i < 2 * NQH; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto mma = [&](int nq, int mh, const f16x8 (&F)[2][2]) __attribute__((always_inline)) {
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](int nq, int mh, const auto& F) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
       for (int i = 0; i < NQH; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < (mh ? NB2 : 2); ++j)
           acc[nq * NQH + i][mh * 2 + j] = mfma16(FA[i][s], F[j][s], acc[nq * NQH + i][mh * 2 + j]);
   };
   auto bar = []() __attribute__((always_inline)) {
@@ -321,13 +366,14 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();
 
-  h10_epilogue<BN>(acc, S, row0, kslice, ks, a, ws);
+  h10_epilogue<BN, MT>(acc, S, row0, kslice, ks, a, ws);
 }
 
-template <int BN>
+template <int BN, int MT>
 __global__ __launch_bounds__(512, 1) void hgemm10_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
                                                           int nmb) {
   extern __shared__ __attribute__((aligned(16))) uint8_t h10lds[];
+  constexpr int BM = H10<BN, MT>::BM;
   const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
   const int kslice = j % ks;
   const int mb = (j / ks) % nmb;
@@ -345,29 +391,32 @@ __global__ __launch_bounds__(512, 1) void hgemm10_kernel(SegList segs, GemvArgs 
   if (a.argmax) a.argmax += m0;
   a.M = min(BM, a.M - m0);
   const int row0 = (tile - S.tile_begin) * BN;       // (host tile counts use BN-row tiles)
-  h10_tile<BN>(S, row0, kslice, ks, a, ws, h10lds);
+  h10_tile<BN, MT>(S, row0, kslice, ks, a, ws, h10lds);
 }
 
-template <int BN>
+template <int BN, int MT>
 int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
-  constexpr int LDS = H10<BN>::LDS;
+  constexpr int LDS = H10<BN, MT>::LDS, BM = H10<BN, MT>::BM;
   const int nmb = (a.M + BM - 1) / BM;
   const int grid = ((ntiles + 7) / 8) * 8 * nmb * ks;
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
-    if (hipFuncSetAttribute((const void*)hgemm10_kernel<BN>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) !=
+    if (hipFuncSetAttribute((const void*)hgemm10_kernel<BN, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) !=
         hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL(hgemm10_kernel<BN>, dim3(grid), dim3(512), LDS, st, sl, a, ks, ws, ntiles, nmb);
+  hipLaunchKernelGGL((hgemm10_kernel<BN, MT>), dim3(grid), dim3(512), LDS, st, sl, a, ks, ws, ntiles, nmb);
   return (int)hipGetLastError();
 }
 
-// bn: weight rows per workgroup tile (256 or 128)
+// bn: weight rows per workgroup tile (256 or 128). Row blocks of 192 instead of 256 where their rounds over the 256 CUs, each three quarters as
+// long, end earlier (Llama-3-8B at 384 rows: gate|up 99 -> 76 us, down 69 -> 57; 1500 rows: o 65 -> 56; 3000: down 308 -> 276).
 int launch_dense10(int bn, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
-  if (bn == 256) return launch_t<256>(sl, ntiles, ks, ws, a, st);
-  if (bn == 128) return launch_t<128>(sl, ntiles, ks, ws, a, st);
+  auto rounds = [&](int bm) { return (long)((ntiles * ((a.M + bm - 1) / bm) * ks + 255) / 256) * bm; };
+  const bool low = rounds(192) < rounds(256);
+  if (bn == 256) return low ? launch_t<256, 3>(sl, ntiles, ks, ws, a, st) : launch_t<256, 4>(sl, ntiles, ks, ws, a, st);
+  if (bn == 128) return low ? launch_t<128, 3>(sl, ntiles, ks, ws, a, st) : launch_t<128, 4>(sl, ntiles, ks, ws, a, st);
   return -1;
 }
 

@@ -409,6 +409,9 @@ def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: 
             raise ValueError(f"qgemv: M={M} rows but x has {x.shape[0]}, y {y.shape[0]}")
         if mode < 0 or waves == 0:
             mode, waves, rt, ks = gemv_config(segs, M) if not mapped else MOE_GEMV
+            if mode == 10 and (x.stride(0) % 8 or y.stride(0) % 4):
+                from . import tuning
+                mode, waves, rt, ks = tuning.dense_heuristic(segs, M, aligned=False)
         if M > 64 and mode == 0:
             # mapped (MoE) rows / path A: chunks of 64 rows
             for m0 in range(0, M, 64):

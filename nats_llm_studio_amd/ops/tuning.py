@@ -90,27 +90,30 @@ def dense_key(segs, M: int) -> str:
     return f"d:{sum(s.w.rows for s in segs)}:{segs[0].w.K}:{_mb(M)}"
 
 
-def dense_heuristic(segs, M: int):
-    """Modes 4/5/6 (dense f16 GEMM) for shapes without a tuned "d:" entry. Decode batches (M < 1024): 128 x 128 tiles
-    on 16 waves (mode 4, wm 2) -- what the tuner picked for nearly every Llama-3-8B / Granite-3.0-2B shape at M = 256 /
-    512, where the r05 rule (256 x 256 tiles from M >= 192) ran Granite's B=512 GEMMs 1.3-1.7x slower
-    (profiles/granite_r06.txt); prefill chunks (M >= 1024): 256-row activation blocks with 256-row weight tiles
-    (mode 5). Then the split-K that minimises (workgroup rounds over the 256 CUs) / ks, with a small per-slice cost."""
-    if M < 1024:
-        mode, bn, wm, waves = (4, 128, 2, 16) if M >= 128 else (4, 128, 2, 8)
-    else:
-        mode, bn, wm, waves = 5, 256, 4, 8
-    bm = 64 * wm
-    tiles = sum((s.w.rows + bn - 1) // bn for s in segs) * ((M + bm - 1) // bm)
-    nkt = segs[0].w.K // 64
-    best, best_ks = None, 1
-    for ks in range(1, 9):
-        if ks > 1 and nkt // ks < 8:
-            break
-        cost = -(-tiles * ks // 256) / ks + 0.03 * ks
-        if best is None or cost < best - 1e-9:
-            best, best_ks = cost, ks
-    return (mode, waves, wm, best_ks)
+# Microseconds of a round of 256 workgroups at K = 4096, by (mode, rt, activation rows of a tile); 5 of them do not grow with
+# K. Mode 10's launcher takes 192 or 256 rows, whichever fills its rounds better. (Llama-3-8B shapes at M = 256 .. 4096, e.g.
+# gate|up at 384 rows 76 us, at 3000 585, Q|K|V at 3000 168, o at 1500 56, down at 4096 375.)
+_ROUND_US = {(10, 1, 256): 106.0, (10, 1, 192): 82.0, (10, 2, 256): 72.0, (10, 2, 192): 48.0, (4, 2, 128): 44.0}
+
+
+def dense_heuristic(segs, M: int, aligned: bool = True):
+    """Dense f16 GEMM for shapes without a tuned "d:" entry, and above the tuned row counts: the cheapest of mode 10 with 256 or 128
+    weight rows and mode 4 with 128 x 128 tiles, by the rounds of tiles over the 256 CUs; split-K slabs are written and read again.
+    (A rule that took mode 4 below 1024 rows and mode 5 above ran a 32000-row head at 300 / 900 / 4096 rows in 161 / 742 / 2846 us;
+    mode 10 takes 108 / 223 / 909.) aligned: the operands' row strides suit mode 10, whose stores are 4 columns wide."""
+    rows, K = sum(s.w.rows for s in segs), segs[0].w.K
+    nkt = K // 64
+    aligned = aligned and all(s.w.rows % 4 == 0 and s.ycol % 4 == 0 for s in segs)
+
+    def us(mode, rt, ks):
+        bn = 256 if (mode, rt) == (10, 1) else 128
+        tiles = sum((s.w.rows + bn - 1) // bn for s in segs) * ks
+        best = min(-(-tiles * -(-M // bm) // 256) * (5.0 + (t - 5.0) * K / ks / 4096)
+                   for (md, r, bm), t in _ROUND_US.items() if (md, r) == (mode, rt))
+        return best + (2.0 + 2e-6 * ks * M * rows if ks > 1 else 0.0)
+    mode, rt, ks = min(((mode, rt, ks) for mode, rt in ([(10, 1), (10, 2)] if aligned else []) + [(4, 2)] for ks in range(1, 9)
+                        if ks == 1 or nkt // ks >= 8), key=lambda c: us(*c))
+    return (mode, 8 if mode == 10 or M < 128 else 16, rt, ks)
 
 
 def select_dense(segs, M: int):
@@ -118,6 +121,8 @@ def select_dense(segs, M: int):
     hit = table().get(dense_key(segs, M))
     if hit is not None and hit[0] < 0:
         return None
+    if M > MBUCKETS[-1]:
+        return dense_heuristic(segs, M)
     return hit if hit is not None else dense_heuristic(segs, M)
 
 

@@ -1,0 +1,76 @@
+"""The dense f16 GEMM (mode 10) where its row blocks change between 192 and 256 rows, and its RoPE epilogue for head widths that its
+8-byte stores take and that they do not."""
+import numpy as np
+import pytest
+import torch
+
+from nats_llm_studio_amd import ops
+from nats_llm_studio_amd.gguf.constants import GGMLType
+from nats_llm_studio_amd.gguf.quants import random_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def weight(rows, K, seed=0):
+    w = ops.QWeight(random_blocks(GGMLType.Q8_0, rows * K, 0.02, np.random.default_rng(seed)), GGMLType.Q8_0, rows, K, "cuda", "w")
+    w.expand_dense()
+    return w
+
+
+def acts(M, K, seed=1):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn((M + 63) // 64 * 64, K, generator=g, device="cuda").to(torch.float16)
+
+
+def relerr(got, want):
+    return float((got.double() - want.double()).norm() / want.double().norm())
+
+
+# rows: 101 weight tiles of 256 (202 of 128) make 192-row blocks the shorter walk at 190, 384 and 700 rows and 256-row blocks at
+# 193 .. 256 and 512 rows, for one of the two tile widths at least
+@pytest.mark.parametrize("rt", [1, 2])
+@pytest.mark.parametrize("M", [190, 193, 256, 257, 384, 385, 512, 700])
+@pytest.mark.parametrize("epi", ["f32", "swiglu"])
+def test_row_blocks(M, rt, epi):
+    rows, K = 25700 - 4 if epi == "f32" else 25600, 256
+    w, x = weight(rows, K), acts(M, K)
+    z = x[:M].float() @ w.d16.float().T
+    if epi == "swiglu":
+        v = z.view(M, rows // 16, 2, 8)
+        z = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, rows // 2)
+    y = torch.full((x.shape[0], z.shape[1]), 7.0, device="cuda", dtype=torch.float32 if epi == "f32" else torch.float16)
+    ops.qgemv([ops.Seg(w)], x, y, M, epi=epi, mode=10, waves=8, rt=rt, ks=1)
+    # sums of 256 products in f32; f16 outputs round to 2^-11
+    assert relerr(y[:M], z) < (1e-6 if epi == "f32" else 5e-4)
+    assert (y[M:] == 7).all()
+
+
+@pytest.mark.parametrize("cfg", [(10, 8, 1, 1), (10, 8, 2, 1), (4, 16, 2, 1), (4, 8, 4, 1)])
+@pytest.mark.parametrize("D,bias", [(64, False), (128, True), (34, True)])
+@pytest.mark.parametrize("M", [70, 300])
+def test_rope_epilogue(cfg, D, bias, M):
+    """Against the same product rotated on the CPU: rows without a cache slot, shuffled slots."""
+    Hq, Hkv, K = 16, 8, 256
+    ws = [weight(h * D, K, s) for s, h in enumerate((Hq, Hkv, Hkv))]
+    segs = [ops.Seg(ws[0], 0), ops.Seg(ws[1], Hq * D), ops.Seg(ws[2], (Hq + Hkv) * D)]
+    x, n = acts(M, K), (Hq + 2 * Hkv) * D
+    pad = x.shape[0]
+    cs = ops.rope_table(400, D, 10000.0, torch.device("cuda"))
+    pos = (torch.arange(pad, dtype=torch.int32, device="cuda") * 7) % 400
+    slot = torch.randperm(pad, generator=torch.Generator().manual_seed(2)).int().cuda()
+    slot[[0, 17, M - 1]] = -1
+    b = torch.randn(n, generator=torch.Generator().manual_seed(3)).cuda() if bias else None
+    outs = []
+    for c, fuse in ((cfg, True), (cfg, False)):
+        q = torch.full((pad, Hq * D), 776.0, dtype=torch.bfloat16, device="cuda")
+        kc, vc = (torch.full((pad, Hkv, D), 776.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        qkv = torch.zeros(pad, n, device="cuda")
+        if fuse:
+            ops.qkv_rope_kv(segs, x, qkv, pos, slot, cs, q, kc, vc, M, Hq, Hkv, D, cfg=c, bias=b)
+        else:
+            ops.qgemv(segs, x, qkv, M, mode=c[0], waves=c[1], rt=c[2], ks=1)
+            q, kc, vc = q.cpu(), kc.cpu(), vc.cpu()
+            ops.rope_kv(qkv.cpu(), pos.cpu(), slot.cpu(), cs.cpu(), q, kc, vc, M, Hq, Hkv, D, bias=None if b is None else b.cpu())
+        outs.append((q.cpu(), kc.cpu(), vc.cpu()))
+    for a, b in zip(*outs):      # one bf16 rounding apart at most, and the same places written
+        assert relerr(a, b) < 2e-3 and ((a == 776) == (b == 776)).all()
