@@ -308,6 +308,7 @@ class Engine:
         kw = {"logit_rows": self.max_logit_rows} if max_logit_rows > self.max_batch else {}
         self.pb = model.step_buffers(max_prefill_tokens, self.max_batch, self.max_blocks, **kw)
         self._fed: Dict[object, _Seq] = {}
+        self._stage: Optional[list] = None      # pinned buffers of _rows_to_host
         pin = self.dev.type == "cuda"
         # decode metadata / next-token host buffers are double-buffered (async decode: step N+1 is
         # prepared and launched while step N's copies may still be in flight)
@@ -474,7 +475,7 @@ class Engine:
         self.graphs.clear()
         self.pf_graphs.clear()
         self.kc = self.vc = self.state = None
-        self.db = self.pb = None
+        self.db = self.pb = self._stage = None
         self.model = None
         if self.dev.type == "cuda":
             torch.cuda.empty_cache()
@@ -683,14 +684,16 @@ class Engine:
     # decode step. Not to be mixed with submitted requests.
     def feed(self, entries) -> List[torch.Tensor]:
         """entries: [(id, tokens, want)]: the next tokens of request `id` (admitted at its first entry) and the places
-        among them whose logits are wanted. Returns one CPU f32 tensor [len(want), vocab] per entry."""
+        among them whose logits are wanted. Returns one CPU f32 tensor [len(want), vocab] per entry (rows of one buffer)."""
         if self.tp is not None:
             raise NotImplementedError("feed: single-GPU engines only")
         if self.running or self.waiting:
             raise RuntimeError("feed: the engine is generating")
         if len(set(e[0] for e in entries)) != len(entries):
             raise ValueError("feed: one entry per request and step")
-        seqs = []
+        # (a decode step of a few hundred requests waits for this loop: a token at a time is checked without an array, entries
+        # without wanted places share one empty result)
+        V, bs, single, seqs = self.cfg.vocab, self.bs, True, []
         for rid, toks, want in entries:
             s = self._fed.get(rid)
             if s is None:
@@ -700,18 +703,20 @@ class Engine:
                 if self.slots is not None:
                     s.state_slot = self.slots.alloc()
                 self._fed[rid] = s
-            if not len(toks):
+            m = len(toks)
+            if not m:
                 raise ValueError("feed: an entry without tokens")
-            if any(not 0 <= int(t) < self.cfg.vocab for t in toks):
+            if not (0 <= int(toks[0]) < V if m == 1 else self._inside(toks, V)):
                 raise ValueError("feed: token outside the vocabulary")
-            if any(not 0 <= int(w) < len(toks) for w in want):
+            if len(want) and any(not 0 <= int(w) < m for w in want):
                 raise ValueError("feed: wanted place outside the entry")
-            n = s.n_fed + len(toks)
+            if m > 1 or not s.n_fed:
+                single = False
+            n = s.n_fed + m
             if n > self.ctx:
                 raise ValueError(f"feed: {n} tokens exceed the context length ({self.ctx})")
-            more = math.ceil(n / self.bs) - len(s.blocks)
-            if more > 0:
-                blocks = self.alloc.alloc(more)
+            if n > len(s.blocks) * bs:
+                blocks = self.alloc.alloc(math.ceil(n / bs) - len(s.blocks))
                 if blocks is None:
                     raise RuntimeError("feed: the cache pool is full")
                 s.blocks += blocks
@@ -719,31 +724,67 @@ class Engine:
                     for hm in self.h_meta_d2:
                         self._tables(hm, self.db.pad)[0][s.row, :len(s.blocks)] = s.blocks
             seqs.append(s)
-        out = [torch.zeros(len(e[2]), self.cfg.vocab) for e in entries]
-        if all(len(e[1]) == 1 and s.n_fed > 0 for e, s in zip(entries, seqs)):
-            self._feed_decode(seqs, entries, out)
+        wants = [len(e[2]) for e in entries]
+        flat = torch.empty(sum(wants), V)                  # every entry's rows, one entry behind the other
+        if single:
+            self._feed_decode(seqs, entries, flat, wants)
         else:
-            self._feed_rows(seqs, entries, out)
-        return out
+            self._feed_rows(seqs, entries, flat, wants)
+        if len(flat) == 0:
+            return [flat] * len(entries)
+        return list(flat.split(wants))
 
-    def _feed_decode(self, seqs, entries, out):
+    @staticmethod
+    def _inside(toks, vocab: int) -> bool:
+        """Whether every token is an id of the vocabulary."""
+        try:
+            a = np.fromiter(map(int, toks), np.int64, len(toks))
+        except OverflowError:
+            return False
+        return bool((a >= 0).all() and (a < vocab).all())
+
+    STAGE_BYTES = 8 << 20        # of each of the two pinned buffers that logits pass on their way to the host
+
+    def _rows_to_host(self, src: torch.Tensor, dst: torch.Tensor):
+        """Copy device rows to pageable host memory, through two pinned buffers: one is emptied while the next copy runs."""
+        if self.dev.type != "cuda":
+            dst.copy_(src)
+            return
+        n, V = dst.shape
+        rows = max(1, self.STAGE_BYTES // (4 * V))
+        if self._stage is None:
+            self._stage = [(torch.empty(min(rows, self.max_logit_rows), V, pin_memory=True), torch.cuda.Event()) for _ in range(2)]
+        rows = len(self._stage[0][0])
+        for c in range(0, n + rows, rows):
+            if c < n:
+                buf, ev = self._stage[c // rows & 1]
+                buf[:min(rows, n - c)].copy_(src[c:c + rows], non_blocking=True)
+                ev.record()
+            if c:
+                buf, ev = self._stage[(c // rows - 1) & 1]
+                ev.synchronize()
+                dst[c - rows:c].copy_(buf[:min(rows, n - c + rows)])
+
+    def _feed_decode(self, seqs, entries, flat, wants):
         for s, e in zip(seqs, entries):
             s.tokens.append(int(e[1][0]))
             if s.row < 0:
                 self._assign_row(s)
-        need = any(len(e[2]) for e in entries)
+        need = len(flat) > 0
         (snap, k) = self._launch(seqs, set(), need)
+        if need:
+            rows = [r for (r, _), w in zip(snap, wants) for _ in range(w)]
+            lg = self.db.logits
+            lg = lg[rows[0]:rows[0] + len(rows)] if rows == list(range(rows[0], rows[0] + len(rows))) else lg[rows]
+            self._rows_to_host(lg, flat)
         if self.dev.type == "cuda":
             self._ev[k].synchronize()
-        if need:
-            lg = self.db.logits[[r for r, _ in snap]].float().cpu()
-            for i, e in enumerate(entries):
-                out[i][:] = lg[i]
 
-    def _feed_rows(self, seqs, entries, out):
+    def _feed_rows(self, seqs, entries, flat, wants):
         """Row batches of at most max_prefill rows and max_logit_rows wanted rows (one batch unless the step is larger)."""
         work = [(i, s, [int(t) for t in e[1]], sorted((int(w), j) for j, w in enumerate(e[2])))
                 for i, (s, e) in enumerate(zip(seqs, entries))]
+        first = [0, *itertools.accumulate(wants)]          # an entry's first row of the results
         done = [0] * len(work)
         while any(done[i] < len(toks) for i, _, toks, _ in work):
             parts, rows, dest, T = [], [], [], 0
@@ -758,7 +799,7 @@ class Engine:
                     continue
                 parts.append((s, s.n_fed, toks[done[i]:done[i] + n]))
                 rows += [T + p - done[i] for p, _ in w]
-                dest += [(i, j) for _, j in w]
+                dest += [first[i] + j for _, j in w]
                 s.tokens += toks[done[i]:done[i] + n]
                 s.n_fed += n
                 done[i] += n
@@ -768,9 +809,13 @@ class Engine:
             self._exec_prefill(T, rows or [0], True, len(parts))
             self.counters["prefill_tokens"] += T
             if rows:
-                lg = self.pb.logits[:len(rows)].float().cpu()
-                for r, (i, j) in enumerate(dest):
-                    out[i][j] = lg[r]
+                lg = self.pb.logits[:len(rows)]
+                if dest == list(range(dest[0], dest[0] + len(dest))):
+                    self._rows_to_host(lg, flat[dest[0]:dest[0] + len(dest)])
+                else:
+                    got = torch.empty(len(rows), self.cfg.vocab)
+                    self._rows_to_host(lg, got)
+                    flat[dest] = got
             elif self.dev.type == "cuda":
                 torch.cuda.current_stream(self.dev).synchronize()
 
@@ -779,7 +824,11 @@ class Engine:
         s = self._fed.pop(rid)
         s.done = True
         self._release_memory(s)
-        self._release_rows()
+        if s.row >= 0:
+            self.rows[s.row] = None
+            s.row = -1
+        if not self._fed:               # (with the last one: what finished generations may have left)
+            self._release_rows()
 
     def _first_tokens(self, seqs: List[_Seq], toks: List[int]):
         now = time.monotonic()

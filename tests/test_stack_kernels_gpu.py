@@ -157,3 +157,20 @@ def test_plain_attention_rows_of_many_sequences(K, dt, H, G, D, window, keep, si
     # f32: the sums of a row; bf16: the output's rounding
     assert relerr(o[:T, :, :D], want) < (2e-6 if dt == "f32" else 3e-3)
     assert (o[:T, :, D:] == 0).all() and (o[T - 1] == 0).all() and (o[T] == 7).all()
+
+
+@pytest.mark.parametrize("n", [1, 6, 7, 8, 14, 15, 50])
+def test_rows_to_host(K, n):
+    """Logits on their way through two pinned buffers of seven rows: fewer, exactly and more than they hold, wanted rows gathered."""
+    from types import SimpleNamespace
+
+    from nats_llm_studio_amd.engine.engine import Engine
+    V = 33
+    eng = SimpleNamespace(dev=torch.device("cuda:0"), STAGE_BYTES=7 * 4 * V + 5, _stage=None, max_logit_rows=64)
+    for k in range(3):                                   # the buffers are used again
+        src = rnd(n + 3, V, seed=k).float().cuda()
+        for rows in (src[:n], src[list(range(n, 0, -1))]):
+            dst = torch.zeros(n, V)
+            Engine._rows_to_host(eng, rows, dst)
+            assert (dst == rows.cpu()).all()
+    assert len(eng._stage[0][0]) == 7
