@@ -767,12 +767,13 @@ __global__ __launch_bounds__(64) void moe_pick_kernel(const float* __restrict__ 
 
 // ---- routed-entry lists of one step: entries (token t, choice j) = t * topk + j grouped by expert (entry order within
 // an expert is arbitrary: rows do not interact), and the (expert, <= bm entries) tiles of the grouped products.
-// One workgroup. PICK: also choose the experts (small steps: one launch less).
+// One workgroup. PICK: also choose the experts (small steps: one launch less). ctx (null: none): rows without keys are a step's
+// padding and get no entries (200 of 256 rows: two experts had half as many rows again, a second tile each).
 template <bool PICK>
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict__ z, long ldz, int T, Route R,
                                                         float* __restrict__ topw, int* __restrict__ sel, int bm,
                                                         int* __restrict__ rows, int* __restrict__ tiles,
-                                                        int* __restrict__ ntiles, int maxtiles) {
+                                                        int* __restrict__ ntiles, int maxtiles, const int* __restrict__ ctx) {
   __shared__ int cnt[ME], off[ME], pos[ME];
   __shared__ float sc[PICK ? PW : 1][PICK ? ME : 1], gs[PICK ? PW : 1][PICK ? ME : 1];
   const int E = R.E, topk = R.topk, n = T * topk;
@@ -784,7 +785,9 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict_
   }
   for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < n; i += 1024) atomicAdd(&cnt[min(max(sel[i], 0), E - 1)], 1);
+  auto live = [&](int i) { return !ctx || ctx[i / topk] > 0; };
+  for (int i = threadIdx.x; i < n; i += 1024)
+    if (live(i)) atomicAdd(&cnt[min(max(sel[i], 0), E - 1)], 1);
   __syncthreads();
   if (threadIdx.x < 64) {
     // one wave: exclusive prefix sums of counts and tile counts, 64 experts at a time
@@ -820,7 +823,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict_
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += 1024) {
     const int e = min(max(sel[i], 0), E - 1);
-    rows[off[e] + atomicAdd(&pos[e], 1)] = i;
+    if (live(i)) rows[off[e] + atomicAdd(&pos[e], 1)] = i;
   }
 }
 
@@ -935,9 +938,9 @@ int nls_stack_argmax(const float* z, long ldz, int V, int* out, int n, void* str
   return (int)hipGetLastError();
 }
 
-// rows: int [T * topk]; tiles: int [maxtiles][4], maxtiles >= min(T * topk, E + T * topk / bm)
+// rows: int [T * topk]; tiles: int [maxtiles][4], maxtiles >= min(T * topk, E + T * topk / bm); ctx: int [T] (null: every row is routed)
 int nls_moe_plan(const float* z, long ldz, int T, int E, int topk, int groups, int keep, int softmax, int gbest, float scale,
-                 float* topw, int* sel, int bm, int* rows, int* tiles, int* ntiles, int maxtiles, void* stream) {
+                 float* topw, int* sel, int bm, int* rows, int* tiles, int* ntiles, int maxtiles, const int* ctx, void* stream) {
   if (T < 1 || E < 1 || E > ME || topk < 1 || topk > E || groups < 1 || E % groups || keep < 1 || bm < 1 ||
       (long)min(keep, groups) * (E / groups) < topk || maxtiles < 1 || gbest < 1 || gbest > 2)
     return -1;
@@ -945,12 +948,12 @@ int nls_moe_plan(const float* z, long ldz, int T, int E, int topk, int groups, i
   hipStream_t st = (hipStream_t)stream;
   if (T <= 32) {
     hipLaunchKernelGGL(moe_plan_kernel<true>, dim3(1), dim3(1024), 0, st, z, ldz, T, R, topw, sel, bm,
-                       rows, tiles, ntiles, maxtiles);
+                       rows, tiles, ntiles, maxtiles, ctx);
     return (int)hipGetLastError();
   }
   hipLaunchKernelGGL(moe_pick_kernel, dim3(T), dim3(64), 0, st, z, ldz, R, topw, sel);
   hipLaunchKernelGGL(moe_plan_kernel<false>, dim3(1), dim3(1024), 0, st, z, ldz, T, R, topw, sel, bm, rows,
-                     tiles, ntiles, maxtiles);
+                     tiles, ntiles, maxtiles, ctx);
   return (int)hipGetLastError();
 }
 

@@ -313,7 +313,7 @@ class MoeFeedForward(_Part):
     def run(self, b: StackBuffers, e: dict, step: "_Step"):
         T, st = step.T, step.st
         e["first"].run(T, st)
-        e["plan"].run(e["z"], T, st)
+        e["plan"].run(e["z"], T, st, step.keys)
         e["up"].run(T, st)
         e["down"].run(T, st)
 
@@ -877,6 +877,7 @@ class _Step:
     st: int
     plan: Optional[_ExpandPlan] = None
     layer: int = 0              # the layer run: its cache and state (its parts may be another run's)
+    keys: Optional[torch.Tensor] = None      # keys of each row (None: no row is padding)
 
 
 # runs of at least this many rows expand (below, the latent-space attention's extra products cost less than the expansion
@@ -1111,7 +1112,7 @@ class StackModel:
             raise ValueError(f"step of {T} rows, buffers hold {b.pad}")
         cfg = self.cfg
         st = K.stream(self.device)
-        step = _Step(T, T if nruns is None else nruns, block_size, st)
+        step = _Step(T, T if nruns is None else nruns, block_size, st, keys=b.ctx_len)
         if row_info is not None and qblocks is not None:
             step.plan = self._expand_plan(b, qblocks, row_info, T, block_size, st)
         rms, groups = cfg.design.norm == "rms", cfg.norm_groups

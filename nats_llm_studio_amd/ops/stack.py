@@ -55,7 +55,7 @@ _SIGS = {
     "nls_gla_step": [P, P, P, L, P, L, P, P, P, I, F, F, P, L, P, I, P, P, L, P, L, P, L, I, I, I, F, I, P],
     "nls_latent_rows": [P, L, I, P, P, L, P, L, I, I, I, P, P, P, P, P, L, I, F, I, P],
     "nls_stack_argmax": [P, L, I, P, I, P],
-    "nls_moe_plan": [P, L, I, I, I, I, I, I, I, F, P, P, I, P, P, P, I, P],
+    "nls_moe_plan": [P, L, I, I, I, I, I, I, I, F, P, P, I, P, P, P, I, P, P],
     "nls_shift_mix": [P, L, P, P, L, P, L, L, P, P, I, I, I, P],
     "nls_wkv_scan": [P, P, P, L, P, L, P, P, L, P, L, P, L, P, L, I, P, I, I, I, I, P],
     "nls_scan_out": [P, L, P, P, L, P, L, I, I, I, F, I, P],
@@ -185,7 +185,8 @@ class Seg:
 
 
 # (weight rows, rows) of lin_gemm's configs
-GEMM_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (256, 256), (64, 64), (192, 128), (256, 256))
+GEMM_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (256, 256), (64, 64), (192, 128), (256, 256),
+              (96, 64), (160, 64), (128, 64), (96, 128))
 
 
 # Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
@@ -235,7 +236,7 @@ class LinLaunch:
             if bm == 16:
                 return False, 1, (4 if self._tiles(16, 16, M) >= 1536 else 8), 1
             if bm == 64:
-                return True, 0
+                return True, 0 if self.f32 else self.balanced(M)
             if bm == 256:
                 return True, 7
             return True, (3 if self._tiles(256, 128, M) >= 224 else 2)
@@ -247,6 +248,8 @@ class LinLaunch:
             return False, 1, (4 if ns <= 16 else 8 if n16 >= 320 or ns <= 32 else 16), 1
         if n16 <= 64:                     # a router's few outputs: split K over a workgroup's waves
             return False, 1, 16, 1
+        if M <= 64 and not self.f32 and ns > 16:
+            return self.few_rows(M, n64)
         if M <= 64:
             if n64 >= 250:
                 return True, 0
@@ -255,6 +258,11 @@ class LinLaunch:
             return True, (0 if M <= 2048 else 1)
         if n64 < 96 and n16 <= 1024:
             return False, 1, 16, 1
+        if M <= 128 and not self.f32:
+            if 160 <= self._tiles(96, 128, M) <= 256:        # 128 x 24576 x 4096: 52 us, 61 on 192 x 128, 65 on 64 x 64
+                return True, 11
+            if n64 > 256 and self._tiles(96, 64, M) <= 256:  # 96 x 10240 x 4096: 34 us, 37 on 64 x 64, 53 on 192 x 128
+                return True, 8
         rate = GEMM_RATE_F32 if self.f32 else GEMM_RATE
         if self.f32 or M > 512:
             cand = list(rate)
@@ -270,6 +278,23 @@ class LinLaunch:
             n, (few, lo, hi) = self._tiles(*GEMM_TILES[c], M), rate[c]
             return -(-n // 256) * GEMM_TILES[c][0] * GEMM_TILES[c][1] / (lo if n <= few else hi)
         return True, min(cand, key=cost)
+
+    def balanced(self, M: int) -> int:
+        """The GEMM config of launches with up to 64 rows to a tile, which read each weight once: the tile whose rounds of 256 workgroups
+        sum up to the fewest weight rows, the largest of equals (four stages also keep such workgroups from sharing a CU while
+        another has none). In a running step at 64 rows and K = 4096 (64 / 96 / 128 / 160 weight rows): N = 35888 85 / 75 / 98 / 73 us, 34816
+        75 / 68 / 92 / 63, 26880 57 / 68 / 54 / 60, 24576 57 / 53 / 57 / 63, 32000 65 / 76 / 68 / 73; eight experts, N = 6144: 99 / 94 / 107 / 119,
+        and N = 4096 at K = 6144: 115 / 99 / 82 / 85."""
+        return min((10, 9, 8, 0), key=lambda c: (-(-self._tiles(*GEMM_TILES[c], M) // 256) * GEMM_TILES[c][0], -GEMM_TILES[c][0]))
+
+    def few_rows(self, M: int, n64: int):
+        """17 to 64 rows, bound by the weights' bytes. Up to 8192 outputs the streaming kernel's two weight tiles fill the chip (48 x 4096 x
+        4096: 20 us, 27 in the GEMM; 24 x 8192: 16, 27)."""
+        if self._tiles(32, 64, M) <= 256:
+            return False, 4, 8, 2
+        if n64 <= 256:                    # 48 x 10240 x 4096: 27 us with 8 stages in flight, 35 streaming; 20 rows: 27, 23
+            return (False, 2, 4, 2) if M <= 32 else (True, 5)
+        return True, self.balanced(M)
 
     def split_config(self, M: int):
         """(config, K splits) of a launch that may split K: about 512 workgroups of 64 x 64 tiles, or 256 of 256 x 128."""
@@ -372,11 +397,12 @@ class MoePlan:
         n = T * self.top
         return max(1, min(n, self.experts), n // bm)
 
-    def run(self, z: torch.Tensor, T: int, st: int):
+    def run(self, z: torch.Tensor, T: int, st: int, ctx_len: Optional[torch.Tensor] = None):
+        """ctx_len: rows without keys (a step's padding) are not routed."""
         _check(lib().nls_moe_plan(z.data_ptr(), z.stride(0), T, self.experts, self.top, self.groups, self.keep,
                                   self.softmax, self.group_best, self.scale, self.topw.data_ptr(), self.sel.data_ptr(), self.bm(T),
                                   self.rows.data_ptr(), self.tiles.data_ptr(), self.ntiles.data_ptr(),
-                                  self.max_tiles(T), st), "nls_moe_plan")
+                                  self.max_tiles(T), _p(ctx_len), st), "nls_moe_plan")
 
 
 # ---------------------------------------------------------------------------

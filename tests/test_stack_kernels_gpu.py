@@ -69,6 +69,37 @@ def test_phased_gemm(K, M, Kd):
     assert (o[:, 32:64] == 7).all() and all((t[M] == 7).all() for t in y.values())
 
 
+@pytest.mark.parametrize("cfg", [8, 9, 10, 11])
+@pytest.mark.parametrize("M,N,Kd", [(17, 96, 70), (64, 160, 192), (65, 161, 256), (129, 500, 330), (40, 1000, 1000)])
+def test_balanced_tiles(K, cfg, M, N, Kd):
+    """Tiles of 96, 128 and 160 weight rows: row and column edges, one to sixteen steps of K (fewer than the stages)."""
+    bf = torch.bfloat16
+    x, w = rnd(M, Kd, seed=1).to(bf), (rnd(N, Kd, seed=2) * Kd ** -0.5).to(bf)
+    y = torch.full((M + 1, N), 7.0, device="cuda")
+    L = K.LinLaunch([K.Seg(K.PackedLinear(w, False, "cuda"), act(x, K.act_ld(Kd)), y[:M])])
+    L._cfg[M] = (True, cfg), 1
+    L.run(M, st())
+    assert relerr(y[:M], x.double() @ w.double().T) < 2e-6 and (y[M] == 7).all()
+
+
+@pytest.mark.parametrize("T", [7, 32, 33, 200])
+def test_padding_rows_are_not_routed(K, T):
+    """Rows without keys get no entries, in both forms of the plan; none at all when every row is padding."""
+    E, top = 8, 2
+    z = rnd(T, E, seed=1).float()
+    ctx = (torch.arange(T, dtype=torch.int32) % 3) * 5
+    plan = K.MoePlan(T, E, top, 1, 1, 1.0, "cuda")
+    for c in (ctx, torch.zeros_like(ctx)):
+        plan.run(z.cuda(), T, st(), c.cuda())
+        n = int(plan.ntiles[0])
+        got = []
+        for e, o, k, _ in plan.tiles[:n].tolist():
+            rows = plan.rows[o:o + k].tolist()
+            assert 1 <= k <= plan.bm(T) and all(plan.sel[r] == e for r in rows)
+            got += rows
+        assert sorted(got) == [i for i in range(T * top) if c[i // top] > 0]
+
+
 @pytest.mark.parametrize("M,N,rows", [(300, 160, 1500), (600, 512, 1200), (700, 160, 1399)])
 def test_tall_split(K, M, N, rows):
     """More rows than a slab was bound for: as many slabs as the buffer holds (4, 2, 1), apart by the launch's rows."""
