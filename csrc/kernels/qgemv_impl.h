@@ -833,9 +833,9 @@ DEVI void mm_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
   };
 
   typedef typename RawOf<T>::type Raw;
-  // weight-stream depth: few-row launches (MT <= 2) are latency-bound on the weight stream (batch-1
+  // weight-stream depth: few rows (NA <= 2) are latency-bound on the weight stream (batch-1
   // gate|up: one 128-row workgroup per CU), so keep 4 super-blocks in flight per wave there
-  constexpr int DEPTH = (MT <= 2 && RT == 1 && sizeof(Raw) <= 80) ? 4 : 2;
+  constexpr int DEPTH = (NA <= 2 && MT <= 4 && RT == 1 && sizeof(Raw) <= 80) ? 4 : 2;
   Raw wA[RT], wB[RT], wC[RT], wD[RT];
   const int sbl = max(sb1 - 1, sb0);
   if (sb0 < sb1) {
@@ -860,7 +860,7 @@ DEVI void mm_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
     load_xh(nxt, 0);
     __builtin_amdgcn_sched_barrier(0);
     const act_t* xb = lds + buf * (MT * 16 * 256);
-    if constexpr (MT >= 4) {
+    if constexpr (NA >= 4 || MT == 8) {
       // large tiles: per-K-step fragments (scales once per super-block), weight buffer reloaded
       // after its last use; x half 0 written after K-steps 0-3, half 1 loaded then, written last
       typename ScOf<T>::type sc[RT];
@@ -990,8 +990,10 @@ DEVI void mm_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
   }
 }
 
-// Active-tile dispatch: only the 8-wave, 2-row-tile, 8-tile instance (the MoE grouped launch) picks NA
-// per block -- {2, 4, 6, 8}, rounded up to even to bound the instantiations; the rest run NA = MT.
+// Active-tile dispatch by the rows of a block (an expert's are known on the device only): the 8-wave, 2-row-tile, 8-tile
+// instance takes {2, 4, 6, 8}, rounded up to even to bound the instantiations, those of 2 to 4 tiles {1, 2, MT}: 24 tokens
+// give eight experts 4 to 11 rows each, so a second tile was only padding (Q5_K gate|up 8 x 8192 x 2048 on (8, 2): 27.7 ->
+// 25.1 us, down 8 x 2048 x 4096 on (4, 1): 19.9 -> 17.5; 64 tokens 34.3 -> 28.5 and 29.5 -> 20.4).
 template <int T, int WAVES, int RT, int MT, bool XL>
 DEVI void mm_tile_na(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, act_t* lds,
                      const int* xm, const int* ym) {
@@ -1001,6 +1003,10 @@ DEVI void mm_tile_na(const Seg& S, int row0, int kslice, int ks, const GemvArgs&
     else if (na <= 4) mm_tile<T, WAVES, RT, MT, XL, 4>(S, row0, kslice, ks, a, ws, lds, xm, ym);
     else if (na <= 6) mm_tile<T, WAVES, RT, MT, XL, 6>(S, row0, kslice, ks, a, ws, lds, xm, ym);
     else mm_tile<T, WAVES, RT, MT, XL, 8>(S, row0, kslice, ks, a, ws, lds, xm, ym);
+  } else if constexpr (MT >= 2 && MT <= 4 && !XL) {
+    if (a.M <= 16) mm_tile<T, WAVES, RT, MT, XL, 1>(S, row0, kslice, ks, a, ws, lds, xm, ym);
+    else if (MT > 2 && a.M <= 32) mm_tile<T, WAVES, RT, MT, XL, 2>(S, row0, kslice, ks, a, ws, lds, xm, ym);
+    else mm_tile<T, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, lds, xm, ym);
   } else {
     mm_tile<T, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, lds, xm, ym);
   }

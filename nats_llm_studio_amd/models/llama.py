@@ -40,7 +40,7 @@ _SPLIT_WG = int(os.environ.get("NLS_ATTN_SPLIT_WG", "256"))
 # split_chunk: 64 keys below 1K of context, 128 above)
 _MIN_CHUNK = int(os.environ.get("NLS_ATTN_MIN_CHUNK", "0"))
 # MoE: tokens per step above which the experts run as ONE grouped LDS-dequant GEMM launch (below: path-A
-# GEMVs over each expert's gathered rows)
+# GEMVs over each expert's gathered rows; few rows to an expert, on either side: path B, tuning.expert_heuristic)
 # (Mixtral-8x7B: B=64 15.2 vs 28.9 ms/step, B=32 15.2 vs 15.6, B=16 14.8 vs 9.7; round-2 sweep)
 _MOE_GEMM_T = int(os.environ.get("NLS_MOE_GEMM_T", "16"))
 # MoE decode at up to this many tokens (<= 4) fuses the FFN input RMSNorm, the router and the route
@@ -622,9 +622,15 @@ class LlamaModel:
         return False
 
     @staticmethod
-    def _moe_gemm_cfg(lw: LayerWeights, rows: int, n_exp: int):
+    def _moe_few_cfg(lw: LayerWeights, T: int, per: float):
+        """Launch configs (gate/up, down) of the expert products at few rows to an expert; {}: the caller's own."""
+        return tuple(dict(zip(("mode", "waves", "rt", "ks"), tuning.expert_heuristic(ws[:8], T, per) or ()))
+                     for ws in (lw.exp_gateup, lw.exp_down))
+
+    @staticmethod
+    def _moe_gemm_cfg(lw: LayerWeights, rows: int, n_exp: int, T: int = 0):
         """Launch configs (gate/up, down, down split-K) of the grouped expert GEMMs for `rows` routed rows
-        over `n_exp` experts."""
+        over `n_exp` experts (T: of so many tokens, 0: not known)."""
         if all(w.d16 is not None for w in lw.exp_gateup + lw.exp_down):
             # f16 expert copies (expand_dense tier 2): the dense DMA GEMM, bandwidth- rather than
             # dequant-bound at ~64 rows per expert (NLS_MOE_DENSE_GU/_DN = mode,waves,rt)
@@ -645,6 +651,8 @@ class LlamaModel:
             # ms/step vs 16.63 with mode 3 split 4 and 18.24 split 2 (profiles/moe_dma_r06.txt; the isolated
             # probe's 168 vs 285 us did not carry over -- the model's mode-2 down runs at ~144 us)
             gu = dict(mode=3, waves=4, rt=6, ks=1)
+        few = LlamaModel._moe_few_cfg(lw, T, rows / n_exp)
+        gu, dn = few[0] or gu, few[1] or dn
         if os.environ.get("NLS_MOE_QCFG_GU"):      # explicit (mode, waves, rt) overrides
             gu = dict(zip(("mode", "waves", "rt"), (int(v) for v in os.environ["NLS_MOE_QCFG_GU"].split(","))), ks=1)
         if os.environ.get("NLS_MOE_QCFG_DN"):
@@ -762,11 +770,13 @@ class LlamaModel:
         # rows in a 256-row block cost 64 rows of MFMA (Mixtral B=256, round-2 sweep: gate/up
         # rt 4 / down rt 4 = 19.6 ms/step, 4/2 = 20.7, 2/2 = 28.3, 1/1 = 43.0)
         gu = dn = {}
+        if not gemm and self.device.type == "cuda" and T * k >= len(self.experts):
+            gu, dn = self._moe_few_cfg(lw, T, T * k / E)
         if not gemm and len(_MOE_GEMV_DN) == 4:
             dn = dict(zip(("mode", "waves", "rt", "ks"), _MOE_GEMV_DN))
         dn_rows = T
         if gemm:
-            gu, dn, kdn = self._moe_gemm_cfg(lw, T * k, E)
+            gu, dn, kdn = self._moe_gemm_cfg(lw, T * k, E, T)
             # down projection (K = d_ff): split K over workgroups when ONE launch covers every routed row
             # (<= 8 local experts, no EP: every y row written by exactly one expert in every K slice);
             # the slabs are indexed by the y row, so that launch's M is the T*k output rows

@@ -86,6 +86,25 @@ def heuristic(segs, M: int):
     return (1, waves, rt, ks)
 
 
+def expert_heuristic(ws, T: int, per: float):
+    """Path B config of a grouped launch over the experts `ws` (<= 8) for T tokens, `per` routed rows to an expert, or None: path A (up
+    to 16 tokens) or the LDS-dequant GEMM. With few rows to an expert the launch is bound by the weights' bytes; path B streams
+    them through registers, skips an expert's unused activation tiles, and wins as soon as its grid covers the 256 CUs.
+    256 weight rows to a workgroup (us, path B / LDS-dequant GEMM / path A): Q5_K 8 x 8192 x 2048 at 8 / 24 / 64 / 96 tokens
+    22 / - / 31, 25 / 40 / 62, 28 / 39 / -, 28 / 42 / -; at 128 37 / 43 even routing, 55 / 53 skewed, so not there; Q4_K 8 x 28672 x 4096 at
+    24 tokens 107 / 197 / 237 (4 waves; with 8 waves 121: more than a workgroup to a CU). 64 weight rows: Q5_K 8 x 2048 x
+    4096 at 16 / 24 / 64 tokens 16 / - / 15, 17 / 31 / 25, 20 / 32 / -; Q4_K 8 x 4096 x 4096 at 8 / 24 / 64 18 / - / 21, 22 / 30 / 39, 25 / 32 / -."""
+    if T < 4 or not all(int(w.type) in (8, 12, 13, 14) for w in ws):
+        return None
+    big = sum((w.rows + 255) // 256 for w in ws)
+    if big >= 256 and T <= 128 and per < 32:
+        return (1, 4 if big > 256 and T <= 32 else 8, 2, 1)
+    small = sum((w.rows + 63) // 64 for w in ws)
+    if (small >= 512 and 4 < T <= 64) or (small >= 256 and 16 < T <= 64):
+        return (1, 4, 1, 1)
+    return None
+
+
 def dense_key(segs, M: int) -> str:
     return f"d:{sum(s.w.rows for s in segs)}:{segs[0].w.K}:{_mb(M)}"
 

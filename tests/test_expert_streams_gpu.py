@@ -1,0 +1,67 @@
+"""Grouped expert products at few rows to an expert (path B of the quantised GEMV: per-expert active tiles) and the rule that sends
+launches there."""
+import numpy as np
+import pytest
+import torch
+
+from nats_llm_studio_amd import ops
+from nats_llm_studio_amd.gguf import quants as Q
+from nats_llm_studio_amd.gguf.constants import GGMLType
+from nats_llm_studio_amd.ops import tuning
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves,rt", [(4, 1), (4, 2), (8, 2)])
+@pytest.mark.parametrize("counts", [(1, 0, 4), (16, 15, 9), (17, 16, 1, 0), (32, 31, 33, 16), (48, 17, 64, 0, 1), (47, 32, 90, 128)])
+@pytest.mark.parametrize("qt", [GGMLType.Q4_K, GGMLType.Q5_K, GGMLType.Q6_K, GGMLType.Q8_0])
+def test_active_tiles(gpu, waves, rt, counts, qt):
+    """Counts at the edges of the 16-row tiles, rows short of a workgroup's tile, a single super-block of K and an odd number. x and
+    the dequantised weights are f16 (a weight is rounded at most twice, d * q and its difference to the minimum), products are summed
+    in 32 bits: |error| <= 2^-9 sum |x| |w|."""
+    rng = np.random.default_rng(len(counts))
+    T = max(max(counts), 4)
+    for N, K in ((272, 256), (144, 1280)):
+        raw = [Q.random_blocks(qt, N * K, 0.05, rng) for _ in counts]
+        ws = [ops.QWeight(r, qt, N, K, gpu) for r in raw]
+        W = [ops.QWeight(r, qt, N, K, "cpu").dense().double() for r in raw]
+        x = torch.randn(T, K, device=gpu).to(ops.ACT_DTYPE)
+        xm = [torch.randperm(T)[:c] for c in counts]
+        y = torch.full((sum(counts) + 1, N), 3.0, device=gpu)
+        act = torch.full((sum(counts) + 1, N // 2), 3.0, device=gpu, dtype=ops.ACT_DTYPE)
+        segs, y0 = [], 0
+        for w, c, m in zip(ws, counts, xm):
+            pad = torch.zeros(T, dtype=torch.int32)
+            pad[:c] = m
+            ym = torch.zeros(T, dtype=torch.int32)
+            ym[:c] = torch.arange(y0, y0 + c)
+            segs.append(ops.Seg(w, 0, pad.to(gpu), ym.to(gpu), torch.tensor([c], dtype=torch.int32, device=gpu)))
+            y0 += c
+        ops.qgemv(segs, x, y, T, epi="f32", mode=1, waves=waves, rt=rt, ks=1)
+        ops.qgemv(segs, x, act, T, epi="swiglu", mode=1, waves=waves, rt=rt, ks=1)
+        xd, y0 = x.cpu().double(), 0
+        for c, m, w in zip(counts, xm, W):
+            ref, e = xd[m] @ w.t(), (xd[m].abs() @ w.abs().t()) * 2.0 ** -9
+            assert ((y[y0:y0 + c].cpu().double() - ref).abs() <= e).all()
+            g, u = (ref.view(c, N // 16, 2, 8)[:, :, i] for i in (0, 1))
+            eg, eu = (e.view(c, N // 16, 2, 8)[:, :, i] for i in (0, 1))
+            want = torch.nn.functional.silu(g) * u
+            bound = 1.1 * eg * (u.abs() + eu) + torch.nn.functional.silu(g).abs() * eu + want.abs() * 2.0 ** -10 + 2.0 ** -14
+            assert ((act[y0:y0 + c].cpu().double() - want.reshape(c, N // 2)).abs() <= bound.reshape(c, N // 2)).all()
+            y0 += c
+        assert (y[y0:] == 3.0).all() and (act[y0:] == 3.0).all()
+
+
+class _W:
+    def __init__(self, rows, type=12):
+        self.rows, self.type = rows, type
+
+
+def test_expert_rule():
+    """Path B only where its grid covers the chip, for the quantised types, and never above 128 tokens."""
+    up, small = [_W(8192)] * 8, [_W(2048)] * 8
+    assert [tuning.expert_heuristic(up, T, T / 4) for T in (1, 3, 4, 32, 128, 129)] == [None, None] + [(1, 8, 2, 1)] * 2 + [None] * 2
+    assert tuning.expert_heuristic([_W(28672)] * 8, 32, 8) == (1, 4, 2, 1) and tuning.expert_heuristic([_W(28672)] * 8, 33, 8.25) == (1, 8, 2, 1)
+    assert [tuning.expert_heuristic(small, T, T / 4) for T in (16, 17, 64, 65)] == [None, (1, 4, 1, 1), (1, 4, 1, 1), None]
+    assert tuning.expert_heuristic([_W(4096)] * 8, 5, 1.25) == (1, 4, 1, 1) and tuning.expert_heuristic([_W(4096)] * 8, 4, 1) is None
+    assert tuning.expert_heuristic([_W(8192)], 32, 8) is None and tuning.expert_heuristic([_W(8192, 1)] * 8, 32, 8) is None
+    assert tuning.expert_heuristic([_W(2048)] * 4 + [_W(2048, 99)] * 4, 32, 8) is None
