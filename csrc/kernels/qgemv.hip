@@ -259,7 +259,17 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
     for (int i = 0; i < nseg; ++i) rl.s[i] = RedSeg{sl.s[i].tile_begin_col, sl.s[i].rows, sl.s[i].ycol, 0};
     rl.nseg = nseg;
     const int nout = epi == EPI_SWIGLU ? cols / 2 : cols;
-    dim3 grid((nout + 255) / 256, M);
+    const size_t ysz = epi == EPI_ACT ? 2 : 4;
+    if (nseg == 1 && epi != EPI_SWIGLU && (((uintptr_t)ws) & 15) == 0 && cols % 4 == 0 &&
+        (epi == EPI_ARGMAX || (ldy % 4 == 0 && segs[0].ycol % 4 == 0 && ((uintptr_t)y) % (4 * ysz) == 0))) {
+      auto k = ks == 2 ? splitk_reduce4_kernel<2> : ks == 4 ? splitk_reduce4_kernel<4> : ks == 8 ? splitk_reduce4_kernel<8> : splitk_reduce4_kernel<0>;
+      hipLaunchKernelGGL(k, dim3((cols + 1023) / 1024, M), dim3(256), 0, st, (const float*)ws, ks, M, cols, segs[0].ycol, a);
+      return (int)hipGetLastError();
+    }
+    // with an arg-max every workgroup ends in an atomic on its row's key, all on neighbouring addresses: about 2048 workgroups in all
+    // (and no atomic for a key that is not larger) instead of one for every 256 columns (32 rows x 32000: 28 -> 16.5 us)
+    const int nwg = (nout + 255) / 256;
+    dim3 grid(argmax ? min(nwg, max(8, 2048 / M)) : nwg, M);
     hipLaunchKernelGGL(splitk_reduce_kernel, grid, dim3(256), 0, st, (const float*)ws, ks, M, cols, rl, a);
     return (int)hipGetLastError();
   }

@@ -353,6 +353,9 @@ def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: 
         if any(s.xmap is not None for s in segs) or M > 16:
             raise ValueError("fused-norm GEMV needs unmapped rows and M <= 16")
         cfg = gemv_config(segs, M)
+        if argmax is not None:
+            from . import tuning
+            cfg = tuning.argmax_config(cfg, segs, M)
         fz = _lib.NlsFuse(xf=xf.data_ptr(), ldxf=xf.stride(0), nw=nw.data_ptr(), eps=float(eps),
                           ssq_in=ssq.data_ptr(), ldss=int(ldss), nss_in=int(nparts))
         cands = [cfg] if cfg[0] in (0, 1) else []
@@ -409,6 +412,9 @@ def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: 
             raise ValueError(f"qgemv: M={M} rows but x has {x.shape[0]}, y {y.shape[0]}")
         if mode < 0 or waves == 0:
             mode, waves, rt, ks = gemv_config(segs, M) if not mapped else MOE_GEMV
+            if argmax is not None and not mapped:
+                from . import tuning
+                mode, waves, rt, ks = tuning.argmax_config((mode, waves, rt, ks), segs, M)
             if mode == 10 and (x.stride(0) % 8 or y.stride(0) % 4):
                 from . import tuning
                 mode, waves, rt, ks = tuning.dense_heuristic(segs, M, aligned=False)

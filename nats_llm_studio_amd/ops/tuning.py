@@ -105,6 +105,16 @@ def expert_heuristic(ws, T: int, per: float):
     return None
 
 
+def argmax_config(cfg, segs, M: int):
+    """Config of a launch with an arg-max: path B unsplit ends in an atomic for every 16 weight rows and token, all on M neighbouring
+    keys (32000 Q6_K rows, K = 4096, (1, 8, 1, 1): 62 us at 2 tokens, 108 at 8, 166 at 24, 248 at 64). Split in two, the reduce
+    takes the maximum with few atomics: 26, 28, 34, 47; at K = 2048 2 / 8 / 24 / 64 tokens 58 / 105 / 150 / 217 -> 18 / 20 /
+    25 / 34, one token 36 -> 19; on 16-row tiles, (1, 8, 1, 2), 24 / 26 / 30 / 36."""
+    if cfg[0] == 1 and 1 in cfg[2:] and M <= 64 and sum(s.w.rows for s in segs) >= 8192 and segs[0].w.K >= 1024:
+        return (1, 4 if M == 1 else 8, 2, 2)
+    return cfg
+
+
 def dense_key(segs, M: int) -> str:
     return f"d:{sum(s.w.rows for s in segs)}:{segs[0].w.K}:{_mb(M)}"
 

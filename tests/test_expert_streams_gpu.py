@@ -65,3 +65,29 @@ def test_expert_rule():
     assert tuning.expert_heuristic([_W(4096)] * 8, 5, 1.25) == (1, 4, 1, 1) and tuning.expert_heuristic([_W(4096)] * 8, 4, 1) is None
     assert tuning.expert_heuristic([_W(8192)], 32, 8) is None and tuning.expert_heuristic([_W(8192, 1)] * 8, 32, 8) is None
     assert tuning.expert_heuristic([_W(2048)] * 4 + [_W(2048, 99)] * 4, 32, 8) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 15, 17, 33, 64])
+@pytest.mark.parametrize("rows,K,qt", [(8192, 1024, GGMLType.Q6_K), (8209, 1280, GGMLType.Q4_K), (32000, 2048, GGMLType.Q8_0)])
+def test_head_argmax(gpu, M, rows, K, qt):
+    """A head's own config: split in two with the maxima from the reduce. The keys are those of the logits it stored (the lowest of
+    equal columns: every row of the second half is there twice), and a second launch into the same keys changes nothing."""
+    raw = Q.random_blocks(qt, rows * K, 0.05, np.random.default_rng(5)).reshape(rows, -1)
+    raw[rows // 2:2 * (rows // 2)] = raw[:rows // 2]
+    seg = [ops.Seg(ops.QWeight(raw.reshape(-1), qt, rows, K, gpu))]
+    assert tuning.argmax_config(ops.gemv_config(seg, M), seg, M)[3] > 1 or ops.gemv_config(seg, M)[0] != 1
+    x = torch.zeros(64, K, dtype=ops.ACT_DTYPE, device=gpu)
+    x[:M] = torch.randn(M, K, device=gpu)
+    y, only = (torch.zeros(64, rows, device=gpu) for _ in range(2))
+    keys, keys2 = (torch.zeros(64, dtype=torch.int64, device=gpu) for _ in range(2))
+    ids = torch.zeros(64, dtype=torch.int32, device=gpu)
+    for _ in range(2):
+        ops.qgemv(seg, x, y, M, argmax=keys)
+    ops.qgemv(seg, x, only, M, epi="argmax", argmax=keys2)
+    assert torch.equal(keys, keys2) and not only.any() and not keys[M:].any()
+    ops.argmax_unpack(keys, M, ids)
+    assert ids[:M].tolist() == y[:M].cpu().numpy().argmax(1).tolist()
+    W = ops.QWeight(raw.reshape(-1), qt, rows, K, "cpu").dense().double()
+    ref, bound = x[:M].cpu().double() @ W.t(), (x[:M].cpu().double().abs() @ W.abs().t()) * 2.0 ** -9
+    assert ((y[:M].cpu().double() - ref).abs() <= bound).all()
