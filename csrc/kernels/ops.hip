@@ -72,19 +72,37 @@ __global__ __launch_bounds__(512) void rmsnorm_kernel(const float* __restrict__ 
 #define NLS_SLAB_RUNTIME 0   // 1: always the runtime-ks kernels (A/B build tag)
 #endif
 // KS > 0: the split count as a constant -- every slab load of the row is issued before the first add (ks is a
-// runtime loop bound otherwise, and each slab's loads wait for the previous add chain); KS = 0: any ks.
-template <int KS>
+// runtime loop bound otherwise, and each slab's loads wait for the previous add chain); KS = 0: any ks (also none).
+// E > 0: the row is also routed (MoE: router logits of the f16 row, as router_logits_kernel multiplies them, then route_one),
+// one launch instead of three: at 32 rows the router and the route took 4.4 us each, behind 4.6 for this one. RT.counts: zeroed before.
+struct RouteArgs {
+  const act_t* wr; float* logits; float* topw; int *counts, *xrows, *yrows, *sel; int k, renorm, cap;
+};
+template <int KS, int E = 0>
 __global__ __launch_bounds__(512) void splitk_add_rmsnorm_kernel(const float* __restrict__ ws, int ks, int M,
                                                                  float alpha, float* __restrict__ x, long ldx,
                                                                  const float* __restrict__ w,
                                                                  act_t* __restrict__ out, long ldo, int D,
-                                                                 float eps) {
+                                                                 float eps, RouteArgs R) {
   __shared__ float sh[8];
   const int m = blockIdx.x;
   float* xr = x + (size_t)m * ldx;
   float4 v[4], wv[4];
   float ss = 0.f;
   const int nk = KS > 0 ? KS : ks;
+  typedef act_t act4 __attribute__((ext_vector_type(4)));
+  float acc_e[E > 0 ? E : 1];
+  act4 wr[E > 0 ? 4 : 1][E > 0 ? E : 1];       // the router's rows do not depend on x: their loads go first
+  if constexpr (E > 0) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc_e[e] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = (threadIdx.x + j * 512) * 4;
+#pragma unroll
+      for (int e = 0; e < E; ++e) wr[j][e] = i < D ? *reinterpret_cast<const act4*>(R.wr + (size_t)e * D + i) : act4{0, 0, 0, 0};
+    }
+  }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int i = (threadIdx.x + j * 512) * 4;
@@ -121,7 +139,6 @@ __global__ __launch_bounds__(512) void splitk_add_rmsnorm_kernel(const float* __
   ss = block_sum<512>(ss, sh);
   const float inv = rsqrtf(ss / (float)D + eps);
   act_t* o = out + (size_t)m * ldo;
-  typedef act_t act4 __attribute__((ext_vector_type(4)));
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int i = (threadIdx.x + j * 512) * 4;
@@ -130,9 +147,37 @@ __global__ __launch_bounds__(512) void splitk_add_rmsnorm_kernel(const float* __
       act4 r = {(act_t)(v[j].x * inv * ww.x), (act_t)(v[j].y * inv * ww.y), (act_t)(v[j].z * inv * ww.z),
                 (act_t)(v[j].w * inv * ww.w)};
       *reinterpret_cast<act4*>(o + i) = r;
+      if constexpr (E > 0) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          const act4 q = wr[j][e];
+          acc_e[e] += (float)r.x * (float)q.x + (float)r.y * (float)q.y + (float)r.z * (float)q.z + (float)r.w * (float)q.w;
+        }
+      }
+    }
+  }
+  if constexpr (E > 0) {
+    __shared__ float red[8][E], lg[E];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const float a = wave_sum(acc_e[e]);
+      if (lane == 0) red[wave][e] = a;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      if (lane < E) {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s += red[i][lane];
+        lg[lane] = s;
+        R.logits[(size_t)m * E + lane] = s;
+      }
+      route_one(lg, m, lane, E, R.k, R.renorm, R.topw, R.counts, R.xrows, R.yrows, R.cap, R.sel);
     }
   }
 }
+
 
 // f32 -> f32 variant (final norm feeding an fp32 reference / lm-head in f32)
 __global__ __launch_bounds__(256) void rmsnorm_f32_kernel(const float* __restrict__ x, long ldx,
@@ -640,8 +685,27 @@ int nls_splitk_add_rmsnorm(const float* ws, int ks, int M, float alpha, float* x
   auto k = kc == 2 ? splitk_add_rmsnorm_kernel<2> : kc == 3 ? splitk_add_rmsnorm_kernel<3>
          : kc == 4 ? splitk_add_rmsnorm_kernel<4> : kc == 1 ? splitk_add_rmsnorm_kernel<1> : splitk_add_rmsnorm_kernel<0>;
   hipLaunchKernelGGL(k, dim3(M), dim3(512), 0, (hipStream_t)stream, ws, ks, M, alpha, x, ldx, w, (act_t*)out, ldo, D,
-                     eps);
+                     eps, RouteArgs{});
   return (int)hipGetLastError();
+}
+
+// ks = 0: no slabs, x is normalised as it is. counts: int [E], zeroed; xrows / yrows: int [E][cap], cap >= M
+int nls_splitk_add_rmsnorm_route(const float* ws, int ks, int M, float alpha, float* x, long ldx, const float* w,
+                                 void* out, long ldo, int D, float eps, const void* wr, int E, int k, int renorm, float* logits,
+                                 float* topw, int* counts, int* xrows, int* yrows, int cap, int* sel, void* stream) {
+  if (M < 1 || D % 4 || D > 8192 || ks < 0 || (ks > 0 && !ws) || k < 1 || k > E || k > 8 || cap < M) return -1;
+  const RouteArgs R{(const act_t*)wr, logits, topw, counts, xrows, yrows, sel, k, renorm, cap};
+#define NLS_AR(EE)                                                                                                        \
+  if (E == EE) {                                                                                                          \
+    auto f = ks == 2 ? splitk_add_rmsnorm_kernel<2, EE> : ks == 4 ? splitk_add_rmsnorm_kernel<4, EE>                      \
+                                                                  : splitk_add_rmsnorm_kernel<0, EE>;                     \
+    hipLaunchKernelGGL(f, dim3(M), dim3(512), 0, (hipStream_t)stream, ws, ks, M, alpha, x, ldx, w, (act_t*)out, ldo, D,   \
+                       eps, R);                                                                                           \
+    return (int)hipGetLastError();                                                                                        \
+  }
+  NLS_AR(2) NLS_AR(4) NLS_AR(8)
+#undef NLS_AR
+  return -1;
 }
 
 int nls_rope_kv(const float* qkv, long ldqkv, int ks, long slab, const float* bias, const int* pos, const int* slot,

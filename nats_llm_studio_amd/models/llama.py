@@ -441,6 +441,7 @@ class LlamaModel:
                 rlogits=torch.zeros(pad, E, dtype=torch.float32, device=dev),
                 topw=torch.zeros(pad * k, dtype=torch.float32, device=dev),
                 counts=torch.zeros(E, dtype=torch.int32, device=dev),
+                lcounts=torch.zeros(len(self.layers), E, dtype=torch.int32, device=dev),
                 xrows=torch.zeros(E * pad, dtype=torch.int32, device=dev),
                 yrows=torch.zeros(E * pad, dtype=torch.int32, device=dev),
                 sel=torch.zeros(pad * k, dtype=torch.int32, device=dev),
@@ -487,6 +488,12 @@ class LlamaModel:
                  and ops.norm_fusable(T, cfg.d_model))
         if fnorm:
             return self._forward_fused_norm(b, kc, vc, T, block_size, n_split, logit_rows, n_logits, need_logits)
+        # more than _MOE_NORM_ROUTE_T tokens: the launch that sums up the o projection and normalises also routes; every layer's
+        # expert counts are zeroed here, by one launch
+        route = (cfg.n_expert and fused and x.is_cuda and T > _MOE_NORM_ROUTE_T and _ROUTER_KERNEL
+                 and all(lw.router16 is not None for lw in self.layers))
+        if route:
+            b.moe["lcounts"].zero_()
         fused_prev = True                       # layer 0's input norm is applied just below
         ops.rmsnorm(x, self.layers[0].attn_norm, b.h, T, cfg.eps)
         for L, lw in enumerate(self.layers):
@@ -502,7 +509,12 @@ class LlamaModel:
                               block_size, cfg.attn_softmax_scale, chunk=-_MIN_CHUNK, n_split=n_split, workspace=b.attn_ws,
                               counters=b.attn_cnt)
             moe_norm = fused and lw.router16 is not None and T <= _MOE_NORM_ROUTE_T
-            moe_routed = False
+            moe_routed, counts = False, None
+            if route:
+                m, counts = b.moe, b.moe["lcounts"][L]
+                moe_routed = ops.qgemv_add_rmsnorm_route(
+                    Seg(lw.wo), b.ao, x, lw.ffn_norm, b.h, T, cfg.residual_scale, cfg.eps, lw.router16, m["rlogits"],
+                    cfg.n_expert_used, m["topw"], counts, m["xrows"], m["yrows"], x.shape[0], sel=m["sel"])
             if moe_norm and _MOE_FOLD_ROUTE and x.is_cuda:
                 # the o projection's last workgroup applies the FFN norm, the router and the route
                 m = b.moe
@@ -527,7 +539,8 @@ class LlamaModel:
             fused_prev = False
             if cfg.n_expert:
                 fused_prev = self._moe(lw, b, T, nxt if (fused or self.ep_exchange) else None,
-                                       lw.ffn_norm if moe_norm and not moe_routed else None, routed=moe_routed)
+                                       lw.ffn_norm if moe_norm and not moe_routed else None, routed=moe_routed,
+                                       counts=counts if moe_routed else None)
             else:
                 ops.qgemv([Seg(lw.gateup)], b.h, b.act, T, epi="swiglu")
                 if fused:
@@ -736,7 +749,8 @@ class LlamaModel:
         return False
 
     def _moe(self, lw: LayerWeights, b: StepBuffers, T: int, next_norm: Optional[torch.Tensor] = None,
-             in_norm: Optional[torch.Tensor] = None, routed: bool = False) -> bool:
+             in_norm: Optional[torch.Tensor] = None, routed: bool = False,
+             counts: Optional[torch.Tensor] = None) -> bool:
         """Top-k routed experts: router GEMV -> route kernel (per-expert row lists on device)
         -> grouped expert GEMVs (tiles of experts with no routed rows exit before reading
         weights) -> deterministic weighted combine into the residual. `in_norm` (<= 4 tokens): b.h is
@@ -748,16 +762,17 @@ class LlamaModel:
         m = b.moe
         k, E = cfg.n_expert_used, cfg.n_expert
         cap = b.x.shape[0]
-        # routed: the o projection already normalised b.h and routed the tokens (ops.qgemv_add_norm_route)
+        counts = m["counts"] if counts is None else counts
+        # routed: the o projection already normalised b.h and routed the tokens (ops.qgemv_add_norm_route, .._rmsnorm_route)
         if in_norm is not None and not routed:
             use_sel = self.device.type == "cuda" and T * k < len(self.experts)
             routed = ops.moe_norm_route(b.x, in_norm, cfg.eps, lw.router16, b.h, m["rlogits"], T, k, m["topw"],
-                                        m["counts"], m["xrows"], m["yrows"], cap, sel=m["sel"] if use_sel else None)
+                                        counts, m["xrows"], m["yrows"], cap, sel=m["sel"] if use_sel else None)
             if not routed:
                 ops.rmsnorm(b.x, in_norm, b.h, T, cfg.eps)
         zeroed = False
         if not routed:
-            zeroed = self._router(lw, b.h, m["rlogits"], T, counts=m["counts"])
+            zeroed = self._router(lw, b.h, m["rlogits"], T, counts=counts)
         # few tokens: path-A GEMV over each expert's gathered rows; many tokens: ONE route and the
         # LDS-dequant GEMM (mode 2) over all experts, each m-block of an expert gathering its rows
         # through xrows and exiting when it lies past the expert's device-side count
@@ -795,10 +810,10 @@ class LlamaModel:
             # the EP exchange needs every (token, slot)'s expert: its owner rank pushes the row
             exch = self.ep_exchange and self.comm.oneshot.ep_ok(n * k, cfg.d_model)
             if not (routed and c0 == 0 and n == T):
-                ops.moe_route(m["rlogits"][c0:], n, k, m["topw"], m["counts"], m["xrows"], m["yrows"], cap,
+                ops.moe_route(m["rlogits"][c0:], n, k, m["topw"], counts, m["xrows"], m["yrows"], cap,
                               sel=m["sel"] if (use_sel or exch) else None, counts_zeroed=zeroed and c0 == 0)
             loc = list(zip(self.experts, lw.exp_gateup, lw.exp_down))
-            segs = [Seg(gu, 0, m["xrows"][e * cap:], m["yrows"][e * cap:], m["counts"][e:e + 1]) for e, gu, _ in loc]
+            segs = [Seg(gu, 0, m["xrows"][e * cap:], m["yrows"][e * cap:], counts[e:e + 1]) for e, gu, _ in loc]
 
             def sel(s0):
                 return (m["sel"], n * k, self.experts[0] + s0) if use_sel else None
@@ -806,7 +821,7 @@ class LlamaModel:
                 ops.qgemv(segs[s0:s0 + 8], b.h[c0:], b.act, n, epi="swiglu", sel=sel(s0), **gu)
             if self.ep and not exch:           # rows routed to other ranks' experts stay zero
                 m["yexp"][:n * k].zero_()
-            segs = [Seg(dn, 0, m["yrows"][e * cap:], m["yrows"][e * cap:], m["counts"][e:e + 1]) for e, _, dn in loc]
+            segs = [Seg(dn, 0, m["yrows"][e * cap:], m["yrows"][e * cap:], counts[e:e + 1]) for e, _, dn in loc]
             for s0 in range(0, len(segs), 8):
                 ops.qgemv(segs[s0:s0 + 8], b.act, m["yexp"], dn_rows if dn.get("ks", 1) > 1 else n, epi="f32",
                           sel=sel(s0), **dn)

@@ -532,6 +532,34 @@ def qgemv_add_rmsnorm(seg: Seg, xin: torch.Tensor, x: torch.Tensor, norm_w: torc
     return rmsnorm(x, norm_w, h, M, eps)
 
 
+def qgemv_add_rmsnorm_route(seg: Seg, xin: torch.Tensor, x: torch.Tensor, nw: torch.Tensor, h: torch.Tensor, M: int,
+                            alpha: float, eps: float, wr: torch.Tensor, logits: torch.Tensor, k: int, topw: torch.Tensor,
+                            counts: torch.Tensor, xrows: torch.Tensor, yrows: torch.Tensor, cap: int, renorm: bool = True,
+                            sel: Optional[torch.Tensor] = None) -> bool:
+    """qgemv_add_rmsnorm, then the router logits of the normalised rows (wr: the router's f16 copy [E, D]) and the top-k route
+    (moe_route) in the launch that normalises. `counts` [E] must be zero before. False (nothing done) where the launch does not apply:
+    the caller then runs qgemv_add_rmsnorm, router_logits and moe_route."""
+    E, D = wr.shape
+    if (not x.is_cuda or seg.xmap is not None or seg.ycol or seg.w.rows != x.shape[1] or D != x.shape[1] or E not in (2, 4, 8)
+            or k > E or D % 8 or D > 8192 or wr.dtype != ACT_DTYPE or not wr.is_contiguous() or logits.stride(0) != E or cap < M):
+        return False
+    mode, waves, rt, ks = gemv_config([seg], M)
+    st, L, ws = _stream_ptr(x), _lib.lib(), None
+    if mode == 0 or ks < 2:
+        ks = 0
+        qgemv([seg], xin, x, M, alpha=alpha, epi="add")
+    else:
+        ws = _workspace(x.device, ks * M * seg.w.rows).data_ptr()
+        arr = _seg_arr([seg], mode)
+        _lib.check(L.nls_qgemv(arr, 1, xin.data_ptr(), xin.stride(0), x.data_ptr(), x.stride(0), M, float(alpha), EPI["slabs"],
+                               None, waves, rt, mode, ks, ws, st), "nls_qgemv")
+    _lib.check(L.nls_splitk_add_rmsnorm_route(ws, ks, M, float(alpha), x.data_ptr(), x.stride(0), nw.data_ptr(), h.data_ptr(),
+                                              h.stride(0), D, float(eps), wr.data_ptr(), E, k, int(renorm), logits.data_ptr(),
+                                              topw.data_ptr(), counts.data_ptr(), xrows.data_ptr(), yrows.data_ptr(), cap,
+                                              _p(sel), st), "nls_splitk_add_rmsnorm_route")
+    return True
+
+
 def qgemv_add_norm_route(seg: Seg, xin: torch.Tensor, x: torch.Tensor, nw: torch.Tensor, h: torch.Tensor, M: int,
                          alpha: float, eps: float, counter: torch.Tensor, wr: torch.Tensor, logits: torch.Tensor, k: int,
                          topw: torch.Tensor, counts: torch.Tensor, xrows: torch.Tensor, yrows: torch.Tensor, cap: int,

@@ -91,3 +91,40 @@ def test_head_argmax(gpu, M, rows, K, qt):
     W = ops.QWeight(raw.reshape(-1), qt, rows, K, "cpu").dense().double()
     ref, bound = x[:M].cpu().double() @ W.t(), (x[:M].cpu().double().abs() @ W.abs().t()) * 2.0 ** -9
     assert ((y[:M].cpu().double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,D,E,k", [(5, 256, 4, 2), (24, 2048, 8, 2), (33, 1280, 2, 1), (64, 4096, 8, 8), (70, 512, 8, 3)])
+@pytest.mark.parametrize("ksplit", [0, 2, 3, 4])
+def test_add_rmsnorm_route(gpu, monkeypatch, M, D, E, k, ksplit):
+    """Projection, residual, norm and route in one call: the rows as qgemv_add_rmsnorm leaves them, and the lists, weights and experts
+    moe_route makes of the logits it reports; those are the f16 rows' products in 32 bits (|error| <= D 2^-24 sum |h| |w|)."""
+    rng = np.random.default_rng(3)
+    raw = Q.random_blocks(GGMLType.Q4_K, D * 1280, 0.05, rng)
+    seg = ops.Seg(ops.QWeight(raw, GGMLType.Q4_K, D, 1280, gpu))
+    monkeypatch.setattr(ops, "gemv_config", lambda segs, M: (1, 8, 1, ksplit) if ksplit else (0, 4, 1, 1))
+    xin, h, h2 = torch.zeros(128, 1280, dtype=ops.ACT_DTYPE, device=gpu), *(torch.zeros(128, D, dtype=ops.ACT_DTYPE, device=gpu) for _ in range(2))
+    xin[:M] = torch.randn(M, 1280, device=gpu)
+    x = torch.randn(128, D, device=gpu)
+    x2, nw = x.clone(), torch.rand(D, device=gpu) + 0.5
+    wr = (torch.randn(E, D, device=gpu) * 0.1).to(ops.ACT_DTYPE)
+    cap = M + 3
+
+    def state():
+        return dict(logits=torch.zeros(128, E, device=gpu), topw=torch.zeros(128 * k, device=gpu),
+                    counts=torch.zeros(E, dtype=torch.int32, device=gpu), xrows=torch.full((E * cap,), -1, dtype=torch.int32, device=gpu),
+                    yrows=torch.full((E * cap,), -1, dtype=torch.int32, device=gpu), sel=torch.zeros(128 * k, dtype=torch.int32, device=gpu))
+    a, b = state(), state()
+    assert ops.qgemv_add_rmsnorm_route(seg, xin, x, nw, h, M, 0.7, 1e-5, wr, a["logits"], k, a["topw"], a["counts"], a["xrows"], a["yrows"],
+                                       cap, sel=a["sel"])
+    ops.qgemv_add_rmsnorm(seg, xin, x2, nw, h2, M, 0.7, 1e-5)
+    assert torch.equal(x, x2) and (h.float() - h2.float()).abs().max() <= 2.0 ** -10 * h2.float().abs().max()
+    hd, wd = h[:M].cpu().double(), wr.cpu().double()
+    assert ((a["logits"][:M].cpu().double() - hd @ wd.t()).abs() <= D * 2.0 ** -24 * (hd.abs() @ wd.abs().t())).all()
+    ops.moe_route(a["logits"], M, k, b["topw"], b["counts"], b["xrows"], b["yrows"], cap, sel=b["sel"])
+    for n in ("topw", "counts", "sel"):
+        assert torch.equal(a[n], b[n])
+    for n in ("xrows", "yrows"):
+        assert torch.equal(a[n].view(E, cap).sort(1).values, b[n].view(E, cap).sort(1).values)
+    assert not ops.qgemv_add_rmsnorm_route(seg, xin, x, nw, h, M, 0.7, 1e-5, wr[:1], a["logits"][:, :1], 1, a["topw"], a["counts"], a["xrows"],
+                                           a["yrows"], cap)
