@@ -41,8 +41,9 @@ __global__ __launch_bounds__(256) void shift_mix_kernel(Mix p) {
   }
 }
 
-// DP: key channels padded to a multiple of 32 (zeros past D)
-template <typename T, int DP, int PARTS, int CPL>
+// DP: key channels padded to a multiple of 32 (zeros past D). VEC: D = DP and 16-byte aligned rows (8 values of an operand's row to
+// a thread: a quarter of the loads' addresses; 3500 tokens, 32 heads of 64: 433 -> 355 us)
+template <typename T, int DP, int PARTS, int CPL, bool VEC>
 __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
   constexpr int WC = 256 / PARTS * CPL;          // value columns per workgroup
   constexpr int CH = DP <= 64 ? 32 : (DP <= 128 ? 16 : 8);   // tokens per staged chunk
@@ -81,40 +82,74 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
     const int i = (threadIdx.x & 15) + 16 * q;
     ur[q] = i < D ? p.u[hb + i] : 0.f;
   }
-  float fr[NV], fk[NV], fw[NV], fv[(CH * WC + 255) / 256];
-  auto fetch = [&](int base) __attribute__((always_inline)) {
+  // these loads have arrived before the first chunk's go out: the loop over tokens would wait for all loads in flight otherwise
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      const int e = threadIdx.x + q * 256, tt = e / DP, i = e % DP;
-      const bool in = tt < CH && base + tt < n && i < D;
-      const size_t row = (size_t)(t0 + min(base + tt, n - 1));
-      fr[q] = in ? ld1(rp + row * p.ld + i) : 0.f;
-      fk[q] = in ? ld1(kp + row * p.ld + i) : 0.f;
-      fw[q] = in ? wp[row * p.ldw + i] : 0.f;
+  for (int c = 0; c < CPL; ++c)
+#pragma unroll
+    for (int i = 0; i < R; ++i) asm volatile("" : "+v"(S[c][i]));
+#pragma unroll
+  for (int q = 0; q < DP / 16; ++q) asm volatile("" : "+v"(ur[q]));
+  // the next chunk, as it lies in memory: no branch and no conversion, which would wait for the load, until it is staged (3500
+  // tokens, 32 heads of 64: 748 us with a branch around each load, 10 round trips to memory a chunk; 433 without)
+  constexpr int NU = (CH * WC + 255) / 256;
+  typedef T tv8 __attribute__((ext_vector_type(8), aligned(16)));
+  typedef float fv8 __attribute__((ext_vector_type(8), aligned(16)));
+  static_assert(!VEC || (CH * DP == 2048 && CH * WC <= 2048), "8 values to a thread");
+  T fr[VEC ? 1 : NV], fk[VEC ? 1 : NV], fv[VEC ? 1 : NU];
+  float fw[VEC ? 1 : NV];
+  tv8 r8, k8, v8;
+  fv8 w8;
+  const int et = threadIdx.x / (DP / 8), ei = threadIdx.x % (DP / 8) * 8;                               // VEC: a thread's token and keys
+  const int vt = threadIdx.x % (CH * WC / 8) / (WC / 8), vi = threadIdx.x % (WC / 8) * 8;                 // and token and columns
+  auto fetch = [&](int base) __attribute__((always_inline)) {
+    if constexpr (VEC) {
+      const size_t row = t0 + min(base + et, n - 1), vrow = t0 + min(base + vt, n - 1);
+      r8 = *reinterpret_cast<const tv8*>(rp + row * p.ld + ei);
+      k8 = *reinterpret_cast<const tv8*>(kp + row * p.ld + ei);
+      w8 = *reinterpret_cast<const fv8*>(wp + row * p.ldw + ei);
+      v8 = *reinterpret_cast<const tv8*>(vp + vrow * p.ld + c0 + vi);
+      return;
     }
 #pragma unroll
-    for (int q = 0; q < (CH * WC + 255) / 256; ++q) {
-      const int e = threadIdx.x + q * 256, tt = e / WC, i = c0 + (e & (WC - 1));
-      const bool in = tt < CH && base + tt < n && i < D;
-      fv[q] = in ? ld1(vp + (size_t)(t0 + min(base + tt, n - 1)) * p.ld + i) : 0.f;
+    for (int q = 0; q < NV; ++q) {
+      const int e = threadIdx.x + q * 256, tt = e / DP, i = min(e % DP, D - 1);
+      const size_t row = (size_t)(t0 + min(base + tt, n - 1));
+      fr[VEC ? 0 : q] = rp[row * p.ld + i];
+      fk[VEC ? 0 : q] = kp[row * p.ld + i];
+      fw[VEC ? 0 : q] = wp[row * p.ldw + i];
+    }
+#pragma unroll
+    for (int q = 0; q < NU; ++q) {
+      const int e = threadIdx.x + q * 256, tt = e / WC, i = min(c0 + (e & (WC - 1)), D - 1);
+      fv[VEC ? 0 : q] = vp[(size_t)(t0 + min(base + tt, n - 1)) * p.ld + i];
     }
   };
   fetch(0);
   for (int base = 0; base < n; base += CH) {
     __syncthreads();
+    if constexpr (VEC) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      const int e = threadIdx.x + q * 256, tt = e / DP, i = e % DP;
-      if (tt < CH) {
-        rs[tt][i] = fr[q];
-        ks[tt][i] = fk[q];
-        ws[tt][i] = fw[q];
+      for (int h = 0; h < 8; h += 4) {
+        *reinterpret_cast<f32x4*>(&rs[et][ei + h]) = f32x4{(float)r8[h], (float)r8[h + 1], (float)r8[h + 2], (float)r8[h + 3]};
+        *reinterpret_cast<f32x4*>(&ks[et][ei + h]) = f32x4{(float)k8[h], (float)k8[h + 1], (float)k8[h + 2], (float)k8[h + 3]};
+        *reinterpret_cast<f32x4*>(&ws[et][ei + h]) = f32x4{w8[h], w8[h + 1], w8[h + 2], w8[h + 3]};
+        *reinterpret_cast<f32x4*>(&vs[vt][vi + h]) = f32x4{(float)v8[h], (float)v8[h + 1], (float)v8[h + 2], (float)v8[h + 3]};
       }
-    }
+    } else {
 #pragma unroll
-    for (int q = 0; q < (CH * WC + 255) / 256; ++q) {
-      const int e = threadIdx.x + q * 256;
-      if (e < CH * WC) vs[e / WC][e & (WC - 1)] = fv[q];
+      for (int q = 0; q < NV; ++q) {
+        const int e = threadIdx.x + q * 256, tt = e / DP, i = e % DP;
+        if (tt < CH) {
+          rs[tt][i] = i < D ? (float)fr[VEC ? 0 : q] : 0.f;
+          ks[tt][i] = i < D ? (float)fk[VEC ? 0 : q] : 0.f;
+          ws[tt][i] = i < D ? fw[VEC ? 0 : q] : 0.f;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < NU; ++q) {
+        const int e = threadIdx.x + q * 256;
+        if (e < CH * WC) vs[e / WC][e & (WC - 1)] = c0 + (e & (WC - 1)) < D ? (float)fv[VEC ? 0 : q] : 0.f;
+      }
     }
     __syncthreads();
     if (base + CH < n) fetch(base + CH);
@@ -126,15 +161,17 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
       if (tt < CH)
 #pragma unroll
         for (int q = 0; q < DP / 16; ++q) a += rs[tt][l + 16 * q] * ur[q] * ks[tt][l + 16 * q];
-#pragma unroll
-      for (int s = 8; s > 0; s >>= 1) a += __shfl_xor(a, s, 64);
+      // (row rotations: the exchanges of a butterfly over 16 lanes without the LDS round trips)
+      a = dpp_add<0x121>(dpp_add<0x122>(dpp_add<0x124>(dpp_add<0x128>(a))));
       if (tt < CH && l == 0) ruk[tt] = a;
     }
     __syncthreads();
-    // 8 tokens at a time, the next token's operands on their way while one is summed; lane part q keeps token q's output
+    // 8 tokens at a time, the next PF tokens' operands on their way while one is summed (a token's arithmetic takes less than
+    // an LDS read); lane part q keeps token q's output
+    constexpr int PF = R <= 4 ? 3 : 1, RB = PF + 1;
     const int m = min(CH, n - base);
-    f32x4 r4[2][R / 4], k4[2][R / 4], w4[2][R / 4];
-    float v1[2][CPL];
+    f32x4 r4[RB][R / 4], k4[RB][R / 4], w4[RB][R / 4];
+    float v1[RB][CPL];
     auto get = [&](int tt, int b) __attribute__((always_inline)) {
 #pragma unroll
       for (int q = 0; q < R / 4; ++q) {
@@ -162,7 +199,8 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
         o[c] = sum_parts<PARTS>(o0 + o1);
       }
     };
-    get(0, 0);
+#pragma unroll
+    for (int i = 0; i < PF; ++i) get(i, i);
     for (int t8 = 0; t8 < m; t8 += 8) {
       float mine[CPL], o[CPL];
 #pragma unroll
@@ -172,17 +210,17 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
       if (last >= 7) {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          get(min(t8 + q + 1, CH - 1), (q & 1) ^ 1);
-          token(q & 1, o);
+          get(min(t8 + q + PF, CH - 1), (q + PF) % RB);
+          token(q % RB, o);
 #pragma unroll
           for (int c = 0; c < CPL; ++c) mine[c] = part == q ? o[c] : mine[c];
         }
       } else {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          get(min(t8 + q + 1, CH - 1), (q & 1) ^ 1);
+          get(min(t8 + q + PF, CH - 1), (q + PF) % RB);
           if (q > last) continue;              // (uniform)
-          token(q & 1, o);
+          token(q % RB, o);
 #pragma unroll
           for (int c = 0; c < CPL; ++c) mine[c] = part == q ? o[c] : mine[c];
         }
@@ -206,14 +244,24 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
     p.prev[(size_t)slot * p.ldp + i] = p.x[(size_t)(t0 + n - 1) * p.ldx + i];
 }
 
+template <typename T, int DP, int PARTS>
+int scan_v(const Scan& p, int nruns, hipStream_t st) {
+  const dim3 grid(p.H * ((p.V + 256 / PARTS - 1) / (256 / PARTS)), nruns);
+  if constexpr (DP >= 64) {
+    auto whole = [](const void* q, long ld, size_t size) { return (uintptr_t)q % 16 == 0 && ld * size % 16 == 0; };
+    if (p.D == DP && whole(p.r, p.ld, sizeof(T)) && whole(p.k, p.ld, sizeof(T)) && whole(p.v, p.ld, sizeof(T)) && whole(p.w, p.ldw, 4)) {
+      hipLaunchKernelGGL((wkv_scan_kernel<T, DP, PARTS, 1, true>), grid, dim3(256), 0, st, p);
+      return (int)hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((wkv_scan_kernel<T, DP, PARTS, 1, false>), grid, dim3(256), 0, st, p);
+  return (int)hipGetLastError();
+}
+
 template <typename T, int DP>
 int scan_d(const Scan& p, int nruns, hipStream_t st) {
-  auto grid = [&](int wc) { return dim3(p.H * ((p.V + wc - 1) / wc), nruns); };
-  if (DP < 64 || p.H * nruns * ((p.V + 31) / 32) >= 256)
-    hipLaunchKernelGGL((wkv_scan_kernel<T, DP, 8, 1>), grid(32), dim3(256), 0, st, p);
-  else
-    hipLaunchKernelGGL((wkv_scan_kernel<T, DP, DP < 64 ? 8 : 16, 1>), grid(16), dim3(256), 0, st, p);
-  return (int)hipGetLastError();
+  if (DP < 64 || p.H * nruns * ((p.V + 31) / 32) >= 256) return scan_v<T, DP, 8>(p, nruns, st);
+  return scan_v<T, DP, DP < 64 ? 8 : 16>(p, nruns, st);
 }
 
 template <typename T>

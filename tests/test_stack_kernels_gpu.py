@@ -205,3 +205,53 @@ def test_rows_to_host(K, n):
             Engine._rows_to_host(eng, rows, dst)
             assert (dst == rows.cpu()).all()
     assert len(eng._stage[0][0]) == 7
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D", [60, 64, 128, 256])
+def test_wkv_scan_loads(K, dt, D):
+    """Runs around a staged chunk's 8 to 32 tokens, one that starts from a state, few heads and enough for the other split: rows on
+    16-byte boundaries (8 values to a thread where D is the padded width) and rows that are not give the same bits, and so does
+    a run in two pieces; against 64 bits sums of a run's n D products, each rounded a few times: 2^-24 (n + D) sums of their magnitudes."""
+    H = 2 if D != 64 else 9
+    lens, pos0 = [1, 31, 32, 33, 70, 40], [0, 0, 0, 0, 0, 5]
+    n = sum(lens)
+    r, k, v = (rnd(n, H * D, seed=i).to(dt) * 0.3 for i in range(3))
+    w, u = torch.sigmoid(rnd(n, H * D, seed=4)).float(), rnd(H * D, seed=5).float()
+    S0 = rnd(len(lens), H * D * D, seed=6).float() * 0.3
+
+    def put(x, off):
+        ld = H * D + (1 if off else 8)
+        flat = torch.zeros(n * ld + 8, dtype=x.dtype, device="cuda")
+        t = flat[off:off + n * ld].view(n, ld)[:, :H * D]
+        t.copy_(x)
+        return t
+
+    def run(off, pieces):
+        S, prev, x = S0.cuda(), torch.zeros(len(lens), 8, device="cuda"), torch.zeros(n, 8, device="cuda")
+        o = torch.zeros(n, H * D, device="cuda")
+        for lo, hi in pieces:
+            rows, t = [], 0
+            for s, (m, p) in enumerate(zip(lens, pos0)):
+                a, b = int(m * lo), int(m * hi)
+                rows.append([t + a, b - a, s, p + a])
+                t += m
+            K.wkv_scan(put(r, off), put(k, off), put(v, off), put(w, off), u.cuda(), o, S, x, prev,
+                       torch.tensor(rows, dtype=torch.int32).cuda(), len(lens), H, D, st())
+        return o.cpu(), S.cpu()
+    o, S = run(0, [(0, 1)])
+    for off, pieces in ((1, [(0, 1)]), (0, [(0, 0.5), (0.5, 1)]), (1, [(0, 0.3), (0.3, 1)])):
+        o1, S1 = run(off, pieces)
+        assert torch.equal(o, o1) and torch.equal(S, S1)
+    t = 0
+    for s, m in enumerate(lens):
+        rr, kk, vv, ww = (x[t:t + m].double().view(m, H, D) for x in (r, k, v, w))
+        uu = u.double().view(H, D, 1)
+        Sd, Sa = (S0[s].double().view(H, D, D) * (pos0[s] > 0) for _ in range(2))
+        Sa = Sa.abs()
+        for i in range(m):
+            kv = kk[i][:, :, None] * vv[i][:, None, :]
+            want, mag = ((Sd + uu * kv) * rr[i][:, :, None]).sum(1), ((Sa + uu.abs() * kv.abs()) * rr[i].abs()[:, :, None]).sum(1)
+            assert ((o[t + i].double().view(H, D) - want).abs() <= 2.0 ** -24 * (i + D + 8) * mag).all()
+            Sd, Sa = ww[i][:, :, None] * Sd + kv, ww[i][:, :, None] * Sa + kv.abs()
+        t += m
