@@ -67,9 +67,9 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(lglds));
   const uint32_t wl = base + (uint32_t)(NW * wave) * 1024u;
   const uint32_t xl = base + G::WST + (uint32_t)(NX * wave) * 1024u;
-  auto dma = [&](int j) __attribute__((always_inline)) {     // step j (clamped) -> stage j % NST
+  auto dma = [&](int j, int stage) __attribute__((always_inline)) {     // step j (clamped) -> stage
     const int jc = jb + min(j, nst - 1);
-    const uint32_t so = (uint32_t)(j % NST) * G::STG;
+    const uint32_t so = (uint32_t)stage * G::STG;
 #pragma unroll
     for (int i = 0; i < NW; ++i) glds16(wsrc[i] + (size_t)jc * 2048, wl + so + i * 1024);
 #pragma unroll
@@ -81,9 +81,9 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
 #pragma unroll
     for (int j = 0; j < MTW; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int xfo = r * 64 + ((g ^ lin_swz(r)) << 4);
-  auto step = [&](int j) __attribute__((always_inline)) {
-    const uint8_t* wb = lglds + (j % NST) * G::STG + lane * 16;
-    const uint8_t* xb = lglds + (j % NST) * G::STG + G::WST + xfo;
+  auto step = [&](int stage) __attribute__((always_inline)) {
+    const uint8_t* wb = lglds + stage * G::STG + lane * 16;
+    const uint8_t* xb = lglds + stage * G::STG + G::WST + xfo;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       u32x4 A[NTW], B[MTW];
@@ -99,17 +99,25 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   };
   constexpr int FL = (NST - 2) * (NW + NX);           // DMA instructions left in flight across the barrier
 #pragma unroll
-  for (int j = 0; j < NST - 1; ++j) dma(j);
+  for (int j = 0; j < NST - 1; ++j) dma(j, j);
   wait_vm_lgkm0<FL>();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  for (int j = 0; j < nst; ++j) {
-    dma(j + NST - 1);                                 // that stage was last read in step j - 1: retired
-    step(j);
+  // step j is in stage j % NST: NST steps to a pass of the loop, so that stages are constants and the accumulators stay where they are
+  auto turn = [&](int j, int stage) __attribute__((always_inline)) {
+    dma(j + NST - 1, (stage + NST - 1) % NST);        // that stage was last read in step j - 1: retired
+    step(stage);
     wait_vm_lgkm0<FL>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-  }
+  };
+  int j0 = 0;
+  for (; j0 + NST <= nst; j0 += NST)
+#pragma unroll
+    for (int s = 0; s < NST; ++s) turn(j0 + s, s);
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (j0 + s < nst) turn(j0 + s, s);                // (uniform)
   wait_vm_lgkm0<0>();                                 // the clamped tail DMAs land before the workgroup's LDS is freed
 #pragma unroll
   for (int j = 0; j < MTW; ++j) {
@@ -143,7 +151,7 @@ template <typename T>
 int gemm_d(LinArgs& a, int cfg, hipStream_t st) {
   switch (cfg) {
     case 0: return gemm_t<T, 64, 64, 2, 2, 3>(a, st);
-    case 1: return gemm_t<T, 128, 64, 4, 1, 2>(a, st);
+    case 1: return gemm_t<T, 128, 64, 4, 1, 3>(a, st);
     case 2: return gemm_t<T, 128, 128, 2, 2, 2>(a, st);
     case 3: return gemm_t<T, 256, 128, 4, 2, 3>(a, st);
     case 4: return gemm_t<T, 256, 256, 4, 2, 2>(a, st);

@@ -195,13 +195,17 @@ GEMM_TILES = ((64, 64), (128, 64), (128, 128), (256, 128), (256, 256), (64, 64),
 # against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 298 against 262 (3).
 GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 0.47, 0.72),
              1: (512, 0.5, 0.63), 0: (1024, 0.45, 0.55)}
-# 32-bit operands: f32 MFMAs leave LDS and waits behind, the small tile loses little and wastes least (900 x 2048 x 7680: 280 us against
-# 488 on 128 x 64 and 703 on 192 x 128; 1500 x 35888 x 4096: 3573 against 3584 on 256 x 128 and 3415 on 192 x 128)
-GEMM_RATE_F32 = {6: (0, 1.0, 1.0), 0: (0, 0.9, 0.9)}
+# 32-bit operands: bound by the f32 MFMAs (75 to 80 % of the time in any tile), so the rounds decide (64 x 64 / 128 x 64 / 192 x 128 / 256 x 128):
+# 900 x 20096 x 2048 727 / 658 / 756 / 771 us, 300 rows 257 / 267 / 377 / 259, 1500 1059 / 987 / - / 1036, 900 x 2048 x 9728 333 / 337 / 868 / 1160.
+GEMM_RATE_F32 = {6: (0, 1.0, 1.0), 3: (0, 0.98, 0.98), 1: (0, 0.955, 0.955), 0: (0, 0.865, 0.865)}
+
+# Launches of 129 to 512 rows that do not fill the chip with 256 x 128 tiles (weight rows x rows of a round by its time): 300 x 4096 x 4096 28 us
+# on 96 x 64, 34 on 64 x 64, 46 on 192 x 128; 200 x 6144 x 4096 27, 32, 49; 160 x 10240 x 4096 45, 37, 47; 400 x 6144 x 2048 27, 29, 29, 28 on 96 x 128.
+GEMM_RATE_MID = {8: (0, 0.47, 0.47), 0: (0, 0.51, 0.51), 11: (0, 0.655, 0.655), 6: (0, 1.1, 1.1)}
 
 
 # Microseconds of a round of 256 workgroups of a tile: fixed + per input column (from rounds at K = 1024 .. 17408)
-ROUND_US = {7: (8.0, 0.0215), 3: (8.0, 0.0151), 6: (8.0, 0.0112)}
+ROUND_US = {7: (8.0, 0.0215), 3: (8.0, 0.0151), 6: (8.0, 0.0112), 10: (5.0, 0.0075)}
 
 
 class LinLaunch:
@@ -268,8 +272,11 @@ class LinLaunch:
             cand = list(rate)
         elif self._tiles(256, 128, M) >= 120:
             cand = [3, 6, 7]
+        elif n64 <= 256:
+            return True, 5
         else:
-            return True, (5 if n64 <= 256 else 0)
+            rate = GEMM_RATE_MID
+            cand = list(rate)
         if 7 in cand and min(s.w.nsub for s in self.segs) < 6:      # (its DMA runs two steps ahead)
             cand.remove(7)
 
@@ -297,7 +304,8 @@ class LinLaunch:
         return True, self.balanced(M)
 
     def split_config(self, M: int):
-        """(config, K splits) of a launch that may split K: about 512 workgroups of 64 x 64 tiles, or 256 of 256 x 128."""
+        """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 25 in two
+        of 128 x 64)."""
         n16 = self._tiles(16, 16, M)
         if M <= 16:
             rt = 1 if M <= 8 else 2
@@ -305,22 +313,30 @@ class LinLaunch:
         if M <= 32:
             return (False, 2, 4, 4 if n16 >= 256 else 2), 8
         big, small = self._tiles(256, 128, M), self._tiles(64, 64, M)
-        if M > 128 and big * 8 >= 256:
-            return (True, 3), -(-256 // big)
-        return (True, 0), -(-512 // small)
+        if self.f32 or small > 256:
+            return ((True, 3), -(-256 // big)) if M > 128 and big * 8 >= 256 else ((True, 0), -(-512 // small))
+        if M <= 64:                       # one workgroup to a CU, 8 stages in flight: 64 x 4096 x 17408 34 us in 8 splits of 64 x 64 with
+            return (True, 5), 256 // small                                      # three, 31 in 4 (and half the slabs), 40 x 4096 x 9216 19, 18
+        c, ks = self.cheapest(M, self.segs[0].slabs)
+        return (True, c), ks
 
-    def tall_split(self, M: int):
-        """(config, K splits) of more rows than slab_rows: as many slabs of M rows as y holds. A narrow product has fewer tiles than
-        there are CUs, or lasts two rounds for a few more; each further slab is written and read again (about 4 TB/s). 2000 x 4096 x
-        17408: 286 us in one round of 256 x 128 -> 222 in two splits of 256 x 256; the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
+    def cheapest(self, M: int, most: int):
+        """(config, splits) of the least time for a launch with up to `most` slabs of K; each further slab is written and read again (about
+        4 TB/s)."""
         s = self.segs[0]
-        most = min(s.slabs, s.y.shape[0] // M, s.w.nsub // 16)
 
         def us(c, ks):
             fixed, per = ROUND_US[c]
             rounds = -(-self._tiles(*GEMM_TILES[c], M) * ks // 256)
             return rounds * (fixed + per * s.w.K / ks) + (ks - 1) * M * s.w.N * 2e-6
-        c, ks = min(((c, ks) for c in ROUND_US for ks in range(1, most + 1)), key=lambda v: us(*v))
+        return min(((c, ks) for c in ROUND_US for ks in range(1, max(1, min(most, s.w.nsub // 16)) + 1)), key=lambda v: us(*v))
+
+    def tall_split(self, M: int):
+        """(config, K splits) of more rows than slab_rows: as many slabs of M rows as y holds. A narrow product has fewer tiles than
+        there are CUs, or lasts two rounds for a few more. 2000 x 4096 x 17408: 286 us in one round of 256 x 128 -> 222 in two splits of
+        256 x 256; the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
+        s = self.segs[0]
+        c, ks = self.cheapest(M, min(s.slabs, s.y.shape[0] // M))
         return ((True, c), ks) if ks > 1 else (self.config(M), 1)
 
     def run(self, M: int, st: int) -> int:

@@ -255,3 +255,46 @@ def test_wkv_scan_loads(K, dt, D):
             assert ((o[t + i].double().view(H, D) - want).abs() <= 2.0 ** -24 * (i + D + 8) * mag).all()
             Sd, Sa = ww[i][:, :, None] * Sd + kv, ww[i][:, :, None] * Sa + kv.abs()
         t += m
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 5, 6, 8, 9, 10, 11])
+def test_tile_steps(K, cfg, f32):
+    """One to nineteen steps of K: fewer than the tile's stages, whole passes of them and every remainder, whole and in two splits. The
+    products are summed in 32 bits: |error| <= 2^-24 K sum |x| |w|."""
+    import ctypes
+    M, N = 70, 200
+    for steps in range(1, 20):
+        Kd = steps * (32 if f32 else 64) - 3
+        dt = torch.float32 if f32 else torch.bfloat16
+        x, w = (rnd(n, Kd, seed=i).to(dt) for i, n in ((steps, M), (50, N)))
+        xa = torch.zeros(M, K.act_ld(Kd), dtype=dt, device="cuda")
+        xa[:, :Kd] = x
+        y = torch.full((2 * M, N), 9.0, device="cuda")
+        p = K.PackedLinear(w, f32, "cuda")
+        a = K.LinLaunch([K.Seg(p, xa, y, slabs=2, slab_rows=M)]).a
+        a.s[0].M = M
+        want, bound = x.double() @ w.double().T, 2.0 ** -24 * (Kd + 8) * (x.double().abs() @ w.double().abs().T)
+        for ks in (1, 2)[:min(2, p.nsub // 2)]:
+            a.s[0].ks = ks
+            K._check(K.lib().nls_lin_gemm(ctypes.byref(a), int(f32), cfg, st()), "gemm")
+            got = y.view(2, M, N)[:ks].sum(0).cpu().double()
+            assert ((got - want).abs() <= bound + 2.0 ** -23 * want.abs()).all(), (steps, ks)
+
+
+def test_split_rule():
+    """Splits of K never more than the slabs or an eighth of the steps, and a tile that takes the launch."""
+    from nats_llm_studio_amd.ops import stack as S
+
+    class W:
+        f32 = False
+
+        def __init__(self, N, Kd):
+            self.N, self.K, self.nsub = N, Kd, -(-Kd // 64) * 2
+    for N, Kd in ((4096, 17408), (2048, 5632), (640, 4096), (36000, 2048)):
+        for M in (17, 33, 64, 65, 128, 129, 300, 512):
+            l = S.LinLaunch.__new__(S.LinLaunch)
+            l.f32, l.segs = False, [type("Sg", (), dict(w=W(N, Kd), slabs=8, y=torch.zeros(1, 1)))()]
+            l._tiles = lambda bn, bm, m, N=N: -(-N // bn) * -(-m // bm)
+            cfg, ks = l.split_config(M)
+            assert ks >= 1 and (not cfg[0] or cfg[1] in (0, 3, 5, 6, 7, 10)) and (M <= 64 or cfg[1] in (0, 3) or ks <= min(8, Kd // 512))
