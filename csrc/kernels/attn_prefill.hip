@@ -263,20 +263,21 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
   const int qpos = pos0 + tw0 + tl;
 
   // ---- staging: thread tid moves chunks e = tid + 512 i (key e / NCH, chunk e % NCH) of K and of V
+  // Cache blocks are read a tile ahead of their rows, and keys past the last one repeat it (masked below): a load behind its
+  // block's, in a branch, waited for every load before it (3000 tokens, 32 heads of 128: 147 -> 130 us)
   typename KVRaw<KV>::raw kr[NLD], vr[NLD];
+  int blk[NLD];
+  auto load_blocks = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) blk[i] = bt[min(t * KT + (tid + 512 * i) / NCH, nkeys - 1) >> bs_shift];
+  };
   auto load_tile = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      const int e = tid + 512 * i, key = e / NCH, ch = e % NCH;
-      const int p = t * KT + key;
-      if (p < nkeys) {
-        const size_t off = ((size_t)(bt[p >> bs_shift] << bs_shift | (p & bsm)) * Hkv + hk) * D + ch * 8;
-        kr[i] = KVRaw<KV>::ld(kc + off);
-        vr[i] = KVRaw<KV>::ld(vc + off);
-      } else {
-        kr[i] = typename KVRaw<KV>::raw{};
-        vr[i] = typename KVRaw<KV>::raw{};
-      }
+      const int e = tid + 512 * i, ch = e % NCH, p = min(t * KT + e / NCH, nkeys - 1);
+      const size_t off = ((size_t)(blk[i] << bs_shift | (p & bsm)) * Hkv + hk) * D + ch * 8;
+      kr[i] = KVRaw<KV>::ld(kc + off);
+      vr[i] = KVRaw<KV>::ld(vc + off);
     }
   };
   auto store_tile = [&](int buf) __attribute__((always_inline)) {
@@ -295,7 +296,9 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
   for (int i = 0; i < NDB; ++i) o[i] = f32x16{};
   float m = -INFINITY, l = 0.f;
 
+  load_blocks(0);
   load_tile(0);
+  load_blocks(1);
   store_tile(0);
   __syncthreads();
   // V^T fragment read: lane (group of 16: q = (l & 15) >> 2 row, p = l & 3 column quad) supplies row
@@ -303,7 +306,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
   const int vq = (lane & 15) >> 2, vp = lane & 3, vhalf = (lane >> 4) & 1;
   for (int t = 0; t < ntile; ++t) {
     const int cur = t & 1;
-    if (t + 1 < ntile) load_tile(t + 1);      // issue early: lands while this tile computes
+    if (t + 1 < ntile) {                      // issue early: lands while this tile computes
+      load_tile(t + 1);
+      load_blocks(t + 2);
+    }
     const int k0 = t * KT;
     if (wact && k0 <= wlast) {
       const uint8_t* kb = lds + cur * 2 * TILEB;
