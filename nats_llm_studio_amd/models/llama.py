@@ -665,7 +665,8 @@ class LlamaModel:
             # probe's 168 vs 285 us did not carry over -- the model's mode-2 down runs at ~144 us)
             gu = dict(mode=3, waves=4, rt=6, ks=1)
         few = LlamaModel._moe_few_cfg(lw, T, rows / n_exp)
-        gu, dn = few[0] or gu, few[1] or dn
+        gu = gu if "NLS_MOE_RT_GU" in os.environ else few[0] or gu
+        dn = dn if "NLS_MOE_RT_DN" in os.environ or kdn > 1 else few[1] or dn
         if os.environ.get("NLS_MOE_QCFG_GU"):      # explicit (mode, waves, rt) overrides
             gu = dict(zip(("mode", "waves", "rt"), (int(v) for v in os.environ["NLS_MOE_QCFG_GU"].split(","))), ks=1)
         if os.environ.get("NLS_MOE_QCFG_DN"):
@@ -785,7 +786,7 @@ class LlamaModel:
         # rows in a 256-row block cost 64 rows of MFMA (Mixtral B=256, round-2 sweep: gate/up
         # rt 4 / down rt 4 = 19.6 ms/step, 4/2 = 20.7, 2/2 = 28.3, 1/1 = 43.0)
         gu = dn = {}
-        if not gemm and self.device.type == "cuda" and T * k >= len(self.experts):
+        if not gemm and self.device.type == "cuda" and T * k >= len(self.experts) and "NLS_MOE_GEMV" not in os.environ:
             gu, dn = self._moe_few_cfg(lw, T, T * k / E)
         if not gemm and len(_MOE_GEMV_DN) == 4:
             dn = dict(zip(("mode", "waves", "rt", "ks"), _MOE_GEMV_DN))
