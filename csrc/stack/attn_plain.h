@@ -11,6 +11,9 @@
 //   O^T += V^T P^T: those registers are the second operand as they stand; 16 bytes of value row 4 g + j at column 64 q + 4 r are
 //   the first operand of the four tiles of columns 64 q + 4 m + e.
 // Loads run one chunk of key columns and two of value columns ahead; nothing goes through LDS but the queries and the merge.
+// A row also meets keys that it does not see (other sequences' and later tokens' of its group, those ahead of its window, the last one
+// repeated), with a weight of 0, which an infinity or NaN among their values turns into NaN: rows whose result is not finite are summed
+// once more over their own keys alone.
 // What bounds it: the matrix pipe on prompts (32 cycles per MFMA, rows past a run's last token included), the walk over a row's keys on
 // small grids. Three prompts of 300 tokens, 16 heads of 128 over 4: 823 us (one workgroup per row and head, a serial walk) -> 43 us;
 // four decoded tokens behind 300 keys: 136 -> 16 us.
@@ -46,16 +49,56 @@ template <typename T> DEVI f32x4 ld4(const T* p) {
   return f32x4{(float)a[0], (float)a[1], (float)a[2], (float)a[3]};
 }
 
+// Row `row` of a workgroup, its token t and query head h, over the keys that it sees. mls: the waves' maxima and sums, w: 64 NW floats.
+template <typename T, int NW>
+DEVI void redo_row(const PA& p, int t, int h, int row, const float* mls, float* w) {
+  constexpr int NT = 64 * NW, C = VB / NT;
+  const int ctx = p.ctx_len[t], low = p.window > 0 ? ctx - p.window : 0, v0 = blockIdx.z * VB, dv = min(p.Dv - v0, VB);
+  const int* bt = p.bt + (size_t)p.tok_seq[t] * p.bts;
+  const T* q = reinterpret_cast<const T*>(p.q) + (size_t)t * p.ldq + (size_t)h * p.qhs;
+  const T* kc = reinterpret_cast<const T*>(p.k) + (size_t)(h / p.gs) * p.khs;
+  const T* vc = reinterpret_cast<const T*>(p.v) + (size_t)(h / p.gs) * p.khs + v0;
+  auto slot = [&](int k) { return ((size_t)bt[k / p.bs] * p.bs + k % p.bs) * p.ldkv; };
+  float m = -INFINITY, l = 0.f, acc[C];
+  for (int i = 0; i < NW; ++i) m = fmaxf(m, mls[i * 32 + row]);
+  for (int i = 0; i < NW; ++i)
+    if (mls[i * 32 + row] != -INFINITY) l += mls[i * 32 + 16 + row] * expf(mls[i * 32 + row] - m);
+  for (int i = 0; i < C; ++i) acc[i] = 0.f;
+  for (int k0 = 0; k0 < ctx; k0 += NT) {
+    const int n = min(NT, ctx - k0);
+    const T* k = kc + slot(k0 + min((int)threadIdx.x, n - 1));
+    float s = 0.f;
+    for (int d = 0; d < p.Dk; d += 4) {
+      const f32x4 x = ld4(k + d);
+      for (int e = 0; e < 4; ++e) s = fmaf((float)q[d + e], x[e], s);
+    }
+    __syncthreads();                               // (the last keys' weights have been read)
+    w[threadIdx.x] = expf(s * p.scale - m);
+    __syncthreads();
+    for (int i = 0; i < n; ++i) {
+      if (k0 + i < low && k0 + i >= p.keep) continue;
+      const T* v = vc + slot(k0 + i);
+      for (int j = 0; j < C; ++j)
+        if ((int)threadIdx.x + NT * j < dv) acc[j] = fmaf(w[i], (float)v[threadIdx.x + NT * j], acc[j]);
+    }
+  }
+  const float f = (l > 0.f ? 1.f / l : 0.f) * (p.gate ? p.gate[(size_t)t * p.ldg + h] : 1.f);
+  T* y = reinterpret_cast<T*>(p.out) + (size_t)t * p.ldo + (size_t)h * p.ohs + v0;
+  for (int j = 0; j < C; ++j)
+    if ((int)threadIdx.x + NT * j < dv) y[threadIdx.x + NT * j] = (T)(acc[j] * f);
+}
+
 // NQ: 64-column blocks of the values; NW: waves
 template <typename T, int NQ, int NW>
 __global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
   constexpr int KC = NQ > 2 ? 4 : 8;               // 16-column steps of a key chunk
-  constexpr int ML = NW * 32;                      // floats of the waves' maxima and sums
+  constexpr int ML = NW * 32 + 16;                 // floats of the waves' maxima and sums, rows that are not finite
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nks = (p.Dk + 15) >> 4, nc = (nks + KC - 1) / KC, ldl = nc * KC * 16 + 4;
   float *mls = sm, *ob = sm + ML, *qs = ob;        // (the merge takes the queries' place)
+  int* bad = reinterpret_cast<int*>(sm + NW * 32);
   const int kh = blockIdx.y / p.sub, h0 = (blockIdx.y % p.sub) * 16;          // key head, first of its query heads
   const int gr = min(p.gs - h0, 16);                                          // query heads of this workgroup
   const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * p.tb, tn = min(p.tb, p.T - t0);      // (later tokens see more keys)
@@ -195,6 +238,7 @@ __global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
   float M = -INFINITY;
 #pragma unroll
   for (int w = 0; w < NW; ++w) M = fmaxf(M, mls[w * 32 + r]);
+  if (threadIdx.x < 16) bad[threadIdx.x] = 0;
   const float f = m == -INFINITY ? 0.f : expf(m - M);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
@@ -221,10 +265,22 @@ __global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
       const size_t tk = t0 + row / gr;
       v *= (ll > 0.f ? 1.f / ll : 0.f) * (p.gate ? p.gate[tk * p.ldg + head(row)] : 1.f);
       T* y = reinterpret_cast<T*>(p.out) + tk * p.ldo + head(row) * p.ohs + v0 + 64 * q + c;
+      bool fin = true;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (64 * q + c + e < dv) y[e] = (T)v[e];
+        if (64 * q + c + e < dv) {
+          y[e] = (T)v[e];
+          fin = fin && fabsf(v[e]) < INFINITY;
+        }
+      if (!fin) bad[row] = 1;
     }
+  }
+  __syncthreads();
+  for (uint64_t again = __ballot(lane < nrow && bad[lane & 15]); again; again &= again - 1) {
+    const int row = __builtin_ctzll(again);
+    const PA* args = (const PA*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));                 // (read anew: kept from the start, they would not fit beside the loop's scalars)
+    redo_row<T, NW>(*args, t0 + row / gr, kh * args->gs + h0 + row % gr, row, mls, ob);
   }
 }
 
@@ -232,7 +288,7 @@ template <typename T, int NQ, int NW>
 int launch_w(const PA& p, dim3 grid, hipStream_t st) {
   constexpr int KC = NQ > 2 ? 4 : 8;
   const int nc = ((p.Dk + 15) / 16 + KC - 1) / KC;
-  const size_t lds = sizeof(float) * (NW * 32 + max(16 * (nc * KC * 16 + 4), NW * 16 * 68));
+  const size_t lds = sizeof(float) * (NW * 32 + 16 + max(16 * (nc * KC * 16 + 4), NW * 16 * 68));
   if (lds > 64 * 1024) {
     static bool attr = false;
     if (!attr && hipFuncSetAttribute((const void*)attn_plain_kernel<T, NQ, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -257,10 +313,14 @@ int launch(PA p, int T_, int H, hipStream_t st) {
       (p.khs & 3) || p.Dv > MAXV || p.bs < 1)
     return -1;
   p.T = T_;
-  // A few tokens are mostly of several sequences, which a group would walk one after another; with many, that costs nothing.
-  p.tb = T_ <= 64 ? 1 : max(1, 16 / p.gs);
   p.sub = (p.gs + 15) / 16;
-  const dim3 grid((T_ + p.tb - 1) / p.tb, H / p.gs * p.sub, (p.Dv + VB - 1) / VB);
+  // Up to 64 tokens each has a workgroup of its own. With more, a workgroup takes as many as leave one workgroup for each CU: a prompt's
+  // tokens share their keys, those of several sequences are walked one after another. (Decoded tokens behind 300 keys, 16 heads of 128
+  // over 4: 100 of them 47 us in groups of 4, 30 in groups of 2; 200, in groups of 4 either way, 52, and 74 in a workgroup each. 16
+  // heads of 64 over 16: 65 tokens 167 us in groups of 16, 57 in groups of 5. One workgroup per row and head: 241, 403, 193 us.)
+  const int heads = H / p.gs * p.sub;
+  p.tb = T_ <= 64 ? 1 : min(max(1, 16 / p.gs), (int)(((long)T_ * heads + 255) / 256));
+  const dim3 grid((T_ + p.tb - 1) / p.tb, heads, (p.Dv + VB - 1) / VB);
   switch ((p.Dv + 63) / 64) {
     case 1: return launch_q<T, 1>(p, grid, st);
     case 2: return launch_q<T, 2>(p, grid, st);

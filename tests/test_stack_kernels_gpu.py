@@ -190,6 +190,47 @@ def test_plain_attention_rows_of_many_sequences(K, dt, H, G, D, window, keep, si
     assert (o[:T, :, D:] == 0).all() and (o[T - 1] == 0).all() and (o[T] == 7).all()
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16"])
+@pytest.mark.parametrize("H,G,D,spread", [(8, 2, 128, 6), (6, 2, 20, 6), (4, 4, 64, 90), (2, 1, 300, 6), (1, 1, 600, 90)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (20, 3)])
+def test_plain_attention_keeps_values_apart(K, dt, H, G, D, spread, window, keep):
+    """An infinity and a NaN among one sequence's values reach the rows that see their keys, and no other: not those of other sequences,
+    not earlier tokens of the same prompt, not tokens whose window has passed them. Runs of several tokens, single tokens, `spread` of
+    them: workgroups with tokens of several sequences."""
+    d = {"f32": torch.float32, "bf16": torch.bfloat16}[dt]
+    Dp, _ = K.head_pad(D)
+    bs, nb = 16, 5
+    runs = [(0, 37), (30, 9)] + [(10 + i % 40, 1) for i in range(spread)] + [(0, 30)]
+    T = sum(n for _, n in runs)
+    assert T > 64
+    perm = torch.randperm(len(runs) * nb, generator=torch.Generator().manual_seed(5)).view(-1, nb)
+    kc, vc = (rnd(perm.numel() * bs, G * Dp, seed=s).to(d) for s in (1, 2))
+    q, gate = rnd(T, H * Dp, seed=3).to(d), rnd(T, H, seed=4).float()
+    seq = torch.tensor([i for i, (_, n) in enumerate(runs) for _ in range(n)], dtype=torch.int32)
+    pos = torch.tensor([p + j for p, n in runs for j in range(n)])
+    hit = {0: 33, 1: 36, 5: 2, len(runs) - 1: 0}               # sequence -> key with an infinity in column 1, a NaN in column 17
+    bad = vc.clone()
+    for i, k in hit.items():
+        bad[perm[i][k // bs] * bs + k % bs, 1::Dp] = math.inf
+        bad[perm[i][k // bs] * bs + k % bs, 17::Dp] = math.nan
+
+    def run(v):
+        out = torch.full((T, H * Dp), 7.0, dtype=d, device="cuda")
+        part = tuple(torch.zeros(1, device="cuda") for _ in range(3))
+        K.gqa_attention(q.cuda(), kc.cuda(), v.cuda(), gate.cuda(), out, part, perm.int().cuda(), bs, seq.cuda(), (pos + 1).int().cuda(),
+                        T, H, G, Dp, False, 1, 0.8 / math.sqrt(D), st(), window=window, keep=keep, sink=False)
+        return out.view(T, H, Dp).cpu()
+    a, b = run(vc), run(bad)
+    at = torch.tensor([hit.get(int(i), 1 << 30) for i in seq])
+    see = (at <= pos) & ((pos - at < window) | (at < keep) if window else torch.ones(T, dtype=torch.bool))
+    assert 0 < int(see.sum()) < T and a.isfinite().all()
+    assert b[see][..., 1].isinf().all() and b[see][..., 17].isnan().all()
+    # a row that is summed again takes its keys one after another: the sum of up to 50 products in another order, and the output's type
+    tol = 2e-6 if dt == "f32" else 3e-3
+    rest = [c for c in range(Dp) if c not in (1, 17)]
+    assert relerr(b[~see], a[~see]) < tol and relerr(b[see][..., rest], a[see][..., rest]) < tol
+
+
 @pytest.mark.parametrize("n", [1, 6, 7, 8, 14, 15, 50])
 def test_rows_to_host(K, n):
     """Logits on their way through two pinned buffers of seven rows: fewer, exactly and more than they hold, wanted rows gathered."""
