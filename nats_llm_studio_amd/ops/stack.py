@@ -222,7 +222,8 @@ class LinLaunch:
         if plan is not None:
             self.a.tiles, self.a.ntiles = plan.tiles.data_ptr(), plan.ntiles.data_ptr()
         self._cfg = {}
-        self.slab_rows = segs[0].slab_rows       # rows from slab to slab of the last run
+        self._rows, self._ldy = segs[0].slab_rows, segs[0].y.stride(0)
+        self.slab_rows = self._rows              # rows from slab to slab of the last run
 
     def _tiles(self, bn: int, bm: int, M: int) -> int:
         """Workgroups of a launch with bn x bm tiles."""
@@ -336,8 +337,24 @@ class LinLaunch:
         there are CUs, or lasts two rounds for a few more. 2000 x 4096 x 17408: 286 us in one round of 256 x 128 -> 222 in two splits of
         256 x 256; the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
         s = self.segs[0]
-        c, ks = self.cheapest(M, min(s.slabs, s.y.shape[0] // M))
+        c, ks = self.cheapest(M, min(s.slabs, s.y.shape[0] // self.slab_step(M)))
         return ((True, c), ks) if ks > 1 else (self.config(M), 1)
+
+    def slab_step(self, M: int) -> int:
+        """Rows from slab to slab: those the segment was bound for, or M of a larger launch, up to a multiple of 4 (the launch that adds
+        the slabs takes no other distances where a row is not whole groups of 4 columns)."""
+        return self._rows if M <= self._rows else (M + 3) & -4
+
+    def choice(self, M: int):
+        """(config, K splits) of a launch of M rows."""
+        s = self.segs[0]
+        splits = s.slabs > 1 and len(self.segs) == 1 and s.w.nsub >= 64
+        if splits and M <= self._rows:
+            cfg, ks = self.split_config(M)
+            return cfg, max(1, min(ks, s.slabs, s.w.nsub // 16))
+        if splits and not self.f32:
+            return self.tall_split(M)
+        return self.config(M), 1
 
     def run(self, M: int, st: int) -> int:
         """Returns the slabs of output rows that were written (1 unless a segment may split K), `slab_rows` rows apart."""
@@ -351,22 +368,10 @@ class LinLaunch:
         if cfg is None:
             if len(self._cfg) > 4096:
                 self._cfg.clear()
-            s = self.segs[0]
-            splits = s.slabs > 1 and len(self.segs) == 1 and s.w.nsub >= 64
-            if splits and M <= s.slab_rows:
-                cfg, ks = self.split_config(M)
-                cfg = cfg, max(1, min(ks, s.slabs, s.w.nsub // 16))
-            elif splits and not self.f32:
-                cfg = self.tall_split(M)
-            else:
-                cfg = self.config(M), 1
-            self._cfg[M] = cfg
+            cfg = self._cfg[M] = self.choice(M)
         cfg, ks = cfg
-        self.a.s[0].ks = ks
-        if ks > 1:
-            s = self.segs[0]
-            self.slab_rows = max(M, s.slab_rows)
-            self.a.s[0].yks = self.slab_rows * s.y.stride(0)
+        self.slab_rows = self.slab_step(M)
+        self.a.s[0].ks, self.a.s[0].yks = ks, self.slab_rows * self._ldy
         if cfg[0]:
             _check(lib().nls_lin_gemm(ctypes.byref(self.a), self.f32, cfg[1], st), "nls_lin_gemm")
         else:

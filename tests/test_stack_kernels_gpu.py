@@ -116,6 +116,23 @@ def test_tall_split(K, M, N, rows):
     assert relerr(z, x.double() @ w.double().T) < 2e-6
 
 
+@pytest.mark.parametrize("N", [1030, 1031, 1032])
+@pytest.mark.parametrize("M", [600, 601, 602, 603])
+def test_tall_split_of_ragged_rows(K, M, N):
+    """Row counts and widths that are no multiples of 4: the slabs stay where the residual's launch reads them, here and in a launch of
+    a single slab behind it."""
+    bf, Kd, rows = torch.bfloat16, 2090, 1300
+    x, w = rnd(rows - 1, Kd, seed=1).to(bf), (rnd(N, Kd, seed=2) * Kd ** -0.5).to(bf)
+    y = torch.full((rows, N), 7.0, device="cuda")
+    L = K.LinLaunch([K.Seg(K.PackedLinear(w, False, "cuda"), act(x, K.act_ld(Kd)), y, slabs=8, slab_rows=128)])
+    for m, splits in ((M, 2), (rows - 1, 1)):
+        n = L.run(m, st())
+        assert n == splits
+        z = torch.zeros(m, N, device="cuda")
+        K.norm_add(y, None, z, None, m, 1e-5, st(), slabs=n, slab_rows=L.slab_rows)
+        assert relerr(z, x[:m].double() @ w.double().T) < 2e-6
+
+
 @pytest.mark.parametrize("T,E", [(700, 3), (1100, 8)])
 def test_phased_gemm_of_experts(K, T, E):
     """Experts' row lists in tiles of 256 rows: several tiles, part tiles, an expert without rows; both products and the choice."""
