@@ -684,15 +684,15 @@ class Engine:
     # decode step. Not to be mixed with submitted requests.
     def feed(self, entries) -> List[torch.Tensor]:
         """entries: [(id, tokens, want)]: the next tokens of request `id` (admitted at its first entry) and the places
-        among them whose logits are wanted. Returns one CPU f32 tensor [len(want), vocab] per entry (rows of one buffer)."""
+        among them whose logits are wanted. Returns one CPU f32 tensor [len(want), vocab] per entry
+        (with memory of its own; entries without wanted places share an empty one)."""
         if self.tp is not None:
             raise NotImplementedError("feed: single-GPU engines only")
         if self.running or self.waiting:
             raise RuntimeError("feed: the engine is generating")
         if len(set(e[0] for e in entries)) != len(entries):
             raise ValueError("feed: one entry per request and step")
-        # (a decode step of a few hundred requests waits for this loop: a token at a time is checked without an array, entries
-        # without wanted places share one empty result)
+        # (a decode step of a few hundred requests waits for this loop: a token at a time is checked without an array)
         V, bs, single, seqs = self.cfg.vocab, self.bs, True, []
         for rid, toks, want in entries:
             s = self._fed.get(rid)
@@ -725,14 +725,13 @@ class Engine:
                         self._tables(hm, self.db.pad)[0][s.row, :len(s.blocks)] = s.blocks
             seqs.append(s)
         wants = [len(e[2]) for e in entries]
-        flat = torch.empty(sum(wants), V)                  # every entry's rows, one entry behind the other
+        none = torch.empty(0, V)           # (shared: a tensor each would be a tenth of 40 steps of 300 requests)
+        out = [torch.empty(w, V) if w else none for w in wants]
         if single:
-            self._feed_decode(seqs, entries, flat, wants)
+            self._feed_decode(seqs, entries, out, wants)
         else:
-            self._feed_rows(seqs, entries, flat, wants)
-        if len(flat) == 0:
-            return [flat] * len(entries)
-        return list(flat.split(wants))
+            self._feed_rows(seqs, entries, out)
+        return out
 
     @staticmethod
     def _inside(toks, vocab: int) -> bool:
@@ -745,12 +744,26 @@ class Engine:
 
     STAGE_BYTES = 8 << 20        # of each of the two pinned buffers that logits pass on their way to the host
 
-    def _rows_to_host(self, src: torch.Tensor, dst: torch.Tensor):
-        """Copy device rows to pageable host memory, through two pinned buffers: one is emptied while the next copy runs."""
+    def _rows_to_host(self, src: torch.Tensor, dst):
+        """Copy device rows to pageable host memory, through two pinned buffers: one is emptied while the next copy runs. dst: a tensor
+        of as many rows, or a list of tensors that take them one after another."""
+        rest = collections.deque([dst] if torch.is_tensor(dst) else dst)
+
+        def put(rows: torch.Tensor):
+            while len(rows):
+                t = rest.popleft()
+                n = min(len(t), len(rows))
+                if n == 1:                                 # (numpy's copy costs a third of torch's here)
+                    np.copyto(t[:1].numpy(), rows[:1].numpy())
+                else:
+                    t[:n].copy_(rows[:n])
+                if n < len(t):
+                    rest.appendleft(t[n:])
+                rows = rows[n:]
         if self.dev.type != "cuda":
-            dst.copy_(src)
+            put(src)
             return
-        n, V = dst.shape
+        n, V = src.shape
         rows = max(1, self.STAGE_BYTES // (4 * V))
         if self._stage is None:
             self._stage = [(torch.empty(min(rows, self.max_logit_rows), V, pin_memory=True), torch.cuda.Event()) for _ in range(2)]
@@ -763,28 +776,27 @@ class Engine:
             if c:
                 buf, ev = self._stage[(c // rows - 1) & 1]
                 ev.synchronize()
-                dst[c - rows:c].copy_(buf[:min(rows, n - c + rows)])
+                put(buf[:min(rows, n - c + rows)])
 
-    def _feed_decode(self, seqs, entries, flat, wants):
+    def _feed_decode(self, seqs, entries, out, wants):
         for s, e in zip(seqs, entries):
             s.tokens.append(int(e[1][0]))
             if s.row < 0:
                 self._assign_row(s)
-        need = len(flat) > 0
+        need = any(wants)
         (snap, k) = self._launch(seqs, set(), need)
         if need:
             rows = [r for (r, _), w in zip(snap, wants) for _ in range(w)]
             lg = self.db.logits
             lg = lg[rows[0]:rows[0] + len(rows)] if rows == list(range(rows[0], rows[0] + len(rows))) else lg[rows]
-            self._rows_to_host(lg, flat)
+            self._rows_to_host(lg, [t for t, w in zip(out, wants) if w])
         if self.dev.type == "cuda":
             self._ev[k].synchronize()
 
-    def _feed_rows(self, seqs, entries, flat, wants):
+    def _feed_rows(self, seqs, entries, out):
         """Row batches of at most max_prefill rows and max_logit_rows wanted rows (one batch unless the step is larger)."""
         work = [(i, s, [int(t) for t in e[1]], sorted((int(w), j) for j, w in enumerate(e[2])))
                 for i, (s, e) in enumerate(zip(seqs, entries))]
-        first = [0, *itertools.accumulate(wants)]          # an entry's first row of the results
         done = [0] * len(work)
         while any(done[i] < len(toks) for i, _, toks, _ in work):
             parts, rows, dest, T = [], [], [], 0
@@ -799,7 +811,11 @@ class Engine:
                     continue
                 parts.append((s, s.n_fed, toks[done[i]:done[i] + n]))
                 rows += [T + p - done[i] for p, _ in w]
-                dest += [first[i] + j for _, j in w]
+                for _, j in w:                             # [entry, first place among its results, past the last one]
+                    if dest and dest[-1][0] == i and dest[-1][2] == j:
+                        dest[-1][2] += 1
+                    else:
+                        dest.append([i, j, j + 1])
                 s.tokens += toks[done[i]:done[i] + n]
                 s.n_fed += n
                 done[i] += n
@@ -809,13 +825,7 @@ class Engine:
             self._exec_prefill(T, rows or [0], True, len(parts))
             self.counters["prefill_tokens"] += T
             if rows:
-                lg = self.pb.logits[:len(rows)]
-                if dest == list(range(dest[0], dest[0] + len(dest))):
-                    self._rows_to_host(lg, flat[dest[0]:dest[0] + len(dest)])
-                else:
-                    got = torch.empty(len(rows), self.cfg.vocab)
-                    self._rows_to_host(lg, got)
-                    flat[dest] = got
+                self._rows_to_host(self.pb.logits[:len(rows)], [out[i][a:b] for i, a, b in dest])
             elif self.dev.type == "cuda":
                 torch.cuda.current_stream(self.dev).synchronize()
 

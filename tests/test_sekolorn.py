@@ -245,6 +245,23 @@ def test_engine_feed_bookkeeping():
         eng.feed([("d", [64], [])])
 
 
+def test_engine_feed_results_are_their_own():
+    """Results share no memory with those of other entries, wherever their rows came from: a kept row keeps no more than itself."""
+    from nats_llm_studio_amd.engine.engine import Engine
+    m = _FakeRecurrent()
+    eng = Engine(m, None, max_batch=4, num_blocks=24, max_prefill_tokens=16, ctx=96, use_graphs=False, max_logit_rows=3)
+    t = [S.tokens(30, 64, i) for i in range(4)]
+    for step in ([(i, t[i][:9], [8, 0, 1, 1]) for i in range(4)], [(i, t[i][9:10], [0] * (i % 2)) for i in range(4)],
+                 [(i, t[i][10:11], [0, 0]) for i in range(4)]):
+        got = eng.feed(step)
+        assert [len(g) for g in got] == [len(e[2]) for e in step]
+        assert len({g.data_ptr() for g in got if len(g)}) == sum(len(g) > 0 for g in got)
+        assert all(g.untyped_storage().nbytes() == 4 * g.numel() for g in got)
+        for (i, toks, want), g in zip(step, got):
+            n = {9: 0, 1: 9 if step[0][1] == t[0][9:10] else 10}[len(toks)]
+            assert [int(r.argmax()) for r in g] == [_fake_next(t[i][:n + w + 1]) for w in want]
+
+
 # ---- the plain implementation against itself
 
 def test_oracle_cut_sequences():
