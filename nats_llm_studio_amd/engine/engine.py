@@ -779,6 +779,8 @@ class Engine:
                 put(buf[:min(rows, n - c + rows)])
 
     def _feed_decode(self, seqs, entries, out, wants):
+        if any(s.row < 0 for s in seqs):
+            self._release_rows()           # (a generation that ended while its next step ran may still hold some)
         for s, e in zip(seqs, entries):
             s.tokens.append(int(e[1][0]))
             if s.row < 0:
@@ -837,7 +839,7 @@ class Engine:
         if s.row >= 0:
             self.rows[s.row] = None
             s.row = -1
-        if not self._fed:               # (with the last one: what finished generations may have left)
+        if not self._fed:
             self._release_rows()
 
     def _first_tokens(self, seqs: List[_Seq], toks: List[int]):

@@ -262,6 +262,29 @@ def test_engine_feed_results_are_their_own():
             assert [int(r.argmax()) for r in g] == [_fake_next(t[i][:n + w + 1]) for w in want]
 
 
+def test_engine_feed_after_a_finished_generation():
+    """A generation that ends at an end-of-sequence token while the next step runs leaves its decode row behind: fed requests get that
+    row, also while others of them live."""
+    from nats_llm_studio_amd.engine.engine import Engine
+    from nats_llm_studio_amd.engine.sampling import SamplingParams
+    p = S.tokens(5, 64, 1)
+    want = list(p)
+    for _ in range(4):
+        want.append(_fake_next(want))
+    eng = Engine(_FakeRecurrent(), None, max_batch=2, num_blocks=24, max_prefill_tokens=16, ctx=96, use_graphs=False, eos_ids=(want[-1],))
+    assert eng.generate(p, SamplingParams(max_tokens=40)).stop_reason == "eosFound" and any(eng.rows)
+    t = {r: S.tokens(20, 64, i) for i, r in enumerate("abc")}
+
+    def step(k, rids):
+        for r, g in zip(rids, eng.feed([(r, t[r][k:k + 1], [0]) for r in rids])):
+            assert int(g[0].argmax()) == _fake_next(t[r][:k + 1])
+    eng.feed([(r, t[r][:7], []) for r in "ab"])
+    step(7, "a")
+    eng.feed_end("a")
+    eng.feed([("c", t["c"][:7], [])])
+    step(7, "bc")
+
+
 # ---- the plain implementation against itself
 
 def test_oracle_cut_sequences():
