@@ -1425,6 +1425,14 @@ class Engine:
             self.waiting.appendleft(s)
 
     def _decode(self, seqs: List[_Seq]):
+        fresh = sum(s.row < 0 for s in seqs)
+        if fresh and fresh > sum(r is None for r in self.rows):
+            # rows of sequences that ended while their next step ran: free once that step is over
+            self._drain()
+            self._release_rows()
+            seqs = [s for s in seqs if not s.done]
+            if not seqs:
+                return
         for s in seqs:
             if s.row < 0:
                 self._assign_row(s)

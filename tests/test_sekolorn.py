@@ -285,6 +285,26 @@ def test_engine_feed_after_a_finished_generation():
     step(7, "bc")
 
 
+def test_engine_full_batch_after_a_finished_generation():
+    """As many requests as there are decode rows, right after a generation that left one of them behind."""
+    from nats_llm_studio_amd.engine.engine import Engine, GenRequest
+    from nats_llm_studio_amd.engine.sampling import SamplingParams
+    want = S.tokens(5, 64, 1)
+    for _ in range(4):
+        want = want + [_fake_next(want)]
+    eng = Engine(_FakeRecurrent(), None, max_batch=2, num_blocks=24, max_prefill_tokens=64, ctx=96, use_graphs=False, eos_ids=(want[-1],))
+    assert eng.generate(want[:5], SamplingParams(max_tokens=40)).stop_reason == "eosFound" and any(eng.rows)
+    prompts = [S.tokens(6, 64, i) for i in (3, 4)]
+    futs = [eng.submit(GenRequest(p, SamplingParams(max_tokens=5, ignore_eos=True))) for p in prompts]
+    for _ in range(30):
+        eng.step()
+    for p, f in zip(prompts, futs):
+        w = list(p)
+        for _ in range(5):
+            w.append(_fake_next(w))
+        assert f.result(0).token_ids == w[6:]
+
+
 # ---- the plain implementation against itself
 
 def test_oracle_cut_sequences():
