@@ -772,7 +772,7 @@ class Engine:
             if c < n:
                 buf, ev = self._stage[c // rows & 1]
                 buf[:min(rows, n - c)].copy_(src[c:c + rows], non_blocking=True)
-                ev.record()
+                ev.record(torch.cuda.current_stream(self.dev))       # (the copy's; another device may be current)
             if c:
                 buf, ev = self._stage[(c // rows - 1) & 1]
                 ev.synchronize()

@@ -265,6 +265,22 @@ def test_rows_to_host(K, n):
     assert len(eng._stage[0][0]) == 7
 
 
+def test_rows_to_host_waits_on_the_engines_device(K, monkeypatch):
+    """The buffers' events are recorded on the stream of the engine's device, not on that of whichever device is current."""
+    from types import SimpleNamespace
+
+    from nats_llm_studio_amd.engine.engine import Engine
+    eng = SimpleNamespace(dev=torch.device("cuda:0"), STAGE_BYTES=1 << 10, _stage=None, max_logit_rows=64)
+    asked, current = [], torch.cuda.current_stream
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: asked.append(device) or current(device))
+    recorded, record = [], torch.cuda.Event.record
+    monkeypatch.setattr(torch.cuda.Event, "record", lambda self, stream=None: recorded.append(stream) or record(self, stream))
+    src, dst = rnd(9, 33).float().cuda(), torch.zeros(9, 33)
+    Engine._rows_to_host(eng, src, dst)
+    assert torch.equal(dst, src.cpu())
+    assert len(recorded) == 2 and all(s == current(eng.dev) for s in recorded) and asked[:2] == [eng.dev] * 2
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("D", [60, 64, 128, 256])
 def test_wkv_scan_loads(K, dt, D):
