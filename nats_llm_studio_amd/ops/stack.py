@@ -296,8 +296,14 @@ class LinLaunch:
         return min((10, 9, 8, 0), key=lambda c: (-(-self._tiles(*GEMM_TILES[c], M) // 256) * GEMM_TILES[c][0], -GEMM_TILES[c][0]))
 
     def few_rows(self, M: int, n64: int):
-        """17 to 64 rows, bound by the weights' bytes. Up to 8192 outputs the streaming kernel's two weight tiles fill the chip (48 x 4096 x
-        4096: 20 us, 27 in the GEMM; 24 x 8192: 16, 27)."""
+        """17 to 64 rows, bound by the weights' bytes: the streaming kernel with the smallest tiles (weight rows x rows) that give each CU
+        no more than one workgroup. 16 x 32 / 32 x 32 / 32 x 64, us: 24 x 4096 x 4096 13.4 / 19.0 / 15.1 (in the GEMM 19.4), 32 x 2048 x 9728
+        28.7 / 40.6 / 33.1, 64 rows of it 31.5 / 42.6 / 52.7; 64 x 4096 x 17408 101.6 / 77.1 / 93.7, 40 rows of it 101.3 / 75.7 / 70.6;
+        64 x 6144 x 2048 19.7 / 17.4 / 14.2."""
+        if self._tiles(16, 32, M) <= 256:
+            return False, 2, 8, 1
+        if M > 48 and self._tiles(32, 32, M) <= 256:
+            return False, 2, 8, 2
         if self._tiles(32, 64, M) <= 256:
             return False, 4, 8, 2
         if n64 <= 256:                    # 48 x 10240 x 4096: 27 us with 8 stages in flight, 35 streaming; 20 rows: 27, 23
