@@ -991,10 +991,11 @@ DEVI void mm_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
 }
 
 // Active-tile dispatch by the rows of a block (an expert's are known on the device only): the 8-wave, 2-row-tile, 8-tile
-// instance takes {2, 4, 6, 8}, rounded up to even to bound the instantiations, those of 2 to 4 tiles {1, 2, MT}: 24 tokens
-// give eight experts 4 to 11 rows each, so a second tile was only padding (Q5_K gate|up 8 x 8192 x 2048 on (8, 2): 27.7 ->
-// 25.1 us, down 8 x 2048 x 4096 on (4, 1): 19.9 -> 17.5; 64 tokens 34.3 -> 28.5 and 29.5 -> 20.4).
-template <int T, int WAVES, int RT, int MT, bool XL>
+// instance takes {2, 4, 6, 8}, rounded up to even to bound the instantiations, those of 2 to 4 tiles (GRP: mapped rows) {1, 2, MT}:
+// 24 tokens give eight experts 4 to 11 rows each, so a second tile was only padding (Q5_K gate|up 8 x 8192 x 2048 on (8, 2): 27.7
+// -> 25.1 us, down 8 x 2048 x 4096 on (4, 1): 19.9 -> 17.5; 64 tokens 34.3 -> 28.5 and 29.5 -> 20.4). Launches whose rows are all
+// there keep the one instance: beside the others it has 20 to 60 registers less (Q6_K 49155 x 2048 at 64 rows 53 us, 64 with them).
+template <int T, int WAVES, int RT, int MT, bool XL, bool GRP>
 DEVI void mm_tile_na(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, act_t* lds,
                      const int* xm, const int* ym) {
   if constexpr (MT == 8 && WAVES == 8 && RT == 2 && !XL) {
@@ -1003,7 +1004,7 @@ DEVI void mm_tile_na(const Seg& S, int row0, int kslice, int ks, const GemvArgs&
     else if (na <= 4) mm_tile<T, WAVES, RT, MT, XL, 4>(S, row0, kslice, ks, a, ws, lds, xm, ym);
     else if (na <= 6) mm_tile<T, WAVES, RT, MT, XL, 6>(S, row0, kslice, ks, a, ws, lds, xm, ym);
     else mm_tile<T, WAVES, RT, MT, XL, 8>(S, row0, kslice, ks, a, ws, lds, xm, ym);
-  } else if constexpr (MT >= 2 && MT <= 4 && !XL) {
+  } else if constexpr (GRP && MT >= 2 && MT <= 4 && !XL) {
     if (a.M <= 16) mm_tile<T, WAVES, RT, MT, XL, 1>(S, row0, kslice, ks, a, ws, lds, xm, ym);
     else if (MT > 2 && a.M <= 32) mm_tile<T, WAVES, RT, MT, XL, 2>(S, row0, kslice, ks, a, ws, lds, xm, ym);
     else mm_tile<T, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, lds, xm, ym);
@@ -1012,7 +1013,7 @@ DEVI void mm_tile_na(const Seg& S, int row0, int kslice, int ks, const GemvArgs&
   }
 }
 
-template <int WAVES, int RT, int MT, int KSET, bool XL = false>
+template <int WAVES, int RT, int MT, int KSET, bool XL = false, bool GRP = false>
 __global__ __launch_bounds__(WAVES * 64) void qmm_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
                                                          int nmb) {
   extern __shared__ __attribute__((aligned(16))) act_t xlds[];
@@ -1051,22 +1052,22 @@ __global__ __launch_bounds__(WAVES * 64) void qmm_kernel(SegList segs, GemvArgs 
   const int row0 = (tile - S.tile_begin) * WAVES * RT * 16;
   if constexpr (KSET == 0) {
     switch (S.type) {
-      case QT_Q4_K: mm_tile_na<QT_Q4_K, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
-      case QT_Q6_K: mm_tile_na<QT_Q6_K, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q4_K: mm_tile_na<QT_Q4_K, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q6_K: mm_tile_na<QT_Q6_K, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
       default: break;
     }
   } else if constexpr (KSET == 1) {
     switch (S.type) {
-      case QT_Q5_K: mm_tile_na<QT_Q5_K, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
-      case QT_Q6_K: mm_tile_na<QT_Q6_K, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
-      case QT_Q8_0: mm_tile_na<QT_Q8_0, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q5_K: mm_tile_na<QT_Q5_K, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q6_K: mm_tile_na<QT_Q6_K, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q8_0: mm_tile_na<QT_Q8_0, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
       default: break;
     }
   } else if constexpr (KSET == 3) {
     switch (S.type) {
-      case QT_Q51: mm_tile_na<QT_Q51, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
-      case QT_Q6_K: mm_tile_na<QT_Q6_K, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
-      case QT_Q8_0: mm_tile_na<QT_Q8_0, WAVES, RT, MT, XL>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q51: mm_tile_na<QT_Q51, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q6_K: mm_tile_na<QT_Q6_K, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
+      case QT_Q8_0: mm_tile_na<QT_Q8_0, WAVES, RT, MT, XL, GRP>(S, row0, kslice, ks, a, ws, xlds, xm, ym); break;
       default: break;
     }
   } else {
@@ -1212,13 +1213,11 @@ template <int WAVES, int RT, int MT, int KSET>
 int launch_b(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st, int nmb) {
   const size_t lds = (size_t)2 * MT * 16 * 256 * sizeof(act_t);
   const int grid = nmb > 1 ? ((ntiles + 7) / 8) * 8 * nmb * ks : ntiles * ks;
+  bool mapped = false;
+  for (int i = 0; i < sl.nseg; ++i) mapped |= sl.s[i].xmap != nullptr || sl.s[i].mcount != nullptr;
   if constexpr (MT == 1) {      // few rows: stage the whole x slice once (XL) when it fits
-    bool mapped = false;
     int kmax = 0;
-    for (int i = 0; i < sl.nseg; ++i) {
-      mapped |= sl.s[i].xmap != nullptr || sl.s[i].mcount != nullptr;
-      kmax = max(kmax, sl.s[i].K);
-    }
+    for (int i = 0; i < sl.nseg; ++i) kmax = max(kmax, sl.s[i].K);
     const size_t xbytes = (size_t)a.M * (((kmax >> 8) + ks - 1) / ks) * 256 * sizeof(act_t);
     if (nmb == 1 && !mapped && xbytes <= XL_LDS_BYTES) {
       const size_t need = a.xf ? xbytes + 64 * sizeof(float) : xbytes;     // + inv-rms scratch
@@ -1231,6 +1230,12 @@ int launch_b(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a
   if constexpr (WAVES == 7) {   // (the 7-wave instance exists for the staged batch-1 path only)
     return -1;
   } else {
+    if constexpr (MT >= 2 && MT <= 4 && KSET != 2)
+      if (mapped) {
+        hipLaunchKernelGGL((qmm_kernel<WAVES, RT, MT, KSET, false, true>), dim3(grid), dim3(WAVES * 64), lds, st, sl, a, ks, ws,
+                           ntiles, nmb);
+        return (int)hipGetLastError();
+      }
     hipLaunchKernelGGL((qmm_kernel<WAVES, RT, MT, KSET>), dim3(grid), dim3(WAVES * 64), lds, st, sl, a, ks, ws,
                        ntiles, nmb);
     return (int)hipGetLastError();
