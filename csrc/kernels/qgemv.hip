@@ -262,8 +262,16 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
     const size_t ysz = epi == EPI_ACT ? 2 : 4;
     if (nseg == 1 && epi != EPI_SWIGLU && (((uintptr_t)ws) & 15) == 0 && cols % 4 == 0 &&
         (epi == EPI_ARGMAX || (ldy % 4 == 0 && segs[0].ycol % 4 == 0 && ((uintptr_t)y) % (4 * ysz) == 0))) {
-      auto k = ks == 2 ? splitk_reduce4_kernel<2> : ks == 4 ? splitk_reduce4_kernel<4> : ks == 8 ? splitk_reduce4_kernel<8> : splitk_reduce4_kernel<0>;
-      hipLaunchKernelGGL(k, dim3((cols + 1023) / 1024, M), dim3(256), 0, st, (const float*)ws, ks, M, cols, segs[0].ycol, a);
+      const int tx = argmax || tiles % 4 || (tile_rows != 128 && tile_rows != 256) || mode == 1 ? 256 : tile_rows / 4;
+#define NLS_R4(TX)                                                                                                     \
+  if (tx == TX) {                                                                                                      \
+    auto k = ks == 2 ? splitk_reduce4_kernel<2, TX> : ks == 4 ? splitk_reduce4_kernel<4, TX>                           \
+           : ks == 8 ? splitk_reduce4_kernel<8, TX> : splitk_reduce4_kernel<0, TX>;                                    \
+    hipLaunchKernelGGL(k, dim3((cols + 4 * TX - 1) / (4 * TX), (M + 256 / TX - 1) / (256 / TX)), dim3(256), 0, st,     \
+                       (const float*)ws, ks, M, cols, segs[0].ycol, a);                                                \
+  }
+      NLS_R4(256) NLS_R4(64) NLS_R4(32)
+#undef NLS_R4
       return (int)hipGetLastError();
     }
     // with an arg-max every workgroup ends in an atomic on its row's key, all on neighbouring addresses: about 2048 workgroups in all

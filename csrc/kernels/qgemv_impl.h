@@ -1140,12 +1140,15 @@ static __global__ void splitk_reduce_kernel(const float* __restrict__ ws, int ks
 
 // The same for one segment whose columns, strides and pointers are multiples of 4 (not SwiGLU): 16-byte loads and stores, one
 // float4 to a thread, KS slabs in flight (0: any number). 32 rows x 32000 in two slabs with the arg-max: 16.5 -> 9.7 us.
-template <int KS>
+// A workgroup takes 4 TX columns of 256 / TX rows. With an arg-max TX = 256, one atomic for 1024 columns. The GEMMs leave the slabs of
+// weight tile t in the L2 of XCD t % 8; workgroups as wide as a tile, in multiples of 8, read them there (256 x 2048 in five slabs, with
+// the product: 19.2 us in 1024 columns to a workgroup, 15.0 in 256).
+template <int KS, int TX>
 __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ ws, int ks, int M, int ntot, int ycol,
                                                              GemvArgs a) {
-  const int b = blockIdx.y, col = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const int b = blockIdx.y * (256 / TX) + threadIdx.x / TX, col = (blockIdx.x * TX + threadIdx.x % TX) * 4;
   unsigned long long best = 0ull;
-  if (col < ntot) {
+  if (col < ntot && (TX == 256 || b < M)) {
     const float* p = ws + (size_t)b * ntot + col;
     const size_t slab = (size_t)M * ntot;
     f32x4 v{0.f, 0.f, 0.f, 0.f};
@@ -1169,14 +1172,14 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __rest
       typedef act_t act4 __attribute__((ext_vector_type(4)));
       *reinterpret_cast<act4*>(reinterpret_cast<act_t*>(a.y) + off) = act4{(act_t)v[0], (act_t)v[1], (act_t)v[2], (act_t)v[3]};
     }
-    if (a.argmax)
+    if (TX == 256 && a.argmax)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const unsigned long long k = argmax_key(v[i], ycol + col + i);
         best = k > best ? k : best;
       }
   }
-  if (a.argmax) reduce_argmax(a.argmax + b, best);
+  if (TX == 256 && a.argmax) reduce_argmax(a.argmax + b, best);
 }
 
 // ---- launch helpers, one kernel type-set (KSET) per translation unit -------------------------

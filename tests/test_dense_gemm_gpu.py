@@ -74,3 +74,21 @@ def test_rope_epilogue(cfg, D, bias, M):
         outs.append((q.cpu(), kc.cpu(), vc.cpu()))
     for a, b in zip(*outs):      # one bf16 rounding apart at most, and the same places written
         assert relerr(a, b) < 2e-3 and ((a == 776) == (b == 776)).all()
+
+
+@pytest.mark.parametrize("cfg", [(10, 8, 1), (10, 8, 2), (5, 16, 2), (4, 8, 2)])
+@pytest.mark.parametrize("rows,K", [(1024, 2304), (1020, 2048), (2048, 1024), (388, 2048), (1536, 2560)])
+def test_split_reduce(cfg, rows, K):
+    """Slabs of a split product and their sum: whole and part workgroups of columns and of rows, where a workgroup has the tile's columns
+    and where it has 1024; every kind of output, two slabs to nine."""
+    w = weight(rows, K)
+    for M in (70, 129, 258, 263):
+        x = acts(M, K)
+        z = x[:M].double() @ w.d16.double().T
+        for ks in (2, 3, 4, 5, 8, 9):
+            for epi, dt in (("f32", torch.float32), ("add", torch.float32), ("act", torch.float16)):
+                y = torch.full((M + 1, rows + 4), 7.0, device="cuda", dtype=dt)
+                ops.qgemv([ops.Seg(w, 4)], x, y, M, epi=epi, mode=cfg[0], waves=cfg[1], rt=cfg[2], ks=ks)
+                # f32 sums of K products; f16 outputs round to 2^-11
+                assert relerr(y[:M, 4:] - (7 if epi == "add" else 0), z) < (5e-4 if epi == "act" else 4e-6), (M, ks, epi)
+                assert (y[M] == 7).all() and (y[:, :4] == 7).all()
