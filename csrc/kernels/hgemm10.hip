@@ -84,7 +84,8 @@ DEVI int unit_rt(int u, int idx) {           // idx: row-tile slot of the unit
 template <int BN, int MT>
 using H10Acc = f32x4[2 * H10<BN, MT>::NQH][MT];
 
-template <int BN, int MT>
+// ROPE: the RoPE epilogue, in kernels of its own: beside it the 256 x 256 tile spilled 21 registers
+template <int BN, int MT, bool ROPE>
 DEVI void h10_epilogue(H10Acc<BN, MT>& acc, const Seg& S, int row0, int kslice, int ks,
                        const GemvArgs& a, float* ws) {
   constexpr int NQH = H10<BN, MT>::NQH;
@@ -94,7 +95,7 @@ DEVI void h10_epilogue(H10Acc<BN, MT>& acc, const Seg& S, int row0, int kslice, 
   const int M = a.M;
   const int g4 = 4 * (lane >> 4), r16 = lane & 15;
   const int nb = row0 + wr * (BN / 2), mb = wc * 16 * MT;
-  if (ks > 1 || a.epi == EPI_SLABS) {
+  if (!ROPE && (ks > 1 || a.epi == EPI_SLABS)) {
 #pragma unroll
     for (int i = 0; i < 2 * NQH; ++i) {
       const int n = nb + 16 * i + g4;
@@ -109,7 +110,7 @@ DEVI void h10_epilogue(H10Acc<BN, MT>& acc, const Seg& S, int row0, int kslice, 
     return;
   }
   const float al = a.alpha;
-  if (a.epi == EPI_ROPE) {
+  if constexpr (ROPE) {
     // RoPE pairs (e, e + 1) of the lane's 4 consecutive weight rows: no cross-lane traffic
     if ((a.D & 3) || (a.ldq & 3)) {
       for (int i = 0; i < 2 * NQH; ++i) {               // (moved up instead of unrolled: the general form is long)
@@ -230,7 +231,7 @@ DEVI void h10_epilogue(H10Acc<BN, MT>& acc, const Seg& S, int row0, int kslice, 
   }
 }
 
-template <int BN, int MT>
+template <int BN, int MT, bool ROPE>
 DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, uint8_t* lds) {
   typedef H10<BN, MT> C;
   constexpr int TB = C::TB, NQH = C::NQH, NA = C::NA, NB2 = C::NB2;
@@ -366,10 +367,10 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();
 
-  h10_epilogue<BN, MT>(acc, S, row0, kslice, ks, a, ws);
+  h10_epilogue<BN, MT, ROPE>(acc, S, row0, kslice, ks, a, ws);
 }
 
-template <int BN, int MT>
+template <int BN, int MT, bool ROPE>
 __global__ __launch_bounds__(512, 1) void hgemm10_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
                                                           int nmb) {
   extern __shared__ __attribute__((aligned(16))) uint8_t h10lds[];
@@ -391,23 +392,28 @@ __global__ __launch_bounds__(512, 1) void hgemm10_kernel(SegList segs, GemvArgs 
   if (a.argmax) a.argmax += m0;
   a.M = min(BM, a.M - m0);
   const int row0 = (tile - S.tile_begin) * BN;       // (host tile counts use BN-row tiles)
-  h10_tile<BN, MT>(S, row0, kslice, ks, a, ws, h10lds);
+  h10_tile<BN, MT, ROPE>(S, row0, kslice, ks, a, ws, h10lds);
 }
 
-template <int BN, int MT>
-int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
+template <int BN, int MT, bool ROPE>
+int launch_e(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   constexpr int LDS = H10<BN, MT>::LDS, BM = H10<BN, MT>::BM;
   const int nmb = (a.M + BM - 1) / BM;
   const int grid = ((ntiles + 7) / 8) * 8 * nmb * ks;
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
-    if (hipFuncSetAttribute((const void*)hgemm10_kernel<BN, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) !=
+    if (hipFuncSetAttribute((const void*)hgemm10_kernel<BN, MT, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) !=
         hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((hgemm10_kernel<BN, MT>), dim3(grid), dim3(512), LDS, st, sl, a, ks, ws, ntiles, nmb);
+  hipLaunchKernelGGL((hgemm10_kernel<BN, MT, ROPE>), dim3(grid), dim3(512), LDS, st, sl, a, ks, ws, ntiles, nmb);
   return (int)hipGetLastError();
+}
+
+template <int BN, int MT>
+int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
+  return a.epi == EPI_ROPE ? launch_e<BN, MT, true>(sl, ntiles, ks, ws, a, st) : launch_e<BN, MT, false>(sl, ntiles, ks, ws, a, st);
 }
 
 // bn: weight rows per workgroup tile (256 or 128). Row blocks of 192 instead of 256 where their rounds over the 256 CUs, each three quarters as
