@@ -417,10 +417,12 @@ int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a
 }
 
 // bn: weight rows per workgroup tile (256 or 128). Row blocks of 192 instead of 256 where their rounds over the 256 CUs, each three quarters as
-// long, end earlier (Llama-3-8B at 384 rows: gate|up 99 -> 76 us, down 69 -> 57; 1500 rows: o 65 -> 56; 3000: down 308 -> 276).
+// long, end earlier (Llama-3-8B at 384 rows: gate|up 99 -> 76 us, down 69 -> 57; 1500 rows: o 65 -> 56; 3000: down 308 -> 276). With 256 weight rows
+// they must end a good deal earlier: 192 x 256 tiles multiply slower, and the last round is seldom full (28672 x 4096, rounds by length: 0.75 at
+// 600 and 1100 rows 193 -> 169 and 292 -> 254 us, 0.875 at 3000 rows 638 -> 674, 0.9 at 2400 527 -> 537, 0.94 at 2048 417 -> 437).
 int launch_dense10(int bn, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   auto rounds = [&](int bm) { return (long)((ntiles * ((a.M + bm - 1) / bm) * ks + 255) / 256) * bm; };
-  const bool low = rounds(192) < rounds(256);
+  const bool low = rounds(192) * 100 < rounds(256) * (bn == 256 ? 85 : 100);
   if (bn == 256) return low ? launch_t<256, 3>(sl, ntiles, ks, ws, a, st) : launch_t<256, 4>(sl, ntiles, ks, ws, a, st);
   if (bn == 128) return low ? launch_t<128, 3>(sl, ntiles, ks, ws, a, st) : launch_t<128, 4>(sl, ntiles, ks, ws, a, st);
   return -1;
