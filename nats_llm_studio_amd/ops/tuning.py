@@ -6,6 +6,7 @@ the table use the heuristic below.
 """
 from __future__ import annotations
 
+import functools
 import json
 import os
 
@@ -130,16 +131,20 @@ def dense_heuristic(segs, M: int, aligned: bool = True):
     weight rows and mode 4 with 128 x 128 tiles, by the rounds of tiles over the 256 CUs; split-K slabs are written and read again.
     (A rule that took mode 4 below 1024 rows and mode 5 above ran a 32000-row head at 300 / 900 / 4096 rows in 161 / 742 / 2846 us;
     mode 10 takes 108 / 223 / 909.) aligned: the operands' row strides suit mode 10, whose stores are 4 columns wide."""
-    rows, K = sum(s.w.rows for s in segs), segs[0].w.K
-    nkt = K // 64
     aligned = aligned and all(s.w.rows % 4 == 0 and s.ycol % 4 == 0 for s in segs)
+    return _dense_rule(tuple(s.w.rows for s in segs), segs[0].w.K, M, aligned)
+
+
+@functools.lru_cache(maxsize=4096)         # (30 to 50 us to work out, and a prompt's launches ask once for each layer and projection)
+def _dense_rule(rows, K: int, M: int, aligned: bool):
+    nkt = K // 64
 
     def us(mode, rt, ks):
         bn = 256 if (mode, rt) == (10, 1) else 128
-        tiles = sum((s.w.rows + bn - 1) // bn for s in segs) * ks
+        tiles = sum((n + bn - 1) // bn for n in rows) * ks
         best = min(-(-tiles * -(-M // bm) // 256) * (5.0 + (t - 5.0) * K / ks / 4096)
                    for (md, r, bm), t in _ROUND_US.items() if (md, r) == (mode, rt))
-        return best + (2.0 + 2e-6 * ks * M * rows if ks > 1 else 0.0)
+        return best + (2.0 + 2e-6 * ks * M * sum(rows) if ks > 1 else 0.0)
     mode, rt, ks = min(((mode, rt, ks) for mode, rt in ([(10, 1), (10, 2)] if aligned else []) + [(4, 2)] for ks in range(1, 9)
                         if ks == 1 or nkt // ks >= 8), key=lambda c: us(*c))
     return (mode, 8 if mode == 10 or M < 128 else 16, rt, ks)
