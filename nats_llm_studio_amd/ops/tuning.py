@@ -11,6 +11,7 @@ import json
 import os
 
 _TABLE = None
+_FORCED = set()        # keys of NLS_TUNING_EXTRA's entries: no rule below changes those launches
 _PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemv_tuning.json")
 MBUCKETS = (1, 2, 4, 8, 16, 32, 48, 64, 128, 256, 512, 1024, 2048)
 
@@ -32,6 +33,7 @@ def table():
     global _TABLE
     if _TABLE is None:
         _TABLE = {}
+        _FORCED.clear()
         if os.path.exists(_PATH):
             with open(_PATH) as f:
                 _TABLE = {k: tuple(v) for k, v in json.load(f).items()}
@@ -44,6 +46,7 @@ def table():
         extra = os.environ.get("NLS_TUNING_EXTRA")
         if extra:
             _TABLE.update({k: tuple(v) for k, v in json.loads(extra).items()})
+            _FORCED.update(json.loads(extra))
     return _TABLE
 
 
@@ -111,6 +114,8 @@ def argmax_config(cfg, segs, M: int):
     keys (32000 Q6_K rows, K = 4096, (1, 8, 1, 1): 62 us at 2 tokens, 108 at 8, 166 at 24, 248 at 64). Split in two, the reduce
     takes the maximum with few atomics: 26, 28, 34, 47; at K = 2048 2 / 8 / 24 / 64 tokens 58 / 105 / 150 / 217 -> 18 / 20 /
     25 / 34, one token 36 -> 19; on 16-row tiles, (1, 8, 1, 2), 24 / 26 / 30 / 36."""
+    if _FORCED and key(segs, M) in _FORCED:
+        return cfg
     if cfg[0] == 1 and 1 in cfg[2:] and M <= 64 and sum(s.w.rows for s in segs) >= 8192 and segs[0].w.K >= 1024:
         return (1, 4 if M == 1 else 8, 2, 2)
     return cfg
@@ -155,7 +160,7 @@ def select_dense(segs, M: int):
     hit = table().get(dense_key(segs, M))
     if hit is not None and hit[0] < 0:
         return None
-    if M > MBUCKETS[-1]:
+    if M > MBUCKETS[-1] and dense_key(segs, M) not in _FORCED:
         return dense_heuristic(segs, M)
     return hit if hit is not None else dense_heuristic(segs, M)
 

@@ -67,6 +67,22 @@ def test_expert_rule():
     assert tuning.expert_heuristic([_W(2048)] * 4 + [_W(2048, 99)] * 4, 32, 8) is None
 
 
+def test_environment_entries_stay(monkeypatch):
+    """A launch config given in the environment is what runs: not split for a head's arg-max, and also above the tuned row counts."""
+    class W(_W):
+        K = 4096
+    head, dense = [ops.Seg(W(32000, 14))], [ops.Seg(W(4096))]
+    monkeypatch.setattr(tuning, "_TABLE", None)
+    monkeypatch.setenv("NLS_TUNING_EXTRA", '{"14:32000:4096:16": [1, 4, 1, 1], "d:4096:4096:2048": [5, 8, 4, 2]}')
+    try:
+        assert tuning.argmax_config(tuning.select(head, 12), head, 12) == (1, 4, 1, 1)
+        assert tuning.argmax_config((1, 4, 1, 1), head, 24) == (1, 8, 2, 2)          # another row count's own
+        assert tuning.select_dense(dense, 3000) == (5, 8, 4, 2) and tuning.select_dense(dense, 1024) != (5, 8, 4, 2)
+    finally:
+        tuning._TABLE = None
+        tuning._FORCED.clear()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 2, 15, 17, 33, 64])
 @pytest.mark.parametrize("rows,K,qt", [(8192, 1024, GGMLType.Q6_K), (8209, 1280, GGMLType.Q4_K), (32000, 2048, GGMLType.Q8_0)])
