@@ -69,6 +69,53 @@ def test_phased_gemm(K, M, Kd):
     assert (o[:, 32:64] == 7).all() and all((t[M] == 7).all() for t in y.values())
 
 
+@pytest.mark.parametrize("M,N,Kd,ks", [(1, 256, 400, 2), (300, 515, 700, 2), (257, 512, 700, 3), (600, 1028, 1100, 5), (1300, 4096, 700, 3),
+                                        (513, 2304, 1300, 6)])
+def test_phased_splits(K, M, N, Kd, ks):
+    """Split products: 3 to 6 steps, not the same to every split, whole and ragged columns, up to 288 tiles, so that a workgroup walks from
+    a split's tile to another split's; each slab holds its own steps' sums."""
+    bf, steps = torch.bfloat16, K.act_ld(Kd) // 64
+    x, w = rnd(M, Kd, seed=1).to(bf), (rnd(N, Kd, seed=2) * Kd ** -0.5).to(bf)
+    y = torch.full((ks * M + 1, N), 7.0, device="cuda")
+    L = K.LinLaunch([K.Seg(K.PackedLinear(w, False, "cuda"), act(x, K.act_ld(Kd)), y, slabs=ks, slab_rows=M)])
+    L._cfg[M] = (True, 7), ks
+    assert L.run(M, st()) == ks and L.slab_rows == M
+    for i in range(ks):
+        k0, k1 = (min(Kd, 64 * (steps * j // ks)) for j in (i, i + 1))
+        assert relerr(y[i * M:(i + 1) * M], x[:, k0:k1].double() @ w[:, k0:k1].double().T) < 2e-6
+    assert (y[ks * M] == 7).all()
+
+
+@pytest.mark.parametrize("M", [200, 600])
+@pytest.mark.parametrize("N", [256, 516, 518])
+def test_phased_gates_and_groups(K, M, N):
+    """256 x 256 tiles: the gated and the weighted epilogues, whole 4-column groups and not, and a batch of groups with columns of their
+    own in x and y."""
+    bf, Kd, G = torch.bfloat16, 250, 3
+    ld = K.act_ld(Kd)
+    x = rnd(M, G * Kd, seed=1).to(bf)
+    X = torch.cat([act(x[:, g * Kd:(g + 1) * Kd], ld) for g in range(G)], 1).contiguous()
+    w = {n: (rnd(N, Kd, seed=10 + i) * Kd ** -0.5).to(bf) for i, n in enumerate(("swiglu", "siluglu", "sigmoid"))}
+    wg = (rnd(G, N, Kd, seed=20) * Kd ** -0.5).to(bf)
+    y = {n: torch.full((M + 1, N if n == "sigmoid" else N // 2), 7.0, dtype=bf, device="cuda") for n in w}
+    yg = torch.full((M + 1, G * (N + 8)), 7.0, device="cuda")
+    segs = [K.Seg(K.PackedLinear(v, False, "cuda"), X, y[n][:M], n, alpha={"swiglu": 0.9, "sigmoid": 1.5}.get(n, 1.0)) for n, v in w.items()]
+    L = K.LinLaunch(segs + [K.Seg(K.PackedLinear(wg, False, "cuda"), X, yg[:M], xgs=ld, ygs=N + 8)])
+    L._cfg[M] = (True, 7), 1
+    L.run(M, st())
+    z = {n: x[:, :Kd].double() @ v.double().T for n, v in w.items()}
+    g, u = z["swiglu"][:, 0::2].clamp(max=0.9), z["swiglu"][:, 1::2].clamp(-0.9, 0.9)
+    silu = torch.nn.functional.silu
+    want = {"swiglu": g * torch.sigmoid(1.702 * g) * (u + 1), "siluglu": silu(z["siluglu"][:, 0::2]) * z["siluglu"][:, 1::2],
+            "sigmoid": 1.5 * torch.sigmoid(z["sigmoid"])}
+    for n, v in want.items():                        # bf16 outputs round to 2^-9
+        assert relerr(y[n][:M], v) < 3e-3 and (y[n][M] == 7).all(), n
+    o = yg.view(M + 1, G, N + 8)
+    for i in range(G):
+        assert relerr(o[:M, i, :N], x[:, i * Kd:(i + 1) * Kd].double() @ wg[i].double().T) < 2e-6
+    assert (o[:, :, N:] == 7).all() and (o[M] == 7).all()
+
+
 @pytest.mark.parametrize("cfg", [8, 9, 10, 11])
 @pytest.mark.parametrize("M,N,Kd", [(17, 96, 70), (64, 160, 192), (65, 161, 256), (129, 500, 330), (40, 1000, 1000)])
 def test_balanced_tiles(K, cfg, M, N, Kd):
@@ -354,21 +401,3 @@ def test_tile_steps(K, cfg, f32):
             K._check(K.lib().nls_lin_gemm(ctypes.byref(a), int(f32), cfg, st()), "gemm")
             got = y.view(2, M, N)[:ks].sum(0).cpu().double()
             assert ((got - want).abs() <= bound + 2.0 ** -23 * want.abs()).all(), (steps, ks)
-
-
-def test_split_rule():
-    """Splits of K never more than the slabs or an eighth of the steps, and a tile that takes the launch."""
-    from nats_llm_studio_amd.ops import stack as S
-
-    class W:
-        f32 = False
-
-        def __init__(self, N, Kd):
-            self.N, self.K, self.nsub = N, Kd, -(-Kd // 64) * 2
-    for N, Kd in ((4096, 17408), (2048, 5632), (640, 4096), (36000, 2048)):
-        for M in (17, 33, 64, 65, 128, 129, 300, 512):
-            l = S.LinLaunch.__new__(S.LinLaunch)
-            l.f32, l.segs = False, [type("Sg", (), dict(w=W(N, Kd), slabs=8, y=torch.zeros(1, 1)))()]
-            l._tiles = lambda bn, bm, m, N=N: -(-N // bn) * -(-m // bm)
-            cfg, ks = l.split_config(M)
-            assert ks >= 1 and (not cfg[0] or cfg[1] in (0, 3, 5, 6, 7, 10)) and (M <= 64 or cfg[1] in (0, 3) or ks <= min(8, Kd // 512))

@@ -29,3 +29,25 @@ def test_few_rows(N, Kd):
         assert not gemm and nw == 8 and grids[mt, rt] <= 256
         smaller = [t for t in grids if t[0] * t[1] < mt * rt and grids[t] <= 256]
         assert all(t == (2, 2) and M <= 48 for t in smaller)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("N,Kd", [(4096, 17408), (4096, 6144), (2048, 5632), (640, 4096), (36000, 2048), (1030, 2090), (96, 8192)])
+@pytest.mark.parametrize("pad", [64, 512, 4096])
+def test_splits_of_a_launch(N, Kd, pad, f32):
+    """What a launch with slabs runs, over the rows a buffer of `pad` takes: no more splits than slabs, than fit the buffer's rows at the
+    distance the launch sets, or than leave 8 sub-tile pairs to each; a config that exists and takes the launch."""
+    bound = min(pad, 512)
+    rows = max(pad, 8 * bound)
+    L = launch(N, Kd, f32, rows, 8, bound)
+    nsub = L.segs[0].w.nsub
+    for M in sorted({m for b in (1, 9, 16, 17, 32, 33, 64, 65, 128, 129, 200, 256, 300, 512, 513, 601, 1000, 1365, 2047, 2049, 3001, 4096)
+                     for m in (b, pad) if m <= pad}):
+        (gemm, c, *more), ks = L.choice(M)
+        step = L.slab_step(M)
+        assert step >= M and step % 4 == 0 and 1 <= ks <= 8 and ks * step <= max(rows, step)
+        assert ks == 1 or nsub // ks >= 16
+        if gemm:
+            assert c in S.GEMM_TILES and (c != 7 or (not f32 and nsub // 2 // ks >= 3))
+        else:
+            assert c in (1, 2, 4) and more[0] in (4, 8, 16) and more[1] in (1, 2, 4)
