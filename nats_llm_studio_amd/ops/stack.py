@@ -204,8 +204,10 @@ GEMM_RATE_F32 = {6: (0, 1.0, 1.0), 3: (0, 0.98, 0.98), 1: (0, 0.955, 0.955), 0: 
 GEMM_RATE_MID = {8: (0, 0.47, 0.47), 0: (0, 0.51, 0.51), 11: (0, 0.655, 0.655), 6: (0, 1.1, 1.1)}
 
 
-# Microseconds of a round of 256 workgroups of a tile: fixed + per input column (from rounds at K = 1024 .. 17408)
-ROUND_US = {7: (8.0, 0.0215), 3: (8.0, 0.0151), 6: (8.0, 0.0112), 10: (5.0, 0.0075)}
+# Microseconds of a round of 256 workgroups of a tile: fixed + per input column (from rounds at K = 512 .. 17408). With the sum of the slabs
+# behind it, 5 / 10 (64 x 64, 128 x 64): 65 x 640 x 4096 in eight splits 12.2 / 14.5 us, 128 x 1030 x 2090 in four 15.2 / 17.6, 65 x 2048 x 5632 in
+# four / eight 16.5 / 18.6.
+ROUND_US = {7: (8.0, 0.0215), 3: (8.0, 0.0151), 6: (8.0, 0.0112), 10: (5.0, 0.0075), 5: (5.0, 0.0042)}
 
 
 class LinLaunch:
@@ -311,8 +313,8 @@ class LinLaunch:
         return True, self.balanced(M)
 
     def split_config(self, M: int):
-        """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 25 in two
-        of 128 x 64)."""
+        """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the
+        five of 192 x 128 that are chosen; 25 in two of 128 x 64)."""
         n16 = self._tiles(16, 16, M)
         if M <= 16:
             rt = 1 if M <= 8 else 2
@@ -344,7 +346,7 @@ class LinLaunch:
         256 x 256; the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
         s = self.segs[0]
         c, ks = self.cheapest(M, min(s.slabs, s.y.shape[0] // self.slab_step(M)))
-        return ((True, c), ks) if ks > 1 else (self.config(M), 1)
+        return ((True, c), ks) if ks > 1 or c == 5 else (self.config(M), 1)
 
     def slab_step(self, M: int) -> int:
         """Rows from slab to slab: those the segment was bound for, or M of a larger launch, up to a multiple of 4 (the launch that adds
