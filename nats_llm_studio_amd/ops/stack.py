@@ -291,11 +291,13 @@ class LinLaunch:
 
     def balanced(self, M: int) -> int:
         """The GEMM config of launches with up to 64 rows to a tile, which read each weight once: the tile whose rounds of 256 workgroups
-        sum up to the fewest weight rows, the largest of equals (four stages also keep such workgroups from sharing a CU while
-        another has none). In a running step at 64 rows and K = 4096 (64 / 96 / 128 / 160 weight rows): N = 35888 85 / 75 / 98 / 73 us, 34816
-        75 / 68 / 92 / 63, 26880 57 / 68 / 54 / 60, 24576 57 / 53 / 57 / 63, 32000 65 / 76 / 68 / 73; eight experts, N = 6144: 99 / 94 / 107 / 119,
-        and N = 4096 at K = 6144: 115 / 99 / 82 / 85."""
-        return min((10, 9, 8, 0), key=lambda c: (-(-self._tiles(*GEMM_TILES[c], M) // 256) * GEMM_TILES[c][0], -GEMM_TILES[c][0]))
+        sum up to the fewest weight rows; of equals the largest (four stages also keep such workgroups from sharing a CU while
+        another has none), up to 40 rows the smallest. In a running step at 64 rows and K = 4096 (64 / 96 / 128 / 160 weight rows): N = 35888
+        85 / 75 / 98 / 73 us, 34816 75 / 68 / 92 / 63, 24576 57 / 53 / 57 / 63; eight experts, N = 6144: 99 / 94 / 107 / 119, and N = 4096 at
+        K = 6144: 115 / 99 / 82 / 85. Equals, 64 / 128 weight rows, one launch after another: 64 x 26880 50.4 / 44.5, 64 x 32000 54.0 / 52.3
+        (in the step 65 / 68), 24 rows 41.7 / 43.7 and 47.8 / 51.0."""
+        small = 1 if M <= 40 and self.plan is None else -1
+        return min((10, 9, 8, 0), key=lambda c: (-(-self._tiles(*GEMM_TILES[c], M) // 256) * GEMM_TILES[c][0], small * GEMM_TILES[c][0]))
 
     def few_rows(self, M: int, n64: int):
         """17 to 64 rows, bound by the weights' bytes: the streaming kernel with the smallest tiles (weight rows x rows) that give each CU

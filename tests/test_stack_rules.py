@@ -51,3 +51,10 @@ def test_splits_of_a_launch(N, Kd, pad, f32):
             assert c in S.GEMM_TILES and (c != 7 or (not f32 and nsub // 2 // ks >= 3))
         else:
             assert c in (1, 2, 4) and more[0] in (4, 8, 16) and more[1] in (1, 2, 4)
+
+
+def test_equal_rounds():
+    """Wide launches of few rows whose rounds sum up to the same weight rows on two tiles: 64 rows to a tile up to 40 rows, then 128."""
+    for N in (26880, 32000, 32768):
+        assert [launch(N, 4096).config(M) for M in (17, 32, 40, 41, 64)] == [(True, 0)] * 3 + [(True, 10)] * 2
+    assert [launch(35888, 4096).config(M) for M in (24, 64)] == [(True, 9)] * 2
