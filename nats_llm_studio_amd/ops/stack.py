@@ -243,7 +243,10 @@ class LinLaunch:
             if bm == 16:
                 return False, 1, (4 if self._tiles(16, 16, M) >= 1536 else 8), 1
             if bm == 64:
-                return True, 0 if self.f32 else self.balanced(M)
+                # short products are over before the deeper tiles' stages pay: 64 x 64 / chosen by rounds, us: 64 experts of 30 rows, 512 x 2048 28 / 41
+                # and 2048 x 512 35 / 48; 8 of 30, 3072 x 2048 22.5 / 25.9; 32 of 30, 4096 x 1536 86 / 94; at 3072 inputs 24.2 / 23.6, from there
+                # on 8 x 4096 x 6144 95 / 79, 8 x 6144 x 4096 79 / 77
+                return True, 0 if self.f32 or self.segs[0].w.K < 3072 else self.balanced(M)
             if bm == 256:
                 return True, 7
             return True, (3 if self._tiles(256, 128, M) >= 224 else 2)

@@ -58,3 +58,12 @@ def test_equal_rounds():
     for N in (26880, 32000, 32768):
         assert [launch(N, 4096).config(M) for M in (17, 32, 40, 41, 64)] == [(True, 0)] * 3 + [(True, 10)] * 2
     assert [launch(35888, 4096).config(M) for M in (24, 64)] == [(True, 9)] * 2
+
+
+def test_short_expert_products():
+    """Experts of a few dozen rows: tiles by rounds only where the inputs are many."""
+    for N, Kd, want in ((512, 2048, 0), (2048, 512, 0), (3072, 2048, 0), (4096, 6144, 10), (6144, 4096, 8)):
+        L = launch(N, Kd)
+        L.plan, L.segs[0].s.rows = S.MoePlan(120, 8, 2, 1, 1, 1.0, "cpu"), 1
+        L.segs[0].w.groups = 8
+        assert L.plan.bm(120) == 64 and L.config(120) == (True, want), (N, Kd)
