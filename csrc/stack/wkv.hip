@@ -167,8 +167,10 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
     }
     __syncthreads();
     // 8 tokens at a time, the next PF tokens' operands on their way while one is summed (a token's arithmetic takes less than
-    // an LDS read); lane part q keeps token q's output
-    constexpr int PF = R <= 4 ? 3 : 1, RB = PF + 1;
+    // an LDS read); lane part q keeps token q's output. Three tokens ahead, unless f32 values wait one by one in the registers
+    // (VEC false): those then leave room for two waves on a SIMD instead of three (100 runs of 50 tokens, 16 heads of 32: 32.7 us
+    // against 26.7 with one token ahead; 8 runs of 300, 10 heads of 60: 52.0 against 49.2)
+    constexpr int PF = R <= 4 && (VEC || sizeof(T) == 2) ? 3 : 1, RB = PF + 1;
     const int m = min(CH, n - base);
     f32x4 r4[RB][R / 4], k4[RB][R / 4], w4[RB][R / 4];
     float v1[RB][CPL];
