@@ -689,7 +689,8 @@ int nls_splitk_add_rmsnorm(const float* ws, int ks, int M, float alpha, float* x
   return (int)hipGetLastError();
 }
 
-// ks = 0: no slabs, x is normalised as it is. counts: int [E], zeroed; xrows / yrows: int [E][cap], cap >= M
+// ks = 0: no slabs, x is normalised as it is. counts: int [E], zeroed; xrows / yrows: int [E][cap], cap >= M. E: the counts that
+// router_logits takes too, the only ones whose router has an f16 copy [E][D]; a thread holds E partial sums.
 int nls_splitk_add_rmsnorm_route(const float* ws, int ks, int M, float alpha, float* x, long ldx, const float* w,
                                  void* out, long ldo, int D, float eps, const void* wr, int E, int k, int renorm, float* logits,
                                  float* topw, int* counts, int* xrows, int* yrows, int cap, int* sel, void* stream) {

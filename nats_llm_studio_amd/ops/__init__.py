@@ -538,7 +538,9 @@ def qgemv_add_rmsnorm_route(seg: Seg, xin: torch.Tensor, x: torch.Tensor, nw: to
                             sel: Optional[torch.Tensor] = None) -> bool:
     """qgemv_add_rmsnorm, then the router logits of the normalised rows (wr: the router's f16 copy [E, D]) and the top-k route
     (moe_route) in the launch that normalises. `counts` [E] must be zero before. False (nothing done) where the launch does not apply:
-    the caller then runs qgemv_add_rmsnorm, router_logits and moe_route."""
+    the caller then runs qgemv_add_rmsnorm, router_logits and moe_route. 2, 4 or 8 experts: as many as router_logits takes and the
+    model keeps that copy for (a thread holds E partial sums, so E is fixed when the kernel is built); routers of other sizes stay
+    packed and are multiplied as any layer is."""
     E, D = wr.shape
     if (not x.is_cuda or seg.xmap is not None or seg.ycol or seg.w.rows != x.shape[1] or D != x.shape[1] or E not in (2, 4, 8)
             or k > E or D % 8 or D > 8192 or wr.dtype != ACT_DTYPE or not wr.is_contiguous() or logits.stride(0) != E or cap < M):

@@ -192,7 +192,7 @@ GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 5: (64, 6
 # Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
 # phased 256 x 256 tile: a round of 256 workgroups took 88 us at K = 4096 (1.24 PFLOP/s, 1.36 over many rounds), one of 3 (256 x 128)
 # 70 us, one of 6 (192 x 128) 54 us, so it wins where rounds fill: 2000 x 35888 490 us against 743 (3) and 652 (6), 512 x 24576 92
-# against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 298 against 262 (3).
+# against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 297 against 269 (3).
 GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 0.47, 0.72),
              1: (512, 0.5, 0.63), 0: (1024, 0.45, 0.55)}
 # 32-bit operands: bound by the f32 MFMAs (75 to 80 % of the time in any tile), so the rounds decide (64 x 64 / 128 x 64 / 192 x 128 / 256 x 128):
@@ -319,7 +319,7 @@ class LinLaunch:
 
     def split_config(self, M: int):
         """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the
-        five of 192 x 128 that are chosen; 25 in two of 128 x 64)."""
+        five of 192 x 128 that are chosen, 25.5 in two of 128 x 64; 41, 34 and 32 with the launch that adds the slabs)."""
         n16 = self._tiles(16, 16, M)
         if M <= 16:
             rt = 1 if M <= 8 else 2
@@ -347,8 +347,8 @@ class LinLaunch:
 
     def tall_split(self, M: int):
         """(config, K splits) of more rows than slab_rows: as many slabs of M rows as y holds. A narrow product has fewer tiles than
-        there are CUs, or lasts two rounds for a few more. 2000 x 4096 x 17408: 286 us in one round of 256 x 128 -> 222 in two splits of
-        256 x 256; the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
+        there are CUs, or lasts two rounds for a few more. 2000 x 4096 x 17408: 269 us in one round of 256 x 128 -> 209 in two splits of
+        256 x 256 (292 -> 230 with the launch that adds the slabs); the passes of 600 tokens of a model 4096 wide 2446 -> 1895 us."""
         s = self.segs[0]
         c, ks = self.cheapest(M, min(s.slabs, s.y.shape[0] // self.slab_step(M)))
         return ((True, c), ks) if ks > 1 or c == 5 else (self.config(M), 1)
