@@ -154,6 +154,7 @@ int gemm_d(LinArgs& a, int cfg, hipStream_t st) {
     case 1: return gemm_t<T, 128, 64, 4, 1, 3>(a, st);
     case 2: return gemm_t<T, 128, 128, 2, 2, 2>(a, st);
     case 3: return gemm_t<T, 256, 128, 4, 2, 3>(a, st);
+    case 4: return gemm_t<T, 256, 256, 4, 2, 2>(a, st);
     case 5: return gemm_t<T, 64, 64, 2, 2, 8>(a, st);
     case 6: return gemm_t<T, 192, 128, 4, 2, 3>(a, st);
     case 8: return gemm_t<T, 96, 64, 2, 2, 4>(a, st);
@@ -168,9 +169,9 @@ int gemm_d(LinArgs& a, int cfg, hipStream_t st) {
 
 extern "C" {
 
-// cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 5 = 64 x 64 with 8 stages in flight
-// (launches of at most one workgroup per CU), 6 = 192 x 128, 7 = 256 x 256 in phases (bf16), 8 = 96 x 64, 9 = 160 x 64,
-// 10 = 128 x 64 with four stages, 11 = 96 x 128
+// cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256 in two stages (either
+// type; a launch's own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
+// 6 = 192 x 128, 7 = 256 x 256 in phases (bf16), 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
   if (cfg == 7) return f32 ? -1 : nls_lin::lin_phased(a, (hipStream_t)stream);

@@ -185,8 +185,8 @@ class Seg:
 
 
 # (weight rows, rows) of lin_gemm's configs
-GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 5: (64, 64), 6: (192, 128), 7: (256, 256), 8: (96, 64),
-              9: (160, 64), 10: (128, 64), 11: (96, 128)}
+GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 4: (256, 256), 5: (64, 64), 6: (192, 128), 7: (256, 256),
+              8: (96, 64), 9: (160, 64), 10: (128, 64), 11: (96, 128)}
 
 
 # Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
