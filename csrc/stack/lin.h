@@ -89,6 +89,7 @@ template <> struct LT<float> {
 // one workgroup's tile: segment, group, split of K, first weight row, first row, rows
 struct LinTile {
   int seg, grp, ks, n0, m0, cnt;
+  bool once;            // no other tile reads these weights
   const int* rows;      // routed: entries of this tile
 };
 
@@ -121,6 +122,7 @@ DEVI bool lin_tile(const LinArgs& a, int id, LinTile& t) {
     t.rows = S.rows + a.tiles[4 * mi + 1];
     t.cnt = a.tiles[4 * mi + 2];
     t.m0 = 0;
+    t.once = (mi == 0 || a.tiles[4 * mi - 4] != t.grp) && (mi + 1 >= *a.ntiles || a.tiles[4 * mi + 4] != t.grp);
   } else {
     q /= nnt;
     t.grp = S.ng == 1 ? 0 : q % S.ng;
@@ -128,6 +130,7 @@ DEVI bool lin_tile(const LinArgs& a, int id, LinTile& t) {
     t.rows = nullptr;
     t.m0 = mi * BM;
     t.cnt = min(BM, S.M - t.m0);
+    t.once = nmt == 1;
   }
   return true;
 }

@@ -7,11 +7,17 @@
 // in flight. Routed rows (experts) are gathered by the DMA's per-lane source addresses.
 // Tile ids are dealt to the 8 XCDs in contiguous ranges, a few m-tiles innermost (lin_tile): the workgroups that run
 // together on an XCD form a block of weight and row tiles and read both through its L2.
+// Weights of a tile that no other one shares (LinTile::once) come with the non-temporal hint: few rows make a launch a read of the weights, and
+// without the hint they push the rows, caches and states of the step out of the caches (us in a running step, without / with: 64 x 35888 x 4096
+// 75.7 / 59.7, 4.9 TB/s, 64 x 32000 68.7 / 55.5, eight experts of 50 rows 94.5 / 76.3 and 83.0 / 78.0). Weights of two row tiles need the L2 for the
+// second one's read: with the hint eight experts of 75 rows took 142 -> 163 us.
+#include <type_traits>
 #include "../kernels/lds_dma.h"
 #include "lin.h"
 
 namespace nls_lin {
 using nls_dma::glds16;
+using nls_dma::glds16_nt;
 using nls_dma::lds_addr;
 using nls_dma::wait_vm_lgkm0;
 
@@ -67,11 +73,14 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr(lglds));
   const uint32_t wl = base + (uint32_t)(NW * wave) * 1024u;
   const uint32_t xl = base + G::WST + (uint32_t)(NX * wave) * 1024u;
-  auto dma = [&](int j, int stage) __attribute__((always_inline)) {     // step j (clamped) -> stage
+  auto dma = [&](int j, int stage, auto once) __attribute__((always_inline)) {     // step j (clamped) -> stage
     const int jc = jb + min(j, nst - 1);
     const uint32_t so = (uint32_t)stage * G::STG;
 #pragma unroll
-    for (int i = 0; i < NW; ++i) glds16(wsrc[i] + (size_t)jc * 2048, wl + so + i * 1024);
+    for (int i = 0; i < NW; ++i) {
+      if constexpr (decltype(once)::value) glds16_nt(wsrc[i] + (size_t)jc * 2048, wl + so + i * 1024);
+      else glds16(wsrc[i] + (size_t)jc * 2048, wl + so + i * 1024);
+    }
 #pragma unroll
     for (int i = 0; i < NX; ++i) glds16(xsrc[i >> 1] + (size_t)(2 * jc + (i & 1)) * L::KS, xl + so + i * 1024);
   };
@@ -98,26 +107,30 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
     }
   };
   constexpr int FL = (NST - 2) * (NW + NX);           // DMA instructions left in flight across the barrier
-#pragma unroll
-  for (int j = 0; j < NST - 1; ++j) dma(j, j);
-  wait_vm_lgkm0<FL>();
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
   // step j is in stage j % NST: NST steps to a pass of the loop, so that stages are constants and the accumulators stay where they are
-  auto turn = [&](int j, int stage) __attribute__((always_inline)) {
-    dma(j + NST - 1, (stage + NST - 1) % NST);        // that stage was last read in step j - 1: retired
+  auto turn = [&](int j, int stage, auto once) __attribute__((always_inline)) {
+    dma(j + NST - 1, (stage + NST - 1) % NST, once);  // that stage was last read in step j - 1: retired
     step(stage);
     wait_vm_lgkm0<FL>();
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  int j0 = 0;
-  for (; j0 + NST <= nst; j0 += NST)
+  auto walk = [&](auto once) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < NST; ++s) turn(j0 + s, s);
+    for (int j = 0; j < NST - 1; ++j) dma(j, j, once);
+    wait_vm_lgkm0<FL>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    int j0 = 0;
+    for (; j0 + NST <= nst; j0 += NST)
 #pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (j0 + s < nst) turn(j0 + s, s);                // (uniform)
+      for (int s = 0; s < NST; ++s) turn(j0 + s, s, once);
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+      if (j0 + s < nst) turn(j0 + s, s, once);        // (uniform)
+  };
+  if (__builtin_amdgcn_readfirstlane(t.once)) walk(std::true_type{});
+  else walk(std::false_type{});
   wait_vm_lgkm0<0>();                                 // the clamped tail DMAs land before the workgroup's LDS is freed
 #pragma unroll
   for (int j = 0; j < MTW; ++j) {

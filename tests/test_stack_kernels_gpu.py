@@ -401,3 +401,21 @@ def test_tile_steps(K, cfg, f32):
             K._check(K.lib().nls_lin_gemm(ctypes.byref(a), int(f32), cfg, st()), "gemm")
             got = y.view(2, M, N)[:ks].sum(0).cpu().double()
             assert ((got - want).abs() <= bound + 2.0 ** -23 * want.abs()).all(), (steps, ks)
+
+
+@pytest.mark.parametrize("T,E", [(24, 4), (100, 8), (300, 8)])
+def test_experts_of_one_and_of_several_tiles(K, T, E):
+    """Experts' row lists in tiles of 64 rows: lists of one tile beside longer ones (their weights are fetched in different ways)."""
+    bf, d, n = torch.bfloat16, 330, 200
+    x, z, w = rnd(T, d, seed=1).to(bf), rnd(T, E, seed=2).float(), (rnd(E, n, d, seed=3) * d ** -0.5).to(bf)
+    z[:, 1] += 2.0
+    plan = K.MoePlan(T, E, 2, 1, 1, 1.0, "cuda")
+    assert plan.bm(T) == 64
+    y, W = torch.zeros(2 * T, n, device="cuda"), K.PackedLinear(w, False, "cuda")
+    plan.run(z.cuda(), T, st())
+    K.LinLaunch([K.Seg(W, act(x, K.act_ld(d)), y, routed=(plan.rows, 2))], plan).run(T, st())
+    sel = plan.sel.cpu().long()
+    rows = sel.bincount(minlength=E)
+    assert T == 24 or (rows.max() > 64 and rows.min() <= 64)
+    want = torch.stack([w[e].double() @ x[i // 2].double() for i, e in enumerate(sel.tolist())])
+    assert relerr(y, want) < 2e-6
