@@ -63,6 +63,7 @@ def replay(eng, lines, out_dir: str, reply):
             rows.numpy().astype("<f4").tofile(os.path.join(out_dir, f"{step['step']}.f32"))
         for rid in step.get("end", []):
             eng.feed_end(rid)
+        eng.feed_wait()
         reply(f"done {step['step']}")
 
 

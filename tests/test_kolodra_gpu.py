@@ -467,6 +467,53 @@ def test_feed_schedules(gpu, tmp_path, dt, name):
 
 
 @pytest.mark.parametrize("dt", DT)
+def test_feed_steps_under_way(gpu, tmp_path, dt):
+    """Steps without wanted places are not waited for: pages that are added, requests that end and others that take their rows, pages
+    and slots while steps are under way, another stream, and a generation behind them change no logits."""
+    from nats_llm_studio_amd.engine.sampling import SamplingParams
+    cfg = S.CONFIGS["uneven"]
+    W = S.make_weights(cfg)
+    eng = engine(load(tmp_path, cfg, W, dt))
+    seqs = {k: S.tokens(60, cfg["vocab"], 20 + i) for i, k in enumerate("abcdef")}
+    want = {k: O.forward(cfg, W, t)[-1:] for k, t in seqs.items()}
+    alone = eng.generate(seqs["a"][:9], SamplingParams(max_tokens=6, ignore_eos=True)).token_ids
+    at = dict.fromkeys(seqs, 0)
+
+    def step(n, *ks, last=()):
+        ent = [(k, seqs[k][at[k]:at[k] + n], [n - 1] if k in last else []) for k in ks]
+        for k in ks:
+            at[k] += n
+        return dict(zip(ks, eng.feed(ent)))
+    step(20, "a", "b")
+    for _ in range(39):
+        step(1, "a", "b")                       # (two pages further)
+    assert eng._flight is not None
+    eng.feed_end("b")                           # not wanted: its row goes to "c"
+    step(30, "c")
+    got = step(1, "a", "c", last="a")["a"]
+    assert at["a"] == 60 and close(got, want["a"], dt)
+    eng.feed_end("a")
+    side = torch.cuda.Stream()
+    step(29, "d")
+    with torch.cuda.stream(side):
+        for _ in range(28):
+            step(1, "c", "d")
+    for _ in range(3):                          # (31 + 28: the two are at their 59th and 57th token)
+        got = step(1, "d", last="d" if at["d"] == 59 else ())
+    assert close(got["d"], want["d"], dt)
+    assert close(step(1, "c", last="c")["c"], want["c"], dt)
+    step(12, "e")
+    step(1, "e")
+    for k in "cde":
+        eng.feed_end(k)
+    assert eng._flight is None and eng.alloc.n_free == eng.num_blocks and len(eng.slots.free) == 4
+    step(12, "f")
+    step(1, "f")                                # left under way and live
+    assert eng.generate(seqs["a"][:9], SamplingParams(max_tokens=6, ignore_eos=True)).token_ids == alone
+    assert eng._flight is None
+
+
+@pytest.mark.parametrize("dt", DT)
 def test_long_prompt_segments(gpu, tmp_path, dt):
     """A prompt long enough that the recurrence runs in segments, alone and beside other runs, then decoded on."""
     cfg = S.CONFIGS["uneven"]

@@ -245,6 +245,31 @@ def test_engine_feed_bookkeeping():
         eng.feed([("d", [64], [])])
 
 
+@pytest.mark.parametrize("n", [8, 9, 30])
+def test_engine_rows_of_many_prompts(n):
+    """The staged rows of few and of many portions: ids, positions, slots, contexts, block tables and runs."""
+    from nats_llm_studio_amd.engine.engine import Engine
+    eng = Engine(_FakeRecurrent(), None, max_batch=32, num_blocks=400, max_prefill_tokens=512, ctx=96, use_graphs=False)
+    rng = np.random.RandomState(n)
+    parts = []
+    for i in range(n):
+        p0, c = int(rng.randint(0, 60)), int(rng.randint(1, 16))
+        s = type("Seq", (), dict(blocks=rng.permutation(400)[:(p0 + c) // 16 + 1].tolist(), state_slot=int(rng.randint(32))))()
+        parts.append((s, p0, rng.randint(0, 64, c).tolist()))
+    T = eng._fill_rows(parts)
+    pad, h = eng.pb.pad, eng.h_meta_p.numpy()
+    bt, runs = eng._tables(eng.h_meta_p, pad)
+    at = 0
+    for i, (s, p0, toks) in enumerate(parts):
+        c = len(toks)
+        pos = list(range(p0, p0 + c))
+        rows = [h[k * pad + at:k * pad + at + c].tolist() for k in range(6)]
+        assert rows == [toks, pos, [s.blocks[p // 16] * 16 + p % 16 for p in pos], [i] * c, [p + 1 for p in pos], [0] * c]
+        assert bt[i, :len(s.blocks)].tolist() == s.blocks and runs[i].tolist() == [at, c, s.state_slot, p0]
+        at += c
+    assert at == T
+
+
 def test_engine_feed_results_are_their_own():
     """Results share no memory with those of other entries, wherever their rows came from: a kept row keeps no more than itself."""
     from nats_llm_studio_amd.engine.engine import Engine
