@@ -328,22 +328,18 @@ DEVI void hgemm_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs&
 
 template <int WM, int BN, int NWV, int NST>
 __global__ __launch_bounds__(64 * NWV, NST == 2 ? 2 : 1) void hgemm_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
-                                                       int nmb) {
+                                                       int nmb, int slots) {
   extern __shared__ __attribute__((aligned(16))) uint8_t hlds[];
   constexpr int BM = HG<WM, BN, NWV, NST>::BM;
-  // (tile, m-block, k-slice) with all m-blocks and k-slices of a tile on one XCD
-  const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
-  const int kslice = j % ks;
-  const int mb = (j / ks) % nmb;
-  const int tile = (j / ks / nmb) * 8 + xcd;
-  if (tile >= ntiles) return;
-  const int m0 = mb * BM;
+  Block b;
+  if (!launch_block<BM>(segs, a, ks, ntiles, nmb, slots, b)) return;
+  const int kslice = b.kslice, tile = b.tile, m0 = b.mb * BM;
   Seg S = segs.s[0];
 #pragma unroll
   for (int s = 1; s < 8; ++s)
     if (s < segs.nseg && tile >= segs.s[s].tile_begin) S = segs.s[s];
   // MoE grouped GEMM (as mode 2): the expert's routed-row count lives on the device; m-blocks past it
-  // exit before issuing any DMA (the grid is sized for every routed row on one expert)
+  // exit before issuing any DMA
   const int mrows = S.mcount ? min(*S.mcount, a.M) : a.M;
   if (m0 >= mrows) return;
   const int* xm = S.xmap ? S.xmap + m0 : nullptr;
@@ -361,7 +357,7 @@ template <int WM, int BN, int NWV, int NST>
 int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   typedef HG<WM, BN, NWV, NST> G;
   const int nmb = (a.M + G::BM - 1) / G::BM;
-  const int grid = ((ntiles + 7) / 8) * 8 * nmb * ks;
+  const int slots = grouped_slots(sl, a, G::BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)hgemm_kernel<WM, BN, NWV, NST>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -369,7 +365,7 @@ int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((hgemm_kernel<WM, BN, NWV, NST>), dim3(grid), dim3(G::NT), G::LDS, st, sl, a, ks, ws, ntiles, nmb);
+  hipLaunchKernelGGL((hgemm_kernel<WM, BN, NWV, NST>), dim3(grid), dim3(G::NT), G::LDS, st, sl, a, ks, ws, ntiles, nmb, slots);
   return (int)hipGetLastError();
 }
 

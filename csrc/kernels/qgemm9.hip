@@ -418,28 +418,23 @@ constexpr int kset_lds() {
 
 // NWV = 8: two waves per SIMD (256 registers); NWV = 4: one wave per SIMD with up to 512 registers, so a
 // wave holds 4 weight tiles x 16 activation tiles of accumulators (half the LDS reads per MFMA).
-// BM = 64 (mode 12, the MoE experts' grouped GEMM): segments may be mapped -- each expert's routed rows are
-// gathered through xmap and scattered through ymap, and m-blocks past the expert's device-side row count
-// exit before reading any weights (the grid is sized for every token on one expert)
-template <int KSET, int RT, int NWV, int BM>
+// MAP (experts): each one's routed rows are gathered through xmap and scattered through ymap; a build of its own, the plain one keeps its
+// registers.
+template <int KSET, int RT, int NWV, int BM, bool MAP>
 __global__ __launch_bounds__(64 * NWV, 1) void qgemm9_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
-                                                          int nmb) {
+                                                          int nmb, int slots) {
   extern __shared__ __attribute__((aligned(16))) uint8_t q9lds[];
-  const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
-  const int kslice = j % ks;
-  const int mb = (j / ks) % nmb;
-  const int tile = (j / ks / nmb) * 8 + xcd;
-  if (tile >= ntiles) return;
-  const int m0 = mb * BM;
+  Block b;
+  if (!launch_block<BM>(segs, a, ks, ntiles, nmb, MAP ? slots : 0, b)) return;
+  const int kslice = b.kslice, tile = b.tile, m0 = b.mb * BM;
   Seg S = segs.s[0];
 #pragma unroll
   for (int s = 1; s < 8; ++s)
     if (s < segs.nseg && tile >= segs.s[s].tile_begin) S = segs.s[s];
-  // mapped rows only at BM 64 (the dispatcher refuses them for mode 9): the 256-row build keeps mode 9's code
-  const int mrows = (BM == 64 && S.mcount) ? min(*S.mcount, a.M) : a.M;
+  const int mrows = (MAP && S.mcount) ? min(*S.mcount, a.M) : a.M;
   if (m0 >= mrows) return;
-  const int* xm = (BM == 64 && S.xmap) ? S.xmap + m0 : nullptr;
-  const int* ym = (BM == 64 && S.ymap) ? S.ymap + m0 : nullptr;
+  const int* xm = (MAP && S.xmap) ? S.xmap + m0 : nullptr;
+  const int* ym = (MAP && S.ymap) ? S.ymap + m0 : nullptr;
   a.m0 = m0;
   if (!xm) a.x += (size_t)m0 * a.ldx;
   const size_t esz = (a.epi == EPI_F32 || a.epi == EPI_ADD_F32 || a.epi == EPI_ARGMAX) ? 4 : 2;
@@ -461,20 +456,20 @@ __global__ __launch_bounds__(64 * NWV, 1) void qgemm9_kernel(SegList segs, GemvA
   }
 }
 
-template <int KSET, int RT, int NWV, int BM>
+template <int KSET, int RT, int NWV, int BM, bool MAP>
 int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   constexpr int lds = kset_lds<KSET, RT, NWV, BM>();
   const int nmb = (a.M + BM - 1) / BM;
-  const int grid = ((ntiles + 7) / 8) * 8 * nmb * ks;
+  const int slots = MAP ? grouped_slots(sl, a, BM) : 0, grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
-    if (hipFuncSetAttribute((const void*)qgemm9_kernel<KSET, RT, NWV, BM>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)qgemm9_kernel<KSET, RT, NWV, BM, MAP>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             lds) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((qgemm9_kernel<KSET, RT, NWV, BM>), dim3(grid), dim3(64 * NWV), lds, st, sl, a, ks, ws, ntiles,
-                     nmb);
+  hipLaunchKernelGGL((qgemm9_kernel<KSET, RT, NWV, BM, MAP>), dim3(grid), dim3(64 * NWV), lds, st, sl, a, ks, ws, ntiles,
+                     nmb, slots);
   return (int)hipGetLastError();
 }
 
@@ -484,9 +479,11 @@ int launch_k(int waves, int rt, int bm, const SegList& sl, int ntiles, int ks, f
   // bm 64 (the round-5 "mode 12" MoE variant, 2.6-3.1x slower than mode 2 on Mixtral's experts) is no longer
   // instantiated: the template keeps the geometry, the default build does not carry the code
   if (bm != 256) return -1;
-  if (waves == 4 && rt == 2) return launch_t<KSET, 2, 4, 256>(sl, ntiles, ks, ws, a, st);
-  if (waves == 8 && rt == 2) return launch_t<KSET, 2, 8, 256>(sl, ntiles, ks, ws, a, st);
-  if (waves == 8 && rt == 1) return launch_t<KSET, 1, 8, 256>(sl, ntiles, ks, ws, a, st);
+  if (sl.s[0].xmap || sl.s[0].ymap || sl.s[0].mcount)
+    return waves == 8 && rt == 2 ? launch_t<KSET, 2, 8, 256, true>(sl, ntiles, ks, ws, a, st) : -1;
+  if (waves == 4 && rt == 2) return launch_t<KSET, 2, 4, 256, false>(sl, ntiles, ks, ws, a, st);
+  if (waves == 8 && rt == 2) return launch_t<KSET, 2, 8, 256, false>(sl, ntiles, ks, ws, a, st);
+  if (waves == 8 && rt == 1) return launch_t<KSET, 1, 8, 256, false>(sl, ntiles, ks, ws, a, st);
   return -1;
 }
 

@@ -297,21 +297,18 @@ DEVI void dma_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
 // other's MFMAs, where the 128 / 256-row blocks own a CU each.
 template <int MT, int KSET>
 __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void qmm_dma_kernel(SegList segs, GemvArgs a, int ks, float* ws,
-                                                                        int ntiles, int nmb) {
+                                                                        int ntiles, int nmb, int slots) {
   extern __shared__ __attribute__((aligned(16))) uint8_t dlds[];
   constexpr int BM = MT * 16;
-  const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
-  const int kslice = j % ks;
-  const int mb = (j / ks) % nmb;
-  const int tile = (j / ks / nmb) * 8 + xcd;
-  if (tile >= ntiles) return;
+  Block b;
+  if (!launch_block<BM>(segs, a, ks, ntiles, nmb, slots, b)) return;
+  const int kslice = b.kslice, tile = b.tile;
   Seg S = segs.s[0];
 #pragma unroll
   for (int s = 1; s < 8; ++s)
     if (s < segs.nseg && tile >= segs.s[s].tile_begin) S = segs.s[s];
-  const int m0 = mb * BM;
+  const int m0 = b.mb * BM;
   // MoE grouped GEMM: the expert's routed-row count lives on the device; m-blocks past it exit before any DMA
-  // (the grid is sized for the worst case, every token on one expert)
   const int mrows = S.mcount ? min(*S.mcount, a.M) : a.M;
   if (m0 >= mrows) return;
   const int* xm = S.xmap ? S.xmap + m0 : nullptr;
@@ -347,7 +344,7 @@ int launch_dma_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArg
   constexpr int BM = MT * 16;
   const int nmb = (a.M + BM - 1) / BM;
   const size_t lds = dma_lds_bytes<MT>();
-  const int grid = ((ntiles + 7) / 8) * 8 * nmb * ks;
+  const int slots = grouped_slots(sl, a, BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)qmm_dma_kernel<MT, KSET>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -355,7 +352,7 @@ int launch_dma_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArg
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((qmm_dma_kernel<MT, KSET>), dim3(grid), dim3(256), lds, st, sl, a, ks, ws, ntiles, nmb);
+  hipLaunchKernelGGL((qmm_dma_kernel<MT, KSET>), dim3(grid), dim3(256), lds, st, sl, a, ks, ws, ntiles, nmb, slots);
   return (int)hipGetLastError();
 }
 

@@ -343,22 +343,18 @@ DEVI void lds_tile_na(int na, const Seg& S, int row0, int kslice, int ks, const 
 
 template <int WM, int KSET>
 __global__ __launch_bounds__(512) void qmm_lds_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
-                                                      int nmb) {
+                                                      int nmb, int slots) {
   extern __shared__ __attribute__((aligned(16))) act_t lds[];
   constexpr int BM = WM * 64;
-  // (tile, m-block, k-slice) with all m-blocks and k-slices of a tile on one XCD
-  const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
-  const int kslice = j % ks;
-  const int mb = (j / ks) % nmb;
-  const int tile = (j / ks / nmb) * 8 + xcd;
-  if (tile >= ntiles) return;
-  const int m0 = mb * BM;
+  Block b;
+  if (!launch_block<BM>(segs, a, ks, ntiles, nmb, slots, b)) return;
+  const int kslice = b.kslice, tile = b.tile, m0 = b.mb * BM;
   Seg S = segs.s[0];
 #pragma unroll
   for (int s = 1; s < 8; ++s)
     if (s < segs.nseg && tile >= segs.s[s].tile_begin) S = segs.s[s];
   // MoE grouped GEMM: the expert's routed-row count lives on the device; m-blocks past it exit
-  // before reading any weights (the grid is sized for the worst case, every token on one expert)
+  // before reading any weights
   const int mrows = S.mcount ? min(*S.mcount, a.M) : a.M;
   if (m0 >= mrows) return;
   const int* xm = S.xmap ? S.xmap + m0 : nullptr;
@@ -393,7 +389,7 @@ int launch_lds_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArg
   constexpr int BM = WM * 64;
   const int nmb = (a.M + BM - 1) / BM;
   const size_t lds = (size_t)2 * (BM + 128) * 64 * sizeof(act_t);
-  const int grid = ((ntiles + 7) / 8) * 8 * nmb * ks;
+  const int slots = grouped_slots(sl, a, BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)qmm_lds_kernel<WM, KSET>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -401,7 +397,7 @@ int launch_lds_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArg
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((qmm_lds_kernel<WM, KSET>), dim3(grid), dim3(512), lds, st, sl, a, ks, ws, ntiles, nmb);
+  hipLaunchKernelGGL((qmm_lds_kernel<WM, KSET>), dim3(grid), dim3(512), lds, st, sl, a, ks, ws, ntiles, nmb, slots);
   return (int)hipGetLastError();
 }
 

@@ -39,6 +39,7 @@ struct NlsFuse {
   const int* sel; int sel_slots, sel_base, pad1;                             // device-selected segments
   const void* wr; int E, topk, renorm, rcap;                                 // MoE route after the norm (onw)
   float* rlogits; float* topw; int* counts; int* xrows; int* yrows; int* rsel;
+  int nrows, pad2;                                                           // rows of a grouped launch (GemvArgs)
 };
 
 // mode 0: path A (waves split K, LDS reduce; mapped rows / MoE capable)
@@ -114,8 +115,10 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
     if (!((waves == 4 && rt == 2) || (waves == 8 && (rt == 2 || rt == 1))) || fz->xf || fz->onw || epi == EPI_ROPE || ldx % 8 ||
         ((epi == EPI_F32 || epi == EPI_ADD_F32 || epi == EPI_ACT) && ldy % 4))
       return -1;
+    const bool mapped = segs[0].xmap || segs[0].ymap || segs[0].mcount;      // (experts: all segments or none)
+    if (mapped && (waves != 8 || rt != 2 || ks > 1)) return -1;
     for (int i = 0; i < nseg; ++i)
-      if (segs[i].xmap || segs[i].ymap || segs[i].mcount || segs[i].ycol % 4) return -1;
+      if ((segs[i].xmap || segs[i].ymap || segs[i].mcount) != mapped || segs[i].ycol % 4) return -1;
   } else if (mode >= 4 && mode <= 6) {
     if ((waves != 8 && waves != 16) || (rt != 2 && rt != 4) || fz->xf || fz->onw || (epi == EPI_ROPE && mode == 6))
       return -1;
@@ -139,11 +142,11 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
   for (int i = 0; i < nseg; ++i) {
     if (segs[i].K % 256 || segs[i].rows < 1) return -1;
     if (epi == EPI_SWIGLU && segs[i].rows % 16) return -1;
-    // mapped rows (MoE): path A, or path B / the LDS-dequant / LDS-DMA / dense GEMMs (modes 1-5) without
+    // mapped rows (MoE): path A, or path B / the LDS-dequant / LDS-DMA / dense GEMMs (modes 1-5, 9 unsplit) without
     // arg-max; split-K only as "mapped split-K" (every segment an expert writing the same output
     // columns of its own y rows, f32 store)
     if ((segs[i].xmap || segs[i].ymap || segs[i].mcount) && mode != 0 &&
-        (!(mode >= 1 && mode <= 5) || argmax || epi == EPI_SLABS || (ks > 1 && !mks)))
+        (!((mode >= 1 && mode <= 5) || mode == 9) || argmax || epi == EPI_SLABS || (ks > 1 && !mks)))
       return -1;
     sl.s[i].w = (const uint8_t*)segs[i].w;
     sl.s[i].xmap = segs[i].xmap;
@@ -218,6 +221,7 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
   a.xrows = fz->xrows;
   a.yrows = fz->yrows;
   a.rsel = fz->rsel;
+  a.nrows = fz->nrows;
   a.ssq_out = fz->ssq_out;
   a.ssq_in = fz->ssq_in;
   a.ldss = fz->ldss;

@@ -70,7 +70,59 @@ struct GemvArgs {
   // norm + router + route launch folded away. counts [E] are zeroed here first.
   const act_t* wr; int E, topk, renorm, rcap;
   float* rlogits; float* topw; int* counts; int* xrows; int* yrows; int* rsel;
+  int nrows;          // grouped launches (grouped_slots): rows of all segments together, at most (0: not known)
 };
+
+// Grouped launches (experts: segments of one shape with device row counts) of the tiled GEMMs. In a grid of (tile, every block of BM rows that an
+// expert might have) most workgroups have no rows and exit at once, at a fixed period of the workgroup ids; an XCD deals its workgroups to the
+// shader engines in turn, so those with rows meet on some of the engines while the others idle (eight experts of 8192 x 2048, 1000 tokens of two
+// each, one block of four with rows: 358 us). So the workgroups number the blocks that do have rows, through the counts, one after another for
+// each weight tile, and those without work are the last of the grid (151 us). The grid holds, for a weight tile, as many blocks as all rows can
+// fill: rows / BM and a part block for each segment.
+inline int grouped_slots(const SegList& sl, const GemvArgs& a, int BM) {
+  for (int s = 0; s < sl.nseg; ++s)
+    if (!sl.s[s].mcount || sl.s[s].rows != sl.s[0].rows) return 0;
+  const int nmb = (a.M + BM - 1) / BM;
+  return a.nrows > 0 ? min(sl.nseg * nmb, a.nrows / BM + sl.nseg) : sl.nseg * nmb;
+}
+
+// Workgroup -> (k slice, block of rows, tile), every block and k slice of a weight tile on one XCD. slots: of a grouped launch, else 0.
+struct Block {
+  int kslice, mb, tile;
+};
+template <int BM>
+DEVI bool launch_block(const SegList& segs, const GemvArgs& a, int ks, int ntiles, int nmb, int slots, Block& b) {
+  const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
+  b.kslice = j % ks;
+  if (!slots) {
+    b.mb = (j / ks) % nmb;
+    b.tile = (j / ks / nmb) * 8 + xcd;
+    return b.tile < ntiles;
+  }
+  const int per = ntiles / segs.nseg;
+  int n[8], all = 0;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    n[s] = s < segs.nseg ? (min(*segs.s[s].mcount, a.M) + BM - 1) / BM : 0;
+    all += n[s];
+  }
+  const int q = j / ks, t = all ? q / all * 8 + xcd : per;
+  if (t >= per) return false;
+  int at = q % all;
+  b.mb = -1;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    if (b.mb < 0 && at < n[s]) {
+      b.mb = at;
+      b.tile = s * per + t;
+    }
+    at -= n[s];
+  }
+  return true;
+}
+inline int block_grid(const SegList& sl, int ntiles, int ks, int nmb, int slots) {
+  return slots ? (ntiles / sl.nseg + 7) / 8 * 8 * slots * ks : (ntiles + 7) / 8 * 8 * nmb * ks;
+}
 
 // inv[m] = 1 / rms of rows m < M from producer partial sums of squares (see GemvArgs::ssq_in); one
 // wave per row, lanes sum the shares in a fixed order; ends with a workgroup barrier

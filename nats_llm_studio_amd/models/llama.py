@@ -650,20 +650,13 @@ class LlamaModel:
             gu = dict(zip(("mode", "waves", "rt"), _MOE_DENSE_GU[:3]), ks=1)
             dn = dict(zip(("mode", "waves", "rt"), _MOE_DENSE_DN[:3]), ks=1)
             return gu, dn, (_MOE_DENSE_DN[3] if len(_MOE_DENSE_DN) > 3 else 1)
-        # few routed rows per expert: 128-row blocks (64 KiB of LDS, two workgroups per CU hide each
-        # other's dequant/barrier waits; Mixtral B=64: 13.8 vs 15.2 ms/step), else 256-row blocks
-        rt = 2 if rows < 32 * n_exp else 4
-        gu = dict(mode=2, waves=8, rt=int(os.environ.get("NLS_MOE_RT_GU", rt)), ks=1)
-        dn = dict(mode=2, waves=8, rt=int(os.environ.get("NLS_MOE_RT_DN", rt)), ks=1)
-        kdn = int(os.environ.get("NLS_MOE_KS_DN", "1"))
-        kquant = all(int(w.type) in (12, 13, 14) for w in lw.exp_gateup + lw.exp_down)   # the DMA GEMM's types
-        if kquant and 32 * n_exp <= rows <= 96 * n_exp and os.environ.get("NLS_MOE_DMA", "1") == "1":
-            # ~32-96 routed rows per expert (Mixtral B=128-384): gate|up on the LDS-DMA GEMM over 96-row blocks at
-            # two workgroups per CU, the DMA gathering each expert's rows (286 -> 260 us per launch in the model).
-            # The down projection stays on mode 2 unsplit: in the model (Mixtral-8x7B B=256, one box) 16.45
-            # ms/step vs 16.63 with mode 3 split 4 and 18.24 split 2 (profiles/moe_dma_r06.txt; the isolated
-            # probe's 168 vs 285 us did not carry over -- the model's mode-2 down runs at ~144 us)
-            gu = dict(mode=3, waves=4, rt=6, ks=1)
+        kdn, dma = int(os.environ.get("NLS_MOE_KS_DN", "1")), os.environ.get("NLS_MOE_DMA", "1") == "1"
+        gu, dn = (dict(zip(("mode", "waves", "rt", "ks"), tuning.expert_gemm(ws[:8], rows / n_exp, dma)))
+                  for ws in (lw.exp_gateup, lw.exp_down))
+        if "NLS_MOE_RT_GU" in os.environ:
+            gu = dict(mode=2, waves=8, rt=int(os.environ["NLS_MOE_RT_GU"]), ks=1)
+        if "NLS_MOE_RT_DN" in os.environ or kdn > 1:
+            dn = dict(mode=2, waves=8, rt=int(os.environ.get("NLS_MOE_RT_DN", 2 if rows < 32 * n_exp else 4)), ks=1)
         few = LlamaModel._moe_few_cfg(lw, T, rows / n_exp)
         gu = gu if "NLS_MOE_RT_GU" in os.environ else few[0] or gu
         dn = dn if "NLS_MOE_RT_DN" in os.environ or kdn > 1 else few[1] or dn
@@ -734,10 +727,10 @@ class LlamaModel:
             M = min(nr, T)                                # an expert gets each token at most once
             segs = [Seg(w, 0, rows[i * cap:], rows[i * cap:], counts[i:i + 1]) for i, w in enumerate(lw.exp_gateup)]
             for s0 in range(0, per, 8):
-                ops.qgemv(segs[s0:s0 + 8], xr, b.act, M, epi="swiglu", **gu)
+                ops.qgemv(segs[s0:s0 + 8], xr, b.act, M, epi="swiglu", routed=nr, **gu)
             segs = [Seg(w, 0, rows[i * cap:], rows[i * cap:], counts[i:i + 1]) for i, w in enumerate(lw.exp_down)]
             for s0 in range(0, per, 8):
-                ops.qgemv(segs[s0:s0 + 8], b.act, m["yexp"], M, epi="f32", **dn)
+                ops.qgemv(segs[s0:s0 + 8], b.act, m["yexp"], M, epi="f32", routed=nr, **dn)
         # combine: the outputs return to the slice's rank in dispatch order -> slot order -> weighted sum
         yb = comm.all_to_all_rows(m["yexp"][:nr], recv, send)
         ys = torch.empty_like(yb)
@@ -801,8 +794,6 @@ class LlamaModel:
             if kdn > 1 and len(self.experts) <= 8 and not self.ep and T * k >= 48 * len(self.experts):
                 dn["ks"] = kdn
                 dn_rows = T * k
-            elif dn.get("mode") == 3:
-                dn = dict(mode=2, waves=8, rt=4, ks=1)      # unsplit, the LDS-dequant GEMM is ahead (285 vs 300 us)
         for c0 in range(0, T, step):
             n = min(step, T - c0)
             # few tokens: the route kernel also lists each (token, slot)'s expert and the expert GEMVs
@@ -819,13 +810,13 @@ class LlamaModel:
             def sel(s0):
                 return (m["sel"], n * k, self.experts[0] + s0) if use_sel else None
             for s0 in range(0, len(segs), 8):
-                ops.qgemv(segs[s0:s0 + 8], b.h[c0:], b.act, n, epi="swiglu", sel=sel(s0), **gu)
+                ops.qgemv(segs[s0:s0 + 8], b.h[c0:], b.act, n, epi="swiglu", sel=sel(s0), routed=n * k, **gu)
             if self.ep and not exch:           # rows routed to other ranks' experts stay zero
                 m["yexp"][:n * k].zero_()
             segs = [Seg(dn, 0, m["yrows"][e * cap:], m["yrows"][e * cap:], counts[e:e + 1]) for e, _, dn in loc]
             for s0 in range(0, len(segs), 8):
                 ops.qgemv(segs[s0:s0 + 8], b.act, m["yexp"], dn_rows if dn.get("ks", 1) > 1 else n, epi="f32",
-                          sel=sel(s0), **dn)
+                          sel=sel(s0), routed=n * k, **dn)
             xs = b.x[c0:c0 + n]
             if exch:
                 # every rank ends with all n * k expert rows (its own pushed, the peers' received): the single-GPU

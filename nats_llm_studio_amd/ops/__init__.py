@@ -342,12 +342,13 @@ def norm_fusable(M: int, K: int) -> bool:
 
 def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: float = 1.0, epi: str = "f32",
           argmax: Optional[torch.Tensor] = None, waves: int = 0, rt: int = 1, mode: int = -1, ks: int = 1,
-          norm=None, sel=None):
+          norm=None, sel=None, routed: int = 0):
     """y (epilogue) alpha * x[:M] @ W^T for each segment. x: f16 [>=pad16(M), K].
     norm = (xf f32 [M, K], w f32 [K], eps[, ssq, ldss, nparts]): the GEMV input is f16(rmsnorm(xf) * w),
     computed inside the kernel (batch <= a few rows; `x` is then ignored on the GPU). With the partial
     sums of squares a qgemv_add_ssq producer left in `ssq`, the kernel skips the reduction pass and the
-    tuned path-B (XL) config stays usable."""
+    tuned path-B (XL) config stays usable.
+    routed: experts' segments together have at most so many rows (their launch then holds few blocks without any)."""
     if norm is not None and x.is_cuda and len(norm) == 6 and norm[3] is not None:
         xf, nw, eps, ssq, ldss, nparts = norm
         if any(s.xmap is not None for s in segs) or M > 16:
@@ -430,6 +431,11 @@ def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: 
         if mode != 0 and ks > 1:
             width = segs[0].w.rows if mapped else sum(s.w.rows for s in segs)   # mapped split-K: shared columns
             ws = _workspace(x.device, ks * M * width).data_ptr()
+        if mapped and routed and mode >= 2:
+            fz = _lib.NlsFuse(nrows=int(routed))
+            _lib.check(L.nls_qgemv_ex(arr, len(arr), x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0), M, float(alpha),
+                                      EPI[epi], _p(argmax), waves, rt, mode, ks, ws, _stream_ptr(x), ctypes.byref(fz)), "nls_qgemv_ex")
+            return y
         rc = L.nls_qgemv(arr, len(arr), x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0), M, float(alpha),
                          EPI[epi], _p(argmax), waves, rt, mode, ks, ws, _stream_ptr(x))
         _lib.check(rc, "nls_qgemv")

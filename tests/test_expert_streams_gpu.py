@@ -144,3 +144,52 @@ def test_add_rmsnorm_route(gpu, monkeypatch, M, D, E, k, ksplit):
         assert torch.equal(a[n].view(E, cap).sort(1).values, b[n].view(E, cap).sort(1).values)
     assert not ops.qgemv_add_rmsnorm_route(seg, xin, x, nw, h, M, 0.7, 1e-5, wr[:1], a["logits"][:, :1], 1, a["topw"], a["counts"], a["xrows"],
                                            a["yrows"], cap)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bound", [False, True])
+@pytest.mark.parametrize("rows", [(0, 1, 257, 256), (96, 97, 0, 0, 600, 5), (0, 0, 0), (255, 64, 128, 129, 300, 1, 0, 40)])
+@pytest.mark.parametrize("mode,waves,rt", [(2, 8, 4), (2, 8, 2), (3, 4, 6), (4, 8, 2), (9, 8, 2)])
+def test_grouped_blocks(gpu, mode, waves, rt, rows, bound):
+    """Blocks of rows of a grouped launch: experts without rows, with whole blocks, with one row more; the number of rows known and not; rows
+    of y that no expert has stay as they are."""
+    E, K, N, T = len(rows), 512, 272, 640
+    raw = [Q.random_blocks(GGMLType.Q5_K, N * K, 0.05, np.random.default_rng(60 + e)) for e in range(E)]
+    ws = [ops.QWeight(r, GGMLType.Q5_K, N, K, gpu) for r in raw]
+    if mode == 4:
+        for w in ws:
+            w.expand_dense()
+    g = torch.Generator().manual_seed(7)
+    x = torch.randn(T, K, generator=g).to(ops.ACT_DTYPE).to(gpu)
+    lists = [torch.randperm(T, generator=g)[:n] for n in rows]
+    at = np.cumsum([0] + list(rows))
+    xr, yr = torch.zeros(E * T, dtype=torch.int32), torch.zeros(E * T, dtype=torch.int32)
+    for e, t in enumerate(lists):
+        xr[e * T:e * T + len(t)] = t.int()
+        yr[e * T:e * T + len(t)] = torch.arange(at[e], at[e + 1]).int()
+    xr, yr, counts = xr.to(gpu), yr.to(gpu), torch.tensor(rows, dtype=torch.int32, device=gpu)
+    y = torch.full((int(at[-1]) + 3, N), 5.0, device=gpu)
+    segs = [ops.Seg(w, 0, xr[e * T:], yr[e * T:], counts[e:e + 1]) for e, w in enumerate(ws)]
+    ops.qgemv(segs, x, y, T, epi="f32", mode=mode, waves=waves, rt=rt, ks=1, routed=int(at[-1]) if bound else 0)
+    assert (y[int(at[-1]):] == 5.0).all()
+    for e, t in enumerate(lists):
+        if len(t):
+            W, xd = ops.QWeight(raw[e], GGMLType.Q5_K, N, K, "cpu").dense().double(), x.cpu().double()[t]
+            got = y[int(at[e]):int(at[e + 1])].cpu().double()
+            assert ((got - xd @ W.t()).abs() <= (xd.abs() @ W.abs().t()) * 2.0 ** -9).all()      # (the bound of test_active_tiles)
+
+
+def test_expert_gemm_rule():
+    """Configs that exist, of types their modes take; the DMA GEMM only where it is allowed."""
+    for type in (7, 8, 12, 13, 14):
+        for N, K in ((8192, 2048), (2048, 4096), (28672, 4096), (4096, 14336), (272, 512)):
+            for E in (1, 2, 4, 8):
+                for per in (0.5, 9, 33, 64, 96, 250, 540, 1000, 4096):
+                    ws = [_W(N, type) for _ in range(E)]
+                    for w in ws:
+                        w.K = K
+                    for dma in (True, False):
+                        mode, waves, rt, ks = tuning.expert_gemm(ws, per, dma)
+                        assert ks == 1 and (mode, waves, rt) in ((2, 8, 4), (2, 8, 2), (3, 4, 6), (9, 8, 2))
+                        assert mode == 2 or type != 7
+                        assert mode != 3 or (dma and type != 8)
