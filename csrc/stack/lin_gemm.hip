@@ -41,11 +41,13 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   typedef LG<BN, BM, WN, WM, NST> G;
   typedef LT<T> L;
   constexpr int NW = G::NW, NX = G::NX, NTW = G::NTW, MTW = G::MTW;
-  const int per = gridDim.x >> 3;
-  const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (id >= ntot) return;
+  int listed, gap;
+  lin_listed(a, BN, listed, gap);
+  ntot -= gap;
+  const int per = (ntot + 7) >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || id >= ntot) return;
   LinTile t;
-  if (!lin_tile<BN, BM>(a, id, t)) return;
+  if (!lin_tile<BN, BM>(a, id < listed ? id : id + gap, t)) return;
   const LinSeg& S = a.s[t.seg];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

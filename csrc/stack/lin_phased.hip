@@ -144,9 +144,8 @@ __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot)
   const int wr = wave >> 2, wc = wave & 3;
   // tile ids are dealt to the XCDs in contiguous ranges, which an XCD's workgroups walk together
   const int xcd = blockIdx.x & 7, nx = gridDim.x >> 3;
-  const LinSeg& R = a.s[0];                              // (only the first segment may be routed)
-  const int listed = R.rows ? ((R.N + PB - 1) / PB) * __builtin_amdgcn_readfirstlane(*a.ntiles) : a.begin[1];
-  const int gap = a.begin[1] - listed;                   // ids that a full list would have
+  int listed, gap;                                       // (of a routed first segment)
+  lin_listed(a, PB, listed, gap);
   ntot -= gap;
   const int per = (ntot + 7) >> 3, last = min(ntot, (xcd + 1) * per);
 
@@ -154,7 +153,7 @@ __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot)
   // others U3; tiles with (tile & 2) == 0 of the rows are U1, the others U2.
   const int ta = (wave & 3) + 8 * (wave >> 2), tb = (wave & 1) + 4 * (wave >> 1);
   auto open = [&](int id, PhTile& p) __attribute__((always_inline)) -> int {      // tile id, if there is one; else -1
-    if (id >= last || !lin_tile<PB, PB, true>(a, id < listed ? id : id + gap, p.t)) return -1;
+    if (id >= last || !lin_tile<PB, PB>(a, id < listed ? id : id + gap, p.t)) return -1;
     p.t.grp = __builtin_amdgcn_readfirstlane(p.t.grp);
     p.t.cnt = __builtin_amdgcn_readfirstlane(p.t.cnt);
     p.t.rows = uniform(p.t.rows);

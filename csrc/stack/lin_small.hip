@@ -11,7 +11,10 @@ __global__ __launch_bounds__(64 * NW) void lin_small_kernel(LinArgs a) {
   constexpr int U = RT * MT >= 8 ? 2 : 4;    // sub-tiles in flight per wave
   typedef LT<T> L;
   LinTile t;
-  if (!lin_tile<16 * RT, 16 * MT>(a, blockIdx.x, t)) return;
+  int listed, gap;
+  lin_listed(a, 16 * RT, listed, gap);
+  const int id = blockIdx.x;
+  if (id >= a.begin[a.nseg] - gap || !lin_tile<16 * RT, 16 * MT>(a, id < listed ? id : id + gap, t)) return;
   const LinSeg& S = a.s[t.seg];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
