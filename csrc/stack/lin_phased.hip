@@ -228,7 +228,6 @@ __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot)
   dma_x(0, x0 += 2 * L::KS, PSTG);
   ph_wait<4>();                                          // step 0 has landed
   ph_barrier();
-  if (wr == 1) ph_barrier();
   for (;;) {
     const LinTile t = nxt.t;
     const int nst = nxt.nst, nid = open(id + nx, nxt);
@@ -237,6 +236,9 @@ __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot)
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // group 1 starts a barrier later and ends with the other one: left apart over the epilogue, it would wait with its last phase until group
+    // 0's epilogue is done, and group 0 for its own
+    if (wr == 1) ph_barrier();
     for (int j = 0; j < nst; ++j, buf ^= PSTG) {
       rd_w(0, buf);
       rd_x(B0, 0, buf);
@@ -273,11 +275,11 @@ __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot)
       ph_wait<6>();
       ph_barrier();
     }
+    if (wr == 0) ph_barrier();
     ph_epilogue(a.s[t.seg], t, acc, t.n0 + 128 * wr + 4 * g, 64 * wc + r);
     if (nid < 0) break;
     id = nid;
   }
-  if (wr == 0) ph_barrier();                             // both groups have met the same number of barriers
   ph_wait<0>();                                          // the staged tail lands before the workgroup's LDS is freed
 }
 
