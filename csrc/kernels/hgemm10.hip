@@ -38,8 +38,9 @@ using nls_dma::lds_addr;
 // weight half of a K-tile buffer and each wave's weight rows halve; the activation half, the phase schedule
 // and the unit order stay, only the DMA instruction counts of the two weight units (and so the counted
 // vmcnt of each phase) change.
-// Row blocks of 64 MT rows: 256 (MT 4), or 192 (MT 3: the second half of a wave's rows is one tile), which 257 .. 384 rows and many
-// larger counts fill better (launch_dense10).
+// Row blocks of 64 MT rows: 256 (MT 4), or 192 (MT 3: the second half of a wave's rows is one tile), which 321 .. 384 rows and many
+// larger counts fill better, or with 128 weight rows 320 (MT 5: the first half is three tiles; 18 KiB of LDS reads for 40 MFMAs of a wave, 14 for
+// 24 at 192 rows), which 257 .. 320 and 513 .. 640 rows fill (launch_dense10).
 constexpr int KT = 64;                       // K per tile
 template <int BN, int MT>
 struct H10 {
@@ -50,13 +51,14 @@ struct H10 {
   static constexpr int RTG = BN / 32;        // 16-row weight tiles per wave group (wr)
   static constexpr int NQH = RTG / 2;        // ... per quadrant half (nq)
   static constexpr int NA = BN / 128;        // DMA instructions per lane of a weight unit (U1: 2)
-  static constexpr int NB2 = MT - 2;         // ... of U2
-  // counted waits: the last three units issued stay in flight (units U0/U3 carry NA, U1 two, U2 NB2)
-  static constexpr int VM_PRO = NA + 2;            // after the prologue: U0(1) U1(1)
-  static constexpr int VM_Q0 = NA + 2 + NB2;       // U0(T+1) U1(T+1) U2(T+1)
-  static constexpr int VM_Q1 = NA + 2 + NB2;       // U1(T+1) U2(T+1) U3(T+1)
+  static constexpr int NB1 = (MT + 1) / 2;   // ... of U1, and tiles of the first half of a wave's rows
+  static constexpr int NB2 = MT - NB1;       // ... of U2
+  // counted waits: the last three units issued stay in flight (units U0/U3 carry NA, U1 NB1, U2 NB2)
+  static constexpr int VM_PRO = NA + NB1;          // after the prologue: U0(1) U1(1)
+  static constexpr int VM_Q0 = NA + NB1 + NB2;     // U0(T+1) U1(T+1) U2(T+1)
+  static constexpr int VM_Q1 = NA + NB1 + NB2;     // U1(T+1) U2(T+1) U3(T+1)
   static constexpr int VM_Q2 = 2 * NA + NB2;       // U2(T+1) U3(T+1) U0(T+2)
-  static constexpr int VM_Q3 = 2 * NA + 2;   // U3(T+1) U0(T+2) U1(T+2)
+  static constexpr int VM_Q3 = 2 * NA + NB1; // U3(T+1) U0(T+2) U1(T+2)
 };
 
 DEVI int swz(int r) { return (0x1320 >> (4 * ((r >> 2) & 3))) & 3; }
@@ -72,11 +74,12 @@ template <int BN, int MT>
 DEVI int unit_rt(int u, int idx) {           // idx: row-tile slot of the unit
   // BN 256: U0: A {0-3, 8-11}; U3: A {4-7, 12-15}. BN 128: U0: A {0-1, 4-5}; U3: A {2-3, 6-7}.
   // U1: B {0,1,4,5,8,9,12,13}; U2: B {2,3,6,7,10,11,14,15}. MT 3: U1: B {0,1,3,4,6,7,9,10}; U2: B {2,5,8,11}
-  constexpr int NQH = H10<BN, MT>::NQH, RTG = H10<BN, MT>::RTG;
+  // MT 5: U1: B {0-2, 5-7, 10-12, 15-17}; U2: B {3,4,8,9,13,14,18,19}
+  constexpr int NQH = H10<BN, MT>::NQH, RTG = H10<BN, MT>::RTG, NB1 = H10<BN, MT>::NB1, NB2 = H10<BN, MT>::NB2;
   if (u == 0) return (idx % NQH) + RTG * (idx / NQH);
   if (u == 3) return NQH + (idx % NQH) + RTG * (idx / NQH);
-  if (u == 1) return (idx & 1) + MT * (idx >> 1);
-  return MT == 4 ? 2 + (idx & 1) + 4 * (idx >> 1) : 2 + MT * idx;
+  if (u == 1) return idx % NB1 + MT * (idx / NB1);
+  return NB1 + idx % NB2 + MT * (idx / NB2);
 }
 
 // ---- epilogue (mode 8's; shared by modes 10 and 11): lane holds weight rows nb + 16i + 4(l >> 4) + e, activation
@@ -234,7 +237,7 @@ DEVI void h10_epilogue(H10Acc<BN, MT>& acc, const Seg& S, int row0, int kslice, 
 template <int BN, int MT, bool ROPE>
 DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, uint8_t* lds) {
   typedef H10<BN, MT> C;
-  constexpr int TB = C::TB, NQH = C::NQH, NA = C::NA, NB2 = C::NB2;
+  constexpr int TB = C::TB, NQH = C::NQH, NA = C::NA, NB1 = C::NB1, NB2 = C::NB2;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 2, wc = wave & 3;
@@ -244,7 +247,7 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
   const int M = a.M;
   const act_t* Wd = reinterpret_cast<const act_t*>(S.w);
 
-  // ---- DMA: unit u of K-tile T -> buffer T & 1. This wave issues subtiles idx = n * wave + j (j < n; n = 2,
+  // ---- DMA: unit u of K-tile T -> buffer T & 1. This wave issues subtiles idx = n * wave + j (j < n; n = NB1, NB2,
   // or NA for a weight unit) of every unit: row-tile unit_rt(u, idx >> 1), k-step idx & 1. Lane L -> row
   // 16 rt + (L >> 2), physical chunk L & 3 <- logical chunk (L & 3) ^ swz(L >> 2).
   const int lc = (lane & 3) ^ swz(lane >> 2);
@@ -253,9 +256,9 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
     const int Tc = t0 + min(T, nkt - 1);       // clamped: past the end re-stages the last tile (same bytes)
     const bool bu = u == 1 || u == 2;
     const uint32_t buf = base + (uint32_t)(T & 1) * TB + (bu ? (uint32_t)C::AB : 0u);
-    const int n = u == 1 ? 2 : u == 2 ? NB2 : NA;
+    const int n = u == 1 ? NB1 : u == 2 ? NB2 : NA;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < 3; ++j) {
       if (j >= n) break;
       const int idx = n * wave + j;
       const int rt = unit_rt<BN, MT>(u, idx >> 1), kstep = idx & 1;
@@ -273,7 +276,7 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
 
   // ---- fragments: lane reads row (l & 15) of a 16-row subtile, logical chunk l >> 4
   const int fro = (lane & 15) * 64 + (((lane >> 4) ^ swz(lane & 15)) << 4);
-  f16x8 FA[NQH][2], FB0[2][2], FB1[NB2][2];
+  f16x8 FA[NQH][2], FB0[NB1][2], FB1[NB2][2];
   auto rdA = [&](int T, int nq) __attribute__((always_inline)) {
     const uint8_t* p = lds + (T & 1) * TB + fro;
 #pragma unroll
@@ -285,9 +288,9 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
   auto rdB = [&](auto& F, int T, int mh) __attribute__((always_inline)) {
     const uint8_t* p = lds + (T & 1) * TB + C::AB + fro;
 #pragma unroll
-    for (int i = 0; i < (mh ? NB2 : 2); ++i)
+    for (int i = 0; i < (mh ? NB2 : NB1); ++i)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) F[i][s] = *reinterpret_cast<const f16x8*>(p + ((wc * MT + mh * 2 + i) * 2 + s) * 1024);
+      for (int s = 0; s < 2; ++s) F[i][s] = *reinterpret_cast<const f16x8*>(p + ((wc * MT + mh * NB1 + i) * 2 + s) * 1024);
   };
   f32x4 acc[2 * NQH][MT];
 #pragma unroll
@@ -300,8 +303,8 @@ DEVI void h10_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
 #pragma unroll
       for (int i = 0; i < NQH; ++i)
 #pragma unroll
-        for (int j = 0; j < (mh ? NB2 : 2); ++j)
-          acc[nq * NQH + i][mh * 2 + j] = mfma16(FA[i][s], F[j][s], acc[nq * NQH + i][mh * 2 + j]);
+        for (int j = 0; j < (mh ? NB2 : NB1); ++j)
+          acc[nq * NQH + i][mh * NB1 + j] = mfma16(FA[i][s], F[j][s], acc[nq * NQH + i][mh * NB1 + j]);
   };
   auto bar = []() __attribute__((always_inline)) {
     __builtin_amdgcn_s_barrier();
@@ -420,10 +423,13 @@ int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a
 // long, end earlier (Llama-3-8B at 384 rows: gate|up 99 -> 76 us, down 69 -> 57; 1500 rows: o 65 -> 56; 3000: down 308 -> 276). With 256 weight rows
 // they must end a good deal earlier: 192 x 256 tiles multiply slower, and the last round is seldom full (28672 x 4096, rounds by length: 0.75 at
 // 600 and 1100 rows 193 -> 169 and 292 -> 254 us, 0.875 at 3000 rows 638 -> 674, 0.9 at 2400 527 -> 537, 0.94 at 2048 417 -> 437).
+// Blocks of 320 rows with 128 weight rows: a round of 224 workgroups reads 28672 x 4096 once, as do two of 192 x 256, for 320 rows instead of 384.
+// In a running step of 320 rows 90.5 (384 rows, 192 x 256) -> 79.6 us, a head of 32000 92 -> 85; 640 rows 172 -> 162 and 186 -> 170.
 int launch_dense10(int bn, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   auto rounds = [&](int bm) { return (long)((ntiles * ((a.M + bm - 1) / bm) * ks + 255) / 256) * bm; };
   const bool low = rounds(192) * 100 < rounds(256) * (bn == 256 ? 85 : 100);
   if (bn == 256) return low ? launch_t<256, 3>(sl, ntiles, ks, ws, a, st) : launch_t<256, 4>(sl, ntiles, ks, ws, a, st);
+  if (bn == 128 && rounds(320) * 100 < (low ? rounds(192) : rounds(256)) * 97) return launch_t<128, 5>(sl, ntiles, ks, ws, a, st);
   if (bn == 128) return low ? launch_t<128, 3>(sl, ntiles, ks, ws, a, st) : launch_t<128, 4>(sl, ntiles, ks, ws, a, st);
   return -1;
 }

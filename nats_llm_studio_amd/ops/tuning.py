@@ -155,9 +155,9 @@ def dense_key(segs, M: int) -> str:
 
 
 # Microseconds of a round of 256 workgroups at K = 4096, by (mode, rt, activation rows of a tile); 5 of them do not grow with
-# K. Mode 10's launcher takes 192 or 256 rows, whichever fills its rounds better. (Llama-3-8B shapes at M = 256 .. 4096, e.g.
+# K. Mode 10's launcher takes 192 or 256 rows, or with 128 weight rows 320, whichever fills its rounds best. (Llama-3-8B shapes at M = 256 .. 4096, e.g.
 # gate|up at 384 rows 76 us, at 3000 585, Q|K|V at 3000 168, o at 1500 56, down at 4096 375.)
-_ROUND_US = {(10, 1, 256): 106.0, (10, 1, 192): 82.0, (10, 2, 256): 72.0, (10, 2, 192): 48.0, (4, 2, 128): 44.0}
+_ROUND_US = {(10, 1, 256): 106.0, (10, 1, 192): 82.0, (10, 2, 256): 72.0, (10, 2, 192): 48.0, (10, 2, 320): 76.0, (4, 2, 128): 44.0}
 
 
 def dense_heuristic(segs, M: int, aligned: bool = True):
@@ -189,7 +189,9 @@ def select_dense(segs, M: int):
     hit = table().get(dense_key(segs, M))
     if hit is not None and hit[0] < 0:
         return None
-    if M > MBUCKETS[-1] and dense_key(segs, M) not in _FORCED:
+    # (257 .. 320 and 513 .. 640 rows fill blocks of 320, which the entries, measured at 512 and 1024 rows, do not take: Llama-3-8B gate|up at 320
+    # rows 97 -> 91 us, o 28 -> 26; at 640 gate|up 172 -> 162, down 94 -> 86, Q|K|V 50 -> 44)
+    if (M > MBUCKETS[-1] or 256 < M <= 320 or 512 < M <= 640) and dense_key(segs, M) not in _FORCED:
         return dense_heuristic(segs, M)
     return hit if hit is not None else dense_heuristic(segs, M)
 

@@ -92,3 +92,45 @@ def test_split_reduce(cfg, rows, K):
                 # f32 sums of K products; f16 outputs round to 2^-11
                 assert relerr(y[:M, 4:] - (7 if epi == "add" else 0), z) < (5e-4 if epi == "act" else 4e-6), (M, ks, epi)
                 assert (y[M] == 7).all() and (y[:, :4] == 7).all()
+
+
+# 320-row blocks with 128 weight rows: 201 weight tiles take them at 257 .. 320 and 513 .. 640 rows; one K step (no successor to stage) to twelve
+@pytest.mark.parametrize("M", [257, 271, 319, 320, 321, 513, 640])
+@pytest.mark.parametrize("K", [256, 768])
+def test_blocks_of_320(M, K):
+    rows = 25700 - 4
+    w, x = weight(rows, K), acts(M, K)
+    z = x[:M].double() @ w.d16.double().T
+    for epi, ks in (("f32", 1), ("add", 1), ("add", 4)):
+        y = torch.full((x.shape[0] + 1, rows), 7.0, device="cuda")
+        ops.qgemv([ops.Seg(w)], x, y, M, epi=epi, mode=10, waves=8, rt=2, ks=ks)
+        assert relerr(y[:M] - (7 if epi == "add" else 0), z) < 4e-6, (epi, ks)       # sums of K products in f32
+        assert (y[M:] == 7).all()
+
+
+def test_blocks_of_320_rope():
+    """144 weight tiles in three segments; D = 34 takes the general stores."""
+    M, K = 300, 256
+    for D, Hq, Hkv in ((128, 128, 8), (34, 504, 24)):
+        ws = [weight(h * D, K, s) for s, h in enumerate((Hq, Hkv, Hkv))]
+        segs = [ops.Seg(ws[0], 0), ops.Seg(ws[1], Hq * D), ops.Seg(ws[2], (Hq + Hkv) * D)]
+        x, n = acts(M, K), (Hq + 2 * Hkv) * D
+        pad = x.shape[0]
+        cs = ops.rope_table(400, D, 10000.0, torch.device("cuda"))
+        pos = (torch.arange(pad, dtype=torch.int32, device="cuda") * 7) % 400
+        slot = torch.randperm(pad, generator=torch.Generator().manual_seed(2)).int().cuda()
+        slot[[0, 17, M - 1]] = -1
+        outs = []
+        for fuse in (True, False):
+            q = torch.full((pad, Hq * D), 776.0, dtype=torch.bfloat16, device="cuda")
+            kc, vc = (torch.full((pad, Hkv, D), 776.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+            qkv = torch.zeros(pad, n, device="cuda")
+            if fuse:
+                ops.qkv_rope_kv(segs, x, qkv, pos, slot, cs, q, kc, vc, M, Hq, Hkv, D, cfg=(10, 8, 2, 1))
+            else:
+                ops.qgemv(segs, x, qkv, M, mode=4, waves=16, rt=2, ks=1)
+                q, kc, vc = q.cpu(), kc.cpu(), vc.cpu()
+                ops.rope_kv(qkv.cpu(), pos.cpu(), slot.cpu(), cs.cpu(), q, kc, vc, M, Hq, Hkv, D)
+            outs.append((q.cpu(), kc.cpu(), vc.cpu()))
+        for a, b in zip(*outs):      # one bf16 rounding apart at most, and the same places written
+            assert relerr(a, b) < 2e-3 and ((a == 776) == (b == 776)).all()
