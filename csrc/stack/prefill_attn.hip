@@ -14,6 +14,10 @@
 // The next tile's loads are in flight in registers while a tile computes (its cache slots one tile ahead of that); one
 // barrier per tile, two LDS buffers. Rows are padded in LDS (K: 16 bytes, V: 64) against bank conflicts. Under a sliding window
 // (with kept first keys) tiles that no row sees are left out. The epilogue applies the head's output gate, if there is one.
+// A tile is a chain (scores, maximum, exponentials, values) with little to overlap in one wave per SIMD, so two workgroups of four waves share a
+// CU: registers are held to 256, and a tile of more than 40 KB has one buffer. Runs of 60 tokens of 64 sequences, 32 heads on 8: 57 us with one
+// workgroup to a CU, 36 so; 6 x 650 87 -> 50; one of 1000 41 -> 34. Where the longest walk is the time, two groups of four waves take every other
+// tile of a workgroup's rows and the second one's sums are added over LDS (2000 tokens of 16 heads on 4: 60 -> 49 us).
 #include "../kernels/common.h"
 
 namespace nls_pfa {
@@ -51,20 +55,31 @@ struct FP {
 };
 constexpr int NO_WINDOW = 1 << 30;
 
-template <int NKU, int NKR, int NDB, int NWV>      // 32-column units: keys unrotated / rotated, values; waves
-__global__ __launch_bounds__(64 * NWV) void flash_prefill_kernel(FP p) {
+// Bytes of a tile in LDS and its buffers. Two workgroups of four row waves share a CU, or the two key groups of one; each has one buffer where
+// two do not fit.
+template <int NKU, int NKR, int NDB, int NWV, int NG>
+struct Fit {
+  static constexpr int KROW = 32 * (NKU + NKR) * 2 + 16, VROW = 32 * NDB * 2 + (NDB > 1 ? 64 : 0);
+  static constexpr int TB = 64 * (KROW + VROW), TWO = NWV == 4 && NDB <= 4 ? 2 : 1;
+  static constexpr int BUFS = 2 * TB * TWO <= 160 * 1024 ? 2 : 1;
+  static constexpr int LDS = NG * BUFS * TB;
+  static_assert(NG == 1 || (TWO == 2 && 64 * NWV * (16 * NDB + 2) * 4 <= LDS), "a group's partial sums take the place of the tiles");
+};
+
+template <int NKU, int NKR, int NDB, int NWV, int NG>      // 32-column units: keys unrotated / rotated, values; waves of rows; key groups
+__global__ __launch_bounds__(64 * NWV * NG, (Fit<NKU, NKR, NDB, NWV, NG>::TWO == 2 ? 2 : 0)) void flash_prefill_kernel(FP p) {
   constexpr bool PAGED = NKR == 0;
   static_assert(!PAGED || NKU == NDB, "grouped form: equal key and value widths");
   constexpr int NT = 64 * NWV, KT = 64;
   constexpr int DKU = 32 * NKU, DR = 32 * NKR, DK = DKU + DR, DV = 32 * NDB;
-  constexpr int KROW = DK * 2 + 16, VROW = DV * 2 + (NDB > 1 ? 64 : 0);
-  constexpr int TB = KT * (KROW + VROW);
+  typedef Fit<NKU, NKR, NDB, NWV, NG> F;
+  constexpr int KROW = F::KROW, VROW = F::VROW, TB = F::TB, BUFS = F::BUFS;
   constexpr int CU = DKU / 8, CR = DR / 8, CV = DV / 8;   // 16-byte chunks per key
   constexpr int NLK = (KT * CU + NT - 1) / NT;                               // grouped: chunks per thread of K, and of V
   constexpr int NLR = (KT * CR + NT - 1) / NT, NLV = (KT * CV + NT - 1) / NT; // latent: of the rotated part, and of V
   constexpr int NLD = PAGED ? 2 * NLK : NLK + NLR + NLV;
   constexpr int NKS = DK / 16;
-  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];              // [2][K tile | V tile]
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_all[];          // [NG][BUFS][K tile | V tile]
 
   const int HK = PAGED ? p.H / p.gs : p.H, gs = PAGED ? p.gs : 1;
   const int kh = blockIdx.x % HK, rest = blockIdx.x / HK;
@@ -73,8 +88,9 @@ __global__ __launch_bounds__(64 * NWV) void flash_prefill_kernel(FP p) {
   const int t0 = blk[0], ntok = blk[1], pos0 = blk[3], xoff = blk[4];
   const int nrow = ntok * gs;
   if (PAGED && row0 >= nrow) return;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = NG == 1 ? 0 : wv / NWV, wave = wv - NWV * grp, tid = threadIdx.x - NT * grp;
+  uint8_t* lds = lds_all + grp * BUFS * TB;
   const int h = lane >> 5, tl = lane & 31;
   const int tw0 = row0 + 32 * wave;
   const int myrow = min(tw0 + tl, nrow - 1), mytok = myrow / gs, head = PAGED ? kh * gs + myrow - mytok * gs : kh;
@@ -106,7 +122,7 @@ __global__ __launch_bounds__(64 * NWV) void flash_prefill_kernel(FP p) {
       for (int i = 0; i < NLR; ++i) sl[i] = p.xmap[xoff + min(tile(t) * KT + (tid + NT * i) / max(CR, 1), nkeys - 1)];
     }
   };
-  load_slots(0);
+  load_slots(grp);
 
   u32x4 st[NLD];
   auto load_tile = [&](int t) __attribute__((always_inline)) {
@@ -170,19 +186,22 @@ __global__ __launch_bounds__(64 * NWV) void flash_prefill_kernel(FP p) {
   f32x16 o[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) o[i] = f32x16{};
-  float m = p.sink ? 0.f : -INFINITY, l = p.sink && h == 0 ? 1.f : 0.f;       // (l: two lanes' shares of a row)
-  load_tile(0);
-  load_slots(1);
-  store_tile(0);
+  float m = p.sink && grp == 0 ? 0.f : -INFINITY, l = p.sink && grp == 0 && h == 0 ? 1.f : 0.f;       // (l: two lanes' shares of a row)
+  if (NG == 1 || grp < ntile) {
+    load_tile(grp);
+    load_slots(grp + NG);
+    store_tile(0);
+  }
   __syncthreads();
   const int vq = (lane & 15) >> 2, vp = lane & 3, vhalf = (lane >> 4) & 1;
-  for (int t = 0; t < ntile; ++t) {
-    const int cur = t & 1, k0 = tile(t) * KT;
-    if (t + 1 < ntile) {
-      load_tile(t + 1);
-      load_slots(t + 2);
+  const int nstep = (ntile + NG - 1) / NG;
+  for (int i = 0; i < nstep; ++i) {
+    const int t = i * NG + grp, cur = i & (BUFS - 1), k0 = tile(t) * KT;
+    if (t + NG < ntile) {
+      load_tile(t + NG);
+      load_slots(t + 2 * NG);
     }
-    if (wact && k0 <= wlast && (k0 < p.keep || k0 + KT > wfirst - p.window + 1)) {
+    if (wact && (NG == 1 || t < ntile) && k0 <= wlast && (k0 < p.keep || k0 + KT > wfirst - p.window + 1)) {
       const uint8_t* kb = lds + cur * TB;
       const uint8_t* vb = kb + KT * KROW;
       f32x16 s[2];
@@ -244,8 +263,29 @@ __global__ __launch_bounds__(64 * NWV) void flash_prefill_kernel(FP p) {
         }
       }
     }
-    if (t + 1 < ntile) store_tile(cur ^ 1);                     // that buffer was last read in tile t - 1
+    if (BUFS == 1) __syncthreads();
+    if (t + NG < ntile) store_tile(BUFS == 2 ? cur ^ 1 : 0);    // (of two, that buffer was last read in the step before)
     __syncthreads();
+  }
+  if constexpr (NG == 2) {                                      // the second group's sums, brought to a common maximum
+    float* ex = reinterpret_cast<float*>(lds_all) + tid;        // [2 + 16 NDB][NT]
+    if (grp) {
+      ex[0] = m;
+      ex[NT] = l;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[(2 + 16 * db + r) * NT] = o[db][r];
+    }
+    __syncthreads();
+    if (grp) return;
+    const float m1 = ex[0], mn = fmaxf(m, m1);
+    const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * sl2), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - mn) * sl2);
+    l = l * a0 + ex[NT] * a1;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * a0 + ex[(2 + 16 * db + r) * NT] * a1;
   }
   l += __shfl_xor(l, 32, 64);
   if (tw0 + tl >= nrow) return;
@@ -271,17 +311,17 @@ __global__ __launch_bounds__(64 * NWV) void flash_prefill_kernel(FP p) {
     }
 }
 
-template <int NKU, int NKR, int NDB, int NWV>
+template <int NKU, int NKR, int NDB, int NWV, int NG = 1>
 int launch_t(const FP& p, int nblocks, hipStream_t st) {
-  constexpr int LDS = 2 * 64 * (32 * (NKU + NKR) * 2 + 16 + 32 * NDB * 2 + (NDB > 1 ? 64 : 0));
+  constexpr int LDS = Fit<NKU, NKR, NDB, NWV, NG>::LDS;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute((const void*)flash_prefill_kernel<NKU, NKR, NDB, NWV>,
+    if (hipFuncSetAttribute((const void*)flash_prefill_kernel<NKU, NKR, NDB, NWV, NG>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((flash_prefill_kernel<NKU, NKR, NDB, NWV>), dim3(nblocks * (p.H / p.gs) * p.nsub), dim3(64 * NWV), LDS,
+  hipLaunchKernelGGL((flash_prefill_kernel<NKU, NKR, NDB, NWV, NG>), dim3(nblocks * (p.H / p.gs) * p.nsub), dim3(64 * NWV * NG), LDS,
                      st, p);
   return (int)hipGetLastError();
 }
@@ -299,18 +339,19 @@ int nls_expand_plan(const int* spans, int nspans, int maxctx, const int* bt, int
   return (int)hipGetLastError();
 }
 
-// dku, dr, dv: expanded widths per head: dku, dv in {32, 64, 128}, dr in {32, 64}; waves 4 or 8 (blocks of 32 * waves rows)
+// waves 4 or 8 (blocks of 32 * waves rows); groups 2: two groups of four waves share the keys of a workgroup's rows
+// dku, dr, dv: expanded widths per head: dku, dv in {32, 64, 128}, dr in {32, 64}
 int nls_latent_prefill(const void* qn, long ldqn, int qns, const void* qr, long ldqr, int qrs, const void* kx,
                        const void* vx, const void* cache, long ldc, const int* xmap, const int* blocks, int nblocks,
                        const float* gate, int ldg, void* out, long ldo, int H, int dku, int dr, int dv, int vdim,
-                       int waves, float scale, void* stream) {
-  if (nblocks < 1 || H < 1 || vdim < 1 || vdim > dv) return -1;
+                       int waves, int groups, float scale, void* stream) {
+  if (nblocks < 1 || H < 1 || (groups != 1 && (groups != 2 || waves != 4)) || vdim < 1 || vdim > dv) return -1;
   FP p{(const __bf16*)qn, (const __bf16*)qr, (const __bf16*)kx, (const __bf16*)vx, (const __bf16*)cache, xmap, blocks,
        gate, (__bf16*)out, ldqn, ldqr, ldc, ldo, qns, qrs, H, vdim, ldg, 1, 1, scale, NO_WINDOW, 0, 0};
   hipStream_t st = (hipStream_t)stream;
 #define NLS_LP(U, R, V) \
   if (dku == 32 * U && dr == 32 * R && dv == 32 * V) \
-    return waves == 8 ? launch_t<U, R, V, 8>(p, nblocks, st) : waves == 4 ? launch_t<U, R, V, 4>(p, nblocks, st) : -1;
+    return waves == 8 ? launch_t<U, R, V, 8>(p, nblocks, st) : waves != 4 ? -1 : groups == 2 ? launch_t<U, R, V, 4, 2>(p, nblocks, st) : launch_t<U, R, V, 4>(p, nblocks, st);
 #define NLS_LPV(U, R) NLS_LP(U, R, 1) NLS_LP(U, R, 2) NLS_LP(U, R, 4)
   NLS_LPV(1, 1) NLS_LPV(2, 1) NLS_LPV(4, 1) NLS_LPV(1, 2) NLS_LPV(2, 2) NLS_LPV(4, 2)
 #undef NLS_LPV
@@ -318,12 +359,13 @@ int nls_latent_prefill(const void* qn, long ldqn, int qns, const void* qr, long 
   return -1;
 }
 
-// Dp: padded head width (32, 64, 128; 256 with 4 waves); k, v: paged [slots][G][Dp]; blocks of up to 32 * waves tokens. window > 0: a
+// Dp: padded head width (32, 64, 128; 256 with 4 waves); k, v: paged [slots][G][Dp]; blocks of up to 32 * waves tokens; groups: as above (at 256 columns
+// one). window > 0: a
 // sliding window with `keep` first keys
 int nls_gqa_prefill(const void* q, long ldq, const void* k, const void* v, const int* xmap, const int* blocks, int nblocks,
-                    const float* gate, int ldg, void* out, long ldo, int H, int G, int Dp, int waves, float scale,
+                    const float* gate, int ldg, void* out, long ldo, int H, int G, int Dp, int waves, int groups, float scale,
                     int window, int keep, int sink, void* stream) {
-  if (nblocks < 1 || G < 1 || H < 1 || H % G || window < 0 || window > NO_WINDOW || keep < 0 || (ldq & 7) || (ldo & 3))
+  if (nblocks < 1 || G < 1 || H < 1 || H % G || window < 0 || window > NO_WINDOW || keep < 0 || (ldq & 7) || (ldo & 3) || (groups != 1 && (groups != 2 || waves != 4)))
     return -1;
   FP p{(const __bf16*)q, (const __bf16*)q, (const __bf16*)k, (const __bf16*)v, nullptr, xmap, blocks, gate, (__bf16*)out, ldq, ldq,
        (long)G * Dp, ldo, Dp, Dp, H, Dp, ldg, H / G, H / G, scale, window ? window : NO_WINDOW, keep, sink};
@@ -334,7 +376,7 @@ int nls_gqa_prefill(const void* q, long ldq, const void* k, const void* v, const
     return launch_t<8, 0, 8, 4>(p, nblocks, st);
   }
 #define NLS_GP(D, N) \
-  if (Dp == D) return waves == 8 ? launch_t<N, 0, N, 8>(p, nblocks, st) : waves == 4 ? launch_t<N, 0, N, 4>(p, nblocks, st) : -1;
+  if (Dp == D) return waves == 8 ? launch_t<N, 0, N, 8>(p, nblocks, st) : waves != 4 ? -1 : groups == 2 ? launch_t<N, 0, N, 4, 2>(p, nblocks, st) : launch_t<N, 0, N, 4>(p, nblocks, st);
   NLS_GP(32, 1) NLS_GP(64, 2) NLS_GP(128, 4)
 #undef NLS_GP
   return Dp == 256 && waves == 4 ? launch_t<8, 0, 8, 4>(p, nblocks, st) : -1;

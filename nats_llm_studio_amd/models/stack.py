@@ -250,7 +250,7 @@ class LatentMixer(_Part):
             kx, vx, lin = self._expansion(b, e, rows, plan)
             lin.run(plan.nx, st)
             K.latent_prefill(e["qn"], self.Dq, e["q"], self.Rp, self.Dp, kx, vx, rows, plan.xmap, plan.blocks, plan.nblocks,
-                             plan.waves, e["gate"], e["ao"], c.heads, self.xk, self.xr, self.xv, c.vdim, c.scale, st)
+                             plan.waves, e["gate"], e["ao"], c.heads, self.xk, self.xr, self.xv, c.vdim, c.scale, st, groups=plan.groups)
         e["o_proj"].run(T, st)
 
     def _expansion(self, b: StackBuffers, e: dict, rows, plan):
@@ -450,7 +450,7 @@ class AttentionPart(_SharedPart):
                             c.scale, st, **self.mask)
         if plan is not None:
             K.gqa_prefill(e["q"], kc, vc, plan.xmap, plan.blocks, plan.nblocks, plan.waves, e["gate"], e["out"], c.heads,
-                          c.kv_heads, self.Dp, c.scale, st, **self.mask)
+                          c.kv_heads, self.Dp, c.scale, st, groups=plan.groups, **self.mask)
 
 
 class GlaPart(_SharedPart):
@@ -857,14 +857,34 @@ def yarn(base: float, dims: int, s) -> tuple:
     return 1.0 / (ramp / s.factor + (1.0 - ramp)), 0.1 * math.log(s.factor) + 1.0
 
 
+def _prompt_waves(att, spans):
+    """(waves, key groups) of a step's prompt attention (csrc/stack/prefill_attn.hip): a workgroup has 32 * waves rows of a head. With four waves two
+    workgroups share a CU. Where there are few of them, or the longest walk over keys (in tiles of 64) outlasts the others, two groups of
+    waves share a workgroup's keys; eight waves, which read keys and values half as often, where long walks fill the chip. us, four waves / two
+    groups / eight waves: 32 heads on 8, 2000 tokens 71 / 65 / 79, 1000 34 / 30 / 40, 3500 154 / 173 / 140, 6 x 650 50 / 69 / 61, 64 x 60
+    36 / 69 / 73; 16 on 4, 2000 tokens 60 / 49 / 73, 3500 110 / 84 / 124; expanded, 16 heads 128 + 64 wide, 3500 125 / 96 / 129."""
+    H = max(q.cfg.heads for q in att)
+    if any(getattr(q, "talk", None) is not None for q in att):
+        return (8 if H * sum(-(-s[1] // 256) for s in spans) >= 256 else 4), 1
+    windows = [getattr(q.cfg, "window", 0) for q in att]
+    seen = max(windows) + 128 if all(windows) else 1 << 30                                    # keys that a block of 128 rows sees
+    walks = [-(-min(s[3] + min(o + 128, s[1]), seen) // 64) for s in spans for o in range(0, s[1], 128)]
+    most, mean = max(walks), H * sum(walks) / 512                                              # (512 workgroups at a time)
+    if most >= 6 and (H * len(walks) <= 256 or (most >= 24 and most >= 1.5 * mean)):
+        return 4, 2
+    return (8 if most >= 48 and mean >= 0.6 * most else 4), 1
+
+
 @dataclass
 class _ExpandPlan:
-    """The runs of a step that take the prompt attention: `nx` context rows, query blocks of 32 * waves tokens."""
+    """The runs of a step that take the prompt attention: `nx` context rows, query blocks of 32 * waves tokens, whose keys `groups` groups of
+    waves share."""
     nx: int
     xmap: torch.Tensor          # [nx] cache slots of the runs' contexts
     blocks: torch.Tensor        # [nblocks][8]
     nblocks: int
     waves: int
+    groups: int
     rest: bool                  # some rows attend row by row
     actx: Optional[torch.Tensor]
 
@@ -1054,12 +1074,11 @@ class StackModel:
             rows += n
         if not spans:
             return None, None
-        H = max(q.cfg.heads for q in att)
-        waves = 8 if H * sum(-(-s[1] // 256) for s in spans) >= 256 else 4
+        waves, groups = _prompt_waves(att, spans)
         q = 32 * waves
         blocks = [(s[0] + o, min(q, s[1] - o), s[2], s[3] + o, s[4], 0, 0, 0) for s in spans for o in range(0, s[1], q)]
         blocks.sort(key=lambda v: -(v[3] + v[1]))
-        info = dict(nspans=len(spans), nblocks=len(blocks), nx=nx, maxctx=max(s[5] for s in spans), waves=waves,
+        info = dict(nspans=len(spans), nblocks=len(blocks), nx=nx, maxctx=max(s[5] for s in spans), waves=waves, groups=groups,
                     rest=rows < T)
         return np.asarray(spans + blocks, dtype=np.int32), info
 
@@ -1092,7 +1111,7 @@ class StackModel:
             actx = self.grown(b, "lat.actx", b.pad, 1, torch.int32).view(-1)
             actx[:T].copy_(b.ctx_len[:T])
         K.expand_plan(qblocks, ns, info["maxctx"], b.block_tables, block_size, xmap, actx, st)
-        return _ExpandPlan(info["nx"], xmap, qblocks[ns:], info["nblocks"], info["waves"], info["rest"], actx)
+        return _ExpandPlan(info["nx"], xmap, qblocks[ns:], info["nblocks"], info["waves"], info["groups"], info["rest"], actx)
 
     # ---- forward
     def _norms(self, b: StackBuffers, i: int) -> dict:

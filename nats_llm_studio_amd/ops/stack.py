@@ -47,7 +47,7 @@ _SIGS = {
     "nls_talk_decode": [P, L, P, P, P, I, I, P, P, I, I, I, I, I, I, F, I, P, P, L, P, L, P, L, P, P, P, I, I, I, P],
     "nls_talk_prefill": [P, L, P, P, P, I, I, P, I, I, I, I, I, I, F, I, P, P, L, P, L, P],
     "nls_gqa_attn": [P, L, P, P, P, I, I, P, P, I, I, I, I, I, F, P, L, P, L, P, P, P, I, I, I, I, I, P],
-    "nls_gqa_prefill": [P, L, P, P, P, P, I, P, I, P, L, I, I, I, I, F, I, I, I, P],
+    "nls_gqa_prefill": [P, L, P, P, P, P, I, P, I, P, L, I, I, I, I, I, F, I, I, I, P],
     "nls_delta_conv": [P, L, P, P, L, P, L, P, L, P, P, I, I, I, I, I, I, I, I, P],
     "nls_delta_scan": [P, P, P, L, P, L, P, L, P, L, P, L, P, P, L, P, L, F, P, L, P, I, I, I, I, I, I, P, P, I, I, P],
     "nls_delta_step": [P, P, P, L, P, L, P, L, P, L, P, P, P, P, I, P, L, P, P, I, L, P, L, P, I, P, P, L, I, I, I, I, F, I, P],
@@ -61,7 +61,7 @@ _SIGS = {
     "nls_scan_out": [P, L, P, P, L, P, L, I, I, I, F, I, P],
     "nls_wkv_step": [P, P, P, L, P, L, P, P, L, P, L, P, L, I, P, I, P, P, L, P, L, I, I, F, I, P],
     "nls_expand_plan": [P, I, I, P, I, I, P, P, P],
-    "nls_latent_prefill": [P, L, I, P, L, I, P, P, P, L, P, P, I, P, I, P, L, I, I, I, I, I, I, F, P],
+    "nls_latent_prefill": [P, L, I, P, L, I, P, P, P, L, P, P, I, P, I, P, L, I, I, I, I, I, I, I, F, P],
     "nls_latent_attn": [P, P, P, P, P, P, I, I, P, P, I, I, I, I, I, F, I, P],
 }
 
@@ -556,12 +556,13 @@ def expand_plan(spans, nspans: int, maxctx: int, block_tables, block_size: int, 
 
 
 def latent_prefill(qn, qns: int, q, Rp: int, qrs: int, kx, vx, cache, xmap, blocks, nblocks: int, waves: int, gate, out,
-                   H: int, dku: int, dr: int, dv: int, vdim: int, scale: float, st: int):
-    """Causal attention of query blocks over expanded keys / values; the rotated parts sit at column Rp of q and cache."""
+                   H: int, dku: int, dr: int, dv: int, vdim: int, scale: float, st: int, groups: int = 1):
+    """Causal attention of query blocks over expanded keys / values; the rotated parts sit at column Rp of q and cache. groups: 2 splits a
+    block's keys between two groups of waves (waves 4)."""
     _check(lib().nls_latent_prefill(qn.data_ptr(), qn.stride(0), qns, q.data_ptr() + Rp * q.element_size(), q.stride(0), qrs,
                                     kx.data_ptr(), vx.data_ptr(), cache.data_ptr() + Rp * cache.element_size(),
                                     cache.stride(0), xmap.data_ptr(), blocks.data_ptr(), nblocks, gate.data_ptr(),
-                                    gate.stride(0), out.data_ptr(), out.stride(0), H, dku, dr, dv, vdim, waves, scale, st),
+                                    gate.stride(0), out.data_ptr(), out.stride(0), H, dku, dr, dv, vdim, waves, groups, scale, st),
            "nls_latent_prefill")
 
 
@@ -741,12 +742,12 @@ def gqa_attention(q, kc, vc, gate, out, part, block_tables, block_size: int, tok
 
 
 def gqa_prefill(q, kc, vc, xmap, blocks, nblocks: int, waves: int, gate, out, H: int, G: int, Dp: int, scale: float, st: int,
-                window: int = 0, keep: int = 0, sink: bool = False):
+                window: int = 0, keep: int = 0, sink: bool = False, groups: int = 1):
     """Causal attention of query blocks over their sequences' paged keys and values (gate, window, keep, sink: as
-    gqa_attention)."""
+    gqa_attention; groups: as latent_prefill)."""
     _check(lib().nls_gqa_prefill(q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), xmap.data_ptr(), blocks.data_ptr(),
                                  nblocks, _p(gate), gate.stride(0) if gate is not None else 0, out.data_ptr(), out.stride(0), H, G,
-                                 Dp, waves, scale, window, keep, int(sink), st), "nls_gqa_prefill")
+                                 Dp, waves, groups, scale, window, keep, int(sink), st), "nls_gqa_prefill")
 
 
 # ---------------------------------------------------------------------------
