@@ -215,10 +215,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const __bf16* __re
 // by 4 (key & 3) (conflict-free transposed reads of 4 keys x 32 dims per half wave). The next tile's K/V
 // are loaded into registers while this tile computes (paged: one block-table lookup per key) and written
 // to the other LDS buffer after it; the rescale of O is skipped when no row max grew.
-// Grid: one workgroup per CU (64 KiB LDS, 2 waves per SIMD); blockIdx -> kv head first, so every query
+// A workgroup of one prompt walks its row block's keys tile by tile, and the last block's walk is the launch's time until there are many. So the
+// block is also taken in halves of 32 tokens (NTB 1: four waves), two workgroups to a CU, or with two groups of four waves (NG 2) that take every
+// other tile of the same rows; the second one's sums are added over LDS. One prompt of 1000 tokens, 32 heads of 128 on 8: 40 us, halves 33, two
+// groups 29; 2000 73 / 65 / 58; from some 4000 on the chip is full and whole blocks, which read K and V half as often, are best (170 / 186 / 194).
+// Grid: one workgroup per CU (64 KiB LDS, 2 waves per SIMD), two of halves; blockIdx -> kv head first, so every query
 // block of a kv head runs on one XCD and shares its K/V through that XCD's L2.
-template <int D, typename KV>
-__global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __restrict__ q, long ldq,
+template <int D, typename KV, int NTB, int NG>
+__global__ __launch_bounds__(256 * NTB * NG, 2) void attn_prefill2_kernel(const __bf16* __restrict__ q, long ldq,
                                                             const KV* __restrict__ kc, const KV* __restrict__ vc,
                                                             const int* __restrict__ block_tables, int bt_stride,
                                                             const int* __restrict__ qblocks, int nqb, int Hkv, int G,
@@ -230,25 +234,30 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
   constexpr int TILEB = KT * ROWB;       // one K (or V) tile
   constexpr int NKS = D / 16;            // k-steps of S^T over the head dim
   constexpr int NDB = D / 32;            // 32-dim blocks of O^T
-  constexpr int NLD = KT * NCH / 512;    // staging chunks per thread per K (and per V) tile
-  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * 2 * TILEB];   // [buf][K | V]
+  constexpr int NT = 256 * NTB;          // threads of a key group
+  constexpr int NLD = KT * NCH / NT;     // staging chunks per thread per K (and per V) tile
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_all[];     // [group][buf][K | V]
 
   const int nq4 = G / 4;
   const int bi = blockIdx.x;
   const int hk = bi % Hkv;
   const int rest = bi / Hkv;
   const int hq4 = rest % nq4;
-  const int qb = nqb - 1 - rest / nq4;   // heaviest (latest) query blocks first
+  const int qr = rest / nq4;             // heaviest (latest) query blocks first
+  const int qb = nqb - 1 - (NTB == 2 ? qr : qr >> 1), half = NTB == 2 ? 0 : 1 - (qr & 1);
   const int t0 = qblocks[qb * 4], ntok = qblocks[qb * 4 + 1], seq = qblocks[qb * 4 + 2], pos0 = qblocks[qb * 4 + 3];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (32 * half >= ntok) return;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = NG == 1 ? 0 : wv >> 2;
+  const int wave = wv - 4 * grp, tid = threadIdx.x - NT * grp;
+  uint8_t* lds = lds_all + grp * 4 * TILEB;
   const int h = lane >> 5, tl = lane & 31;
   const int head = hk * G + hq4 * 4 + (wave & 3);
-  const int tw0 = 32 * (wave >> 2);      // the wave's first token of the block
+  const int tw0 = 32 * (NTB == 2 ? wave >> 2 : half);      // the wave's first token of the block
   const int* bt = block_tables + (size_t)seq * bt_stride;
   const int bsm = (1 << bs_shift) - 1;
   const float sl2 = scale * LOG2E_P;
-  const int nkeys = pos0 + ntok;
+  const int nkeys = pos0 + (NTB == 2 ? ntok : min(ntok, tw0 + 32));
   const int ntile = (nkeys + KT - 1) / KT;
   const int wlast = pos0 + min(tw0 + 31, ntok - 1);   // the wave's last valid token position
   const bool wact = tw0 < ntok;
@@ -262,19 +271,19 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
   }
   const int qpos = pos0 + tw0 + tl;
 
-  // ---- staging: thread tid moves chunks e = tid + 512 i (key e / NCH, chunk e % NCH) of K and of V
+  // ---- staging: thread tid moves chunks e = tid + NT i (key e / NCH, chunk e % NCH) of K and of V
   // Cache blocks are read a tile ahead of their rows, and keys past the last one repeat it (masked below): a load behind its
   // block's, in a branch, waited for every load before it (3000 tokens, 32 heads of 128: 147 -> 130 us)
   typename KVRaw<KV>::raw kr[NLD], vr[NLD];
   int blk[NLD];
   auto load_blocks = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) blk[i] = bt[min(t * KT + (tid + 512 * i) / NCH, nkeys - 1) >> bs_shift];
+    for (int i = 0; i < NLD; ++i) blk[i] = bt[min(t * KT + (tid + NT * i) / NCH, nkeys - 1) >> bs_shift];
   };
   auto load_tile = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      const int e = tid + 512 * i, ch = e % NCH, p = min(t * KT + e / NCH, nkeys - 1);
+      const int e = tid + NT * i, ch = e % NCH, p = min(t * KT + e / NCH, nkeys - 1);
       const size_t off = ((size_t)(blk[i] << bs_shift | (p & bsm)) * Hkv + hk) * D + ch * 8;
       kr[i] = KVRaw<KV>::ld(kc + off);
       vr[i] = KVRaw<KV>::ld(vc + off);
@@ -285,7 +294,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
     uint8_t* vb = kb + TILEB;
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
-      const int e = tid + 512 * i, key = e / NCH, ch = e % NCH;
+      const int e = tid + NT * i, key = e / NCH, ch = e % NCH;
       *reinterpret_cast<u32x4*>(kb + key * ROWB + ((ch ^ (key & (NCH - 1) & 15)) << 4)) = KVRaw<KV>::bf16(kr[i]);
       *reinterpret_cast<u32x4*>(vb + key * ROWB + ((ch ^ (((key & 3) << 2) & (NCH - 1))) << 4)) = KVRaw<KV>::bf16(vr[i]);
     }
@@ -296,22 +305,25 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
   for (int i = 0; i < NDB; ++i) o[i] = f32x16{};
   float m = -INFINITY, l = 0.f;
 
-  load_blocks(0);
-  load_tile(0);
-  load_blocks(1);
-  store_tile(0);
+  load_blocks(grp);
+  if (NG == 1 || grp < ntile) {
+    load_tile(grp);
+    load_blocks(grp + NG);
+    store_tile(0);
+  }
   __syncthreads();
   // V^T fragment read: lane (group of 16: q = (l & 15) >> 2 row, p = l & 3 column quad) supplies row
   // kbase + q (and + 8), dims 32 db + 16 ((l >> 4) & 1) + 4 p
   const int vq = (lane & 15) >> 2, vp = lane & 3, vhalf = (lane >> 4) & 1;
-  for (int t = 0; t < ntile; ++t) {
-    const int cur = t & 1;
-    if (t + 1 < ntile) {                      // issue early: lands while this tile computes
-      load_tile(t + 1);
-      load_blocks(t + 2);
+  const int nstep = (ntile + NG - 1) / NG;
+  for (int i = 0; i < nstep; ++i) {
+    const int t = i * NG + grp, cur = i & 1;
+    if (t + NG < ntile) {                     // issue early: lands while this tile computes
+      load_tile(t + NG);
+      load_blocks(t + 2 * NG);
     }
     const int k0 = t * KT;
-    if (wact && k0 <= wlast) {
+    if (wact && (NG == 1 || t < ntile) && k0 <= wlast) {
       const uint8_t* kb = lds + cur * 2 * TILEB;
       const uint8_t* vb = kb + TILEB;
       // ---- S^T = K Q^T
@@ -382,12 +394,32 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
         }
       }
     }
-    if (t + 1 < ntile) {
-      store_tile(cur ^ 1);                    // write late: the other buffer was last read in tile t - 1
+    if (t + NG < ntile) {
+      store_tile(cur ^ 1);                    // write late: the other buffer was last read in the step before
     }
     __syncthreads();
   }
   // ---- normalise and store: lane holds O[token tw0 + tl][32 db + 8 g + 4 h + 0..3] in o[db][4 g .. 4 g + 3]
+  if constexpr (NG == 2) {                    // the second group's sums, brought to a common maximum
+    float* ex = reinterpret_cast<float*>(lds_all) + tid;      // [2 + 16 NDB][NT]
+    if (grp) {
+      ex[0] = m;
+      ex[NT] = l;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ex[(2 + 16 * db + r) * NT] = o[db][r];
+    }
+    __syncthreads();
+    if (grp) return;
+    const float m1 = ex[0], mn = fmaxf(m, m1);
+    const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * sl2), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - mn) * sl2);
+    l = l * a0 + ex[NT] * a1;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * a0 + ex[(2 + 16 * db + r) * NT] * a1;
+  }
   l += __shfl_xor(l, 32, 64);
   const int tok = tw0 + tl;
   if (wact && tok < ntok) {
@@ -406,38 +438,51 @@ __global__ __launch_bounds__(512, 1) void attn_prefill2_kernel(const __bf16* __r
 
 }  // namespace
 
+template <int D, typename KV, int NTB, int NG>
+int attn_prefill2_launch(const void* q, long ldq, const void* kc, const void* vc, const int* block_tables, int bt_stride,
+                         const int* qblocks, int nqb, int Hkv, int G, int bs_shift, float scale, void* out, long ldo,
+                         hipStream_t st) {
+  constexpr int LDS = NG * 4 * 64 * D * 2;
+  static_assert(NG == 1 || 256 * NTB * (2 + D / 2) * 4 <= LDS, "a group's partial sums take the place of the tiles");
+  static bool attr = false;
+  if (!attr) {
+    if (hipFuncSetAttribute((const void*)attn_prefill2_kernel<D, KV, NTB, NG>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+      return -1;
+    attr = true;
+  }
+  hipLaunchKernelGGL((attn_prefill2_kernel<D, KV, NTB, NG>), dim3(nqb * (3 - NTB) * Hkv * (G / 4)), dim3(256 * NTB * NG), LDS, st, (const __bf16*)q,
+                     ldq, (const KV*)kc, (const KV*)vc, block_tables, bt_stride, qblocks, nqb, Hkv, G, bs_shift, scale, (act_t*)out, ldo);
+  return (int)hipGetLastError();
+}
+
+// form 0: blocks of 64 tokens, one workgroup to a CU; 1: halves of 32, two to a CU; 2: halves whose keys two groups of waves share
 template <typename KV>
 int attn_prefill2_impl(const void* q, long ldq, const void* kc, const void* vc, const int* block_tables, int bt_stride,
                        const int* qblocks, int nqb, int Hq, int Hkv, int D, int block_size, float scale, void* out,
-                       long ldo, void* stream) {
+                       long ldo, int form, void* stream) {
   if (Hq % Hkv || (Hq / Hkv) % 4 || (D != 64 && D != 128) || nqb < 1 || block_size < 1 ||
-      (block_size & (block_size - 1)))
+      (block_size & (block_size - 1)) || form < 0 || form > 2)
     return -1;
-  const int G = Hq / Hkv;
-  const int bs_shift = __builtin_ctz(block_size);
-  dim3 grid(nqb * Hkv * (G / 4));
-  hipStream_t st = (hipStream_t)stream;
-  if (D == 128)
-    hipLaunchKernelGGL((attn_prefill2_kernel<128, KV>), grid, dim3(512), 0, st, (const __bf16*)q, ldq, (const KV*)kc,
-                       (const KV*)vc, block_tables, bt_stride, qblocks, nqb, Hkv, G, bs_shift, scale, (act_t*)out, ldo);
-  else
-    hipLaunchKernelGGL((attn_prefill2_kernel<64, KV>), grid, dim3(512), 0, st, (const __bf16*)q, ldq, (const KV*)kc,
-                       (const KV*)vc, block_tables, bt_stride, qblocks, nqb, Hkv, G, bs_shift, scale, (act_t*)out, ldo);
-  return (int)hipGetLastError();
+#define NLS_PF2(DD, NTB, NG) \
+  attn_prefill2_launch<DD, KV, NTB, NG>(q, ldq, kc, vc, block_tables, bt_stride, qblocks, nqb, Hkv, Hq / Hkv, __builtin_ctz(block_size), scale, \
+                                        out, ldo, (hipStream_t)stream)
+  if (D == 128) return form == 0 ? NLS_PF2(128, 2, 1) : form == 1 ? NLS_PF2(128, 1, 1) : NLS_PF2(128, 1, 2);
+  return form == 0 ? NLS_PF2(64, 2, 1) : form == 1 ? NLS_PF2(64, 1, 1) : NLS_PF2(64, 1, 2);
+#undef NLS_PF2
 }
 
 extern "C" int nls_attn_prefill(const void* q, long ldq, const void* kc, const void* vc, const int* block_tables,
                                  int bt_stride, const int* qblocks, int nqb, int Hq, int Hkv, int D, int block_size,
-                                 float scale, void* out, long ldo, void* stream) {
+                                 float scale, void* out, long ldo, int form, void* stream) {
   return attn_prefill2_impl<__bf16>(q, ldq, kc, vc, block_tables, bt_stride, qblocks, nqb, Hq, Hkv, D, block_size,
-                                    scale, out, ldo, stream);
+                                    scale, out, ldo, form, stream);
 }
 
 extern "C" int nls_attn_prefill8(const void* q, long ldq, const void* kc, const void* vc, const int* block_tables,
                                    int bt_stride, const int* qblocks, int nqb, int Hq, int Hkv, int D, int block_size,
-                                   float scale, void* out, long ldo, void* stream) {
+                                   float scale, void* out, long ldo, int form, void* stream) {
   return attn_prefill2_impl<uint8_t>(q, ldq, kc, vc, block_tables, bt_stride, qblocks, nqb, Hq, Hkv, D, block_size,
-                                     scale, out, ldo, stream);
+                                     scale, out, ldo, form, stream);
 }
 
 template <typename KV>

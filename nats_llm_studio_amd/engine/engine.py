@@ -961,7 +961,8 @@ class Engine:
     def _pf_forward(self, Tb: int, need_logits: bool):
         ld, qd = self._pf_dev
         return self.model.forward(self.pb, self.kc, self.vc, Tb, self.bs, self.model.n_splits(Tb),
-                                  logit_rows=ld[:1], n_logits=1, qblocks=qd[:1], nqb=1, need_logits=need_logits)
+                                  logit_rows=ld[:1], n_logits=1, qblocks=qd[:1], nqb=1, need_logits=need_logits,
+                                  **({"qform": 2} if hasattr(self.model, "prefill_form") else {}))     # (one block, behind any context)
 
     def _capture_prefill(self, key):
         """Capture the prefill graph `key` on the current metadata (the caller ran the same forward eagerly)."""
@@ -984,6 +985,8 @@ class Engine:
                 info = {"row_info": ri}
         else:
             qb = ops.prefill_blocks(h[3 * pad:4 * pad], h[pad:2 * pad], T) if self.prefill_attn else None
+            if qb is not None and hasattr(self.model, "prefill_form"):
+                info = {"qform": self.model.prefill_form(qb)}
         key = self._pf_graph_key(T, rows, qb, need_logits)
         if key is not None:
             # rows T .. Tb-1 of the token bucket: no KV writes (slot -1), position 0 (the RoPE table), no attention

@@ -462,13 +462,17 @@ class LlamaModel:
             return 1
         return int(min(_SPLIT_CAP, max(1, _SPLIT_WG // wg)))
 
+    def prefill_form(self, qblocks) -> int:
+        """Form of the prompt attention for a step's query blocks (host side)."""
+        return ops.prefill_form(qblocks, self.Hkv * max(1, self.Hq // self.Hkv // 4))
+
     # ------------------------------------------------------------------ forward
     def forward(self, b: StepBuffers, kc: torch.Tensor, vc: torch.Tensor, T: int, block_size: int,
                 n_split: int = 1, logit_rows: Optional[torch.Tensor] = None, n_logits: Optional[int] = None,
                 qblocks: Optional[torch.Tensor] = None, nqb: int = 0, feed_prev: bool = False,
-                need_logits: bool = True):
+                need_logits: bool = True, qform: int = 0):
         """Runs T tokens through the model; leaves greedy ids in b.next_ids[:n] and logits in b.logits[:n].
-        With `qblocks` (prompt chunks, ops.prefill_blocks) attention runs the MFMA flash-prefill kernel."""
+        With `qblocks` (prompt chunks, ops.prefill_blocks) attention runs the MFMA flash-prefill kernel in its form `qform`."""
         cfg = self.cfg
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         x = b.x
@@ -503,7 +507,7 @@ class LlamaModel:
                             self.rope_neox, bias=lw.qkv_bias)
             if qblocks is not None and nqb > 0 and ops.attention_prefill_ok(Hq, Hkv, D):
                 ops.attention_prefill(b.q, kc[L], vc[L], b.block_tables, qblocks, nqb, b.tok_seq, b.ctx_len, b.ao,
-                                      T, Hq, Hkv, D, block_size, cfg.attn_softmax_scale)
+                                      T, Hq, Hkv, D, block_size, cfg.attn_softmax_scale, qform)
             else:
                 ops.attention(b.q, kc[L], vc[L], b.block_tables, b.tok_seq, b.ctx_len, b.ao, T, Hq, Hkv, D,
                               block_size, cfg.attn_softmax_scale, chunk=-_MIN_CHUNK, n_split=n_split, workspace=b.attn_ws,

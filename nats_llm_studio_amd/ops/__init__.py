@@ -844,20 +844,36 @@ def prefill_blocks(tok_seq, pos, T: int):
     return np.asarray(out, dtype=np.int32).reshape(-1, 4)
 
 
+def prefill_form(qblocks, units: int) -> int:
+    """Form of attention_prefill for the blocks of a step, with `units` workgroups (key heads x fours of query heads) to a block: 0, 64 tokens to a
+    workgroup, one to a CU; 1, 32 tokens, two to a CU; 2, 32 tokens whose keys two groups of waves share, where the longest walk (in tiles of 64
+    keys) outlasts the others or there are few workgroups. us of forms 0 / 1 / 2, 32 heads of 128 on 8: one prompt of 600 tokens 27 / 22 / 20, 1000
+    40 / 33 / 29, 2000 73 / 65 / 58, 3000 109 / 101 / 124, 4096 170 / 186 / 194, 1000 behind 4000 175 / 145 / 116; 6 x 650 55 / 52 / 62, 64 x 60
+    26 / 22 / 34, 300 x 20 54 / 61 / 126; 16 heads on 4, 3000 tokens 103 / 86 / 68."""
+    qb = np.asarray(qblocks)
+    if not len(qb):
+        return 0
+    walks = -(-(qb[:, 1] + qb[:, 3]) // 64)
+    most, mean, n = int(walks.max()), float(walks.sum()) * units / 256, len(qb) * units
+    if most >= 6 and (2 * n <= 256 or (most >= 16 and most >= 1.75 * mean)):
+        return 2
+    return 1 if most >= 1.2 * mean or (most <= 12 and n <= 640) else 0
+
+
 def attention_prefill_ok(Hq: int, Hkv: int, D: int) -> bool:
     return Hq % Hkv == 0 and (Hq // Hkv) % 4 == 0 and D in (64, 128)
 
 
 def attention_prefill(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, block_tables: torch.Tensor,
                       qblocks: torch.Tensor, nqb: int, tok_seq: torch.Tensor, ctx_len: torch.Tensor,
-                      out: torch.Tensor, T: int, Hq: int, Hkv: int, D: int, block_size: int, scale: float):
+                      out: torch.Tensor, T: int, Hq: int, Hkv: int, D: int, block_size: int, scale: float, form: int = 0):
     """Causal MFMA flash attention over the paged cache for prompt chunks (query blocks of PREFILL_QT tokens,
-    ops.prefill_blocks)."""
+    ops.prefill_blocks; form: ops.prefill_form)."""
     if q.is_cuda:
         _lib.check(_kv_fn("nls_attn_prefill_v1" if PREFILL_V1 else "nls_attn_prefill", kc)(q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(),
                                                block_tables.data_ptr(), block_tables.stride(0), qblocks.data_ptr(),
                                                nqb, Hq, Hkv, D, block_size, float(scale), out.data_ptr(),
-                                               out.stride(0), _stream_ptr(q)), "nls_attn_prefill")
+                                               out.stride(0), *(() if PREFILL_V1 else (form,)), _stream_ptr(q)), "nls_attn_prefill")
         return out
     return attention(q, kc, vc, block_tables, tok_seq, ctx_len, out, T, Hq, Hkv, D, block_size, scale)
 

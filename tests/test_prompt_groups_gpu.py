@@ -1,10 +1,12 @@
-"""Prompt attention whose keys two groups of waves share: walks of one tile (the second group has none), of two and of odd counts, windows, keys
+"""Prompt attention (of the stacks, and of GGUF models) in halves of a block and where two groups of waves share the keys: walks of one tile (the second group has none), of two and of odd counts, windows, keys
 of one group only that outweigh the other's, and the choice between the forms."""
 import types
 
+import numpy as np
 import pytest
 import torch
 
+from nats_llm_studio_amd import ops
 from nats_llm_studio_amd.models.stack import _prompt_waves
 from nats_llm_studio_amd.ops import stack as K
 
@@ -109,3 +111,41 @@ def test_expanded(dku, dr, dv, vdim):
 def test_choice(heads, window, spans, want):
     att = [types.SimpleNamespace(cfg=types.SimpleNamespace(heads=heads, window=window))]
     assert _prompt_waves(att, [(0, n, 0, p, 0, p + n, 0, 0) for p, n in spans]) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("kvt", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("D,G,Hkv", [(128, 4, 2), (64, 8, 1)])
+def test_gguf_forms(form, kvt, D, G, Hkv):
+    bs, g, H = 16, torch.Generator(device="cuda").manual_seed(D), G * Hkv
+    pages = max(-(-(p + n) // bs) for p, n in RUNS)
+    bt = torch.randperm(len(RUNS) * pages, generator=torch.Generator().manual_seed(1)).view(len(RUNS), pages).int().cuda()
+    q = torch.randn(T, H, D, generator=g, device="cuda").bfloat16()
+    k, v = (torch.randn(NX, Hkv, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    loud(k, q[:, ::G])
+    k, v = k.to(kvt), v.to(kvt)
+    kc, vc = (torch.zeros(bt.numel() * bs, Hkv, D, device="cuda").to(kvt) for _ in range(2))
+    x = 0
+    for r, (p, n) in enumerate(RUNS):
+        at = torch.arange(p + n, device="cuda")
+        at = bt[r, at // bs].long() * bs + at % bs
+        for c, t in ((kc, k), (vc, v)):
+            c.view(torch.uint8 if kvt.itemsize == 1 else torch.int16)[at] = t[x:x + p + n].view(torch.uint8 if kvt.itemsize == 1 else torch.int16)
+        x += p + n
+    seq = np.concatenate([np.full(n, r) for r, (_, n) in enumerate(RUNS)])
+    pos = np.concatenate([np.arange(p, p + n) for p, n in RUNS])
+    qb = ops.prefill_blocks(seq, pos, T)
+    out = torch.full((T + 1, H * D), 7.0, dtype=ops.ACT_DTYPE, device="cuda")
+    ops.attention_prefill(q.view(T, -1), kc, vc, bt, torch.from_numpy(qb).cuda(), len(qb), None, None, out, T, H, Hkv, D, bs, D ** -0.5, form)
+    assert (out[T] == 7).all()
+    check(out[:T].view(T, H, D), q, k.float().repeat_interleave(G, 1), v.float().repeat_interleave(G, 1), D ** -0.5)
+
+
+@pytest.mark.parametrize("units,runs,want", [
+    (8, [(0, 21)], 1), (8, [(0, 300)], 1), (8, [(0, 1000)], 2), (8, [(0, 2000)], 2), (8, [(0, 3000)], 1), (8, [(0, 4096)], 0), (4, [(0, 3000)], 2),
+    (8, [(4000, 1000)], 2), (8, [(0, 60)] * 64, 1), (8, [(0, 20)] * 300, 0), (4, [(0, 8000)], 0)])
+def test_gguf_choice(units, runs, want):
+    seq = np.concatenate([np.full(n, r) for r, (_, n) in enumerate(runs)])
+    pos = np.concatenate([np.arange(p, p + n) for p, n in runs])
+    assert ops.prefill_form(ops.prefill_blocks(seq, pos, len(seq)), units) == want
