@@ -402,23 +402,27 @@ __global__ __launch_bounds__(256 * NTB * NG, 2) void attn_prefill2_kernel(const 
   // ---- normalise and store: lane holds O[token tw0 + tl][32 db + 8 g + 4 h + 0..3] in o[db][4 g .. 4 g + 3]
   if constexpr (NG == 2) {                    // the second group's sums, brought to a common maximum
     float* ex = reinterpret_cast<float*>(lds_all) + tid;      // [2 + 16 NDB][NT]
-    if (grp) {
-      ex[0] = m;
-      ex[NT] = l;
+    if (ntile == 1) {                         // (a short prompt in the form of a captured launch: there are none)
+      if (grp) return;
+    } else {
+      if (grp) {
+        ex[0] = m;
+        ex[NT] = l;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) ex[(2 + 16 * db + r) * NT] = o[db][r];
+      }
+      __syncthreads();
+      if (grp) return;
+      const float m1 = ex[0], mn = fmaxf(m, m1);
+      const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * sl2), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - mn) * sl2);
+      l = l * a0 + ex[NT] * a1;
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) ex[(2 + 16 * db + r) * NT] = o[db][r];
+        for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * a0 + ex[(2 + 16 * db + r) * NT] * a1;
     }
-    __syncthreads();
-    if (grp) return;
-    const float m1 = ex[0], mn = fmaxf(m, m1);
-    const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * sl2), a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - mn) * sl2);
-    l = l * a0 + ex[NT] * a1;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[db][r] = o[db][r] * a0 + ex[(2 + 16 * db + r) * NT] * a1;
   }
   l += __shfl_xor(l, 32, 64);
   const int tok = tw0 + tl;
