@@ -1657,6 +1657,7 @@ class Engine:
         if not self.use_graphs:
             return
         self._drain()
+        self.feed_wait()                   # (a queued step's upload reads the staging buffers that are cleared here)
         self._precapture_prefill()
         pad = self.db.pad
         h = self.h_meta_d2[0].numpy()

@@ -514,6 +514,27 @@ def test_feed_steps_under_way(gpu, tmp_path, dt):
 
 
 @pytest.mark.parametrize("dt", DT)
+def test_capture_behind_feed_steps(gpu, tmp_path, dt):
+    """Graphs captured while prompt and decode steps are queued: the steps keep their tokens."""
+    cfg = S.CONFIGS["uneven"]
+    W = S.make_weights(cfg)
+    eng = engine(load(tmp_path, cfg, W, dt))
+    t = S.tokens(40, cfg["vocab"], 31)
+    want = O.forward(cfg, W, t)[-1:]
+    eng.feed([("a", t[:30], [])])
+    torch.cuda._sleep(20_000_000)                # (the uploads of what follows wait behind it)
+    for i in range(30, 33):
+        eng.feed([("a", t[i:i + 1], [])])
+    eng.capture_all()
+    torch.cuda._sleep(20_000_000)
+    eng.feed([("a", t[33:37], [])])
+    eng.capture_all([1])
+    for i in range(37, 40):
+        (got,) = eng.feed([("a", t[i:i + 1], [0] if i == 39 else [])])
+    assert close(got, want, dt)
+
+
+@pytest.mark.parametrize("dt", DT)
 def test_long_prompt_segments(gpu, tmp_path, dt):
     """A prompt long enough that the recurrence runs in segments, alone and beside other runs, then decoded on."""
     cfg = S.CONFIGS["uneven"]

@@ -270,6 +270,32 @@ def test_engine_rows_of_many_prompts(n):
     assert at == T
 
 
+class _Queued:
+    """Stands for the stream of a queued feed step: notes what waits for it."""
+    def __init__(self, log):
+        self.log, self.device = log, torch.device("cuda:0")
+
+    def synchronize(self):
+        self.log.append("wait")
+
+
+def test_engine_capture_waits_for_feed_steps(monkeypatch):
+    """The staging buffers that a queued step's upload may still read are cleared only when it is over."""
+    from nats_llm_studio_amd.engine.engine import Engine
+    eng = Engine(_FakeRecurrent(), None, max_batch=2, num_blocks=8, max_prefill_tokens=16, ctx=96, use_graphs=False)
+    eng.feed([("a", [5, 6, 7], [])])
+    eng.feed([("a", [8], [])])
+    log, staged = [], [h.clone() for h in eng.h_meta_d2]
+    eng.use_graphs, eng._flight = True, _Queued(log)
+    eng._flight.synchronize = lambda: log.append([torch.equal(a, b) for a, b in zip(eng.h_meta_d2, staged)])
+    monkeypatch.setattr(eng, "_precapture_prefill", lambda: log.append("prefill"))
+    monkeypatch.setattr(eng, "_capture", lambda *a, **k: log.append("decode"))
+    eng.capture_all([2])
+    assert log[:3] == [[True, True], "prefill", "decode"] and eng._flight is None
+    (got,) = eng.feed([("a", [9], [0])])
+    assert int(got[0].argmax()) == _fake_next([5, 6, 7, 8, 9])
+
+
 def test_engine_feed_results_are_their_own():
     """Results share no memory with those of other entries, wherever their rows came from: a kept row keeps no more than itself."""
     from nats_llm_studio_amd.engine.engine import Engine
