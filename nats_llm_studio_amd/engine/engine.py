@@ -450,11 +450,11 @@ class Engine:
         if self.thread is not None:
             self.thread.join()
             self.thread = None
-        try:
-            self._drain()
-            self.feed_wait()
-        except Exception:
-            pass
+        for settle in (self._drain, self.feed_wait):       # (a failed step does not keep the queued ones from being waited for)
+            try:
+                settle()
+            except Exception:
+                pass
         self.stop_followers()
         for s in list(self.running) + list(self.waiting):
             self._finish(s, "cancelled", "engineShutdown")

@@ -296,6 +296,20 @@ def test_engine_capture_waits_for_feed_steps(monkeypatch):
     assert int(got[0].argmax()) == _fake_next([5, 6, 7, 8, 9])
 
 
+def test_engine_shutdown_waits_for_feed_steps(monkeypatch):
+    """Also where the generation's last step failed: what the queued steps use is freed next."""
+    from nats_llm_studio_amd.engine.engine import Engine
+    eng = Engine(_FakeRecurrent(), None, max_batch=2, num_blocks=8, max_prefill_tokens=16, ctx=96, use_graphs=False)
+    log = []
+    eng._flight = _Queued(log)
+
+    def failed():
+        raise RuntimeError("step")
+    monkeypatch.setattr(eng, "_drain", failed)
+    eng.unload()
+    assert log == ["wait"] and eng.kc is None
+
+
 def test_engine_feed_results_are_their_own():
     """Results share no memory with those of other entries, wherever their rows came from: a kept row keeps no more than itself."""
     from nats_llm_studio_amd.engine.engine import Engine
