@@ -22,6 +22,7 @@ import os
 import math
 import threading
 import time
+import weakref
 from collections import defaultdict, deque
 from concurrent.futures import Future
 from dataclasses import dataclass, field
@@ -218,6 +219,8 @@ class _Seq:
 
 
 class Engine:
+    _queued = weakref.WeakSet()             # engines that have queued feed steps
+
     def __init__(self, model, tokenizer=None, max_batch: int = 64, block_size: int = 16,
                  num_blocks: Optional[int] = None, max_prefill_tokens: int = 2048, use_graphs: bool = True,
                  ctx: Optional[int] = None, kv_mem_fraction: float = 0.5, eos_ids: Seq[int] = (),
@@ -508,6 +511,7 @@ class Engine:
         hm, clk = self.host_ms, time.perf_counter
         t0 = clk()
         self.feed_wait()                   # (requests that were fed and not ended)
+        self._other_streams()
         self._expire()
         self._admit()
         t1 = clk()
@@ -720,8 +724,7 @@ class Engine:
             raise RuntimeError("feed: the engine is generating")
         if len(set(e[0] for e in entries)) != len(entries):
             raise ValueError("feed: one entry per request and step")
-        if self._flight is not None and self._flight != torch.cuda.current_stream(self.dev):
-            self.feed_wait()
+        self._other_streams()
         # (a decode step of a few hundred requests waits for this loop: a token at a time is checked without an array)
         V, bs, single, seqs = self.cfg.vocab, self.bs, True, []
         for rid, toks, want in entries:
@@ -815,6 +818,20 @@ class Engine:
         if st is not None:
             st.synchronize()
 
+    def _fly(self):
+        self._flight = torch.cuda.current_stream(self.dev)
+        Engine._queued.add(self)
+
+    def _other_streams(self):
+        """Wait for queued feed steps that are not on the current stream, those of other engines too: the launches of all engines share the
+        split-K workspace."""
+        for e in list(Engine._queued):
+            st = e._flight
+            if st is not None:
+                cur = torch.cuda.current_stream(st.device)
+                if st != cur:
+                    st.synchronize()
+
     def _feed_decode(self, seqs, entries, out, wants):
         cuda = self.dev.type == "cuda"
         if any(s.row < 0 for s in seqs):
@@ -831,7 +848,7 @@ class Engine:
             self._ev[self._kbuf ^ 1].synchronize()         # the staging buffer's last step
         (snap, k) = self._launch(seqs, set(), need, fetch=False)
         if cuda and not need:
-            self._flight = torch.cuda.current_stream(self.dev)
+            self._fly()
             return
         if need:
             for t, w in zip(out, wants):   # (pages of the results, 3 ms of 300 rows, while the device is busy)
@@ -876,10 +893,11 @@ class Engine:
             self._fill_rows(parts)
             self._exec_prefill(T, rows or [0], True, len(parts))
             self.counters["prefill_tokens"] += T
-            if self.dev.type == "cuda":
-                self._flight = None if rows else torch.cuda.current_stream(self.dev)
             if rows:
+                self._flight = None
                 self._rows_to_host(self.pb.logits[:len(rows)], [out[i][a:b] for i, a, b in dest])
+            elif self.dev.type == "cuda":
+                self._fly()
 
     def feed_end(self, rid):
         """The request is finished: its blocks, state slot and decode row are free again."""

@@ -310,6 +310,28 @@ def test_engine_shutdown_waits_for_feed_steps(monkeypatch):
     assert log == ["wait"] and eng.kc is None
 
 
+def test_engines_on_two_streams(monkeypatch):
+    """Feeding or generating with one engine waits for steps that another one has queued on another stream (they share a workspace), not
+    for those on the same stream."""
+    from nats_llm_studio_amd.engine.engine import Engine
+    from nats_llm_studio_amd.engine.sampling import SamplingParams
+    a, b = (Engine(_FakeRecurrent(), None, max_batch=2, num_blocks=8, max_prefill_tokens=16, ctx=96, use_graphs=False) for _ in range(2))
+    log, cur = [], _Queued([])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev=None: cur)
+    a._flight = cur
+    Engine._queued.add(a)
+    b.feed([("x", [1, 2], [])])
+    assert not log and not cur.log
+    a._flight = _Queued(log)
+    b.feed([("x", [3, 4], [])])
+    assert log == ["wait"]
+    b.feed_end("x")
+    a._flight = _Queued(log)
+    b.generate([1, 2, 3], SamplingParams(max_tokens=1, ignore_eos=True))
+    assert len(log) >= 2
+    a._flight = None
+
+
 def test_engine_feed_results_are_their_own():
     """Results share no memory with those of other entries, wherever their rows came from: a kept row keeps no more than itself."""
     from nats_llm_studio_amd.engine.engine import Engine
