@@ -1099,6 +1099,8 @@ class StackModel:
         key = ("grown", name, cols)
         t = b.shared.get(key)
         if t is None or t.shape[0] < rows:
+            if t is not None and t.is_cuda:            # (a queued step on another stream than the one it was made on may still use it)
+                t.record_stream(torch.cuda.current_stream(t.device))
             b.shared[key] = None
             t = b.shared[key] = torch.zeros(K.pad_to(rows, 1024), cols, dtype=dtype or self.dtype, device=self.device)
         return t

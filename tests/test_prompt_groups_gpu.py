@@ -149,3 +149,22 @@ def test_gguf_choice(units, runs, want):
     seq = np.concatenate([np.full(n, r) for r, (_, n) in enumerate(runs)])
     pos = np.concatenate([np.arange(p, p + n) for p, n in runs])
     assert ops.prefill_form(ops.prefill_blocks(seq, pos, len(seq)), units) == want
+
+
+@pytest.mark.gpu
+def test_grown_scratch_of_a_queued_step():
+    """A scratch that a queued launch of a side stream still uses is not handed out again when a larger one takes its place."""
+    from nats_llm_studio_amd.models.stack import StackModel
+    m, b = types.SimpleNamespace(dtype=torch.float32, device="cuda"), types.SimpleNamespace(shared={})
+    t = StackModel.grown(m, b, "x", 1024, 4096)
+    at, side = t.data_ptr(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(50_000_000)
+        t.fill_(3.0)
+        del t
+        StackModel.grown(m, b, "x", 2048, 4096)
+    assert not side.query()
+    other = torch.empty(1024, 4096, device="cuda")
+    assert other.data_ptr() != at
+    torch.cuda.synchronize()
