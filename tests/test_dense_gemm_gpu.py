@@ -108,6 +108,26 @@ def test_blocks_of_320(M, K):
         assert (y[M:] == 7).all()
 
 
+@pytest.mark.parametrize("M", [257, 300, 320, 513, 640])
+def test_blocks_of_320_gate_and_head(M):
+    """The other epilogues of 320-row blocks: SwiGLU, and a head's arg-max with its logits and alone."""
+    rows, K = 25600, 256                         # 200 weight tiles
+    w, x = weight(rows, K), acts(M, K)
+    z = x[:M].double() @ w.d16.double().T
+    v = z.view(M, rows // 16, 2, 8)
+    want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, rows // 2)
+    y = torch.full((x.shape[0] + 1, rows // 2), 7.0, device="cuda", dtype=torch.float16)
+    ops.qgemv([ops.Seg(w)], x, y, M, epi="swiglu", mode=10, waves=8, rt=2, ks=1)
+    assert relerr(y[:M], want) < 5e-4 and (y[M:] == 7).all()                       # f16 outputs round to 2^-11
+    logits = torch.full((M + 1, rows), 7.0, device="cuda")
+    for epi in ("f32", "argmax"):
+        keys, ids = torch.zeros(M + 1, dtype=torch.int64, device="cuda"), torch.full((M + 1,), -1, dtype=torch.int32, device="cuda")
+        ops.qgemv([ops.Seg(w)], x, logits, M, epi=epi, argmax=keys, mode=10, waves=8, rt=2, ks=1)
+        ops.argmax_unpack(keys, M, ids)
+        assert (ids[:M].long() == logits[:M].argmax(1)).all() and int(keys[M]) == 0 and int(ids[M]) == -1, epi
+    assert relerr(logits[:M], z) < 4e-6 and (logits[M:] == 7).all()
+
+
 def test_blocks_of_320_rope():
     """144 weight tiles in three segments; D = 34 takes the general stores."""
     M, K = 300, 256

@@ -179,6 +179,44 @@ def test_grouped_blocks(gpu, mode, waves, rt, rows, bound):
             assert ((got - xd @ W.t()).abs() <= (xd.abs() @ W.abs().t()) * 2.0 ** -9).all()      # (the bound of test_active_tiles)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("qt", [GGMLType.Q4_K, GGMLType.Q5_K, GGMLType.Q6_K, GGMLType.Q8_0])
+@pytest.mark.parametrize("rows", [(0, 1, 257, 256), (96, 513, 0)])
+def test_grouped_gate_and_down(gpu, qt, rows):
+    """Mode 9 as the experts of long prompts run it: gate and up with the gate applied to scattered rows, then the down projection from them;
+    weight rows that are no multiple of 256, one super-block of K and several. Bounds: test_active_tiles."""
+    E, T, n = len(rows), 600, sum(rows)
+    rng, g = np.random.default_rng(n), torch.Generator().manual_seed(n)
+    for K, F in ((256, 768), (1280, 256)):
+        N = 2 * F - 112                                       # (a whole number of 16-row tiles)
+        gu, dn = ([Q.random_blocks(qt, a * b, 0.05, rng) for _ in rows] for a, b in ((N, K), (K - 16, F)))
+        wg, wd = [ops.QWeight(r, qt, N, K, gpu) for r in gu], [ops.QWeight(r, qt, K - 16, F, gpu) for r in dn]
+        lists, at = [torch.randperm(T, generator=g)[:c] for c in rows], np.cumsum((0,) + rows)
+        ys = torch.randperm(n, generator=g).int()             # (an expert's rows of y are anywhere)
+        xr, yr = torch.zeros(E * T, dtype=torch.int32), torch.zeros(E * T, dtype=torch.int32)
+        for e, t in enumerate(lists):
+            xr[e * T:e * T + len(t)], yr[e * T:e * T + len(t)] = t.int(), ys[at[e]:at[e + 1]]
+        x = torch.randn(T, K, generator=g).to(ops.ACT_DTYPE).to(gpu)
+        act = torch.full((n + 1, F), 3.0, device=gpu, dtype=ops.ACT_DTYPE)
+        act[:n, N // 2:] = 0
+        y = torch.full((n + 1, K - 16), 3.0, device=gpu)
+        xr, yr, counts = xr.to(gpu), yr.to(gpu), torch.tensor(rows, dtype=torch.int32, device=gpu)
+        for ws, a, b, epi in ((wg, x, act, "swiglu"), (wd, act, y, "f32")):
+            segs = [ops.Seg(w, 0, (xr if a is x else yr)[e * T:], yr[e * T:], counts[e:e + 1]) for e, w in enumerate(ws)]
+            ops.qgemv(segs, a, b, T, epi=epi, mode=9, waves=8, rt=2, ks=1, routed=n)
+        assert (act[n] == 3.0).all() and (y[n] == 3.0).all() and (act[:n, N // 2:] == 0).all()
+        for e, t in enumerate(lists):
+            W, at_y = ops.QWeight(gu[e], qt, N, K, "cpu").dense().double(), ys[at[e]:at[e + 1]].long()
+            xd, c = x.cpu().double()[t], len(t)
+            ref, err = xd @ W.t(), (xd.abs() @ W.abs().t()) * 2.0 ** -9
+            a, u, ea, eu = (v.view(c, N // 16, 2, 8)[:, :, i].reshape(c, N // 2) for v in (ref, err) for i in (0, 1))
+            want = torch.nn.functional.silu(a) * u
+            bound = 1.1 * ea * (u.abs() + eu) + torch.nn.functional.silu(a).abs() * eu + want.abs() * 2.0 ** -10 + 2.0 ** -14
+            assert ((act.cpu().double()[at_y, :N // 2] - want).abs() <= bound).all()
+            D, ad = ops.QWeight(dn[e], qt, K - 16, F, "cpu").dense().double(), act.cpu().double()[at_y]
+            assert ((y.cpu().double()[at_y] - ad @ D.t()).abs() <= (ad.abs() @ D.abs().t()) * 2.0 ** -9).all()
+
+
 def test_expert_gemm_rule():
     """Configs that exist, of types their modes take; the DMA GEMM only where it is allowed."""
     for type in (7, 8, 12, 13, 14):
