@@ -357,7 +357,7 @@ template <int WM, int BN, int NWV, int NST>
 int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   typedef HG<WM, BN, NWV, NST> G;
   const int nmb = (a.M + G::BM - 1) / G::BM;
-  const int slots = grouped_slots(sl, a, G::BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
+  const int slots = grouped_slots(sl, a, ntiles, G::BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)hgemm_kernel<WM, BN, NWV, NST>, hipFuncAttributeMaxDynamicSharedMemorySize,

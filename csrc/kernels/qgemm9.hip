@@ -460,7 +460,7 @@ template <int KSET, int RT, int NWV, int BM, bool MAP>
 int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   constexpr int lds = kset_lds<KSET, RT, NWV, BM>();
   const int nmb = (a.M + BM - 1) / BM;
-  const int slots = MAP ? grouped_slots(sl, a, BM) : 0, grid = block_grid(sl, ntiles, ks, nmb, slots);
+  const int slots = MAP ? grouped_slots(sl, a, ntiles, BM) : 0, grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)qgemm9_kernel<KSET, RT, NWV, BM, MAP>, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -344,7 +344,7 @@ int launch_dma_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArg
   constexpr int BM = MT * 16;
   const int nmb = (a.M + BM - 1) / BM;
   const size_t lds = dma_lds_bytes<MT>();
-  const int slots = grouped_slots(sl, a, BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
+  const int slots = grouped_slots(sl, a, ntiles, BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)qmm_dma_kernel<MT, KSET>, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -389,7 +389,7 @@ int launch_lds_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArg
   constexpr int BM = WM * 64;
   const int nmb = (a.M + BM - 1) / BM;
   const size_t lds = (size_t)2 * (BM + 128) * 64 * sizeof(act_t);
-  const int slots = grouped_slots(sl, a, BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
+  const int slots = grouped_slots(sl, a, ntiles, BM), grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
     if (hipFuncSetAttribute((const void*)qmm_lds_kernel<WM, KSET>, hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -76,13 +76,18 @@ struct GemvArgs {
 // Grouped launches (experts: segments of one shape with device row counts) of the tiled GEMMs. In a grid of (tile, every block of BM rows that an
 // expert might have) most workgroups have no rows and exit at once, at a fixed period of the workgroup ids; an XCD deals its workgroups to the
 // shader engines in turn, so those with rows meet on some of the engines while the others idle (eight experts of 8192 x 2048, 1000 tokens of two
-// each, one block of four with rows: 358 us). So the workgroups number the blocks that do have rows, through the counts, one after another for
-// each weight tile, and those without work are the last of the grid (151 us). The grid holds, for a weight tile, as many blocks as all rows can
-// fill: rows / BM and a part block for each segment.
-inline int grouped_slots(const SegList& sl, const GemvArgs& a, int BM) {
+// each, one block of four with rows: 358 us). So the workgroups number the blocks that do have rows, through the counts, and those without work
+// are the last of the grid (151 us). The grid holds, for a weight tile, as many blocks as all rows can fill: rows / BM and a part block for each
+// segment. All experts' blocks for each tile in turn while their rows (16 MB) stay in the caches; else expert by expert, the tiles of all experts
+// dealt to the XCDs in turn (28672 x 4096 at 768 and 1500 rows in blocks of 96 1891 -> 1776 and 3544 -> 3439 us, 4096 x 4096 at 1000 365 -> 338;
+// but 2816 x 2048 at 256 rows in blocks of 256 69 -> 90, 2048 x 768 34 -> 37). Reading the counts costs a workgroup 0.5 to 1 us (2048 x 768 at 10
+// rows 12.2 us without, 13.1 with), so grids with one block to an expert, or whose workgroups with rows have a CU each however they are spread,
+// stay as they are.
+inline int grouped_slots(const SegList& sl, const GemvArgs& a, int ntiles, int BM) {
   for (int s = 0; s < sl.nseg; ++s)
     if (!sl.s[s].mcount || sl.s[s].rows != sl.s[0].rows) return 0;
   const int nmb = (a.M + BM - 1) / BM;
+  if (nmb == 1 || ntiles * min(nmb, 4) <= 256) return 0;
   return a.nrows > 0 ? min(sl.nseg * nmb, a.nrows / BM + sl.nseg) : sl.nseg * nmb;
 }
 
@@ -100,24 +105,35 @@ DEVI bool launch_block(const SegList& segs, const GemvArgs& a, int ks, int ntile
     return b.tile < ntiles;
   }
   const int per = ntiles / segs.nseg;
-  int n[8], all = 0;
+  int n[8], all = 0, at = j / ks, row = 0, nb = 0, seg = 0, t0 = 0;
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
     n[s] = s < segs.nseg ? (min(*segs.s[s].mcount, a.M) + BM - 1) / BM : 0;
     all += n[s];
   }
-  const int q = j / ks, t = all ? q / all * 8 + xcd : per;
-  if (t >= per) return false;
-  int at = q % all;
-  b.mb = -1;
+  if (at >= ((per + 7) >> 3) * all) return false;
+  const bool few = all * segs.s[0].K <= (8 << 20) / BM;
+  if (few) {
+    row = at / all;
+    if (row * 8 + xcd >= per) return false;
+    at -= row * all;
+  }
 #pragma unroll
   for (int s = 0; s < 8; ++s) {
-    if (b.mb < 0 && at < n[s]) {
-      b.mb = at;
-      b.tile = s * per + t;
+    const int f = few ? xcd : (xcd - s * per) & 7, size = few ? n[s] : ((per - f + 7) >> 3) * n[s];
+    if (nb) continue;
+    if (at < size) {
+      nb = n[s];
+      seg = s;
+      t0 = f;
+    } else {
+      at -= size;
     }
-    at -= n[s];
   }
+  if (!nb) return false;
+  if (!few) row = at / nb;
+  b.mb = few ? at : at - row * nb;
+  b.tile = seg * per + t0 + 8 * row;
   return true;
 }
 inline int block_grid(const SegList& sl, int ntiles, int ks, int nmb, int slots) {

@@ -180,6 +180,36 @@ def test_grouped_blocks(gpu, mode, waves, rt, rows, bound):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K", [256, 5120])
+@pytest.mark.parametrize("mode,waves,rt,ks", [(2, 8, 4, 1), (2, 8, 2, 1), (2, 8, 2, 2), (3, 4, 6, 1), (3, 4, 6, 2), (4, 8, 2, 1), (9, 8, 2, 1)])
+def test_grouped_lists(gpu, mode, waves, rt, ks, K):
+    """Grids that number the blocks with rows: all experts' blocks for a weight tile in turn (K 256), and expert by expert (K 5120); 19 weight
+    tiles of 128 and 10 of 256, so the XCDs have unequal shares; K whole and split."""
+    rows, N, T = (0, 1, 257, 256, 513, 96, 600, 40), 2320, 640
+    E, n, g = len(rows), sum(rows), torch.Generator().manual_seed(K)
+    ws = [ops.QWeight(Q.random_blocks(GGMLType.Q5_K, N * K, 0.05, np.random.default_rng(e)), GGMLType.Q5_K, N, K, gpu) for e in range(2)]
+    dense = [w.dense(torch.float32).double() for w in ws]
+    if mode == 4:
+        for w in ws:
+            w.expand_dense()
+    x = torch.randn(T, K, generator=g).to(ops.ACT_DTYPE).to(gpu)
+    lists, at = [torch.randperm(T, generator=g)[:c] for c in rows], np.cumsum((0,) + rows)
+    ys = torch.randperm(n, generator=g).int()
+    xr, yr = torch.zeros(E * T, dtype=torch.int32), torch.zeros(E * T, dtype=torch.int32)
+    for e, t in enumerate(lists):
+        xr[e * T:e * T + len(t)], yr[e * T:e * T + len(t)] = t.int(), ys[at[e]:at[e + 1]]
+    xr, yr, counts = xr.to(gpu), yr.to(gpu), torch.tensor(rows, dtype=torch.int32, device=gpu)
+    segs = [ops.Seg(ws[e % 2], 0, xr[e * T:], yr[e * T:], counts[e:e + 1]) for e in range(E)]
+    y = torch.full((n + 1, N), 5.0, device=gpu)
+    ops.qgemv(segs, x, y, n if ks > 1 else T, epi="f32", mode=mode, waves=waves, rt=rt, ks=ks, routed=n)
+    assert (y[n] == 5.0).all()
+    for e, t in enumerate(lists):
+        W, xd = dense[e % 2], x[t.to(gpu)].double()
+        got = y[ys[at[e]:at[e + 1]].long().to(gpu)].double()
+        assert ((got - xd @ W.t()).abs() <= (xd.abs() @ W.abs().t()) * 2.0 ** -9).all(), e      # (the bound of test_active_tiles)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("qt", [GGMLType.Q4_K, GGMLType.Q5_K, GGMLType.Q6_K, GGMLType.Q8_0])
 @pytest.mark.parametrize("rows", [(0, 1, 257, 256), (96, 513, 0)])
 def test_grouped_gate_and_down(gpu, qt, rows):
