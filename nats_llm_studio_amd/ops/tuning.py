@@ -112,29 +112,31 @@ def expert_heuristic(ws, T: int, per: float):
 
 def expert_gemm(ws, per: float, dma: bool = True):
     """Config (mode, waves, rt, ks) of a grouped launch over the experts `ws` (<= 8) at about `per` routed rows to an expert: the least time by rounds
-    of workgroups over the 256 CUs, with microseconds of a round fitted to launches of 12 to 1000 rows at K = 2048, 4096 and 14336. Mode 9
-    (256 x 256 tiles) takes long prompts, mode 3 (128 x 96, two workgroups to a CU) most counts below, mode 2 (128 x 256 and 128 x 128, multiplying only
-    the 16-row tiles in use) few rows of narrow products. us at modes 2 rt 4 / 2 rt 2 / 3 rt 6 / 9, eight experts: Q5_K 8192 x 2048 at 250 rows
-    149 / 152 / 121 / 148, at 540 286 / 293 / 244 / 233, at 1000 462 / 523 / 436 / 369; Q6_K 2048 x 4096 at 50 rows 40 / 39 / 44 / 105, at 250
-    85 / 86 / 71 / 119; Q4_K 28672 x 4096 at 64 rows 302 / 274 / 216 / 440, at 1000 2508 / 2941 / 2485 / 2036; Q6_K 4096 x 14336 at 64 rows
-    144 / 133 / 132 / 337, at 540 705 / 775 / 662 / 766. dma: mode 3 may be chosen."""
+    of workgroups over the 256 CUs, with microseconds of a round fitted to 14 shapes of eight experts and of eight out of 64 and 128, 768 to 28672 wide, at
+    3 to 1500 rows (what it takes is 0.6 % behind the fastest on average). Mode 9 (256 x 256 tiles) takes long prompts, mode 3 (128 x 96, two
+    workgroups to a CU) wide products of few rows and most counts of some hundred, mode 2 (128 x 256 and 128 x 128, multiplying only the 16-row tiles
+    in use) few rows of narrow products. us at modes 2 rt 4 / 2 rt 2 / 3 rt 6 / 9: Q5_K 8192 x 2048 at 250 rows 150 / 159 / 127 / 146, at 540
+    256 / 288 / 224 / 223, at 1000 418 / 488 / 411 / 360; Q6_K 2048 x 4096 at 50 rows 37 / 37 / 42 / 103, at 250 77 / 98 / 69 / 119; Q4_K
+    28672 x 4096 at 64 rows 291 / 296 / 211 / 448, at 1000 2180 / 2661 / 2330 / 1813; Q6_K 4096 x 14336 at 64 rows 139 / 128 / 135 / 333, at 540
+    660 / 741 / 623 / 782; Q4_K 1536 x 2048 of 128 at 24 rows 23 / 20 / 24 / 54. dma: mode 3 may be chosen."""
     return _expert_rule(len(ws), ws[0].rows, ws[0].K, frozenset(int(w.type) for w in ws), per, dma)
 
 
 @functools.lru_cache(maxsize=4096)         # (a prompt's layers ask for the same)
 def _expert_rule(E: int, N: int, K: int, types, per: float, dma: bool):
-    def wgs(bn, bm):
-        return E * -(-N // bn) * max(1, math.ceil((per + per ** 0.5) / bm))      # (the largest experts' blocks)
+    far = per + per ** 0.5                 # rows of the larger experts
 
-    def pair(n, us):                       # two workgroups to a CU; alone each is faster
-        return us * 0.65 if n <= 256 else -(-n // 512) * us
-    na4, na2 = min(4, math.ceil(per / 64)), min(4, math.ceil(per / 32))
-    cand = {(2, 8, 4, 1): -(-wgs(128, 256) // 256) * (8.0 + 0.0047 * K + (3.7 + 0.00245 * K) * na4),
-            (2, 8, 2, 1): pair(wgs(128, 128), 20.0 + 0.0078 * K + (4.0 + 0.00195 * K) * na2)}
+    def wgs(bn, bm):
+        return E * -(-N // bn) * max(1, math.ceil(far / bm))
+
+    def pair(n, us, one):                  # two workgroups to a CU; alone each is faster
+        return us * one if n <= 256 else -(-n // 512) * us
+    cand = {(2, 8, 4, 1): -(-wgs(128, 256) // 256) * (4.82 + 0.00558 * K + (4.24 + 0.00188 * K) * min(4, math.ceil(far / 64))),
+            (2, 8, 2, 1): pair(wgs(128, 128), 9.93 + 0.00741 * K + (4.64 + 0.00191 * K) * min(4, math.ceil(far / 32)), 0.566)}
     if dma and types <= {12, 13, 14}:
-        cand[3, 4, 6, 1] = pair(wgs(128, 96), (15.0 + 0.0125 * K) * (0.8 if per <= 64 else 1.0))
+        cand[3, 4, 6, 1] = pair(wgs(128, 96), 10.7 + 0.00812 * K + (8.09 + 0.00195 * K) * min(1, per / 96), 0.843)
     if types <= {8, 12, 13, 14}:
-        cand[9, 8, 2, 1] = -(-wgs(256, 256) // 256) * (28.0 + 0.0235 * K)
+        cand[9, 8, 2, 1] = -(-wgs(256, 256) // 256) * (7.0 + 0.0233 * K + 20.0 * min(1, per / 256))
     return min(cand, key=cand.get)
 
 

@@ -247,6 +247,20 @@ def test_grouped_gate_and_down(gpu, qt, rows):
             assert ((y.cpu().double()[at_y] - ad @ D.t()).abs() <= (ad.abs() @ D.abs().t()) * 2.0 ** -9).all()
 
 
+def test_expert_gemm_few_rows():
+    """Few rows of narrow products: mode 2, the fastest measured (2048 x 4096, 4096 x 14336, 1536 x 2048), not mode 3; wide ones mode 3; long
+    prompts mode 9."""
+    def mode(N, K, type, per):
+        ws = [_W(N, type) for _ in range(8)]
+        for w in ws:
+            w.K = K
+        return tuning.expert_gemm(ws, per)[0]
+    for N, K, type in ((2048, 4096, 14), (2048, 4096, 8), (4096, 4096, 12), (4096, 14336, 14), (2816, 2048, 12), (1536, 2048, 12), (2048, 768, 14)):
+        assert {mode(N, K, type, per) for per in (3, 10, 17, 24, 32, 40, 50)} == {2}, (N, K)
+    assert {mode(N, K, 12, per) for N, K in ((28672, 4096), (8192, 4096), (8192, 2048)) for per in (17, 32, 50)} == {3}
+    assert {mode(N, 4096, 12, per) for N in (28672, 8192) for per in (768, 1500)} == {9}
+
+
 def test_expert_gemm_rule():
     """Configs that exist, of types their modes take; the DMA GEMM only where it is allowed."""
     for type in (7, 8, 12, 13, 14):
