@@ -156,10 +156,18 @@ def dense_key(segs, M: int) -> str:
     return f"d:{sum(s.w.rows for s in segs)}:{segs[0].w.K}:{_mb(M)}"
 
 
-# Microseconds of a round of 256 workgroups at K = 4096, by (mode, rt, activation rows of a tile); 5 of them do not grow with
-# K. Mode 10's launcher takes 192 or 256 rows, or with 128 weight rows 320, whichever fills its rounds best. (Llama-3-8B shapes at M = 256 .. 4096, e.g.
-# gate|up at 384 rows 76 us, at 3000 585, Q|K|V at 3000 168, o at 1500 56, down at 4096 375.)
-_ROUND_US = {(10, 1, 256): 106.0, (10, 1, 192): 82.0, (10, 2, 256): 72.0, (10, 2, 192): 48.0, (10, 2, 320): 76.0, (4, 2, 128): 44.0}
+# Microseconds of a round of workgroups, one to a CU: fixed (prologue, stores), and for 4096 of K, by (mode, rt, activation rows of a block). Fitted to
+# 11700 launches of 33 shapes, 2048 to 152064 rows, K 2048 to 28672, at 70 to 4096 rows (each within 5 % on average).
+_ROUND_US = {(10, 1, 256): (11.5, 101.5), (10, 1, 192): (8.5, 80.0), (10, 2, 256): (7.0, 60.0), (10, 2, 192): (6.0, 48.0), (10, 2, 320): (7.5, 71.5),
+             (4, 2, 128): (4.5, 40.0)}
+
+
+def _rows10(rt: int, tiles: int, M: int, ks: int) -> int:
+    """Rows of mode 10's blocks: the launcher's choice (launch_dense10 of hgemm10.hip)."""
+    def rounds(bm):
+        return -(-tiles * -(-M // bm) * ks // 256) * bm
+    low = 192 if rounds(192) * 100 < rounds(256) * (85 if rt == 1 else 100) else 256
+    return 320 if rt == 2 and rounds(320) * 100 < rounds(low) * 97 else low
 
 
 def dense_heuristic(segs, M: int, aligned: bool = True):
@@ -177,10 +185,17 @@ def _dense_rule(rows, K: int, M: int, aligned: bool):
 
     def us(mode, rt, ks):
         bn = 256 if (mode, rt) == (10, 1) else 128
-        tiles = sum((n + bn - 1) // bn for n in rows) * ks
-        best = min(-(-tiles * -(-M // bm) // 256) * (5.0 + (t - 5.0) * K / ks / 4096)
-                   for (md, r, bm), t in _ROUND_US.items() if (md, r) == (mode, rt))
-        return best + (2.0 + 2e-6 * ks * M * sum(rows) if ks > 1 else 0.0)
+        tiles = sum((n + bn - 1) // bn for n in rows)
+        bm = _rows10(rt, tiles, M, ks) if mode == 10 else 128
+        fixed, per = _ROUND_US[mode, rt, bm]
+        # one XCD's workgroups (it has every eighth weight tile) in rounds of its 32 CUs; a round that is not full takes 0.78 of its time at least
+        full, part = divmod(-(-tiles // 8) * -(-M // bm) * ks, 32)
+        n = full + (0.78 + 0.22 * part / 32 if part else 0)
+        t = n * (fixed + per * K / ks / 4096)
+        if bm == 320 and n > 4:
+            t *= 1.05                     # (12288 x 4096 at 3200 rows 355 us, 313 on 256 x 256; 28672 x 4096 at 2880 7 % behind)
+        slabs = ks * M * sum(rows)        # (f32 values; from 64 MB on they leave the caches)
+        return t + ((7.0 if ks > 6 and M > 192 else 3.0) + 1.2e-6 * slabs + 4e-6 * max(0, slabs - (16 << 20)) if ks > 1 else 0.0)
     mode, rt, ks = min(((mode, rt, ks) for mode, rt in ([(10, 1), (10, 2)] if aligned else []) + [(4, 2)] for ks in range(1, 9)
                         if ks == 1 or nkt // ks >= 8), key=lambda c: us(*c))
     return (mode, 8 if mode == 10 or M < 128 else 16, rt, ks)
@@ -191,10 +206,15 @@ def select_dense(segs, M: int):
     hit = table().get(dense_key(segs, M))
     if hit is not None and hit[0] < 0:
         return None
-    # (257 .. 320 and 513 .. 640 rows fill blocks of 320, which the entries, measured at 512 and 1024 rows, do not take: Llama-3-8B gate|up at 320
-    # rows 97 -> 91 us, o 28 -> 26; at 640 gate|up 172 -> 162, down 94 -> 86, Q|K|V 50 -> 44)
-    if (M > MBUCKETS[-1] or 256 < M <= 320 or 512 < M <= 640) and dense_key(segs, M) not in _FORCED:
-        return dense_heuristic(segs, M)
+    # (the entries of 257 .. 320 and 513 .. 640 rows were measured at 512 and 1024, where other splits and blocks fill the rounds. us, entry / rule:
+    # 28672 x 4096 at 320 rows, in blocks of 320, 89 / 81; 4096 x 4096 28.5 / 26.7 and 8192 x 8192 67 / 63, in four parts of K on blocks of 192;
+    # 6144 x 4096 at 640 on mode 4 53 / 46, 10240 x 8192 149 / 120, 3584 x 3584 35 either way. 57344 x 8192 at 320 rows has an entry of its own: two
+    # rounds of 320-row blocks there take 310 to 400, as the card holds its clock, 192 x 256 340 to 350)
+    if dense_key(segs, M) not in _FORCED:
+        if 256 < M <= 320 or 512 < M <= 640:
+            hit = table().get(f"d:{sum(s.w.rows for s in segs)}:{segs[0].w.K}:{320 if M <= 320 else 640}")
+        elif M > MBUCKETS[-1]:
+            hit = None
     return hit if hit is not None else dense_heuristic(segs, M)
 
 

@@ -67,6 +67,23 @@ def test_expert_rule():
     assert tuning.expert_heuristic([_W(2048)] * 4 + [_W(2048, 99)] * 4, 32, 8) is None
 
 
+def test_dense_rule_counts_an_xcds_rounds():
+    """28 weight tiles give four XCDs a tile more than the others: three parts of K, or nine blocks of rows, are two rounds there. us of what the
+    rule took when it counted the whole chip's workgroups and of what it must take: 3584 x 3584 at 300 rows 31 / 23, at 513 35 / 31, at 2880
+    114 / 76; 3584 x 18944 at 513 118 / 100, at 2880 557 / 345; 20480 x 8192 at 1920 631 / 575; 12288 x 4096 at 3200 358 / 313; 57344 x 8192 at
+    320 391 / 347 (an entry)."""
+    def pick(rows, K, M):
+        w = _W(rows)
+        w.K = K
+        return tuning.select_dense([ops.Seg(w)], M)
+    for rows, K, M, slow in ((3584, 3584, 300, (4, 16, 2, 3)), (3584, 3584, 513, (10, 8, 2, 3)), (3584, 3584, 2880, (10, 8, 2, 1)),
+                             (3584, 18944, 513, (10, 8, 2, 3)), (3584, 18944, 2880, (10, 8, 2, 1)), (20480, 8192, 1920, (10, 8, 2, 1)),
+                             (12288, 4096, 3200, (10, 8, 2, 1)), (57344, 8192, 320, (10, 8, 2, 1))):
+        assert pick(rows, K, M) != slow, (rows, K, M)
+    # blocks of 320 rows where they are the shorter walk
+    assert pick(28672, 4096, 300) == pick(28672, 4096, 640) == pick(128256, 4096, 320) == (10, 8, 2, 1)
+
+
 def test_environment_entries_stay(monkeypatch):
     """A launch config given in the environment is what runs: not split for a head's arg-max, and also above the tuned row counts."""
     class W(_W):
