@@ -35,14 +35,20 @@ struct LG {
   static_assert(LDS <= 160 * 1024, "LDS");
 };
 
-template <typename T, int BN, int BM, int WN, int WM, int NST>
+// How a launch's weights are fetched: without the hint, with it, or as each tile asks (LinTile::once). Kernels of their own: one with both walks is
+// twice the code, which a step's launches feel. Steps of four layers at 64 / 96 / 128 rows, us, both walks in a kernel / one: 148 MB of weights
+// 180 / 181, 198 / 190, 207 / 194, 221 MB 210 / 205, 201 / 196, 209 / 202, 529 MB 236 / 234, 308 / 288, 321 / 298; without the hint 184, 189, 193;
+// 198, 195, 202; 255, 306, 323.
+enum Fetch : int { KEEP, STREAM, BY_TILE };
+
+template <typename T, int BN, int BM, int WN, int WM, int NST, int FETCH>
 __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int ntot) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lglds[];
   typedef LG<BN, BM, WN, WM, NST> G;
   typedef LT<T> L;
   constexpr int NW = G::NW, NX = G::NX, NTW = G::NTW, MTW = G::MTW;
-  int listed, gap;
-  lin_listed(a, BN, listed, gap);
+  int listed = ntot, gap = 0;
+  if constexpr (FETCH == BY_TILE) lin_listed(a, BN, listed, gap);      // (a routed segment is fetched by tile)
   ntot -= gap;
   const int per = (ntot + 7) >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || id >= ntot) return;
@@ -131,8 +137,12 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
     for (int s = 0; s < NST - 1; ++s)
       if (j0 + s < nst) turn(j0 + s, s, once);        // (uniform)
   };
-  if (__builtin_amdgcn_readfirstlane(t.once)) walk(std::true_type{});
-  else walk(std::false_type{});
+  if constexpr (FETCH == BY_TILE) {
+    if (__builtin_amdgcn_readfirstlane(t.once)) walk(std::true_type{});
+    else walk(std::false_type{});
+  } else {
+    walk(std::integral_constant<bool, FETCH == STREAM>{});
+  }
   wait_vm_lgkm0<0>();                                 // the clamped tail DMAs land before the workgroup's LDS is freed
 #pragma unroll
   for (int j = 0; j < MTW; ++j) {
@@ -145,21 +155,32 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   }
 }
 
-template <typename T, int BN, int BM, int WN, int WM, int NST>
-int gemm_t(LinArgs& a, hipStream_t st) {
+template <typename T, int BN, int BM, int WN, int WM, int NST, int FETCH>
+int gemm_f(const LinArgs& a, int n, hipStream_t st) {
   typedef LG<BN, BM, WN, WM, NST> G;
-  const int n = lin_count(a, BN, BM);
-  if (n < 1) return -1;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute((const void*)lin_gemm_kernel<T, BN, BM, WN, WM, NST>,
+    if (hipFuncSetAttribute((const void*)lin_gemm_kernel<T, BN, BM, WN, WM, NST, FETCH>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((lin_gemm_kernel<T, BN, BM, WN, WM, NST>), dim3((n + 7) / 8 * 8), dim3(64 * G::NWV), G::LDS, st,
+  hipLaunchKernelGGL((lin_gemm_kernel<T, BN, BM, WN, WM, NST, FETCH>), dim3((n + 7) / 8 * 8), dim3(64 * G::NWV), G::LDS, st,
                      a, n);
   return (int)hipGetLastError();
+}
+
+template <typename T, int BN, int BM, int WN, int WM, int NST>
+int gemm_t(LinArgs& a, hipStream_t st) {
+  const int n = lin_count(a, BN, BM);
+  if (n < 1) return -1;
+  int once = 0, several = 0;                          // segments of one row tile, and of more
+  for (int i = 0; i < a.nseg; ++i) {
+    once |= a.s[i].rows || a.s[i].M <= BM;
+    several |= a.s[i].rows || a.s[i].M > BM;
+  }
+  if (!once) return gemm_f<T, BN, BM, WN, WM, NST, KEEP>(a, n, st);
+  return several ? gemm_f<T, BN, BM, WN, WM, NST, BY_TILE>(a, n, st) : gemm_f<T, BN, BM, WN, WM, NST, STREAM>(a, n, st);
 }
 
 template <typename T>

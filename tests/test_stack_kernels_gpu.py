@@ -419,3 +419,22 @@ def test_experts_of_one_and_of_several_tiles(K, T, E):
     assert T == 24 or (rows.max() > 64 and rows.min() <= 64)
     want = torch.stack([w[e].double() @ x[i // 2].double() for i, e in enumerate(sel.tolist())])
     assert relerr(y, want) < 2e-6
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_fetch_of_one_and_of_two_row_tiles(K, f32):
+    """Launches of one row tile fetch their weights with the non-temporal hint, those of more without: rows at and past a tile's edge. Inputs are
+    exact in both types, products are summed in 32 bits."""
+    x, w = (rnd(257, 150, seed=1) * 64).round() / 64, (rnd(300, 150, seed=2) * 64).round() / 64
+    dt = torch.float32 if f32 else torch.bfloat16
+    x, w = x.to(torch.bfloat16).double(), w.to(torch.bfloat16).double()
+    xa = torch.zeros(257, K.act_ld(150), dtype=dt, device="cuda")
+    xa[:, :150] = x.to(dt)
+    p = K.PackedLinear(w, f32, "cuda")
+    for cfg, (bn, bm) in K.GEMM_TILES.items():
+        for M in (bm, bm + 1) if cfg != 7 else ():
+            y = torch.full((M + 1, 300), 7.0, device="cuda")
+            L = K.LinLaunch([K.Seg(p, xa, y)])
+            L.config = lambda M, c=cfg: (True, c)
+            L.run(M, st())
+            assert relerr(y[:M], x[:M] @ w.T) < 2e-6 and (y[M] == 7).all(), (cfg, M)
