@@ -5,16 +5,21 @@
 
 namespace nls_lin {
 
-template <typename T, int MT, int NW, int RT>
+// LISTED: the first segment is routed (apart, since the branch on it and its loads cost every other launch some 60 ns)
+template <typename T, int MT, int NW, int RT, bool LISTED>
 __global__ __launch_bounds__(64 * NW) void lin_small_kernel(LinArgs a) {
   __shared__ f32x4 red[NW][RT * MT][64];
   constexpr int U = RT * MT >= 8 ? 2 : 4;    // sub-tiles in flight per wave
   typedef LT<T> L;
   LinTile t;
-  int listed, gap;
-  lin_listed(a, 16 * RT, listed, gap);
-  const int id = blockIdx.x;
-  if (id >= a.begin[a.nseg] - gap || !lin_tile<16 * RT, 16 * MT>(a, id < listed ? id : id + gap, t)) return;
+  int id = blockIdx.x;
+  if constexpr (LISTED) {
+    int listed, gap;
+    lin_listed(a, 16 * RT, listed, gap);
+    if (id >= a.begin[a.nseg] - gap) return;
+    if (id >= listed) id += gap;
+  }
+  if (!lin_tile<16 * RT, 16 * MT>(a, id, t)) return;
   const LinSeg& S = a.s[t.seg];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -85,7 +90,8 @@ template <typename T, int MT, int NW, int RT>
 int small_t(LinArgs& a, hipStream_t st) {
   const int n = lin_count(a, 16 * RT, 16 * MT);
   if (n < 1) return -1;
-  hipLaunchKernelGGL((lin_small_kernel<T, MT, NW, RT>), dim3(n), dim3(64 * NW), 0, st, a);
+  if (a.s[0].rows) hipLaunchKernelGGL((lin_small_kernel<T, MT, NW, RT, true>), dim3(n), dim3(64 * NW), 0, st, a);
+  else hipLaunchKernelGGL((lin_small_kernel<T, MT, NW, RT, false>), dim3(n), dim3(64 * NW), 0, st, a);
   return (int)hipGetLastError();
 }
 
