@@ -44,9 +44,10 @@ using nls_dma::lds_addr;
 
 constexpr int LDS_MAX = 160 * 1024;
 
-// NWV waves x RT weight tiles over BM activation rows (256; mode 12: 64, the MoE experts' routed rows):
+constexpr int BM = 256;                                          // activation rows of a workgroup
+// NWV waves x RT weight tiles over BM activation rows:
 // activation / raw-weight DMA instructions per wave per stage / super-block (NWV*RT tile-blocks), the ring depth
-template <int T, int RT, int NWV, int BM = 256>
+template <int T, int RT, int NWV>
 struct Geo {
   static constexpr int XS = BM * 64;                             // bytes of one activation stage [BM][32] f16
   static constexpr int XI = XS / 1024 / NWV;
@@ -118,10 +119,10 @@ struct Cnt {
   static constexpr int v = (NS - 3) * XI + ((P >= 2 && P <= NS - 1) ? NW : 0);
 };
 
-template <int T, int RT, int NWV, int BM = 256>
+template <int T, int RT, int NWV>
 DEVI void q9_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, uint8_t* lds,
                   const int* xm = nullptr, const int* ym = nullptr) {
-  typedef Geo<T, RT, NWV, BM> G;
+  typedef Geo<T, RT, NWV> G;
   constexpr int NS = G::NS, NW = G::NW, TB = G::TB, XI = G::XI, XS = G::XS;
   constexpr int MT = BM / 16;
   const int lane = threadIdx.x & 63;
@@ -247,24 +248,6 @@ DEVI void q9_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
 #pragma unroll
     for (int i = 0; i < RT; ++i) wf[i] = wn[i];
   };
-  // BM 64 (one group of 4 activation tiles per stage): the stages alternate between XA and XB, each stage
-  // requesting the next one's fragments before its MFMAs, and its MFMAs carry ALL the next stage's weight
-  // dequantisation
-  auto stage64 = [&](int j, int pn, auto ODD) __attribute__((always_inline)) {
-    constexpr bool odd = decltype(ODD)::value;
-    f16x8* cur = odd ? XB : XA;
-    f16x8* nxt = odd ? XA : XB;
-    __builtin_amdgcn_s_setprio(1);
-    rdg(nxt, j + 1, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    mmv(cur, 0, [&]() __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < RT; ++i) wn[i] = frag(i, pn);
-    });
-    __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-    for (int i = 0; i < RT; ++i) wf[i] = wn[i];
-  };
 
   if (nst > 0) {
     dma_w(0);
@@ -301,10 +284,7 @@ DEVI void q9_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
 #pragma unroll
           for (int i = 0; i < RT; ++i) prep_sc<T>(raw[i], g, sc[i]);
         }
-        if constexpr (BM == 64)
-          stage64(j0 + p, (p + 1) & 7, std::integral_constant<bool, (p & 1) != 0>{});
-        else
-          stage(j0 + p, (p + 1) & 7);
+        stage(j0 + p, (p + 1) & 7);
       };
       step(std::integral_constant<int, 0>{});
       step(std::integral_constant<int, 1>{});
@@ -320,8 +300,8 @@ DEVI void q9_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();
 
-  // ---- epilogue: lane holds weight rows nb0 + 16i + 4g + e and activation row 16m + r (mapped: output row
-  // ym[16m + r]; mapped split-K slabs are indexed by the output row, one shared segment column range)
+  // ---- epilogue: lane holds weight rows nb0 + 16i + 4g + e and activation row 16m + r (mapped, unsplit only: output row
+  // ym[16m + r])
   const int g4 = 4 * g;
   const int nb0 = row0 + wave * RT * 16;
   auto yrow = [&](int mm) __attribute__((always_inline)) { return ym ? ym[mm] : mm; };
@@ -334,9 +314,7 @@ DEVI void q9_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
       for (int m = 0; m < MT; ++m) {
         const int mm = 16 * m + r;
         if (mm >= M) continue;
-        const size_t srow = ym ? (size_t)ym[mm] : (size_t)(a.m0 + mm);
-        const int scol = ym ? n : S.tile_begin_col + n;
-        *reinterpret_cast<f32x4*>(ws + ((size_t)kslice * a.mtot + srow) * a.pad + scol) = acc[i][m];
+        *reinterpret_cast<f32x4*>(ws + ((size_t)kslice * a.mtot + a.m0 + mm) * a.pad + S.tile_begin_col + n) = acc[i][m];
       }
     }
     return;
@@ -409,18 +387,17 @@ DEVI void q9_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a,
 
 // the formats of one kernel type-set (dispatcher's kset: 0 = Q4_K/Q6_K, 1 = Q5_K/Q6_K/Q8_0,
 // 3 = Q51/Q6_K/Q8_0) and the LDS they need
-template <int KSET, int RT, int NWV, int BM>
+template <int KSET, int RT, int NWV>
 constexpr int kset_lds() {
-  return KSET == 0 ? (Geo<QT_Q4_K, RT, NWV, BM>::LDS > Geo<QT_Q6_K, RT, NWV, BM>::LDS ? Geo<QT_Q4_K, RT, NWV, BM>::LDS
-                                                                                      : Geo<QT_Q6_K, RT, NWV, BM>::LDS)
-                   : LDS_MAX;
+  constexpr int a = Geo<QT_Q4_K, RT, NWV>::LDS, b = Geo<QT_Q6_K, RT, NWV>::LDS;
+  return KSET == 0 ? (a > b ? a : b) : LDS_MAX;
 }
 
 // NWV = 8: two waves per SIMD (256 registers); NWV = 4: one wave per SIMD with up to 512 registers, so a
 // wave holds 4 weight tiles x 16 activation tiles of accumulators (half the LDS reads per MFMA).
 // MAP (experts): each one's routed rows are gathered through xmap and scattered through ymap; a build of its own, the plain one keeps its
 // registers.
-template <int KSET, int RT, int NWV, int BM, bool MAP>
+template <int KSET, int RT, int NWV, bool MAP>
 __global__ __launch_bounds__(64 * NWV, 1) void qgemm9_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles,
                                                           int nmb, int slots) {
   extern __shared__ __attribute__((aligned(16))) uint8_t q9lds[];
@@ -443,57 +420,52 @@ __global__ __launch_bounds__(64 * NWV, 1) void qgemm9_kernel(SegList segs, GemvA
   a.M = min(BM, mrows - m0);
   const int row0 = (tile - S.tile_begin) * 16 * RT * NWV;
   if constexpr (KSET == 0) {
-    if (S.type == QT_Q4_K) q9_tile<QT_Q4_K, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
-    else q9_tile<QT_Q6_K, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    if (S.type == QT_Q4_K) q9_tile<QT_Q4_K, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    else q9_tile<QT_Q6_K, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
   } else if constexpr (KSET == 1) {
-    if (S.type == QT_Q5_K) q9_tile<QT_Q5_K, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
-    else if (S.type == QT_Q8_0) q9_tile<QT_Q8_0, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
-    else q9_tile<QT_Q6_K, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    if (S.type == QT_Q5_K) q9_tile<QT_Q5_K, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    else if (S.type == QT_Q8_0) q9_tile<QT_Q8_0, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    else q9_tile<QT_Q6_K, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
   } else {
-    if (S.type == QT_Q51) q9_tile<QT_Q51, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
-    else if (S.type == QT_Q8_0) q9_tile<QT_Q8_0, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
-    else q9_tile<QT_Q6_K, RT, NWV, BM>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    if (S.type == QT_Q51) q9_tile<QT_Q51, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    else if (S.type == QT_Q8_0) q9_tile<QT_Q8_0, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
+    else q9_tile<QT_Q6_K, RT, NWV>(S, row0, kslice, ks, a, ws, q9lds, xm, ym);
   }
 }
 
-template <int KSET, int RT, int NWV, int BM, bool MAP>
+template <int KSET, int RT, int NWV, bool MAP>
 int launch_t(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
-  constexpr int lds = kset_lds<KSET, RT, NWV, BM>();
+  constexpr int lds = kset_lds<KSET, RT, NWV>();
   const int nmb = (a.M + BM - 1) / BM;
   const int slots = MAP ? grouped_slots(sl, a, ntiles, BM) : 0, grid = block_grid(sl, ntiles, ks, nmb, slots);
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
-    if (hipFuncSetAttribute((const void*)qgemm9_kernel<KSET, RT, NWV, BM, MAP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (hipFuncSetAttribute((const void*)qgemm9_kernel<KSET, RT, NWV, MAP>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             lds) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((qgemm9_kernel<KSET, RT, NWV, BM, MAP>), dim3(grid), dim3(64 * NWV), lds, st, sl, a, ks, ws, ntiles,
+  hipLaunchKernelGGL((qgemm9_kernel<KSET, RT, NWV, MAP>), dim3(grid), dim3(64 * NWV), lds, st, sl, a, ks, ws, ntiles,
                      nmb, slots);
   return (int)hipGetLastError();
 }
 
 template <int KSET>
-int launch_k(int waves, int rt, int bm, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a,
-             hipStream_t st) {
-  // bm 64 (the round-5 "mode 12" MoE variant, 2.6-3.1x slower than mode 2 on Mixtral's experts) is no longer
-  // instantiated: the template keeps the geometry, the default build does not carry the code
-  if (bm != 256) return -1;
+int launch_k(int waves, int rt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
   if (sl.s[0].xmap || sl.s[0].ymap || sl.s[0].mcount)
-    return waves == 8 && rt == 2 ? launch_t<KSET, 2, 8, 256, true>(sl, ntiles, ks, ws, a, st) : -1;
-  if (waves == 4 && rt == 2) return launch_t<KSET, 2, 4, 256, false>(sl, ntiles, ks, ws, a, st);
-  if (waves == 8 && rt == 2) return launch_t<KSET, 2, 8, 256, false>(sl, ntiles, ks, ws, a, st);
-  if (waves == 8 && rt == 1) return launch_t<KSET, 1, 8, 256, false>(sl, ntiles, ks, ws, a, st);
+    return waves == 8 && rt == 2 ? launch_t<KSET, 2, 8, true>(sl, ntiles, ks, ws, a, st) : -1;
+  if (waves == 4 && rt == 2) return launch_t<KSET, 2, 4, false>(sl, ntiles, ks, ws, a, st);
+  if (waves == 8 && rt == 2) return launch_t<KSET, 2, 8, false>(sl, ntiles, ks, ws, a, st);
+  if (waves == 8 && rt == 1) return launch_t<KSET, 1, 8, false>(sl, ntiles, ks, ws, a, st);
   return -1;
 }
 
 // waves x rt weight tiles of 16 rows per workgroup: (4, 2) | (8, 2) | (8, 1) (4 x 4 spills: 256 accumulators
 // plus the pipelined fragments exceed 512 registers) over 256 activation rows; kset as the dispatcher's
-int launch_q9(int kset, int waves, int rt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a,
-              hipStream_t st, int bm) {
-  if (kset == 0) return launch_k<0>(waves, rt, bm, sl, ntiles, ks, ws, a, st);
-  if (kset == 1) return launch_k<1>(waves, rt, bm, sl, ntiles, ks, ws, a, st);
-  if (kset == 3) return launch_k<3>(waves, rt, bm, sl, ntiles, ks, ws, a, st);
+int launch_q9(int kset, int waves, int rt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
+  if (kset == 0) return launch_k<0>(waves, rt, sl, ntiles, ks, ws, a, st);
+  if (kset == 1) return launch_k<1>(waves, rt, sl, ntiles, ks, ws, a, st);
+  if (kset == 3) return launch_k<3>(waves, rt, sl, ntiles, ks, ws, a, st);
   return -1;
 }
 
