@@ -862,7 +862,8 @@ def _prompt_waves(att, spans):
     workgroups share a CU. Where there are few of them, or the longest walk over keys (in tiles of 64) outlasts the others, two groups of
     waves share a workgroup's keys; eight waves, which read keys and values half as often, where long walks fill the chip. us, four waves / two
     groups / eight waves: 32 heads on 8, 2000 tokens 71 / 65 / 79, 1000 34 / 30 / 40, 3500 154 / 173 / 140, 6 x 650 50 / 69 / 61, 64 x 60
-    36 / 69 / 73; 16 on 4, 2000 tokens 60 / 49 / 73, 3500 110 / 84 / 124; expanded, 16 heads 128 + 64 wide, 3500 125 / 96 / 129."""
+    36 / 69 / 73; 16 on 4, 2000 tokens 60 / 49 / 73, 3500 110 / 84 / 124; expanded, 16 heads 128 + 64 wide, 3500 125 / 96 / 129, 32 heads, 128 x 19,
+    some behind up to 2000, 90 / 160 / 149."""
     H = max(q.cfg.heads for q in att)
     if any(getattr(q, "talk", None) is not None for q in att):
         return (8 if H * sum(-(-s[1] // 256) for s in spans) >= 256 else 4), 1
@@ -870,7 +871,8 @@ def _prompt_waves(att, spans):
     seen = max(windows) + 128 if all(windows) else 1 << 30                                    # keys that a block of 128 rows sees
     walks = [-(-min(s[3] + min(o + 128, s[1]), seen) // 64) for s in spans for o in range(0, s[1], 128)]
     most, mean = max(walks), H * sum(walks) / 512                                              # (512 workgroups at a time)
-    if most >= 6 and (H * len(walks) <= 256 or (most >= 24 and most >= 1.5 * mean)):
+    halves = H * sum(-(-w // 2) + 1 for w in walks) / 256                                      # (256 at a time, and the sums to add)
+    if most >= 6 and (H * len(walks) <= 256 or (most >= 24 and most >= 1.5 * mean and halves <= 0.8 * most)):
         return 4, 2
     return (8 if most >= 48 and mean >= 0.6 * most else 4), 1
 

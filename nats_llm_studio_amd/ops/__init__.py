@@ -849,14 +849,19 @@ def prefill_form(qblocks, units: int) -> int:
     workgroup, one to a CU; 1, 32 tokens, two to a CU; 2, 32 tokens whose keys two groups of waves share, where the longest walk (in tiles of 64
     keys) outlasts the others or there are few workgroups. us of forms 0 / 1 / 2, 32 heads of 128 on 8: one prompt of 600 tokens 27 / 22 / 20, 1000
     40 / 33 / 29, 2000 73 / 65 / 58, 3000 109 / 101 / 124, 4096 170 / 186 / 194, 1000 behind 4000 175 / 145 / 116; 6 x 650 55 / 52 / 62, 64 x 60
-    26 / 22 / 34, 300 x 20 54 / 61 / 126; 16 heads on 4, 3000 tokens 103 / 86 / 68."""
+    26 / 22 / 34, 300 x 20 54 / 61 / 126; 16 heads on 4, 3000 tokens 103 / 86 / 68; 64 heads on 16, 230 and 1000 tokens 45 / 41 / 49. Blocks of 32 tokens
+    and less leave every other workgroup of forms 1 and 2 without any: 64 heads on 16, 16 x 23, some behind up to 800, 27 / 29 / 25, 64 heads of 64 on 8,
+    128 x 24 behind up to 4000 100 / 112 / 126."""
     qb = np.asarray(qblocks)
     if not len(qb):
         return 0
     walks = -(-(qb[:, 1] + qb[:, 3]) // 64)
     most, mean, n = int(walks.max()), float(walks.sum()) * units / 256, len(qb) * units
-    if most >= 6 and (2 * n <= 256 or (most >= 16 and most >= 1.75 * mean)):
+    short = 2 * int((qb[:, 1] > 32).sum()) < len(qb)
+    if most >= 6 and (2 * n <= 256 or (most >= (16 if short else 24) and most >= 1.75 * mean and not (short and n > 1024))):
         return 2
+    if short and 2 * n > 256:
+        return 0
     return 1 if most >= 1.2 * mean or (most <= 12 and n <= 640) else 0
 
 

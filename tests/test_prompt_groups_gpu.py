@@ -151,6 +151,21 @@ def test_gguf_choice(units, runs, want):
     assert ops.prefill_form(ops.prefill_blocks(seq, pos, len(seq)), units) == want
 
 
+@pytest.mark.parametrize("units,runs,want", [
+    (16, [(0, 229), (0, 1006)], 1), (16, [(p, 24) for p in [0] * 96 + [30, 80, 200, 500] * 7 + [3973] * 4], 0), (16, [(795, 23)] + [(0, 23)] * 15, 0), (2, [(4781, 18)] * 8 + [(0, 18)] * 56, 2)])
+def test_gguf_choice_of_unlike_runs(units, runs, want):
+    """us of forms 0 / 1 / 2: 45 / 41 / 49 for the first, 100 / 112 / 126 for the second, 27 / 29 / 25 for one like the third."""
+    seq = np.concatenate([np.full(n, r) for r, (_, n) in enumerate(runs)])
+    pos = np.concatenate([np.arange(p, p + n) for p, n in runs])
+    assert ops.prefill_form(ops.prefill_blocks(seq, pos, len(seq)), units) == want
+
+
+def test_choice_of_many_short_runs_behind_contexts():
+    """Walks of one tile waste a second group of waves: 90 us with four waves, 160 with two groups, 149 with eight."""
+    att = [types.SimpleNamespace(cfg=types.SimpleNamespace(heads=32, window=0))]
+    assert _prompt_waves(att, [(0, 19, 0, p, 0, p + 19, 0, 0) for p in [0] * 96 + [30, 80, 200, 500] * 7 + [1971] * 4]) == (4, 1)
+
+
 @pytest.mark.gpu
 def test_grown_scratch_of_a_queued_step():
     """A scratch that a queued launch of a side stream still uses is not handed out again when a larger one takes its place."""
