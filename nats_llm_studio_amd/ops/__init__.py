@@ -855,9 +855,14 @@ def prefill_form(qblocks, units: int) -> int:
     qb = np.asarray(qblocks)
     if not len(qb):
         return 0
-    walks = -(-(qb[:, 1] + qb[:, 3]) // 64)
-    most, mean, n = int(walks.max()), float(walks.sum()) * units / 256, len(qb) * units
-    short = 2 * int((qb[:, 1] > 32).sum()) < len(qb)
+    if len(qb) <= 32:                      # (ahead of a prompt's first launch: 1 us for one block, arrays take 8)
+        rows = qb.tolist()
+        walks = [(r[1] + r[3] + 63) // 64 for r in rows]
+        most, total, long = max(walks), sum(walks), sum(r[1] > 32 for r in rows)
+    else:
+        walks = (qb[:, 1] + qb[:, 3] + 63) // 64
+        most, total, long = int(walks.max()), int(walks.sum()), int((qb[:, 1] > 32).sum())
+    mean, n, short = total * units / 256, len(qb) * units, 2 * long < len(qb)
     if most >= 6 and (2 * n <= 256 or (most >= (16 if short else 24) and most >= 1.75 * mean and not (short and n > 1024))):
         return 2
     if short and 2 * n > 256:
