@@ -220,6 +220,7 @@ class _Seq:
 
 class Engine:
     _queued = weakref.WeakSet()             # engines that have queued feed steps
+    _several = False                        # there are two of them
 
     def __init__(self, model, tokenizer=None, max_batch: int = 64, block_size: int = 16,
                  num_blocks: Optional[int] = None, max_prefill_tokens: int = 2048, use_graphs: bool = True,
@@ -313,6 +314,7 @@ class Engine:
         self._fed: Dict[object, _Seq] = {}
         self._stage: Optional[list] = None      # pinned buffers of _rows_to_host
         self._flight = None                     # stream of feed steps that nothing has waited for
+        self._flown = False                     # there have been such steps
         pin = self.dev.type == "cuda"
         # decode metadata / next-token host buffers are double-buffered (async decode: step N+1 is
         # prepared and launched while step N's copies may still be in flight)
@@ -820,12 +822,15 @@ class Engine:
 
     def _fly(self):
         self._flight = torch.cuda.current_stream(self.dev)
-        Engine._queued.add(self)
+        if not self._flown:
+            self._flown = True
+            Engine._queued.add(self)
+            Engine._several = len(Engine._queued) > 1
 
     def _other_streams(self):
         """Wait for queued feed steps that are not on the current stream, those of other engines too: the launches of all engines share the
         split-K workspace."""
-        for e in list(Engine._queued):
+        for e in list(Engine._queued) if Engine._several or not self._flown else (self,):     # (the set costs a decode step 2 us)
             st = e._flight
             if st is not None:
                 cur = torch.cuda.current_stream(st.device)
