@@ -771,17 +771,13 @@ class LlamaModel:
         zeroed = False
         if not routed:
             zeroed = self._router(lw, b.h, m["rlogits"], T, counts=counts)
-        # few tokens: path-A GEMV over each expert's gathered rows; many tokens: ONE route and the
-        # LDS-dequant GEMM (mode 2) over all experts, each m-block of an expert gathering its rows
-        # through xrows and exiting when it lies past the expert's device-side count
+        # few tokens: path-A GEMV over each expert's gathered rows; many tokens: ONE route and a tiled GEMM over
+        # all experts (tuning.expert_gemm: mode 2, 3 or 9), whose workgroups are the blocks that have rows by the
+        # experts' device-side counts, each gathering its rows through xrows
         gemm = T > _MOE_GEMM_T and self.device.type == "cuda"
         # path-A chunks of <= 32 tokens: the mapped GEMV then runs with <= 2 activation tiles, whose
         # kernels keep every fragment in registers (3-4 tiles spill: -Rpass-analysis scratch > 0)
         step = T if gemm else 32
-        # m-block = 64*rt rows. Every m-block re-dequantises the expert's weights, so the largest block
-        # wins; the GEMM multiplies only the block's real 16-row tiles (qgemm_impl.h NA), so ~64 routed
-        # rows in a 256-row block cost 64 rows of MFMA (Mixtral B=256, round-2 sweep: gate/up
-        # rt 4 / down rt 4 = 19.6 ms/step, 4/2 = 20.7, 2/2 = 28.3, 1/1 = 43.0)
         gu = dn = {}
         if not gemm and self.device.type == "cuda" and T * k >= len(self.experts) and "NLS_MOE_GEMV" not in os.environ:
             gu, dn = self._moe_few_cfg(lw, T, T * k / E)
