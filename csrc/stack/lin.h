@@ -1,7 +1,7 @@
 // Linear layers on packed bf16 / f32 weights (gfx950): the operand layout, launch descriptors and epilogues shared
-// by the few-row kernel (lin_small.hip) and the tiled MFMA GEMM (lin_gemm.hip).
+// by the few-row kernel (lin_small.hip) and the tiled MFMA GEMMs (lin_gemm.hip, lin_phased.hip; f32 lin_split.hip).
 //
-//   y[m, n] = epi(sum_k x[m, k] * W[n, k])        x, W: bf16 (f32 accumulate) or f32 (f32 MFMA throughout)
+//   y[m, n] = epi(sum_k x[m, k] * W[n, k])        x, W: bf16 (f32 accumulate) or f32 (few rows: f32 MFMA; GEMM: lin_split.hip)
 //
 // Packed weights: [N / 16 tiles][K / KS sub-tiles] of 1 KiB. A sub-tile is 16 rows x 64 bytes (KS = 32 bf16 or 16
 // f32 values) in MFMA fragment order: lane 16 g + r owns bytes 16 (16 g + r) .. +16 = row r, k = EL g .. EL g + EL - 1

@@ -1,6 +1,6 @@
-// Tiled MFMA GEMM on packed bf16 / f32 weights (prompt chunks, large decode batches, routed experts with many rows).
+// Tiled MFMA GEMM on packed bf16 weights (prompt chunks, large decode batches, routed experts with many rows).
 //
-// BN weight rows x BM activation rows per workgroup; K advances two 1 KiB sub-tiles (64 bf16 / 32 f32 values) per
+// BN weight rows x BM activation rows per workgroup; K advances two 1 KiB sub-tiles (64 values) per
 // step. Both operands arrive by LDS-DMA into NST-deep rings: weight sub-tiles verbatim (already in fragment order),
 // activation sub-tiles with the 16-byte chunks of a row permuted on the DMA source (chunk ^ swz(row)), so every
 // fragment is one conflict-free ds_read_b128. One raw barrier per step with a counted vmcnt leaves the later stages
@@ -22,6 +22,7 @@ using nls_dma::lds_addr;
 using nls_dma::wait_vm_lgkm0;
 
 int lin_phased(LinArgs& a, hipStream_t st);      // lin_phased.hip
+int lin_split(LinArgs& a, int cfg, hipStream_t st);      // lin_split.hip
 
 template <int BN, int BM, int WN, int WM, int NST>
 struct LG {
@@ -41,10 +42,11 @@ struct LG {
 // 198, 195, 202; 255, 306, 323.
 enum Fetch : int { KEEP, STREAM, BY_TILE };
 
-template <typename T, int BN, int BM, int WN, int WM, int NST, int FETCH>
+template <int BN, int BM, int WN, int WM, int NST, int FETCH>
 __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int ntot) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lglds[];
   typedef LG<BN, BM, WN, WM, NST> G;
+  typedef __bf16 T;
   typedef LT<T> L;
   constexpr int NW = G::NW, NX = G::NX, NTW = G::NTW, MTW = G::MTW;
   int listed = ntot, gap = 0;
@@ -155,22 +157,22 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   }
 }
 
-template <typename T, int BN, int BM, int WN, int WM, int NST, int FETCH>
+template <int BN, int BM, int WN, int WM, int NST, int FETCH>
 int gemm_f(const LinArgs& a, int n, hipStream_t st) {
   typedef LG<BN, BM, WN, WM, NST> G;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute((const void*)lin_gemm_kernel<T, BN, BM, WN, WM, NST, FETCH>,
+    if (hipFuncSetAttribute((const void*)lin_gemm_kernel<BN, BM, WN, WM, NST, FETCH>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((lin_gemm_kernel<T, BN, BM, WN, WM, NST, FETCH>), dim3((n + 7) / 8 * 8), dim3(64 * G::NWV), G::LDS, st,
+  hipLaunchKernelGGL((lin_gemm_kernel<BN, BM, WN, WM, NST, FETCH>), dim3((n + 7) / 8 * 8), dim3(64 * G::NWV), G::LDS, st,
                      a, n);
   return (int)hipGetLastError();
 }
 
-template <typename T, int BN, int BM, int WN, int WM, int NST>
+template <int BN, int BM, int WN, int WM, int NST>
 int gemm_t(LinArgs& a, hipStream_t st) {
   const int n = lin_count(a, BN, BM);
   if (n < 1) return -1;
@@ -179,24 +181,24 @@ int gemm_t(LinArgs& a, hipStream_t st) {
     once |= a.s[i].rows || a.s[i].M <= BM;
     several |= a.s[i].rows || a.s[i].M > BM;
   }
-  if (!once) return gemm_f<T, BN, BM, WN, WM, NST, KEEP>(a, n, st);
-  return several ? gemm_f<T, BN, BM, WN, WM, NST, BY_TILE>(a, n, st) : gemm_f<T, BN, BM, WN, WM, NST, STREAM>(a, n, st);
+  if (!once) return gemm_f<BN, BM, WN, WM, NST, KEEP>(a, n, st);
+  return several ? gemm_f<BN, BM, WN, WM, NST, BY_TILE>(a, n, st) : gemm_f<BN, BM, WN, WM, NST, STREAM>(a, n, st);
 }
 
-template <typename T>
-int gemm_d(LinArgs& a, int cfg, hipStream_t st) {
+int lin_gemm(LinArgs& a, int cfg, hipStream_t st) {
   switch (cfg) {
-    case 0: return gemm_t<T, 64, 64, 2, 2, 3>(a, st);
-    case 1: return gemm_t<T, 128, 64, 4, 1, 3>(a, st);
-    case 2: return gemm_t<T, 128, 128, 2, 2, 2>(a, st);
-    case 3: return gemm_t<T, 256, 128, 4, 2, 3>(a, st);
-    case 4: return gemm_t<T, 256, 256, 4, 2, 2>(a, st);
-    case 5: return gemm_t<T, 64, 64, 2, 2, 8>(a, st);
-    case 6: return gemm_t<T, 192, 128, 4, 2, 3>(a, st);
-    case 8: return gemm_t<T, 96, 64, 2, 2, 4>(a, st);
-    case 9: return gemm_t<T, 160, 64, 2, 2, 4>(a, st);
-    case 10: return gemm_t<T, 128, 64, 2, 2, 4>(a, st);
-    case 11: return gemm_t<T, 96, 128, 2, 2, 4>(a, st);
+    case 0: return gemm_t<64, 64, 2, 2, 3>(a, st);
+    case 1: return gemm_t<128, 64, 4, 1, 3>(a, st);
+    case 2: return gemm_t<128, 128, 2, 2, 2>(a, st);
+    case 3: return gemm_t<256, 128, 4, 2, 3>(a, st);
+    case 4: return gemm_t<256, 256, 4, 2, 2>(a, st);
+    case 5: return gemm_t<64, 64, 2, 2, 8>(a, st);
+    case 6: return gemm_t<192, 128, 4, 2, 3>(a, st);
+    case 7: return lin_phased(a, st);
+    case 8: return gemm_t<96, 64, 2, 2, 4>(a, st);
+    case 9: return gemm_t<160, 64, 2, 2, 4>(a, st);
+    case 10: return gemm_t<128, 64, 2, 2, 4>(a, st);
+    case 11: return gemm_t<96, 128, 2, 2, 4>(a, st);
   }
   return -1;
 }
@@ -205,14 +207,13 @@ int gemm_d(LinArgs& a, int cfg, hipStream_t st) {
 
 extern "C" {
 
-// cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256 in two stages (either
-// type; a launch's own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
-// 6 = 192 x 128, 7 = 256 x 256 in phases (bf16), 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128
+// cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256 in two stages (a launch's
+// own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
+// 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128. f32: 0, 1 and 2; the
+// others but 7 run on the one of these with their rows, at most 128.
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
-  if (cfg == 7) return f32 ? -1 : nls_lin::lin_phased(a, (hipStream_t)stream);
-  return f32 ? nls_lin::gemm_d<float>(a, cfg, (hipStream_t)stream)
-             : nls_lin::gemm_d<__bf16>(a, cfg, (hipStream_t)stream);
+  return f32 ? nls_lin::lin_split(a, cfg, (hipStream_t)stream) : nls_lin::lin_gemm(a, cfg, (hipStream_t)stream);
 }
 
 }  // extern "C"

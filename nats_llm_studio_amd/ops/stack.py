@@ -1,7 +1,7 @@
 """Device ops of the config-driven decoder stacks: ctypes bindings of `_stack.so` (csrc/stack/*.hip, gfx950).
 
 GPU tensors only: there is no eager form of these ops, a missing library raises. Operands are bf16 (f32 accumulation,
-f32 norms / routing / softmax / recurrences) or, for 32-bit models, f32 throughout (f32 MFMA)."""
+f32 norms / routing / softmax / recurrences) or, for 32-bit models, f32 throughout (f32 MFMA, or f32 in three bf16 parts)."""
 from __future__ import annotations
 
 import ctypes
@@ -195,9 +195,12 @@ GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 4: (256, 
 # against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 297 against 269 (3).
 GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 0.47, 0.72),
              1: (512, 0.5, 0.63), 0: (1024, 0.45, 0.55)}
-# 32-bit operands: bound by the f32 MFMAs (75 to 80 % of the time in any tile), so the rounds decide (64 x 64 / 128 x 64 / 192 x 128 / 256 x 128):
-# 900 x 20096 x 2048 727 / 658 / 756 / 771 us, 300 rows 257 / 267 / 377 / 259, 1500 1059 / 987 / - / 1036, 900 x 2048 x 9728 333 / 337 / 868 / 1160.
-GEMM_RATE_F32 = {6: (0, 1.0, 1.0), 3: (0, 0.98, 0.98), 1: (0, 0.955, 0.955), 0: (0, 0.865, 0.865)}
+# 32-bit operands (lin_split.hip): microseconds of 32 input columns on a CU that runs one workgroup of a tile, more for each further one, and how
+# many run together. The measured times of 12 shapes x 7 row counts x 3 tiles x 1 to 8 splits lie 8 % around it (a launch: 8 us and the slabs' sum
+# more), the tile and splits it picks 2 % above the best. 64 x 64 / 128 x 64 / 128 x 128, us: 900 x 20096 x 2048 467 / 432 / 394 (f32 MFMAs 658),
+# 1500 x 35888 x 4096 2621 / 2223 / 2020 (3440), 130 x 4096 x 4096 112 / 142 / 211 and in four splits of the first 63; 900 x 2048 x 9728 323 / 364 / 504 and in
+# four splits of the last 206 (333).
+SPLIT_US = {0: (0.72, 0.32, 6), 1: (1.01, 0.54, 4), 2: (1.64, 0.94, 3)}
 
 # Launches of 129 to 512 rows that do not fill the chip with 256 x 128 tiles (weight rows x rows of a round by its time): 300 x 4096 x 4096 28 us
 # on 96 x 64, 34 on 64 x 64, 46 on 192 x 128; 200 x 6144 x 4096 27, 32, 49; 160 x 10240 x 4096 45, 37, 47; 400 x 6144 x 2048 27, 29, 29, 28 on 96 x 128.
@@ -242,11 +245,13 @@ class LinLaunch:
             bm = self.plan.bm(M)
             if bm == 16:
                 return False, 1, (4 if self._tiles(16, 16, M) >= 1536 else 8), 1
+            if self.f32:
+                return True, min((0, 1) if bm == 64 else (2,), key=lambda c: self.split_us(c, M))
             if bm == 64:
                 # short products are over before the deeper tiles' stages pay: 64 x 64 / chosen by rounds, us: 64 experts of 30 rows, 512 x 2048 28 / 41
                 # and 2048 x 512 35 / 48; 8 of 30, 3072 x 2048 22.5 / 25.9; 32 of 30, 4096 x 1536 86 / 94; at 3072 inputs 24.2 / 23.6, from there
                 # on 8 x 4096 x 6144 95 / 79, 8 x 6144 x 4096 79 / 77
-                return True, 0 if self.f32 or self.segs[0].w.K < 3072 else self.balanced(M)
+                return True, 0 if self.segs[0].w.K < 3072 else self.balanced(M)
             if bm == 256:
                 return True, 7
             return True, (3 if self._tiles(256, 128, M) >= 224 else 2)
@@ -268,13 +273,15 @@ class LinLaunch:
             return True, (0 if M <= 2048 else 1)
         if n64 < 96 and n16 <= 1024:
             return False, 1, 16, 1
-        if M <= 128 and not self.f32:
+        if self.f32:
+            return True, min(SPLIT_US, key=lambda c: self.split_us(c, M))
+        if M <= 128:
             if 160 <= self._tiles(96, 128, M) <= 256:        # 128 x 24576 x 4096: 52 us, 61 on 192 x 128, 65 on 64 x 64
                 return True, 11
             if n64 > 256 and self._tiles(96, 64, M) <= 256:  # 96 x 10240 x 4096: 34 us, 37 on 64 x 64, 53 on 192 x 128
                 return True, 8
-        rate = GEMM_RATE_F32 if self.f32 else GEMM_RATE
-        if self.f32 or M > 512:
+        rate = GEMM_RATE
+        if M > 512:
             cand = list(rate)
         elif self._tiles(256, 128, M) >= 120:
             cand = [3, 6, 7]
@@ -317,6 +324,12 @@ class LinLaunch:
             return (False, 2, 4, 2) if M <= 32 else (True, 5)
         return True, self.balanced(M)
 
+    def split_us(self, c: int, M: int, ks: int = 1) -> float:
+        """About the microseconds of an f32 launch on tile c in ks splits of K (without the 8 us that any takes)."""
+        one, more, together = SPLIT_US[c]
+        full, rest = divmod(-(-self._tiles(*GEMM_TILES[c], M) * ks // 256), together)
+        return max(s.w.nsub for s in self.segs) / (2 * ks) * (full * (one + more * (together - 1)) + (one + more * (rest - 1) if rest else 0))
+
     def split_config(self, M: int):
         """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the
         five of 192 x 128 that are chosen, 25.5 in two of 128 x 64; 41, 34 and 32 with the launch that adds the slabs)."""
@@ -327,7 +340,10 @@ class LinLaunch:
         if M <= 32:
             return (False, 2, 4, 4 if n16 >= 256 else 2), 8
         big, small = self._tiles(256, 128, M), self._tiles(64, 64, M)
-        if self.f32 or small > 256:
+        if self.f32:
+            c, ks = self.cheapest(M, self.segs[0].slabs)
+            return (True, c), ks
+        if small > 256:
             return ((True, 3), -(-256 // big)) if M > 128 and big * 8 >= 256 else ((True, 0), -(-512 // small))
         if M <= 64:                       # one workgroup to a CU, 8 stages in flight: 64 x 4096 x 17408 34 us in 8 splits of 64 x 64 with
             return (True, 5), 256 // small                                      # three, 31 in 4 (and half the slabs), 40 x 4096 x 9216 19, 18
@@ -340,10 +356,12 @@ class LinLaunch:
         s = self.segs[0]
 
         def us(c, ks):
+            if self.f32:
+                return self.split_us(c, M, ks) + (ks - 1) * M * s.w.N * 2e-6
             fixed, per = ROUND_US[c]
             rounds = -(-self._tiles(*GEMM_TILES[c], M) * ks // 256)
             return rounds * (fixed + per * s.w.K / ks) + (ks - 1) * M * s.w.N * 2e-6
-        return min(((c, ks) for c in ROUND_US for ks in range(1, max(1, min(most, s.w.nsub // 16)) + 1)), key=lambda v: us(*v))
+        return min(((c, ks) for c in (SPLIT_US if self.f32 else ROUND_US) for ks in range(1, max(1, min(most, s.w.nsub // 16)) + 1)), key=lambda v: us(*v))
 
     def tall_split(self, M: int):
         """(config, K splits) of more rows than slab_rows: as many slabs of M rows as y holds. A narrow product has fewer tiles than
@@ -365,7 +383,7 @@ class LinLaunch:
         if splits and M <= self._rows:
             cfg, ks = self.split_config(M)
             return cfg, max(1, min(ks, s.slabs, s.w.nsub // 16))
-        if splits and not self.f32:
+        if splits:
             return self.tall_split(M)
         return self.config(M), 1
 
