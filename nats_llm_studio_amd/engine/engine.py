@@ -15,6 +15,7 @@ each decode step:
 """
 from __future__ import annotations
 
+import array
 import collections
 import hashlib
 import itertools
@@ -653,13 +654,13 @@ class Engine:
                     runs[si] = (T, n, s.state_slot, p0)
                 T += n
             return T
-        # all parts at once (200 prompts of 20 tokens 1.6 -> 0.3 ms, nothing runs on the device meanwhile; six of 650 take 0.2 either way, a single
-        # one 15 us longer)
+        # all parts at once (200 prompts of 20 tokens 1.6 -> 0.3 ms, nothing runs on the device meanwhile; a single one takes 15 us longer so)
         count = np.fromiter((len(p[2]) for p in parts), np.int64, len(parts))
         first = np.fromiter((p[1] for p in parts), np.int64, len(parts))
         start = np.cumsum(count) - count
         T = int(count.sum())
-        ids[:T] = np.fromiter(itertools.chain.from_iterable(p[2] for p in parts), np.int64, T)
+        ids[:T] = (np.concatenate([p[2] for p in parts]) if isinstance(parts[0][2], np.ndarray) else
+                   np.fromiter(itertools.chain.from_iterable(p[2] for p in parts), np.int64, T))
         seq = np.repeat(np.arange(len(parts)), count)
         pr = np.arange(T) + (first - start)[seq]
         for si, (s, _, _) in enumerate(parts):
@@ -728,7 +729,8 @@ class Engine:
             raise ValueError("feed: one entry per request and step")
         self._other_streams()
         # (a decode step of a few hundred requests waits for this loop: a token at a time is checked without an array)
-        V, bs, single, seqs = self.cfg.vocab, self.bs, True, []
+        V, bs, single, seqs, ids = self.cfg.vocab, self.bs, True, [], []
+        tables = None
         for rid, toks, want in entries:
             s = self._fed.get(rid)
             if s is None:
@@ -741,7 +743,13 @@ class Engine:
             m = len(toks)
             if not m:
                 raise ValueError("feed: an entry without tokens")
-            if not (0 <= int(toks[0]) < V if m == 1 else self._inside(toks, V)):
+            if m == 1:
+                a = int(toks[0])
+                inside = 0 <= a < V
+            else:
+                a = self._token_array(toks)
+                inside = a is not None and a.view(np.uint64).max() < V
+            if not inside:
                 raise ValueError("feed: token outside the vocabulary")
             if len(want) and any(not 0 <= int(w) < m for w in want):
                 raise ValueError("feed: wanted place outside the entry")
@@ -757,26 +765,40 @@ class Engine:
                 old = len(s.blocks)
                 s.blocks += blocks
                 if s.row >= 0:             # (entries that a step under way does not read)
-                    for hm in self.h_meta_d2:
-                        self._tables(hm, self.db.pad)[0][s.row, old:len(s.blocks)] = blocks
+                    if tables is None:     # (300 requests that take their next block in one step: 0.6 ms of views)
+                        tables = [self._tables(hm, self.db.pad)[0] for hm in self.h_meta_d2]
+                    for bt in tables:
+                        bt[s.row, old:len(s.blocks)] = blocks
             seqs.append(s)
+            ids.append(a)
         wants = [len(e[2]) for e in entries]
         none = torch.empty(0, V)           # (shared: a tensor each would be a tenth of 40 steps of 300 requests)
         out = [torch.empty(w, V) if w else none for w in wants]
         if single:
-            self._feed_decode(seqs, entries, out, wants)
+            self._feed_decode(seqs, ids, out, wants)
         else:
-            self._feed_rows(seqs, entries, out)
+            self._feed_rows(seqs, ids, entries, out)
         return out
 
     @staticmethod
-    def _inside(toks, vocab: int) -> bool:
-        """Whether every token is an id of the vocabulary."""
+    def _token_array(toks) -> Optional[np.ndarray]:
+        """Tokens as an array, once: what follows (checks, staging) takes slices of it, since the device waits for a prompt's first launch (3500
+        tokens 0.36 -> 0.2 ms). None: one of them is past 64 bits."""
         try:
-            a = np.fromiter(map(int, toks), np.int64, len(toks))
+            if type(toks) is list:
+                try:
+                    return np.frombuffer(array.array("q", toks), np.int64)
+                except TypeError:          # (not all of them are whole numbers by type)
+                    pass
+            return np.fromiter(map(int, toks), np.int64, len(toks))
         except OverflowError:
-            return False
-        return bool((a >= 0).all() and (a < vocab).all())
+            return None
+
+    @staticmethod
+    def _touch(out):
+        """Write to each page of the results ahead of the copy (3 ms of 300 rows, 0.1 of six), while the device is busy."""
+        for t in out:
+            t.numpy().reshape(-1)[::1024] = 0
 
     STAGE_BYTES = 8 << 20        # of each of the two pinned buffers that logits pass on their way to the host
 
@@ -837,15 +859,15 @@ class Engine:
                 if st != cur:
                     st.synchronize()
 
-    def _feed_decode(self, seqs, entries, out, wants):
+    def _feed_decode(self, seqs, ids, out, wants):
         cuda = self.dev.type == "cuda"
         if any(s.row < 0 for s in seqs):
             if cuda:
                 for ev in self._ev:        # rows change hands in both staging buffers: no decode step may have its upload ahead
                     ev.synchronize()
             self._release_rows()           # (a generation that ended while its next step ran may still hold some)
-        for s, e in zip(seqs, entries):
-            s.tokens.append(int(e[1][0]))
+        for s, t in zip(seqs, ids):
+            s.tokens.append(t)
             if s.row < 0:
                 self._assign_row(s, sampled=False)
         need = any(wants)
@@ -856,9 +878,7 @@ class Engine:
             self._fly()
             return
         if need:
-            for t, w in zip(out, wants):   # (pages of the results, 3 ms of 300 rows, while the device is busy)
-                if w:
-                    t.numpy().reshape(-1)[::1024] = 0
+            self._touch(t for t, w in zip(out, wants) if w)
             rows = [r for (r, _), w in zip(snap, wants) for _ in range(w)]
             lg = self.db.logits
             lg = lg[rows[0]:rows[0] + len(rows)] if rows == list(range(rows[0], rows[0] + len(rows))) else lg[rows]
@@ -867,10 +887,10 @@ class Engine:
             self._flight = None            # (all of them are ahead of this one on its stream)
             self._ev[k].synchronize()
 
-    def _feed_rows(self, seqs, entries, out):
+    def _feed_rows(self, seqs, ids, entries, out):
         """Row batches of at most max_prefill rows and max_logit_rows wanted rows (one batch unless the step is larger)."""
-        work = [(i, s, [int(t) for t in e[1]], sorted((int(w), j) for j, w in enumerate(e[2])))
-                for i, (s, e) in enumerate(zip(seqs, entries))]
+        work = [(i, s, np.full(1, a) if isinstance(a, int) else a, sorted((int(w), j) for j, w in enumerate(e[2])))
+                for i, (s, a, e) in enumerate(zip(seqs, ids, entries))]
         done = [0] * len(work)
         while any(done[i] < len(toks) for i, _, toks, _ in work):
             parts, rows, dest, T = [], [], [], 0
@@ -890,7 +910,6 @@ class Engine:
                         dest[-1][2] += 1
                     else:
                         dest.append([i, j, j + 1])
-                s.tokens += toks[done[i]:done[i] + n]
                 s.n_fed += n
                 done[i] += n
                 T += n
@@ -898,9 +917,13 @@ class Engine:
             self._fill_rows(parts)
             self._exec_prefill(T, rows or [0], True, len(parts))
             self.counters["prefill_tokens"] += T
+            for s, _, toks in parts:
+                s.tokens += toks.tolist()
             if rows:
                 self._flight = None
-                self._rows_to_host(self.pb.logits[:len(rows)], [out[i][a:b] for i, a, b in dest])
+                dst = [out[i][a:b] for i, a, b in dest]
+                self._touch(dst)
+                self._rows_to_host(self.pb.logits[:len(rows)], dst)
             elif self.dev.type == "cuda":
                 self._fly()
 
