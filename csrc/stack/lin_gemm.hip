@@ -11,6 +11,9 @@
 // without the hint they push the rows, caches and states of the step out of the caches (us in a running step, without / with: 64 x 35888 x 4096
 // 75.7 / 59.7, 4.9 TB/s, 64 x 32000 68.7 / 55.5, eight experts of 50 rows 94.5 / 76.3 and 83.0 / 78.0). Weights of two row tiles need the L2 for the
 // second one's read: with the hint eight experts of 75 rows took 142 -> 163 us.
+// A CU takes in some 50 GB/s of a launch's operands whatever its waves and stages (96 workgroups read cold weights at 4.7 TB/s, 256 at 6.8), and
+// the activation rows count as much as the weights: the 64 x 32 tile brings half as many of them as 64 x 64 (16 x 10240 x 4096 18.2 / 19.2 us, 24 rows
+// 20.0 / 20.5; streamed with the rows from the caches, lin_small.hip, 23.7 and 24).
 #include <type_traits>
 #include "../kernels/lds_dma.h"
 #include "lin.h"
@@ -199,6 +202,7 @@ int lin_gemm(LinArgs& a, int cfg, hipStream_t st) {
     case 9: return gemm_t<160, 64, 2, 2, 4>(a, st);
     case 10: return gemm_t<128, 64, 2, 2, 4>(a, st);
     case 11: return gemm_t<96, 128, 2, 2, 4>(a, st);
+    case 12: return gemm_t<64, 32, 2, 1, 8>(a, st);
   }
   return -1;
 }
@@ -209,8 +213,8 @@ extern "C" {
 
 // cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256 in two stages (a launch's
 // own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
-// 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128. f32: 0, 1 and 2; the
-// others but 7 run on the one of these with their rows, at most 128.
+// 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128, 12 = 64 x 32 with 8 stages.
+// f32: 0, 1 and 2; the others but 7 run on one of these.
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
   return f32 ? nls_lin::lin_split(a, cfg, (hipStream_t)stream) : nls_lin::lin_gemm(a, cfg, (hipStream_t)stream);

@@ -186,7 +186,7 @@ class Seg:
 
 # (weight rows, rows) of lin_gemm's configs
 GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 4: (256, 256), 5: (64, 64), 6: (192, 128), 7: (256, 256),
-              8: (96, 64), 9: (160, 64), 10: (128, 64), 11: (96, 128)}
+              8: (96, 64), 9: (160, 64), 10: (128, 64), 11: (96, 128), 12: (64, 32)}
 
 
 # Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
@@ -258,6 +258,10 @@ class LinLaunch:
         n16, n64 = self._tiles(16, 16, M), self._tiles(64, 64, M)
         ns = max(s.w.nsub for s in self.segs)
         if M <= 16:
+            # 16 rows, streaming / GEMM, us: 10240 x 4096 23.7 / 18.2, 12288 x 2048 14.3 / 12.4, 17944 x 2048 18.7 / 16.4, 34816 x 4096 58.1 / 50.4, 8192 x
+            # 2048 and narrower 9 / 11; 9 rows 19.2 / 18.7, 11.4 / 12.4, 17.4 / 16.9, 52.3 / 50.2
+            if M > 12 and not self.f32 and ns >= 64 and n64 > 128:
+                return True, 12 if n64 <= 256 else self.balanced(M)
             if M > 8 and n16 >= 1024:
                 return False, 1, 4, 2
             return False, 1, (4 if ns <= 16 else 8 if n16 >= 320 or ns <= 32 else 16), 1
@@ -320,8 +324,8 @@ class LinLaunch:
             return False, 2, 8, 2
         if self._tiles(32, 64, M) <= 256:
             return False, 4, 8, 2
-        if n64 <= 256:                    # 48 x 10240 x 4096: 27 us with 8 stages in flight, 35 streaming; 20 rows: 27, 23
-            return (False, 2, 4, 2) if M <= 32 else (True, 5)
+        if n64 <= 256:                    # 48 x 10240 x 4096: 27 us with 8 stages in flight, 35 streaming; 24 rows: 20 on 64 x 32, 24
+            return (True, 5) if M > 32 else (True, 12) if self.segs[0].w.nsub >= 64 else (False, 2, 4, 2)
         return True, self.balanced(M)
 
     def split_us(self, c: int, M: int, ks: int = 1) -> float:
@@ -334,6 +338,10 @@ class LinLaunch:
         """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the
         five of 192 x 128 that are chosen, 25.5 in two of 128 x 64; 41, 34 and 32 with the launch that adds the slabs)."""
         n16 = self._tiles(16, 16, M)
+        # 64 x 32 tiles, one to a CU. 16 rows, streaming / these, us: 4096 x 17408 27.5 / 25.6, 4096 x 8192 15.3 / 14.6, 4096 x 4096 9.1 / 9.6, 2048 x 8704 9.9
+        # / 10.3; 24 rows 27.5 / 26.8, 18.1 / 15.8, 11.5 / 10.6, 12.7 / 12.0, with half the slabs at 4096 columns
+        if not self.f32 and (16 < M <= 32 or 12 < M <= 16 and n16 >= 256 and self.segs[0].w.K >= 8192):
+            return (True, 12), -(-256 // self._tiles(64, 32, M))
         if M <= 16:
             rt = 1 if M <= 8 else 2
             return (False, 1, 8, rt), -(-512 * rt // (2 * n16)) if M > 8 else -(-512 // n16)
