@@ -6,6 +6,7 @@
 // registers, PARTS neighbouring lanes cover the keys and close the sum with in-row lane exchanges (DPP). Few runs take
 // many key parts (short per-token chains on all CUs). Tokens are staged in LDS in chunks of CH as f32, the next chunk's
 // loads in flight while the current one runs.
+#include <type_traits>
 #include "scan.h"
 
 namespace nls_wkv {
@@ -246,12 +247,171 @@ __global__ __launch_bounds__(256) void wkv_scan_kernel(Scan p) {
     p.prev[(size_t)slot * p.ldp + i] = p.x[(size_t)(t0 + n - 1) * p.ldx + i];
 }
 
+// Sums of eight values over 32 lanes each: every exchange adds two of them, one for each half of the lanes (19 instructions; 8 x 5 one by one). Lane
+// 16 a + 4 x + b ends with the sum of value a + 2 b.
+DEVI float sum8_32(const float (&o)[8], int lane) {
+  float h[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, o[2 * i]), __builtin_bit_cast(uint32_t, o[2 * i + 1]), false, false);
+    h[i] = __builtin_bit_cast(float, (uint32_t)s[0]) + __builtin_bit_cast(float, (uint32_t)s[1]);
+  }
+  auto pair = [&](float a, float b, bool hi, auto dpp) __attribute__((always_inline)) {
+    const int send = __builtin_bit_cast(int, hi ? a : b);
+    return (hi ? b : a) + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, send, decltype(dpp)::value, 0xf, 0xf, true));
+  };
+  const float x = pair(h[0], h[1], lane & 1, std::integral_constant<int, 0xB1>{}), y = pair(h[2], h[3], lane & 1, std::integral_constant<int, 0xB1>{});
+  return dpp_add<0x124>(dpp_add<0x128>(pair(x, y, lane & 2, std::integral_constant<int, 0x4E>{})));
+}
+
+// The scan of few runs, up to two workgroups for each CU. A wave takes a token's time to issue and to close its sums (240 cycles of the form above,
+// however many waves share the CU), so here a column's keys lie over 32 lanes, two columns to a wave, the sums of eight tokens are closed together,
+// and the next chunk is staged in a second buffer while one is summed, with a barrier for each. 3500 tokens, 32 heads of 64: 349 -> 261 us, 64 heads
+// 373 -> 362; 2000 tokens, 16 and 32 heads of 128: 301 -> 199 and 308 -> 271; with four workgroups to a CU it would be slower (4 x 900, 32 heads of 64:
+// 121 above, 173).
+template <typename T, int DP, bool VEC>
+__global__ __launch_bounds__(256) void wkv_few_kernel(Scan p) {
+  constexpr int WC = 8, CH = 2048 / DP, R = DP / 32, LR = DP + 4, RQ = R < 4 ? 2 : 4, PF = 3, RB = PF + 1;
+  struct Chunk {
+    float r[CH][LR], k[CH][LR], w[CH][LR], v[CH][WC], ruk[CH];
+  };
+  __shared__ __attribute__((aligned(16))) Chunk ch[2];
+  typedef T tv8 __attribute__((ext_vector_type(8), aligned(16)));
+  typedef float fv8 __attribute__((ext_vector_type(8), aligned(16)));
+  typedef float fq __attribute__((ext_vector_type(RQ)));
+  const int* run = p.runs + 4 * blockIdx.y;
+  const int t0 = run[0], n = run[1], slot = run[2], pos0 = run[3];
+  if (slot < 0 || n < 1) return;
+  const int head = blockIdx.x / (DP / WC), c0 = blockIdx.x % (DP / WC) * WC;
+  const int lane = threadIdx.x & 63, part = lane & 31, col = 2 * (threadIdx.x >> 6) + (lane >> 5), j = c0 + col;
+  const size_t hb = (size_t)head * DP;
+  const T *rp = (const T*)p.r + hb, *kp = (const T*)p.k + hb, *vp = (const T*)p.v + hb;
+  const float* wp = p.w + hb;
+  float* st = p.state + (size_t)slot * p.sstride + hb * DP;
+  const int et = threadIdx.x / (DP / 8), ei = threadIdx.x % (DP / 8) * 8, vt = threadIdx.x % CH;         // a thread's token and keys, its token's values
+  float S[R], u[8];
+#pragma unroll
+  for (int i = 0; i < R; ++i) S[i] = pos0 > 0 ? st[(size_t)(part * R + i) * DP + j] : 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) u[i] = p.u[hb + ei + i];
+  // (arrived before the first chunk's loads go out, which the loop over tokens would wait for otherwise)
+#pragma unroll
+  for (int i = 0; i < R; ++i) asm volatile("" : "+v"(S[i]));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(u[i]));
+  tv8 r8, k8, v8;
+  fv8 w8;
+  auto fetch = [&](int base) __attribute__((always_inline)) {        // (rows past the run: its last one)
+    const size_t row = t0 + min(base + et, n - 1), vrow = t0 + min(base + vt, n - 1);
+    if constexpr (!VEC) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        r8[e] = rp[row * p.ld + ei + e];
+        k8[e] = kp[row * p.ld + ei + e];
+        w8[e] = wp[row * p.ldw + ei + e];
+        v8[e] = vp[vrow * p.ld + c0 + e];
+      }
+      return;
+    }
+    r8 = *reinterpret_cast<const tv8*>(rp + row * p.ld + ei);
+    k8 = *reinterpret_cast<const tv8*>(kp + row * p.ld + ei);
+    w8 = *reinterpret_cast<const fv8*>(wp + row * p.ldw + ei);
+    v8 = *reinterpret_cast<const tv8*>(vp + vrow * p.ld + c0);
+  };
+  auto stage = [&](Chunk& c) __attribute__((always_inline)) {
+    float a = 0.f;
+#pragma unroll
+    for (int h = 0; h < 8; h += 4) {
+      *reinterpret_cast<f32x4*>(&c.r[et][ei + h]) = f32x4{(float)r8[h], (float)r8[h + 1], (float)r8[h + 2], (float)r8[h + 3]};
+      *reinterpret_cast<f32x4*>(&c.k[et][ei + h]) = f32x4{(float)k8[h], (float)k8[h + 1], (float)k8[h + 2], (float)k8[h + 3]};
+      *reinterpret_cast<f32x4*>(&c.w[et][ei + h]) = f32x4{w8[h], w8[h + 1], w8[h + 2], w8[h + 3]};
+      *reinterpret_cast<f32x4*>(&c.v[vt][h]) = f32x4{(float)v8[h], (float)v8[h + 1], (float)v8[h + 2], (float)v8[h + 3]};
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a += (float)r8[e] * u[e] * (float)k8[e];
+    a = sum_parts<DP == 64 ? 8 : 16>(a);
+    if (DP == 256) a += __shfl_xor(a, 16, 64);
+    if (ei == 0) c.ruk[et] = a;
+  };
+  fetch(0);
+  stage(ch[0]);
+  fetch(CH);
+  __syncthreads();
+  int b = 0;
+  for (int base = 0; base < n; base += CH, b ^= 1) {
+    stage(ch[b ^ 1]);
+    fetch(base + 2 * CH);
+    const Chunk& c = ch[b];
+    const int m = min(CH, n - base);
+    fq r4[RB][R / RQ], k4[RB][R / RQ], w4[RB][R / RQ];
+    float v1[RB];
+    auto get = [&](int tt, int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < R / RQ; ++q) {
+        r4[s][q] = *reinterpret_cast<const fq*>(&c.r[tt][part * R + RQ * q]);
+        k4[s][q] = *reinterpret_cast<const fq*>(&c.k[tt][part * R + RQ * q]);
+        w4[s][q] = *reinterpret_cast<const fq*>(&c.w[tt][part * R + RQ * q]);
+      }
+      v1[s] = c.v[tt][col];
+    };
+    auto token = [&](int s) __attribute__((always_inline)) {
+      float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+      for (int q = 0; q < R / RQ; ++q)
+#pragma unroll
+        for (int e = 0; e < RQ; e += 2) {
+          const int i = RQ * q + e;
+          o0 = fmaf(r4[s][q][e], S[i], o0);
+          o1 = fmaf(r4[s][q][e + 1], S[i + 1], o1);
+          S[i] = fmaf(w4[s][q][e], S[i], k4[s][q][e] * v1[s]);
+          S[i + 1] = fmaf(w4[s][q][e + 1], S[i + 1], k4[s][q][e + 1] * v1[s]);
+        }
+      return o0 + o1;
+    };
+#pragma unroll
+    for (int i = 0; i < PF; ++i) get(i, i);
+    for (int t8 = 0; t8 < m; t8 += 8) {
+      float o[8];
+      const int last = m - 1 - t8;
+      if (last >= 7) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          get(min(t8 + q + PF, CH - 1), (q + PF) % RB);
+          o[q] = token(q % RB);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          get(min(t8 + q + PF, CH - 1), (q + PF) % RB);
+          o[q] = 0.f;
+          if (q <= last) o[q] = token(q % RB);           // (uniform)
+        }
+      }
+      const float sum = sum8_32(o, lane);
+      const int q = (lane >> 4 & 1) | (lane & 3) << 1, tt = t8 + q;
+      if (!(lane & 12) && q <= last) p.o[(size_t)(t0 + base + tt) * p.ldo + hb + j] = fmaf(c.ruk[tt], c.v[tt][col], sum);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < R; ++i) st[(size_t)(part * R + i) * DP + j] = S[i];
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < p.width; i += gridDim.x * 256)
+    p.prev[(size_t)slot * p.ldp + i] = p.x[(size_t)(t0 + n - 1) * p.ldx + i];
+}
+
 template <typename T, int DP, int PARTS>
 int scan_v(const Scan& p, int nruns, hipStream_t st) {
   const dim3 grid(p.H * ((p.V + 256 / PARTS - 1) / (256 / PARTS)), nruns);
   if constexpr (DP >= 64) {
     auto whole = [](const void* q, long ld, size_t size) { return (uintptr_t)q % 16 == 0 && ld * size % 16 == 0; };
-    if (p.D == DP && whole(p.r, p.ld, sizeof(T)) && whole(p.k, p.ld, sizeof(T)) && whole(p.v, p.ld, sizeof(T)) && whole(p.w, p.ldw, 4)) {
+    const bool vec = p.D == DP && whole(p.r, p.ld, sizeof(T)) && whole(p.k, p.ld, sizeof(T)) && whole(p.v, p.ld, sizeof(T)) && whole(p.w, p.ldw, 4);
+    if (PARTS == 16 && p.D == DP && p.H * nruns * (DP / 8) <= 512) {
+      const dim3 few(p.H * (DP / 8), nruns);
+      if (vec) hipLaunchKernelGGL((wkv_few_kernel<T, DP, true>), few, dim3(256), 0, st, p);
+      else hipLaunchKernelGGL((wkv_few_kernel<T, DP, false>), few, dim3(256), 0, st, p);
+      return (int)hipGetLastError();
+    }
+    if (vec) {
       hipLaunchKernelGGL((wkv_scan_kernel<T, DP, PARTS, 1, true>), grid, dim3(256), 0, st, p);
       return (int)hipGetLastError();
     }
