@@ -507,7 +507,7 @@ class GlaPart(_SharedPart):
                        e["g"], e["out"], H, D, V, eps, st)
             return
         n = step.nruns
-        shape = K.gla_shape(T, n, H, V)
+        shape = K.gla_shape(T, n, H, V, D, step.longest)
         seg = None
         if shape[0] > 1:
             seg = (self.m.grown(b, "gla.seg", n * shape[0], H * D * V, torch.float32),
@@ -559,7 +559,7 @@ class LightningPart(_SharedPart):
         if T == n and V % 4 == 0 and V <= 1024:
             K.gla_step(e["q"], e["k"], e["v"], self.a, None, 1.0, S, b.runs, T, None, None, None, H, D, V, eps, st, o=e["o"])
         else:
-            shape = K.gla_shape(T, n, H, V)
+            shape = K.gla_shape(T, n, H, V, D, step.longest)
             seg = None
             if shape[0] > 1:
                 seg = (self.m.grown(b, "gla.seg", n * shape[0], H * D * V, torch.float32),
@@ -638,7 +638,7 @@ class DeltaPart(_SharedPart):
             K.delta_step(*qkv, None if own else e["a"], (e["low"], self.a2r, self.dt, self.rate), None if own else e["g"],
                          (e["lowg"], self.g2r), self.ld, S, b.runs, T, self.norm, e["out"], H, G, D, V, eps, st)
             return
-        shape = K.delta_shape(T, n, H, D, V)
+        shape = K.delta_shape(T, n, H, D, V, step.longest)
         seg = None
         if shape[0] > 1:
             seg = (self.m.grown(b, "delta.seg", n * shape[0], H * D * V, torch.float32),
@@ -900,6 +900,7 @@ class _Step:
     plan: Optional[_ExpandPlan] = None
     layer: int = 0              # the layer run: its cache and state (its parts may be another run's)
     keys: Optional[torch.Tensor] = None      # keys of each row (None: no row is padding)
+    longest: Optional[int] = None            # rows of the longest run, if known
 
 
 # runs of at least this many rows expand (below, the latent-space attention's extra products cost less than the expansion
@@ -1128,14 +1129,14 @@ class StackModel:
     def forward(self, b: StackBuffers, kc, vc, T: int, block_size: int, n_split: int = 1,
                 logit_rows: Optional[torch.Tensor] = None, n_logits: Optional[int] = None, qblocks=None, nqb: int = 0,
                 feed_prev: bool = False, need_logits: bool = True, state=None, nruns: Optional[int] = None,
-                row_info: Optional[dict] = None, taps: Optional[list] = None):
+                row_info: Optional[dict] = None, taps: Optional[list] = None, longest: Optional[int] = None):
         """One step of T rows: logits (of `logit_rows`, or of every row) in b.logits[:n], their greedy ids in
-        b.next_ids[:n]. `taps` (a list) receives the residual after every layer."""
+        b.next_ids[:n]. `taps` (a list) receives the residual after every layer. nruns, longest: runs of rows, rows of the longest."""
         if T < 1 or T > b.pad:
             raise ValueError(f"step of {T} rows, buffers hold {b.pad}")
         cfg = self.cfg
         st = K.stream(self.device)
-        step = _Step(T, T if nruns is None else nruns, block_size, st, keys=b.ctx_len)
+        step = _Step(T, T if nruns is None else nruns, block_size, st, keys=b.ctx_len, longest=longest)
         if row_info is not None and qblocks is not None:
             step.plan = self._expand_plan(b, qblocks, row_info, T, block_size, st)
         rms, groups = cfg.design.norm == "rms", cfg.norm_groups

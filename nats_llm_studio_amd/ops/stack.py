@@ -6,6 +6,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+from functools import lru_cache
 from typing import List, Optional
 
 import torch
@@ -622,12 +623,44 @@ def scan_out(o, norm, gate, out, H: int, D: int, T: int, eps: float, st: int):
                               out.stride(0), H, D, T, eps, int(out.dtype == torch.float32), st), "nls_scan_out")
 
 
-def gla_shape(T: int, nruns: int, H: int, V: int):
-    """(segments, groups of 64 value columns per workgroup) of a gla_scan launch: two workgroups per CU from segments of at
-    least 64 tokens, unless whole runs already give one."""
+# A chunked recurrence over 65 to 128 channels and more than 64 value columns, in microseconds: a workgroup has a CU to itself, so
+# what counts is whole rounds of 256 of them, each as long as a segment. (launches, a token of the last pass, a token of the pass
+# that finds what the segments end with, what segments add, the chain of their states: per segment in all, per segment of a run,
+# workgroups of that pass per one of the last.) Fitted to 400 launches of 1 to 64 runs of 60 to 3500 tokens, 16 and 32 heads of
+# 128 x 128, 1 to 16 segments: the count it picks is 0.6 % (gla) and 0.2 % (delta) behind the fastest on average.
+SEGMENT_US = {"gla": (32.4, 0.3424, 0.1862, -10.0, 0.05, 0.0, 1), "delta": (52.5, 0.59, 0.35, -36.0, 0.2215, 9.0, 2)}
+
+
+def segments_us(kind: str, tokens: int, wgs: float, nseg: int) -> float:
+    """What a scan takes with nseg segments of its longest run (tokens); wgs: workgroups of that length, segments aside."""
+    a, tok, tok_local, b, chain, link, lanes = SEGMENT_US[kind]
+    size = -(-tokens // nseg) + 63 & ~63               # (segments are whole chunks of 64 tokens, the last one what is left)
+    m = -(-tokens // size)
+    size = min(size, tokens)
+    us = a + -(-wgs * m // 256) * size * tok
+    return us + (b + -(-wgs * lanes * (m - 1) // 256) * size * tok_local + chain * wgs * m + link * m if m > 1 else 0)
+
+
+@lru_cache(maxsize=1024)
+def segments(kind: str, T: int, tokens: int, wgs: int, most: int) -> int:
+    """The fastest number of segments, up to `most`, of a scan over T rows whose runs have at most `tokens`; wgs: workgroups of
+    one run."""
+    return min(range(1, max(1, min(-(-tokens // 64), most)) + 1), key=lambda s: segments_us(kind, tokens, wgs * T / tokens, s))
+
+
+def gla_shape(T: int, nruns: int, H: int, V: int, D: int = 64, longest: Optional[int] = None):
+    """(segments, groups of 64 value columns per workgroup) of a gla_scan launch; longest: tokens of the longest run, if known.
+    Up to 64 channels two workgroups per CU from segments of 64 tokens and more, unless whole runs already give one (2.7 % behind
+    the fastest count on average; there a CU holds several workgroups). With 65 to 128 channels that rule was 11 % behind, as it
+    does not see a last round that is nearly empty (32 heads of 128 x 128, bf16: 6 runs of 650 tokens 382 us with 3
+    segments, 265 with 1; 1 run of 333 tokens 93 us with 5, 63 with 6): the count is the one that segments_us finds fastest."""
     nt = 1 if V <= 64 else 2
-    wgs = H * -(-V // (64 * nt)) * nruns
-    return 1 if wgs >= 256 else max(1, min(-(-512 // wgs), (T - nruns + 1) // 64, 16)), nt
+    wgs = H * -(-V // (64 * nt))
+    n = T - nruns + 1 if longest is None else longest
+    most = min(-(-512 // (wgs * nruns)), 16)             # (what bounds the scratch, too)
+    if 64 < D <= 128 and nt == 2:
+        return segments("gla", T, longest or -(-T // nruns), wgs, most), nt
+    return 1 if wgs * nruns >= 256 else max(1, min(most, -(-n // 64))), nt
 
 
 def gla_scan(q, k, v, a, qscale: float, o, norm, gate, out, state, runs, nruns: int, H: int, D: int, V: int, eps: float, shape,
@@ -675,12 +708,18 @@ def delta_conv(z, w, y, fac, state, runs, tok_seq, T: int, nruns: int, H: int, G
                                 nruns, H, G, D, V, w.shape[1], int(z.dtype == torch.float32), st), "nls_delta_conv")
 
 
-def delta_shape(T: int, nruns: int, H: int, D: int, V: int):
-    """(segments, groups of 64 value columns per workgroup) of a delta_scan launch. Segments cost a second pass over the tokens
-    with D more columns, so they start where whole runs fill less than half the CUs, and stay longer."""
+def delta_shape(T: int, nruns: int, H: int, D: int, V: int, longest: Optional[int] = None):
+    """(segments, groups of 64 value columns per workgroup) of a delta_scan launch, as gla_shape. Segments cost a second pass over
+    the tokens with D more columns: up to 64 channels they start where whole runs fill less than half the CUs, and stay longer
+    (at 16 heads of 128 x 128 that rule was 5.5 % behind the fastest count on average: 6 runs of 650 tokens 517 us with 3
+    segments, 444 with the 1 that segments_us finds)."""
     nt = 1 if V <= 64 else 2
-    wgs = H * -(-V // (64 * nt)) * nruns
-    return 1 if wgs >= 128 else max(1, min(-(-256 // wgs), (T - nruns + 1) // 128, 16)), nt
+    wgs = H * -(-V // (64 * nt))
+    n = T - nruns + 1 if longest is None else longest
+    most = min(-(-256 // (wgs * nruns)), 16)             # (what bounds the scratch, too)
+    if 64 < D <= 128 and nt == 2:
+        return segments("delta", T, longest or -(-T // nruns), wgs, most), nt
+    return 1 if wgs * nruns >= 128 else max(1, min(most, n // 128)), nt
 
 
 def delta_scan(q, k, v, fac, beta, a, o, norm, gate, out, state, runs, nruns: int, H: int, G: int, D: int, V: int, eps: float,
