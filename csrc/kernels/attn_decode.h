@@ -105,8 +105,21 @@ struct AttnMask {
   int window = 0, keep = 0, sink = 0;
 };
 
-template <typename KV, int WAVES, int D, typename OUT = act_t, bool WIN = false>
-__global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
+template <int WAVES, int D>
+constexpr int attn_decode_lds() {
+  // per wave: one 32-key V tile (8 KiB; a wave's LDS ops run in order, so the next group's V is written
+  // after this group's transposed reads without a second buffer); the space is reused for the cross-wave
+  // merge and the split merge at the end
+  constexpr int VB = WAVES * 32 * D * 2, MB = WAVES > 1 ? (2 * WAVES * 16 + WAVES * 16 * D) * 4 : 0,
+                CB = (16 * 64 + 64 * WAVES * 4) * 4;
+  return VB > MB ? (VB > CB ? VB : CB) : (MB > CB ? MB : CB);
+}
+
+// by of gy: workgroup of token t's heads; Vsm: attn_decode_lds() bytes. AHEAD: the next keys' loads are in flight under a group's
+// arithmetic (at D = 128 220 registers, without it 168).
+template <typename KV, int WAVES, int D, typename OUT, bool WIN, bool AHEAD = true>
+DEVI void attn_decode_body(
+    uint8_t* Vsm, int t, int by, int gy, int split,
     const __bf16* __restrict__ q, long ldq, const KV* __restrict__ kc, const KV* __restrict__ vc,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
     const int* __restrict__ ctx_len, int Hkv, int Gq, int bs, float scale, int chunk, int n_split,
@@ -117,16 +130,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
   constexpr int NCH = D / 8, LPR = NCH, RPI = 64 / LPR, NVL = KG / RPI;   // V: chunks per row, lanes per row,
                                                                           // rows per load, loads per 32 keys
   typedef KVRaw<KV> R;
-  // per wave: one 32-key V tile (8 KiB; a wave's LDS ops run in order, so the next group's V is written
-  // after this group's transposed reads without a second buffer); the space is reused for the cross-wave
-  // merge and the split merge at the end
-  constexpr int VB = WAVES * KG * D * 2, MB = WAVES > 1 ? (2 * WAVES * 16 + WAVES * 16 * D) * 4 : 0,
-                CB = (16 * 64 + 64 * WAVES * 4) * 4;
-  constexpr int SMEM = VB > MB ? (VB > CB ? VB : CB) : (MB > CB ? MB : CB);
-  __shared__ __attribute__((aligned(16))) uint8_t Vsm[SMEM];
-  const int t = blockIdx.x, split = blockIdx.z;
-  const int nhb = (Gq + 15) >> 4, kh = nhb == 1 ? (int)blockIdx.y : (int)blockIdx.y / nhb;
-  const int hofs = nhb == 1 ? 0 : ((int)blockIdx.y - kh * nhb) * 16;
+  const int nhb = (Gq + 15) >> 4, kh = nhb == 1 ? by : by / nhb;
+  const int hofs = nhb == 1 ? 0 : (by - kh * nhb) * 16;
   const int G = min(Gq - hofs, 16), h0 = kh * Gq + hofs;       // this workgroup's query heads: h0 .. h0 + G - 1
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -218,15 +223,19 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
   // wave w takes the 32-key groups w, w + WAVES, ... of the workgroup's range
   const int ngrp_all = end > start ? (end - start + KG - 1) / KG : 0;
   const int ngrp = ngrp_all > wave ? (ngrp_all - wave + WAVES - 1) / WAVES : 0;
-  if (ngrp > 0) {
+  if (AHEAD && ngrp > 0) {
     load(start + wave * KG, kr, vr);
     store_v(0, vr);
   }
   for (int j = 0; j < ngrp; ++j) {
     const int base = start + (j * WAVES + wave) * KG;
     typename R::raw kn[2][NKK], vn[NVL];
-    const bool more = j + 1 < ngrp;
+    const bool more = AHEAD && j + 1 < ngrp;
     if (more) load(base + WAVES * KG, kn, vn);
+    if constexpr (!AHEAD) {
+      load(base, kr, vr);
+      store_v(0, vr);
+    }
     // ---- S^T = K Q^T: s[nt][i] = S[head r][key base + 16 nt + 4 g + i]
     f32x4 s[2];
 #pragma unroll
@@ -365,7 +374,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0) {
-    int* cp = cnt + (size_t)t * gridDim.y + blockIdx.y;
+    int* cp = cnt + (size_t)t * gy + by;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const int old = __hip_atomic_fetch_add(cp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -380,6 +389,19 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
   if (!last) return;
   merge_splits<WAVES, D>(part_o, part_ml, t, h0, G, Hq, n_split, na, out, ldo, gate, ldg,
                          reinterpret_cast<float*>(Vsm));
+}
+
+template <typename KV, int WAVES, int D, typename OUT = act_t, bool WIN = false>
+__global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
+    const __bf16* __restrict__ q, long ldq, const KV* __restrict__ kc, const KV* __restrict__ vc,
+    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
+    const int* __restrict__ ctx_len, int Hkv, int Gq, int bs, float scale, int chunk, int n_split,
+    OUT* __restrict__ out, long ldo, float* __restrict__ part_o, float* __restrict__ part_ml,
+    int* __restrict__ cnt, const float* __restrict__ gate, long ldg, AttnMask mask) {
+  __shared__ __attribute__((aligned(16))) uint8_t Vsm[attn_decode_lds<WAVES, D>()];
+  attn_decode_body<KV, WAVES, D, OUT, WIN>(Vsm, blockIdx.x, blockIdx.y, gridDim.y, blockIdx.z, q, ldq, kc, vc, block_tables,
+                                           bt_stride, tok_seq, ctx_len, Hkv, Gq, bs, scale, chunk, n_split, out, ldo, part_o,
+                                           part_ml, cnt, gate, ldg, mask);
 }
 
 }  // namespace nls_attn

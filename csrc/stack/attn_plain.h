@@ -51,9 +51,9 @@ template <typename T> DEVI f32x4 ld4(const T* p) {
 
 // Row `row` of a workgroup, its token t and query head h, over the keys that it sees. mls: the waves' maxima and sums, w: 64 NW floats.
 template <typename T, int NW>
-DEVI void redo_row(const PA& p, int t, int h, int row, const float* mls, float* w) {
+DEVI void redo_row(const PA& p, int t, int h, int row, int bz, const float* mls, float* w) {
   constexpr int NT = 64 * NW, C = VB / NT;
-  const int ctx = p.ctx_len[t], low = p.window > 0 ? ctx - p.window : 0, v0 = blockIdx.z * VB, dv = min(p.Dv - v0, VB);
+  const int ctx = p.ctx_len[t], low = p.window > 0 ? ctx - p.window : 0, v0 = bz * VB, dv = min(p.Dv - v0, VB);
   const int* bt = p.bt + (size_t)p.tok_seq[t] * p.bts;
   const T* q = reinterpret_cast<const T*>(p.q) + (size_t)t * p.ldq + (size_t)h * p.qhs;
   const T* kc = reinterpret_cast<const T*>(p.k) + (size_t)(h / p.gs) * p.khs;
@@ -88,22 +88,21 @@ DEVI void redo_row(const PA& p, int t, int h, int row, const float* mls, float* 
     if ((int)threadIdx.x + NT * j < dv) y[threadIdx.x + NT * j] = (T)(acc[j] * f);
 }
 
-// NQ: 64-column blocks of the values; NW: waves
+// NQ: 64-column blocks of the values; NW: waves. (bx, by, bz) of gx: workgroup; sm: plain_lds() bytes. PA is the kernel's first argument.
 template <typename T, int NQ, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
+DEVI void attn_plain_body(float* sm, const PA& p, int bx, int by, int bz, int gx) {
   constexpr int KC = NQ > 2 ? 4 : 8;               // 16-column steps of a key chunk
   constexpr int ML = NW * 32 + 16;                 // floats of the waves' maxima and sums, rows that are not finite
-  extern __shared__ __attribute__((aligned(16))) float sm[];
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nks = (p.Dk + 15) >> 4, nc = (nks + KC - 1) / KC, ldl = nc * KC * 16 + 4;
   float *mls = sm, *ob = sm + ML, *qs = ob;        // (the merge takes the queries' place)
   int* bad = reinterpret_cast<int*>(sm + NW * 32);
-  const int kh = blockIdx.y / p.sub, h0 = (blockIdx.y % p.sub) * 16;          // key head, first of its query heads
+  const int kh = by / p.sub, h0 = (by % p.sub) * 16;          // key head, first of its query heads
   const int gr = min(p.gs - h0, 16);                                          // query heads of this workgroup
-  const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * p.tb, tn = min(p.tb, p.T - t0);      // (later tokens see more keys)
+  const int t0 = (gx - 1 - bx) * p.tb, tn = min(p.tb, p.T - t0);      // (later tokens see more keys)
   const int nrow = tn * gr;
-  const int v0 = blockIdx.z * VB, dv = min(p.Dv - v0, VB);                    // this workgroup's value columns
+  const int v0 = bz * VB, dv = min(p.Dv - v0, VB);                            // this workgroup's value columns
   const T* kc = reinterpret_cast<const T*>(p.k) + (size_t)kh * p.khs;
   const T* vc = reinterpret_cast<const T*>(p.v) + (size_t)kh * p.khs + v0;
   auto head = [&](int row) { return (size_t)kh * p.gs + h0 + row % gr; };
@@ -280,15 +279,24 @@ __global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
     const int row = __builtin_ctzll(again);
     const PA* args = (const PA*)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));                 // (read anew: kept from the start, they would not fit beside the loop's scalars)
-    redo_row<T, NW>(*args, t0 + row / gr, kh * args->gs + h0 + row % gr, row, mls, ob);
+    redo_row<T, NW>(*args, t0 + row / gr, kh * args->gs + h0 + row % gr, row, bz, mls, ob);
   }
 }
 
 template <typename T, int NQ, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  attn_plain_body<T, NQ, NW>(sm, p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x);
+}
+
+inline size_t plain_lds(int Dk, int NQ, int NW) {
+  const int KC = NQ > 2 ? 4 : 8, nc = ((Dk + 15) / 16 + KC - 1) / KC;
+  return sizeof(float) * (NW * 32 + 16 + max(16 * (nc * KC * 16 + 4), NW * 16 * 68));
+}
+
+template <typename T, int NQ, int NW>
 int launch_w(const PA& p, dim3 grid, hipStream_t st) {
-  constexpr int KC = NQ > 2 ? 4 : 8;
-  const int nc = ((p.Dk + 15) / 16 + KC - 1) / KC;
-  const size_t lds = sizeof(float) * (NW * 32 + 16 + max(16 * (nc * KC * 16 + 4), NW * 16 * 68));
+  const size_t lds = plain_lds(p.Dk, NQ, NW);
   if (lds > 64 * 1024) {
     static bool attr = false;
     if (!attr && hipFuncSetAttribute((const void*)attn_plain_kernel<T, NQ, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -300,18 +308,20 @@ int launch_w(const PA& p, dim3 grid, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// four waves once they fill the chip, eight (which halve the walk over a row's keys) on smaller grids
+inline bool small(dim3 grid) { return (long)grid.x * grid.y <= 512; }
+
 template <typename T, int NQ>
 int launch_q(const PA& p, dim3 grid, hipStream_t st) {
-  // four waves once they fill the chip, eight (which halve the walk over a row's keys) on smaller grids
-  if (NQ <= 4 && (long)grid.x * grid.y <= 512) return launch_w<T, NQ, NQ <= 4 ? 8 : 4>(p, grid, st);
+  if (NQ <= 4 && small(grid)) return launch_w<T, NQ, NQ <= 4 ? 8 : 4>(p, grid, st);
   return launch_w<T, NQ, 4>(p, grid, st);
 }
 
-template <typename T>
-int launch(PA p, int T_, int H, hipStream_t st) {
+// the launch's tokens per workgroup and grid; false: refused
+inline bool prepare(PA& p, int T_, int H, dim3& grid) {
   if (T_ < 1 || H < 1 || H > 65535 || p.gs < 1 || H % p.gs || p.Dk < 4 || p.Dk > MAXK || (p.Dk & 3) || p.Dv < 1 || (p.ldkv & 3) ||
       (p.khs & 3) || p.Dv > MAXV || p.bs < 1)
-    return -1;
+    return false;
   p.T = T_;
   p.sub = (p.gs + 15) / 16;
   // Up to 64 tokens each has a workgroup of its own. With more, a workgroup takes as many as leave one workgroup for each CU: a prompt's
@@ -320,7 +330,14 @@ int launch(PA p, int T_, int H, hipStream_t st) {
   // heads of 64 over 16: 65 tokens 167 us in groups of 16, 57 in groups of 5. One workgroup per row and head: 241, 403, 193 us.)
   const int heads = H / p.gs * p.sub;
   p.tb = T_ <= 64 ? 1 : min(max(1, 16 / p.gs), (int)(((long)T_ * heads + 255) / 256));
-  const dim3 grid((T_ + p.tb - 1) / p.tb, heads, (p.Dv + VB - 1) / VB);
+  grid = dim3((T_ + p.tb - 1) / p.tb, heads, (p.Dv + VB - 1) / VB);
+  return true;
+}
+
+template <typename T>
+int launch(PA p, int T_, int H, hipStream_t st) {
+  dim3 grid;
+  if (!prepare(p, T_, H, grid)) return -1;
   switch ((p.Dv + 63) / 64) {
     case 1: return launch_q<T, 1>(p, grid, st);
     case 2: return launch_q<T, 2>(p, grid, st);

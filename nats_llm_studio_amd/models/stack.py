@@ -428,13 +428,19 @@ class AttentionPart(_SharedPart):
                      self.scratch(b, "attn.cnt", 1, _SPLIT_WG + self.groups, torch.int32))
         return e
 
-    def run(self, b, e, cache, state, step: "_Step"):
-        c, st, T = self.cfg, step.st, step.T
-        kc, vc = cache[0], cache[1]
+    def rows(self, b, e, cache, step: "_Step"):
+        c, kc, vc, T, st = self.cfg, cache[0], cache[1], step.T, step.st
         K.attn_rows(e["qp"], e["kp"], e["vp"], self.qn, self.kn, self.cs, b.pos, b.slot, e["q"], kc, vc, T, c.heads,
                     c.kv_heads, c.dim, self.Dp, c.rot_dims, self.m.cfg.eps, st, V=c.vdim,
                     head_norm=self.m.cfg.design.attn_qk_norm == "head", key_tiles=self.talk is not None and self.talk_plan.mfma)
-        plan = step.plan
+
+    def splits(self, T: int) -> int:
+        return max(1, min(_SPLIT_CAP, _SPLIT_WG // (T * self.groups))) if self.mfma else 1
+
+    def run(self, b, e, cache, state, step: "_Step"):
+        c, st, T, plan = self.cfg, step.st, step.T, step.plan
+        kc, vc = cache[0], cache[1]
+        self.rows(b, e, cache, step)
         if self.talk is not None:
             args = (self.talk_plan, e["q"], kc, vc, self.talk, e["gate"], e["out"])
             if plan is None or plan.rest:
@@ -444,9 +450,8 @@ class AttentionPart(_SharedPart):
                 K.talk_prefill(*args, b.block_tables, step.block_size, plan.blocks, plan.nblocks, plan.waves, c.vdim, c.scale, st)
             return
         if plan is None or plan.rest:
-            ns = max(1, min(_SPLIT_CAP, _SPLIT_WG // (T * self.groups))) if self.mfma else 1
             K.gqa_attention(e["q"], kc, vc, e["gate"], e["out"], e["part"], b.block_tables, step.block_size, b.tok_seq,
-                            b.ctx_len if plan is None else plan.actx, T, c.heads, c.kv_heads, self.Dp, self.mfma, ns,
+                            b.ctx_len if plan is None else plan.actx, T, c.heads, c.kv_heads, self.Dp, self.mfma, self.splits(T),
                             c.scale, st, **self.mask)
         if plan is not None:
             K.gqa_prefill(e["q"], kc, vc, plan.xmap, plan.blocks, plan.nblocks, plan.waves, e["gate"], e["out"], c.heads,
@@ -744,6 +749,12 @@ class SharedNormLayer:
         self.parts = [PARTS[c.kind](model, i, c, p + "mix." + sub, scale) for c, sub, scale in mixer_parts(L.mixer)]
         self.norm2 = None
         self.mixers = len(self.parts)
+        self.both = 0                    # decoded tokens whose attention and recurrence go in one launch
+        if [type(q) for q in self.parts] == [AttentionPart, GlaPart]:
+            q, r = self.parts
+            if q.talk is None and r.a2r is not None:
+                self.both = K.attn_step_fits(q.cfg.heads, q.cfg.kv_heads, q.Dp, q.mfma, q.cfg.window, r.cfg.heads, r.cfg.dim,
+                                             r.cfg.vdim, model.f32)
         if L.mlp is not None:
             self.parts.append(PARTS[L.mlp.kind](model, i, L.mlp, p + "mlp."))
             if model.cfg.design.norm_place == "parallel":
@@ -774,12 +785,25 @@ class SharedNormLayer:
         for launch in b.launches[key, "in"]:
             launch.run(step.T, step.st)
         caches = kc.get(step.layer, {})
-        for j, (q, e) in enumerate(zip(self.parts, b.launches[key, "parts"])):
+        parts = list(enumerate(zip(self.parts, b.launches[key, "parts"])))
+        if step.T == step.nruns and step.plan is None and step.T <= self.both:
+            self._both(b, *(e for _, (_, e) in parts[:2]), caches[0], state, step)
+            parts = parts[2:]
+        for j, (q, e) in parts:
             q.run(b, e, caches.get(j), state, step)
         out = b.launches[key, "out"]
         n = out.run(step.T, step.st)
         K.norm_add(self.m.slabs(b), None, b.x, fin.pop("copy", None), step.T, cfg.eps, step.st, rms=cfg.design.norm == "rms",
                    slabs=n, slab_rows=out.slab_rows, **fin)
+
+    def _both(self, b, e, f, cache, state, step: "_Step"):
+        q, r = self.parts[:2]
+        c, g, T = q.cfg, r.cfg, step.T
+        q.rows(b, e, cache, step)
+        K.attn_step(e["q"], cache[0], cache[1], e["gate"], e["out"], e["part"], q.splits(T), b.block_tables, step.block_size,
+                    b.tok_seq, b.ctx_len, T, c.heads, c.kv_heads, q.Dp, c.scale, q.mask["sink"], f["q"], f["k"], f["v"], None,
+                    (f["low"], r.a2r, r.a2b, 1.0 / g.tau), g.dim ** -0.5, state["S"], b.runs, r.norm, f["g"], f["out"], g.heads, g.dim,
+                    g.vdim, self.m.cfg.eps, step.st)
 
 
 class SandwichNormLayer:

@@ -54,6 +54,8 @@ _SIGS = {
     "nls_delta_step": [P, P, P, L, P, L, P, L, P, L, P, P, P, P, I, P, L, P, P, I, L, P, L, P, I, P, P, L, I, I, I, I, F, I, P],
     "nls_gla_scan": [P, P, P, L, P, L, F, P, L, P, P, L, P, L, F, P, L, P, I, I, I, I, I, P, P, I, I, P],
     "nls_gla_step": [P, P, P, L, P, L, P, P, P, I, F, F, P, L, P, I, P, P, L, P, L, P, L, I, I, I, F, I, P],
+    "nls_attn_step": [P, L, P, P, P, I, I, P, P, I, I, I, I, F, P, L, P, L, I, I, P, P, P, P, P, P, L, P, L, P, P, P, I, F, F, P, L, P, P, P, L, P,
+                      L, P, L, I, I, I, F, I, P],
     "nls_latent_rows": [P, L, I, P, P, L, P, L, I, I, I, P, P, P, P, P, L, I, F, I, P],
     "nls_stack_argmax": [P, L, I, P, I, P],
     "nls_moe_plan": [P, L, I, I, I, I, I, I, I, F, P, P, I, P, P, P, I, P, P],
@@ -693,6 +695,35 @@ def gla_step(q, k, v, a, gate_in, qscale: float, state, runs, nruns: int, norm, 
                               gate.stride(0) if gate is not None else 0, _p(out), out.stride(0) if out is not None else 0, _p(o),
                               o.stride(0) if o is not None else 0, H, D, V, eps, int(q.dtype == torch.float32), st),
            "nls_gla_step")
+
+
+def attn_step_fits(AH: int, AG: int, Dp: int, mfma: bool, window: int, H: int, D: int, V: int, f32: bool) -> int:
+    """The most tokens whose attention and recurrence attn_step takes in one launch where that is the faster way (0: none): any
+    number in bf16, with one exception of 90 sizes 4 to 50 % less than one behind the other; in 32 bits (a workgroup per CU) up to
+    512 states (20 % less; 1024: 5 to 35 % more)."""
+    if window or V % 4 or V > 1024 or -(-D // (256 // (V // 4))) > 16:
+        return 0
+    if f32:
+        return 512 // max(H, attn_groups(AH, AG)) if Dp <= 256 else 0
+    return 1 << 30 if mfma and Dp in (64, 128) else 0
+
+
+def attn_step(aq, kc, vc, agate, aout, part, ns: int, block_tables, block_size: int, tok_seq, ctx_len, T: int, AH: int, AG: int, Dp: int,
+              scale: float, sink: bool, q, k, v, a, gate_in, qscale: float, state, runs, norm, gate, out, H: int, D: int, V: int,
+              eps: float, st: int):
+    """gqa_attention of T single tokens without a window, and gla_step with a norm on the same tokens, in one launch."""
+    po, pm, cnt = part
+    if ns > 1 and (po.numel() < T * AH * ns * Dp or pm.numel() < T * AH * ns * 2 or cnt.numel() < T * attn_groups(AH, AG)):
+        raise ValueError("attn_step: split workspace too small")
+    lo, a2, b, ia = gate_in if a is None else (None, None, None, 0.0)
+    _check(lib().nls_attn_step(aq.data_ptr(), aq.stride(0), kc.data_ptr(), vc.data_ptr(), block_tables.data_ptr(),
+                               block_tables.stride(0), block_size, tok_seq.data_ptr(), ctx_len.data_ptr(), T, AH, AG, Dp, scale,
+                               _p(agate), agate.stride(0) if agate is not None else 0, aout.data_ptr(), aout.stride(0), int(sink), ns,
+                               po.data_ptr(), pm.data_ptr(), cnt.data_ptr(),
+                               q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), _p(a), a.stride(0) if a is not None else 0,
+                               _p(lo), _p(a2), _p(b), a2.shape[1] if a2 is not None else 0, ia, qscale, state.data_ptr(),
+                               state.stride(0), runs.data_ptr(), norm.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(),
+                               out.stride(0), None, 0, H, D, V, eps, int(q.dtype == torch.float32), st), "nls_attn_step")
 
 
 # ---------------------------------------------------------------------------
