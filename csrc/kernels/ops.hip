@@ -557,6 +557,68 @@ __global__ __launch_bounds__(512) void moe_norm_route_kernel(
   if (wave < T) route_one(lg[wave], wave, lane, E, k, renorm, topw, counts, xrows, yrows, cap, sel);
 }
 
+// The same for 2 to 4 tokens of up to 4096 columns: four waves to a token, all tokens at once. One after another each token took its own
+// loads and two block-wide sums: 4 tokens of 4096 columns, 8 experts 16.1 -> 11.2 us, 2 tokens 10.1 -> 8.3, 3 of 2048 12.1 -> 8.0.
+template <int E>
+__global__ __launch_bounds__(1024) void moe_norm_route4_kernel(
+    const float* __restrict__ x, long ldx, const float* __restrict__ nw, float eps, int D,
+    const act_t* __restrict__ wr, act_t* __restrict__ h, long ldh, float* __restrict__ logits, int T, int k,
+    int renorm, float* __restrict__ topw, int* __restrict__ counts, int* __restrict__ xrows, int* __restrict__ yrows,
+    int cap, int* __restrict__ sel) {
+  __shared__ float sh[16];
+  __shared__ float red[16][E];
+  __shared__ float lg[4][E];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t = tid >> 8, c = (tid & 255) * 4;
+  for (int e = tid; e < E; e += blockDim.x) counts[e] = 0;
+  typedef act_t act4 __attribute__((ext_vector_type(4)));
+  float4 v[4], wv[4];
+  act4 w4[4][E];
+  const float* xr = x + (size_t)t * ldx;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = c + j * 1024;
+    v[j] = i < D ? *reinterpret_cast<const float4*>(xr + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    wv[j] = i < D ? *reinterpret_cast<const float4*>(nw + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int e = 0; e < E; ++e) w4[j][e] = i < D ? *reinterpret_cast<const act4*>(wr + (size_t)e * D + i) : act4{0, 0, 0, 0};
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+  ss = wave_sum(ss);
+  if (lane == 0) sh[wave] = ss;
+  __syncthreads();
+  const float inv = rsqrtf((sh[4 * t] + sh[4 * t + 1] + sh[4 * t + 2] + sh[4 * t + 3]) / (float)D + eps);
+  float acc[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = c + j * 1024;
+    const act4 r = {(act_t)(v[j].x * inv * wv[j].x), (act_t)(v[j].y * inv * wv[j].y), (act_t)(v[j].z * inv * wv[j].z),
+                    (act_t)(v[j].w * inv * wv[j].w)};
+    if (i < D) *reinterpret_cast<act4*>(h + (size_t)t * ldh + i) = r;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      acc[e] += (float)r.x * (float)w4[j][e].x + (float)r.y * (float)w4[j][e].y + (float)r.z * (float)w4[j][e].z +
+                (float)r.w * (float)w4[j][e].w;
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const float a = wave_sum(acc[e]);
+    if (lane == 0) red[wave][e] = a;
+  }
+  __syncthreads();
+  if (tid < T * E) {
+    const int u = tid / E, e = tid - u * E;
+    const float s2 = red[4 * u][e] + red[4 * u + 1][e] + red[4 * u + 2][e] + red[4 * u + 3][e];
+    lg[u][e] = s2;
+    logits[(size_t)u * E + e] = s2;
+  }
+  __syncthreads();
+  if (wave < T) route_one(lg[wave], wave, lane, E, k, renorm, topw, counts, xrows, yrows, cap, sel);
+}
+
 // MoE router logits for many tokens (prefill chunks, decode batches > 4): logits[t][e] = h[t] . Wr[e] with Wr
 // the router's f16 copy [E][D]. The router is E (2-8) rows: the GEMV/GEMM tiles (128 weight rows per
 // workgroup, 128-row activation blocks) ran it on M / 128 workgroups with 15/16 of each MFMA idle -- ~50 us per
@@ -831,6 +893,11 @@ int nls_moe_norm_route(const float* x, long ldx, const float* nw, float eps, int
   if (T < 1 || T > 4 || D % 4 || D > 8192 || k < 1 || k > E || ldx % 4 || ldh % 4) return -1;
   hipStream_t st = (hipStream_t)stream;
 #define NLS_MNR(EE)                                                                                              \
+  if (E == EE && T > 1 && D <= 4096) {                                                                         \
+    hipLaunchKernelGGL(moe_norm_route4_kernel<EE>, dim3(1), dim3(256 * T), 0, st, x, ldx, nw, eps, D, (const act_t*)wr, \
+                       (act_t*)h, ldh, logits, T, k, renorm, topw, counts, xrows, yrows, cap, sel);             \
+    return (int)hipGetLastError();                                                                             \
+  }                                                                                                            \
   if (E == EE) {                                                                                               \
     hipLaunchKernelGGL(moe_norm_route_kernel<EE>, dim3(1), dim3(512), 0, st, x, ldx, nw, eps, D, (const act_t*)wr, \
                        (act_t*)h, ldh, logits, T, k, renorm, topw, counts, xrows, yrows, cap, sel);             \
