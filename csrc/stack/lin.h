@@ -283,6 +283,112 @@ DEVI void lin_store4(const LinSeg& S, int grp, int ks, int n, int yr, f32x4 v) {
   }
 }
 
+// The epilogue of a lane's NI x NJ blocks of 4 columns: columns n + 16 i of rows row0 + 16 j. Rows, column offsets, a column's constants and
+// the choice of the epilogue are taken out of the blocks where whole 4-column groups are written; the rest goes through lin_store4. (Row
+// lists, positions and biases are loads: with one of them in each block, a tile of experts took 35 us longer. And the general
+// epilogue in every block is a walk through code that has not run yet, block by block: 66 x 2048 x 64 without an epilogue 5.6 -> 4.8 us, with
+// sigpow 8.1 -> 5.9, 4000 rows 26.5 -> 19.0; each GEMM launch of a step lost 1 to 2 us to it, 600 rows in 32 bits 4 %.)
+template <typename T, int E, int NI, int NJ>
+DEVI void lin_store(const LinSeg& S, const LinTile& t, const f32x4 (&acc)[NI][NJ], int n, int row0, const int (&yr)[NJ]) {
+  typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  constexpr bool GLU = E == LE_GEGLU || E == LE_SWIGLU || E == LE_SILUGLU, BIAS = E == LE_DECAY || E == LE_SIGPOW;
+  const bool act = sizeof(T) == 2 && S.yact;
+  int col[NI], nr[NI];
+  float b[BIAS ? NI : 1][4], p[E == LE_SIGPOW ? NI : 1][4], gt[NJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int c = n + 16 * i, nb = S.cb < S.N ? c / S.cb : 0;
+    nr[i] = c - nb * S.cb;
+    col[i] = GLU ? c >> 1 : nb * S.cstep + nr[i];
+    if constexpr (BIAS)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        b[i][e] = S.bias[min(c, S.N - 4) + e];
+        if constexpr (E == LE_SIGPOW) p[i][e] = S.gate ? S.gate[min(c, S.N - 4) + e] : S.alpha;
+      }
+  }
+  const float* cs[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    if constexpr (E == LE_ROPE) cs[j] = S.cs + (size_t)S.pos[yr[j]] * S.half * 2;
+    if constexpr (E == LE_GATE) gt[j] = S.gate[(size_t)yr[j] * S.ldg + t.grp];
+  }
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    if (row0 + 16 * j >= t.cnt) break;
+    const size_t o = (size_t)yr[j] * S.ldy + (size_t)t.grp * S.ygs + (size_t)t.ks * S.yks;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if (n + 16 * i >= S.N) break;
+      f32x4 v = acc[i][j];
+      if constexpr (GLU) {
+        float u[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          u[e] = E == LE_SWIGLU ? lin_swiglu(v[2 * e], v[2 * e + 1], S.alpha)
+                                : (E == LE_SILUGLU ? v[2 * e] * lin_sigmoid(v[2 * e]) : lin_gelu(v[2 * e])) * v[2 * e + 1];
+        if constexpr (sizeof(T) == 2) *reinterpret_cast<bf2*>(reinterpret_cast<__bf16*>(S.y) + o + col[i]) = bf2{(__bf16)u[0], (__bf16)u[1]};
+        else *reinterpret_cast<float2*>(reinterpret_cast<float*>(S.y) + o + col[i]) = float2{u[0], u[1]};
+        continue;
+      }
+      if constexpr (E == LE_ROPE) {
+        if (nr[i] < 2 * S.half) {                        // (half is even: both pairs turn or none)
+          const f32x4 w = *reinterpret_cast<const f32x4*>(cs[j] + nr[i]);
+          v = f32x4{v[0] * w[0] - v[1] * w[1], v[1] * w[0] + v[0] * w[1], v[2] * w[2] - v[3] * w[3], v[3] * w[2] + v[2] * w[3]};
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (E == LE_SILU) v[e] = v[e] * lin_sigmoid(v[e]);
+        if constexpr (E == LE_TANH) v[e] = tanhf(v[e]);
+        if constexpr (E == LE_SIGMOID) v[e] = S.alpha * lin_sigmoid(v[e]);
+        if constexpr (E == LE_RELU2) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
+        if constexpr (E == LE_DECAY) v[e] = expf(-expf(v[e] + b[i][e]));
+        if constexpr (E == LE_SIGPOW) v[e] = lin_sigpow(v[e] + b[i][e], p[i][e]);
+        if constexpr (E == LE_GATE) v[e] *= gt[j];
+      }
+      if (act) *reinterpret_cast<bf4*>(reinterpret_cast<__bf16*>(S.y) + o + col[i]) = bf4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+      else *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(S.y) + o + col[i]) = v;
+    }
+  }
+}
+
+template <typename T, int NI, int NJ>
+DEVI void lin_epilogue(const LinSeg& S, const LinTile& t, f32x4 (&acc)[NI][NJ], int n, int row0) {
+  const bool glu = S.epi == LE_GEGLU || S.epi == LE_SWIGLU || S.epi == LE_SILUGLU;
+  const bool whole = !(S.N & 3) && !((S.ldy | S.ygs | S.yks | S.cstep) & 3) && (!glu || S.yact || sizeof(T) == 4);
+  int yr[NJ], xr;
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) lin_row(S, t, row0 + 16 * j, xr, yr[j]);
+#define NLS_LE(E) \
+  case E: lin_store<T, E, NI, NJ>(S, t, acc, n, row0, yr); return;
+  switch (whole ? S.epi : -1) {
+    NLS_LE(LE_NONE) NLS_LE(LE_SILU) NLS_LE(LE_SIGMOID) NLS_LE(LE_RELU2) NLS_LE(LE_GEGLU) NLS_LE(LE_SWIGLU) NLS_LE(LE_SILUGLU)
+    case LE_ROPE:
+      if (!(S.half & 1)) {
+        lin_store<T, LE_ROPE, NI, NJ>(S, t, acc, n, row0, yr);
+        return;
+      }
+    default: break;
+  }
+  if constexpr (NI * NJ < 32)                 // (the largest tiles have no registers for a column's constants)
+    switch (whole ? S.epi : -1) {
+      NLS_LE(LE_TANH) NLS_LE(LE_DECAY) NLS_LE(LE_GATE) NLS_LE(LE_SIGPOW)
+      default: break;
+    }
+#undef NLS_LE
+  // (a loop over the blocks of 16 columns that moves them up: the general epilogue unrolled NI NJ times is more code than the product)
+  for (int i = 0; i < NI; ++i) {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (row0 + 16 * j < t.cnt) lin_store4<T>(S, t.grp, t.ks, n + 16 * i, yr[j], acc[0][j]);
+#pragma unroll
+      for (int k = 0; k + 1 < NI; ++k) acc[k][j] = acc[k + 1][j];
+    }
+  }
+}
+
 // swizzle of a row's four 16-byte chunks in an activation sub-tile of the LDS
 DEVI int lin_swz(int r) { return (0x1320 >> (4 * ((r >> 2) & 3))) & 3; }
 

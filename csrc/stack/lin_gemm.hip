@@ -26,6 +26,7 @@ using nls_dma::wait_vm_lgkm0;
 
 int lin_phased(LinArgs& a, hipStream_t st);      // lin_phased.hip
 int lin_split(LinArgs& a, int cfg, hipStream_t st);      // lin_split.hip
+int lin_thin(LinArgs& a, hipStream_t st);        // lin_thin.hip
 
 template <int BN, int BM, int WN, int WM, int NST>
 struct LG {
@@ -149,15 +150,7 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
     walk(std::integral_constant<bool, FETCH == STREAM>{});
   }
   wait_vm_lgkm0<0>();                                 // the clamped tail DMAs land before the workgroup's LDS is freed
-#pragma unroll
-  for (int j = 0; j < MTW; ++j) {
-    const int row = 16 * (wm * MTW + j) + r;
-    if (row >= t.cnt) continue;
-    int xr, yr;
-    lin_row(S, t, row, xr, yr);
-#pragma unroll
-    for (int i = 0; i < NTW; ++i) lin_store4<T>(S, t.grp, t.ks, t.n0 + 16 * (wn * NTW + i) + 4 * g, yr, acc[i][j]);
-  }
+  lin_epilogue<T>(S, t, acc, t.n0 + 16 * wn * NTW + 4 * g, 16 * wm * MTW + r);
 }
 
 template <int BN, int BM, int WN, int WM, int NST, int FETCH>
@@ -203,6 +196,7 @@ int lin_gemm(LinArgs& a, int cfg, hipStream_t st) {
     case 10: return gemm_t<128, 64, 2, 2, 4>(a, st);
     case 11: return gemm_t<96, 128, 2, 2, 4>(a, st);
     case 12: return gemm_t<64, 32, 2, 1, 8>(a, st);
+    case 13: return lin_thin(a, st);
   }
   return -1;
 }
@@ -213,7 +207,8 @@ extern "C" {
 
 // cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256 in two stages (a launch's
 // own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
-// 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128, 12 = 64 x 32 with 8 stages.
+// 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128, 12 = 64 x 32 with 8 stages,
+// 13 = 64 x 128 straight from memory (K up to 128, no routed rows).
 // f32: 0, 1 and 2; the others but 7 run on one of these.
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);

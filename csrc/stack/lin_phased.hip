@@ -49,92 +49,6 @@ struct PhTile {
   int nst;                                               // steps
 };
 
-// The epilogue of a lane's 8 x 4 blocks. Rows, column offsets and the choice of the epilogue are taken out of the blocks where whole
-// 4-column groups are written; the rest goes through lin_store4. (Row lists and positions are loads: with one of them in each block,
-// a tile of experts took 35 us longer.)
-template <int E>
-DEVI void ph_store(const LinSeg& S, const LinTile& t, const f32x4 (&acc)[8][4], int n, int row0, const int (&yr)[4]) {
-  typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
-  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-  constexpr bool GLU = E == LE_GEGLU || E == LE_SWIGLU || E == LE_SILUGLU;
-  int col[8], nr[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int c = n + 16 * i, nb = S.cb < S.N ? c / S.cb : 0;
-    nr[i] = c - nb * S.cb;
-    col[i] = GLU ? c >> 1 : nb * S.cstep + nr[i];
-  }
-  const float* cs[4];
-  if constexpr (E == LE_ROPE)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) cs[j] = S.cs + (size_t)S.pos[yr[j]] * S.half * 2;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (row0 + 16 * j >= t.cnt) break;
-    const size_t o = (size_t)yr[j] * S.ldy + (size_t)t.grp * S.ygs + (size_t)t.ks * S.yks;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      if (n + 16 * i >= S.N) break;
-      f32x4 v = acc[i][j];
-      if constexpr (GLU) {
-        float u[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e)
-          u[e] = E == LE_SWIGLU ? lin_swiglu(v[2 * e], v[2 * e + 1], S.alpha)
-                                : (E == LE_SILUGLU ? v[2 * e] * lin_sigmoid(v[2 * e]) : lin_gelu(v[2 * e])) * v[2 * e + 1];
-        *reinterpret_cast<bf2*>(reinterpret_cast<__bf16*>(S.y) + o + col[i]) = bf2{(__bf16)u[0], (__bf16)u[1]};
-        continue;
-      }
-      if constexpr (E == LE_ROPE) {
-        if (nr[i] < 2 * S.half) {                        // (half is even: both pairs turn or none)
-          const f32x4 w = *reinterpret_cast<const f32x4*>(cs[j] + nr[i]);
-          v = f32x4{v[0] * w[0] - v[1] * w[1], v[1] * w[0] + v[0] * w[1], v[2] * w[2] - v[3] * w[3], v[3] * w[2] + v[2] * w[3]};
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if constexpr (E == LE_SILU) v[e] = v[e] * lin_sigmoid(v[e]);
-        if constexpr (E == LE_SIGMOID) v[e] = S.alpha * lin_sigmoid(v[e]);
-        if constexpr (E == LE_RELU2) v[e] = fmaxf(v[e], 0.f) * fmaxf(v[e], 0.f);
-      }
-      if (S.yact) *reinterpret_cast<bf4*>(reinterpret_cast<__bf16*>(S.y) + o + col[i]) = bf4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-      else *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(S.y) + o + col[i]) = v;
-    }
-  }
-}
-
-DEVI void ph_epilogue(const LinSeg& S, const LinTile& t, f32x4 (&acc)[8][4], int n, int row0) {
-  const bool glu = S.epi == LE_GEGLU || S.epi == LE_SWIGLU || S.epi == LE_SILUGLU;
-  const bool whole = !(S.N & 3) && !((S.ldy | S.ygs | S.yks | S.cstep) & 3) && (!glu || S.yact);
-  int yr[4], xr;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) lin_row(S, t, row0 + 16 * j, xr, yr[j]);
-  switch (whole ? S.epi : -1) {
-    case LE_NONE: ph_store<LE_NONE>(S, t, acc, n, row0, yr); break;
-    case LE_SILU: ph_store<LE_SILU>(S, t, acc, n, row0, yr); break;
-    case LE_SIGMOID: ph_store<LE_SIGMOID>(S, t, acc, n, row0, yr); break;
-    case LE_RELU2: ph_store<LE_RELU2>(S, t, acc, n, row0, yr); break;
-    case LE_GEGLU: ph_store<LE_GEGLU>(S, t, acc, n, row0, yr); break;
-    case LE_SWIGLU: ph_store<LE_SWIGLU>(S, t, acc, n, row0, yr); break;
-    case LE_SILUGLU: ph_store<LE_SILUGLU>(S, t, acc, n, row0, yr); break;
-    case LE_ROPE:
-      if (!(S.half & 1)) {
-        ph_store<LE_ROPE>(S, t, acc, n, row0, yr);
-        break;
-      }
-    default:
-      // (a loop over the blocks of 16 columns that moves them up: the general epilogue unrolled 32 times is more code than the loop)
-      for (int i = 0; i < 8; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (row0 + 16 * j < t.cnt) lin_store4<__bf16>(S, t.grp, t.ks, n + 16 * i, yr[j], acc[0][j]);
-#pragma unroll
-          for (int k = 0; k < 7; ++k) acc[k][j] = acc[k + 1][j];
-        }
-      }
-  }
-}
-
 __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot) {
   extern __shared__ __attribute__((aligned(16))) uint8_t phlds[];
   typedef LT<__bf16> L;
@@ -276,7 +190,7 @@ __global__ __launch_bounds__(512, 1) void lin_phased_kernel(LinArgs a, int ntot)
       ph_barrier();
     }
     if (wr == 0) ph_barrier();
-    ph_epilogue(a.s[t.seg], t, acc, t.n0 + 128 * wr + 4 * g, 64 * wc + r);
+    lin_epilogue<__bf16>(a.s[t.seg], t, acc, t.n0 + 128 * wr + 4 * g, 64 * wc + r);
     if (nid < 0) break;
     id = nid;
   }

@@ -172,14 +172,12 @@ __global__ __launch_bounds__(64 * NWV, WPE) void lin_split_kernel(LinArgs a, int
     for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) odd |= !(fabsf(acc[q][i][e]) < __builtin_inff());
-  const bool again = __any(odd);
+  if (__any(odd))
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int row = 16 * i + r;
-    int xr0, yr;
-    lin_row(S, t, row, xr0, yr);
-    if (again) {
-      const float* x = (const float*)S.x + (size_t)xr0 * S.ldx + (size_t)t.grp * S.xgs + 32 * jb + 4 * g;
+    for (int i = 0; i < MT; ++i) {
+      int xr, yr;
+      lin_row(S, t, 16 * i + r, xr, yr);
+      const float* x = (const float*)S.x + (size_t)xr * S.ldx + (size_t)t.grp * S.xgs + 32 * jb + 4 * g;
 #pragma unroll
       for (int q = 0; q < RT; ++q) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
@@ -187,10 +185,7 @@ __global__ __launch_bounds__(64 * NWV, WPE) void lin_split_kernel(LinArgs a, int
         acc[q][i] = v;
       }
     }
-    if (row >= t.cnt) continue;
-#pragma unroll
-    for (int q = 0; q < RT; ++q) lin_store4<float>(S, t.grp, t.ks, t.n0 + 16 * (RT * wave + q) + 4 * g, yr, acc[q][i]);
-  }
+  lin_epilogue<float>(S, t, acc, t.n0 + 16 * RT * wave + 4 * g, r);
 }
 
 template <int NWV, int RT, int MT, int WPE>

@@ -190,6 +190,7 @@ class Seg:
 # (weight rows, rows) of lin_gemm's configs
 GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 4: (256, 256), 5: (64, 64), 6: (192, 128), 7: (256, 256),
               8: (96, 64), 9: (160, 64), 10: (128, 64), 11: (96, 128), 12: (64, 32)}
+THIN = 13                # config of products of up to 128 inputs straight from memory, 64 weight rows x 128 rows
 
 
 # Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
@@ -276,8 +277,11 @@ class LinLaunch:
             if n64 >= 250:
                 return True, 0
             return False, 2, (4 if ns <= 16 else 8), (2 if M > 32 or n16 >= 640 else 1)
-        if ns <= 4:                       # a step or two of K: all epilogue
-            return True, (0 if M <= 2048 else 1)
+        if ns <= 4:                       # a step or two of K: all epilogue. 64 x 64 / 128 x 64 / straight from memory, us: 600 x 2048 x 64
+            # 7.2 / 8.0 / 7.8, 2000 12.3 / 11.0 / 10.9, 4000 19.0 / 18.0 / 16.9; 4000 x 4096 x 64 25.4 / 23.5 / 19.2, 600 x 4096 x 128 7.8 / 7.9 / 8.7
+            if not self.f32 and self._tiles(64, 128, M) >= 512:
+                return True, THIN
+            return True, (0 if M <= 2048 or not self.f32 else 1)
         if n64 < 96 and n16 <= 1024:
             return False, 1, 16, 1
         if self.f32:
