@@ -701,7 +701,7 @@ struct Route {
 };
 
 DEVI void pick_experts(const float* __restrict__ z, const Route& R, int lane, float* sc, float* gs, float* __restrict__ topw,
-                       int* __restrict__ sel) {
+                       int* __restrict__ sel, int* kept = nullptr) {
   const int E = R.E, topk = R.topk, groups = R.groups, keep = R.keep;
   const float scale = R.scale;
   if (R.softmax) {
@@ -762,6 +762,7 @@ DEVI void pick_experts(const float* __restrict__ z, const Route& R, int lane, fl
     if (lane == 0) {
       topw[j] = bv * scale;
       sel[j] = be;
+      if (kept) kept[j] = be;
     }
     if (lane == (be & 63)) sc[be] = -4.f;
     __builtin_amdgcn_wave_barrier();
@@ -770,7 +771,7 @@ DEVI void pick_experts(const float* __restrict__ z, const Route& R, int lane, fl
 }
 
 constexpr int ME = 512;       // experts per layer
-constexpr int PW = 8;         // waves that choose experts in moe_plan_kernel<true>
+constexpr int PW = 16, PE = 256;      // tokens (a wave each) and experts of moe_plan_kernel<true>
 
 __global__ __launch_bounds__(64) void moe_pick_kernel(const float* __restrict__ z, long ldz, Route R, float* __restrict__ topw,
                                                       int* __restrict__ sel) {
@@ -789,19 +790,20 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict_
                                                         int* __restrict__ rows, int* __restrict__ tiles,
                                                         int* __restrict__ ntiles, int maxtiles, const int* __restrict__ ctx) {
   __shared__ int cnt[ME], off[ME], pos[ME];
-  __shared__ float sc[PICK ? PW : 1][PICK ? ME : 1], gs[PICK ? PW : 1][PICK ? ME : 1];
+  __shared__ float sc[PICK ? PW : 1][PICK ? PE : 1], gs[PICK ? PW : 1][PICK ? PE : 1];
+  __shared__ int kept[PICK ? PW * PE : 1];    // (the choices: from memory each pass over them is a round trip)
   const int E = R.E, topk = R.topk, n = T * topk;
   if constexpr (PICK) {
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    for (int t = w; w < PW && t < T; t += PW)
-      pick_experts(z + (size_t)t * ldz, R, lane, sc[w], gs[w], topw + (size_t)t * topk, sel + (size_t)t * topk);
-    __threadfence_block();
+    const int t = threadIdx.x >> 6;
+    if (t < T)
+      pick_experts(z + (size_t)t * ldz, R, threadIdx.x & 63, sc[t], gs[t], topw + (size_t)t * topk, sel + (size_t)t * topk, kept + t * topk);
   }
+  auto choice = [&](int i) { return min(max(PICK ? kept[i] : sel[i], 0), E - 1); };
   for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
   __syncthreads();
   auto live = [&](int i) { return !ctx || ctx[i / topk] > 0; };
   for (int i = threadIdx.x; i < n; i += 1024)
-    if (live(i)) atomicAdd(&cnt[min(max(sel[i], 0), E - 1)], 1);
+    if (live(i)) atomicAdd(&cnt[choice(i)], 1);
   __syncthreads();
   if (threadIdx.x < 64) {
     // one wave: exclusive prefix sums of counts and tile counts, 64 experts at a time
@@ -836,7 +838,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const float* __restrict_
   }
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += 1024) {
-    const int e = min(max(sel[i], 0), E - 1);
+    const int e = choice(i);
     if (live(i)) rows[off[e] + atomicAdd(&pos[e], 1)] = i;
   }
 }
@@ -960,7 +962,9 @@ int nls_moe_plan(const float* z, long ldz, int T, int E, int topk, int groups, i
     return -1;
   const Route R{E, topk, groups, keep, softmax, gbest, scale};
   hipStream_t st = (hipStream_t)stream;
-  if (T <= 32) {
+  // One launch while every token has a wave of its own (us, one / two launches: 8 experts, 16 tokens 6.1 / 6.6; 64 experts 8.7 at 8, 9.6 at 16 /
+  // 9.2; with 8 waves 16 and 32 tokens took 8.3 and 13.5, 15.2 and 26.8; 512 experts, 5 tokens 60.5 / 47.5)
+  if (T <= PW && E <= PE) {
     hipLaunchKernelGGL(moe_plan_kernel<true>, dim3(1), dim3(1024), 0, st, z, ldz, T, R, topw, sel, bm,
                        rows, tiles, ntiles, maxtiles, ctx);
     return (int)hipGetLastError();
