@@ -940,6 +940,7 @@ class StackModel:
 
     format = "safetensors"
     prefill_graphs = False        # (the captured single-prompt prefill of the GGUF families)
+    run_lengths = True            # forward takes the longest run's rows
 
     def __init__(self, path: str, device="cuda:0", dtype: torch.dtype = torch.bfloat16, shard: ShardSpec = ShardSpec(),
                  comm=None, ctx: Optional[int] = None):
