@@ -1025,7 +1025,7 @@ class Engine:
         pad = b.pad
         h = self.h_meta_p.numpy()
         info = {}
-        if nruns and getattr(self.model, "run_lengths", False):
+        if nruns and self.slots is not None and getattr(self.model, "run_lengths", False):       # (others have no table of runs)
             info["longest"] = int(self._tables(self.h_meta_p, pad)[1][:nruns, 1].max())
         if hasattr(self.model, "row_blocks"):
             qb, ri = self.model.row_blocks(h[3 * pad:4 * pad], h[pad:2 * pad], T) if self.prefill_attn else (None, None)
