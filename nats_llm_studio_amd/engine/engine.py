@@ -913,12 +913,14 @@ class Engine:
                 s.n_fed += n
                 done[i] += n
                 T += n
-            self._next_prefill_buf()
-            self._fill_rows(parts)
-            self._exec_prefill(T, rows or [0], True, len(parts))
+            try:
+                self._next_prefill_buf()
+                self._fill_rows(parts)
+                self._exec_prefill(T, rows or [0], True, len(parts))
+            finally:                                       # (behind the launch, but with n_fed also where it fails)
+                for s, _, toks in parts:
+                    s.tokens += toks.tolist()
             self.counters["prefill_tokens"] += T
-            for s, _, toks in parts:
-                s.tokens += toks.tolist()
             if rows:
                 self._flight = None
                 dst = [out[i][a:b] for i, a, b in dest]
