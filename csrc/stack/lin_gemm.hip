@@ -209,7 +209,7 @@ extern "C" {
 // own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
 // 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128, 12 = 64 x 32 with 8 stages,
 // 13 = 64 x 128 straight from memory (K up to 128, no routed rows).
-// f32: 0, 1 and 2; the others but 7 run on one of these.
+// f32: 0, 1 and 2; the others run on one of these, but for 7 and 13 and for routed rows on 4, which are refused.
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
   return f32 ? nls_lin::lin_split(a, cfg, (hipStream_t)stream) : nls_lin::lin_gemm(a, cfg, (hipStream_t)stream);

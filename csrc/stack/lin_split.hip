@@ -204,6 +204,9 @@ int split_t(LinArgs& a, hipStream_t st) {
 }
 
 int lin_split(LinArgs& a, int cfg, hipStream_t st) {
+  if (cfg == 4)                                      // (lists in tiles of 256 rows do not fit the 128 of the tile it runs on)
+    for (int i = 0; i < a.nseg; ++i)
+      if (a.s[i].rows) return -1;
   switch (cfg) {
     case 0: case 5: case 12: return split_t<4, 1, 4, 4>(a, st);
     case 1: case 8: case 9: case 10: return split_t<4, 2, 4, 4>(a, st);

@@ -249,6 +249,8 @@ class LinLaunch:
             bm = self.plan.bm(M)
             if bm == 16:
                 return False, 1, (4 if self._tiles(16, 16, M) >= 1536 else 8), 1
+            if bm == 256:                 # (refused in 32 bits, whose tiles have up to 128 rows)
+                return True, 7
             if self.f32:
                 return True, min((0, 1) if bm == 64 else (2,), key=lambda c: self.split_us(c, M))
             if bm == 64:
@@ -256,8 +258,6 @@ class LinLaunch:
                 # and 2048 x 512 35 / 48; 8 of 30, 3072 x 2048 22.5 / 25.9; 32 of 30, 4096 x 1536 86 / 94; at 3072 inputs 24.2 / 23.6, from there
                 # on 8 x 4096 x 6144 95 / 79, 8 x 6144 x 4096 79 / 77
                 return True, 0 if self.segs[0].w.K < 3072 else self.balanced(M)
-            if bm == 256:
-                return True, 7
             return True, (3 if self._tiles(256, 128, M) >= 224 else 2)
         n16, n64 = self._tiles(16, 16, M), self._tiles(64, 64, M)
         ns = max(s.w.nsub for s in self.segs)

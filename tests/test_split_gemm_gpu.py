@@ -77,3 +77,19 @@ def test_routed_rows(K, T):
     sel = plan.sel.cpu().long()
     want = torch.stack([w[e].double() @ x[i // 2].double() for i, e in enumerate(sel.tolist())])
     assert ((y.cpu().double() - want).norm() / want.norm()).item() < 2e-6
+
+
+def test_lists_of_256_rows(K):
+    """Tiles of a list that are taller than any 32-bit one are refused, by the launch's own choice and as a config."""
+    T, d, n, E = 700, 320, 200, 4
+    plan = K.MoePlan(T, E, 2, 1, 1, 1.0, "cuda", tall=True)
+    assert plan.bm(T) == 256
+    plan.run(torch.randn(T, E, device="cuda"), T, st())
+    y = torch.full((2 * T, n), 7.0, device="cuda")
+    L = K.LinLaunch([K.Seg(K.PackedLinear(torch.randn(E, n, d), True, "cuda"), torch.zeros(T, K.act_ld(d), device="cuda"), y, routed=(plan.rows, 2))], plan)
+    for cfg in (None, 4):
+        if cfg is not None:
+            L._cfg[T] = (True, cfg), 1
+        with pytest.raises(RuntimeError):
+            L.run(T, st())
+    assert (y == 7).all()
