@@ -7,7 +7,7 @@
 // A wave owns RT tiles of 16 weight rows, whose sub-tiles it loads straight into registers (they are in fragment order, nobody shares them) and
 // splits there. The activation rows are shared: a stage of them (BM rows x 32 values) is loaded into registers two stages ahead, split once
 // per workgroup and written to LDS as fragments. Both operands take a lane's eight k from the two f32 sub-tiles of a step (4 g .. + 3 of each).
-// A tile whose sums are not all finite is computed again with the f32 MFMA: an infinite operand has no parts.
+// Sums that are not finite are computed again with the f32 MFMA, the wave's others stay: an infinite operand has no parts.
 //
 // Against 64 bits 900 x 20096 x 2048 is off by 7.0e-7 of its norm (f32 MFMAs 8.1e-7), 1500 x 4096 x 17408 by 2.15e-6 (2.36e-6): six products
 // of 32 inputs are 6 K / 32 roundings of a sum, where the f32 MFMA rounds at each input. 1500 x 35888 x 4096 runs at 217 TFLOP/s (f32 MFMAs 128),
@@ -182,7 +182,9 @@ __global__ __launch_bounds__(64 * NWV, WPE) void lin_split_kernel(LinArgs a, int
       for (int q = 0; q < RT; ++q) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < 2 * nst; ++k) v = L::mma(ld16(wp[q] + (size_t)k * 1024), ld16(x + k * L::KS), v);
-        acc[q][i] = v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (!(fabsf(acc[q][i][e]) < __builtin_inff())) acc[q][i][e] = v[e];
       }
     }
   lin_epilogue<float>(S, t, acc, t.n0 + 16 * RT * wave + 4 * g, r);

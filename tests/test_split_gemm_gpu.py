@@ -93,3 +93,15 @@ def test_lists_of_256_rows(K):
         with pytest.raises(RuntimeError):
             L.run(T, st())
     assert (y == 7).all()
+
+
+@pytest.mark.parametrize("cfg", [0, 1, 2])
+def test_rows_beside_values_without_parts(K, cfg):
+    """Sums of finite rows and columns have the same bits whatever the others of their tile hold."""
+    g = torch.Generator().manual_seed(2)
+    x, w = torch.randn(140, 160, generator=g), torch.randn(140, 160, generator=g)
+    plain = launch(K, x.cuda(), w.cuda(), cfg)
+    x[3, 7], x[70, 9], w[20, 5], w[100, 2] = float("inf"), float("nan"), float("-inf"), 3.4e38
+    got = launch(K, x.cuda(), w.cuda(), cfg)
+    rows, cols = [r for r in range(140) if r not in (3, 70)], [c for c in range(140) if c not in (20, 100)]
+    assert torch.equal(got[rows][:, cols], plain[rows][:, cols]) and not got[3, cols].isfinite().any()
