@@ -7,7 +7,8 @@
 // A wave owns RT tiles of 16 weight rows, whose sub-tiles it loads straight into registers (they are in fragment order, nobody shares them) and
 // splits there. The activation rows are shared: a stage of them (BM rows x 32 values) is loaded into registers two stages ahead, split once
 // per workgroup and written to LDS as fragments. Both operands take a lane's eight k from the two f32 sub-tiles of a step (4 g .. + 3 of each).
-// Sums that are not finite are computed again with the f32 MFMA, the wave's others stay: an infinite operand has no parts.
+// Sums that are not finite, and those below 2^-80, are computed again with the f32 MFMA, the wave's others stay: an infinite operand has no parts,
+// and rows of operands below 2^-110 have fewer digits in theirs (beside operands up to 2^20 their sums are such).
 //
 // Against 64 bits 900 x 20096 x 2048 is off by 7.0e-7 of its norm (f32 MFMAs 8.1e-7), 1500 x 4096 x 17408 by 2.15e-6 (2.36e-6): six products
 // of 32 inputs are 6 K / 32 roundings of a sum, where the f32 MFMA rounds at each input. 1500 x 35888 x 4096 runs at 217 TFLOP/s (f32 MFMAs 128),
@@ -50,6 +51,13 @@ DEVI Parts split8(const u32x4& u, const u32x4& v) {
     p.l[i] = pk_bf16(a, b);
   }
   return p;
+}
+
+// Whether a sum is computed again with the f32 MFMA (a zero stays: rows of zeros are common). In integers, which leaves no branch: with one the
+// first sum of a block was compiled to the value it had.
+DEVI bool again(float v) {
+  const uint32_t m = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+  return (m >= 0x7f800000u) | (m - 1 < 0x17800000u - 1);       // inf and NaN, below 2^-80
 }
 
 template <int NWV, int RT, int MT, int WPE>
@@ -171,7 +179,7 @@ __global__ __launch_bounds__(64 * NWV, WPE) void lin_split_kernel(LinArgs a, int
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) odd |= !(fabsf(acc[q][i][e]) < __builtin_inff());
+      for (int e = 0; e < 4; ++e) odd |= again(acc[q][i][e]);
   if (__any(odd))
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -182,9 +190,9 @@ __global__ __launch_bounds__(64 * NWV, WPE) void lin_split_kernel(LinArgs a, int
       for (int q = 0; q < RT; ++q) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         for (int k = 0; k < 2 * nst; ++k) v = L::mma(ld16(wp[q] + (size_t)k * 1024), ld16(x + k * L::KS), v);
+        asm volatile("" : "+v"(acc[q][i]));          // (looked at anew: kept from above, the answers would not fit beside the rest)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (!(fabsf(acc[q][i][e]) < __builtin_inff())) acc[q][i][e] = v[e];
+        for (int e = 0; e < 4; ++e) acc[q][i][e] = again(acc[q][i][e]) ? v[e] : acc[q][i][e];
       }
     }
   lin_epilogue<float>(S, t, acc, t.n0 + 16 * RT * wave + 4 * g, r);

@@ -105,3 +105,16 @@ def test_rows_beside_values_without_parts(K, cfg):
     got = launch(K, x.cuda(), w.cuda(), cfg)
     rows, cols = [r for r in range(140) if r not in (3, 70)], [c for c in range(140) if c not in (20, 100)]
     assert torch.equal(got[rows][:, cols], plain[rows][:, cols]) and not got[3, cols].isfinite().any()
+
+
+@pytest.mark.parametrize("cfg", [0, 1, 2])
+@pytest.mark.parametrize("ex,ew", [(-100, 0), (-111, 0), (-118, 5), (-123, 0), (0, -119), (-60, -55)])
+def test_small_values(K, cfg, ex, ew):
+    """Operands, themselves normal numbers, whose parts or whose parts' products would lie below those: the bound of 32-bit products. Few
+    inputs of one sign, so that an operand's missing digits show and no sum passes below the normal numbers itself."""
+    g = torch.Generator().manual_seed(-ex)
+    x, w = ((torch.rand(70, 4, generator=g) + 1) * 2.0 ** e for e in (ex, ew))
+    x[1] = 0
+    got = launch(K, x.cuda(), w.cuda(), cfg).double()
+    want, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    assert ((got - want).abs() <= 2.0 ** -24 * 12 * mag).all() and not got[1].any()
