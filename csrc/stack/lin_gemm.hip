@@ -1,6 +1,7 @@
-// Tiled MFMA GEMM on packed bf16 weights (prompt chunks, large decode batches, routed experts with many rows).
+// Tiled MFMA GEMM on packed bf16 weights (prompt chunks, large decode batches, routed experts with many rows), and on f32 weights where a CU has
+// one workgroup (beyond that lin_split.hip is the faster one).
 //
-// BN weight rows x BM activation rows per workgroup; K advances two 1 KiB sub-tiles (64 values) per
+// BN weight rows x BM activation rows per workgroup; K advances two 1 KiB sub-tiles (64 bf16 / 32 f32 values) per
 // step. Both operands arrive by LDS-DMA into NST-deep rings: weight sub-tiles verbatim (already in fragment order),
 // activation sub-tiles with the 16-byte chunks of a row permuted on the DMA source (chunk ^ swz(row)), so every
 // fragment is one conflict-free ds_read_b128. One raw barrier per step with a counted vmcnt leaves the later stages
@@ -46,11 +47,10 @@ struct LG {
 // 198, 195, 202; 255, 306, 323.
 enum Fetch : int { KEEP, STREAM, BY_TILE };
 
-template <int BN, int BM, int WN, int WM, int NST, int FETCH>
+template <typename T, int BN, int BM, int WN, int WM, int NST, int FETCH>
 __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int ntot) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lglds[];
   typedef LG<BN, BM, WN, WM, NST> G;
-  typedef __bf16 T;
   typedef LT<T> L;
   constexpr int NW = G::NW, NX = G::NX, NTW = G::NTW, MTW = G::MTW;
   int listed = ntot, gap = 0;
@@ -153,22 +153,22 @@ __global__ __launch_bounds__(64 * WN * WM) void lin_gemm_kernel(LinArgs a, int n
   lin_epilogue<T>(S, t, acc, t.n0 + 16 * wn * NTW + 4 * g, 16 * wm * MTW + r);
 }
 
-template <int BN, int BM, int WN, int WM, int NST, int FETCH>
+template <typename T, int BN, int BM, int WN, int WM, int NST, int FETCH>
 int gemm_f(const LinArgs& a, int n, hipStream_t st) {
   typedef LG<BN, BM, WN, WM, NST> G;
   static bool attr = false;
   if (!attr) {
-    if (hipFuncSetAttribute((const void*)lin_gemm_kernel<BN, BM, WN, WM, NST, FETCH>,
+    if (hipFuncSetAttribute((const void*)lin_gemm_kernel<T, BN, BM, WN, WM, NST, FETCH>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((lin_gemm_kernel<BN, BM, WN, WM, NST, FETCH>), dim3((n + 7) / 8 * 8), dim3(64 * G::NWV), G::LDS, st,
+  hipLaunchKernelGGL((lin_gemm_kernel<T, BN, BM, WN, WM, NST, FETCH>), dim3((n + 7) / 8 * 8), dim3(64 * G::NWV), G::LDS, st,
                      a, n);
   return (int)hipGetLastError();
 }
 
-template <int BN, int BM, int WN, int WM, int NST>
+template <typename T, int BN, int BM, int WN, int WM, int NST>
 int gemm_t(LinArgs& a, hipStream_t st) {
   const int n = lin_count(a, BN, BM);
   if (n < 1) return -1;
@@ -177,25 +177,25 @@ int gemm_t(LinArgs& a, hipStream_t st) {
     once |= a.s[i].rows || a.s[i].M <= BM;
     several |= a.s[i].rows || a.s[i].M > BM;
   }
-  if (!once) return gemm_f<BN, BM, WN, WM, NST, KEEP>(a, n, st);
-  return several ? gemm_f<BN, BM, WN, WM, NST, BY_TILE>(a, n, st) : gemm_f<BN, BM, WN, WM, NST, STREAM>(a, n, st);
+  if (!once) return gemm_f<T, BN, BM, WN, WM, NST, KEEP>(a, n, st);
+  return several ? gemm_f<T, BN, BM, WN, WM, NST, BY_TILE>(a, n, st) : gemm_f<T, BN, BM, WN, WM, NST, STREAM>(a, n, st);
 }
 
 int lin_gemm(LinArgs& a, int cfg, hipStream_t st) {
   switch (cfg) {
-    case 0: return gemm_t<64, 64, 2, 2, 3>(a, st);
-    case 1: return gemm_t<128, 64, 4, 1, 3>(a, st);
-    case 2: return gemm_t<128, 128, 2, 2, 2>(a, st);
-    case 3: return gemm_t<256, 128, 4, 2, 3>(a, st);
-    case 4: return gemm_t<256, 256, 4, 2, 2>(a, st);
-    case 5: return gemm_t<64, 64, 2, 2, 8>(a, st);
-    case 6: return gemm_t<192, 128, 4, 2, 3>(a, st);
+    case 0: return gemm_t<__bf16, 64, 64, 2, 2, 3>(a, st);
+    case 1: return gemm_t<__bf16, 128, 64, 4, 1, 3>(a, st);
+    case 2: return gemm_t<__bf16, 128, 128, 2, 2, 2>(a, st);
+    case 3: return gemm_t<__bf16, 256, 128, 4, 2, 3>(a, st);
+    case 4: return gemm_t<__bf16, 256, 256, 4, 2, 2>(a, st);
+    case 5: return gemm_t<__bf16, 64, 64, 2, 2, 8>(a, st);
+    case 6: return gemm_t<__bf16, 192, 128, 4, 2, 3>(a, st);
     case 7: return lin_phased(a, st);
-    case 8: return gemm_t<96, 64, 2, 2, 4>(a, st);
-    case 9: return gemm_t<160, 64, 2, 2, 4>(a, st);
-    case 10: return gemm_t<128, 64, 2, 2, 4>(a, st);
-    case 11: return gemm_t<96, 128, 2, 2, 4>(a, st);
-    case 12: return gemm_t<64, 32, 2, 1, 8>(a, st);
+    case 8: return gemm_t<__bf16, 96, 64, 2, 2, 4>(a, st);
+    case 9: return gemm_t<__bf16, 160, 64, 2, 2, 4>(a, st);
+    case 10: return gemm_t<__bf16, 128, 64, 2, 2, 4>(a, st);
+    case 11: return gemm_t<__bf16, 96, 128, 2, 2, 4>(a, st);
+    case 12: return gemm_t<__bf16, 64, 32, 2, 1, 8>(a, st);
     case 13: return lin_thin(a, st);
   }
   return -1;
@@ -209,10 +209,13 @@ extern "C" {
 // own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
 // 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128, 12 = 64 x 32 with 8 stages,
 // 13 = 64 x 128 straight from memory (K up to 128, no routed rows).
-// f32: 0, 1 and 2; the others run on one of these, but for 7 and 13 and for routed rows on 4, which are refused.
+// f32: 5 = 64 x 64 on the f32 MFMA in three stages, 0, 1 and 2 in bf16 parts; the others run on one of these, but for 7 and 13 and for routed
+// rows on 4, which are refused.
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
-  return f32 ? nls_lin::lin_split(a, cfg, (hipStream_t)stream) : nls_lin::lin_gemm(a, cfg, (hipStream_t)stream);
+  using namespace nls_lin;
+  hipStream_t st = (hipStream_t)stream;
+  return !f32 ? lin_gemm(a, cfg, st) : cfg == 5 ? gemm_t<float, 64, 64, 2, 2, 3>(a, st) : lin_split(a, cfg, st);
 }
 
 }  // extern "C"

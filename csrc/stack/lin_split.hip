@@ -218,7 +218,7 @@ int lin_split(LinArgs& a, int cfg, hipStream_t st) {
     for (int i = 0; i < a.nseg; ++i)
       if (a.s[i].rows) return -1;
   switch (cfg) {
-    case 0: case 5: case 12: return split_t<4, 1, 4, 4>(a, st);
+    case 0: case 12: return split_t<4, 1, 4, 4>(a, st);
     case 1: case 8: case 9: case 10: return split_t<4, 2, 4, 4>(a, st);
     case 2: case 3: case 4: case 6: case 11: return split_t<4, 2, 8, 3>(a, st);
   }

@@ -199,12 +199,14 @@ THIN = 13                # config of products of up to 128 inputs straight from 
 # against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 297 against 269 (3).
 GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 0.47, 0.72),
              1: (512, 0.5, 0.63), 0: (1024, 0.45, 0.55)}
-# 32-bit operands (lin_split.hip): microseconds of 32 input columns on a CU that runs one workgroup of a tile, more for each further one, and how
-# many run together. The measured times of 12 shapes x 7 row counts x 3 tiles x 1 to 8 splits lie 8 % around it (a launch: 8 us and the slabs' sum
-# more), the tile and splits it picks 2 % above the best. 64 x 64 / 128 x 64 / 128 x 128, us: 900 x 20096 x 2048 467 / 432 / 394 (f32 MFMAs 658),
-# 1500 x 35888 x 4096 2621 / 2223 / 2020 (3440), 130 x 4096 x 4096 112 / 142 / 211 and in four splits of the first 63; 900 x 2048 x 9728 323 / 364 / 504 and in
-# four splits of the last 206 (333).
-SPLIT_US = {0: (0.72, 0.32, 6), 1: (1.01, 0.54, 4), 2: (1.64, 0.94, 3)}
+# 32-bit operands: microseconds of 32 input columns on a CU that runs one workgroup of a tile, more for each further one, and how many run
+# together; 0 to 2 in bf16 parts (lin_split.hip), 5 on the f32 MFMA (1.3 us more a launch). One workgroup to a CU splits and multiplies in turn, and
+# the f32 MFMA is the faster one: 64 x 64, parts / f32, us: 65 x 4096 x 12288 356 / 226, 64 x 16384 x 4096 130 / 88, 256 x 2048 x 8704 249 / 162, in eight
+# splits 64 x 2048 x 8704 41 / 28.6; with two it loses (128 x 10240 x 4096 138 / 147), with four it takes 1.4 times as long. Up to 128 inputs
+# parts win (64 x 2048 x 128 6.9 / 7.6). 22 shapes x 16 row counts x 4 tiles x 1 to 8 splits lie 6 % around it, the tile it picks is 0.1 % behind the
+# fastest on average, tile and splits 1.2 %. 64 x 64 / 128 x 64 / 128 x 128 in parts, us: 900 x 20096 x 2048 467 / 432 / 394 (f32 658), 1500 x 35888 x 4096
+# 2621 / 2223 / 2020 (3440).
+SPLIT_US = {0: (0.78, 0.30, 6), 1: (1.09, 0.49, 4), 2: (1.66, 0.87, 3), 5: (0.57, 0.57, 3)}
 
 # Launches of 129 to 512 rows that do not fill the chip with 256 x 128 tiles (weight rows x rows of a round by its time): 300 x 4096 x 4096 28 us
 # on 96 x 64, 34 on 64 x 64, 46 on 192 x 128; 200 x 6144 x 4096 27, 32, 49; 160 x 10240 x 4096 45, 37, 47; 400 x 6144 x 2048 27, 29, 29, 28 on 96 x 128.
@@ -252,7 +254,7 @@ class LinLaunch:
             if bm == 256:                 # (refused in 32 bits, whose tiles have up to 128 rows)
                 return True, 7
             if self.f32:
-                return True, min((0, 1) if bm == 64 else (2,), key=lambda c: self.split_us(c, M))
+                return True, min((5, 0, 1) if bm == 64 else (2,), key=lambda c: self.split_us(c, M))
             if bm == 64:
                 # short products are over before the deeper tiles' stages pay: 64 x 64 / chosen by rounds, us: 64 experts of 30 rows, 512 x 2048 28 / 41
                 # and 2048 x 512 35 / 48; 8 of 30, 3072 x 2048 22.5 / 25.9; 32 of 30, 4096 x 1536 86 / 94; at 3072 inputs 24.2 / 23.6, from there
@@ -275,7 +277,7 @@ class LinLaunch:
             return self.few_rows(M, n64)
         if M <= 64:
             if n64 >= 250:
-                return True, 0
+                return True, min((5, 0), key=lambda c: self.split_us(c, M)) if self.f32 else 0
             return False, 2, (4 if ns <= 16 else 8), (2 if M > 32 or n16 >= 640 else 1)
         if ns <= 4:                       # a step or two of K: all epilogue. 64 x 64 / 128 x 64 / straight from memory, us: 600 x 2048 x 64
             # 7.2 / 8.0 / 7.8, 2000 12.3 / 11.0 / 10.9, 4000 19.0 / 18.0 / 16.9; 4000 x 4096 x 64 25.4 / 23.5 / 19.2, 600 x 4096 x 128 7.8 / 7.9 / 8.7
@@ -336,10 +338,11 @@ class LinLaunch:
         return True, self.balanced(M)
 
     def split_us(self, c: int, M: int, ks: int = 1) -> float:
-        """About the microseconds of an f32 launch on tile c in ks splits of K (without the 8 us that any takes)."""
+        """About the microseconds of an f32 launch on tile c in ks splits of K (without the 5 us that any takes)."""
         one, more, together = SPLIT_US[c]
         full, rest = divmod(-(-self._tiles(*GEMM_TILES[c], M) * ks // 256), together)
-        return max(s.w.nsub for s in self.segs) / (2 * ks) * (full * (one + more * (together - 1)) + (one + more * (rest - 1) if rest else 0))
+        step = full * (one + more * (together - 1)) + (one + more * (rest - 1) if rest else 0)
+        return max(s.w.nsub for s in self.segs) / (2 * ks) * step + (1.3 if c == 5 else 0)
 
     def split_config(self, M: int):
         """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the

@@ -118,3 +118,25 @@ def test_small_values(K, cfg, ex, ew):
     got = launch(K, x.cuda(), w.cuda(), cfg).double()
     want, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     assert ((got - want).abs() <= 2.0 ** -24 * 12 * mag).all() and not got[1].any()
+
+
+@pytest.mark.parametrize("cfg", [0, 1, 5])
+def test_routed_rows_on_each_tile(K, cfg):
+    """Lists in tiles of 64 rows on every 32-bit tile that takes them: lists of one tile, of two and of few rows."""
+    T, d, n, E = 130, 330, 200, 4
+    g = torch.Generator().manual_seed(3)
+    x, z, w = torch.randn(T, d, generator=g), torch.randn(T, E, generator=g), torch.randn(E, n, d, generator=g) * d ** -0.5
+    z[:, 1] += 2.0
+    plan = K.MoePlan(T, E, 2, 1, 1, 1.0, "cuda")
+    assert plan.bm(T) == 64
+    plan.run(z.cuda(), T, st())
+    xa = torch.zeros(T, K.act_ld(d), device="cuda")
+    xa[:, :d] = x
+    y = torch.full((2 * T + 1, n), 7.0, device="cuda")
+    L = K.LinLaunch([K.Seg(K.PackedLinear(w, True, "cuda"), xa, y, routed=(plan.rows, 2))], plan)
+    L._cfg[T] = (True, cfg), 1
+    L.run(T, st())
+    sel = plan.sel.cpu().long()
+    assert sel.bincount(minlength=E).max() > 64
+    want = torch.stack([w[e].double() @ x[i // 2].double() for i, e in enumerate(sel.tolist())])
+    assert ((y[:-1].cpu().double() - want).norm() / want.norm()).item() < 2e-6 and (y[-1] == 7).all()

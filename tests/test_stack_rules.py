@@ -67,3 +67,13 @@ def test_short_expert_products():
         L.plan, L.segs[0].s.rows = S.MoePlan(120, 8, 2, 1, 1, 1.0, "cpu"), 1
         L.segs[0].w.groups = 8
         assert L.plan.bm(120) == 64 and L.config(120) == (True, want), (N, Kd)
+
+
+def test_tiles_of_32_bits():
+    """One workgroup to a CU at most: the f32 MFMA, unless the inputs are few; more of them: bf16 parts. Splits of K count as workgroups."""
+    for N, Kd, M in ((4096, 12288, 65), (4096, 12288, 256), (16384, 4096, 64), (2048, 512, 512), (1030, 2090, 900)):
+        assert launch(N, Kd, True).config(M) == (True, 5)
+    for N, Kd, M in ((4096, 12288, 257), (16384, 4096, 65), (35888, 4096, 33), (2048, 64, 200), (2048, 128, 200)):
+        assert launch(N, Kd, True).config(M)[1] in (0, 1, 2)
+    assert launch(2048, 8704, True, 4096, 8, 512).choice(64) == ((True, 5), 8)
+    assert launch(2048, 8704, True, 8192, 8, 512).choice(900)[0][1] in (0, 1, 2)
