@@ -348,10 +348,13 @@ class LinLaunch:
         """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the
         five of 192 x 128 that are chosen, 25.5 in two of 128 x 64; 41, 34 and 32 with the launch that adds the slabs)."""
         n16 = self._tiles(16, 16, M)
-        # 64 x 32 tiles, one to a CU. 16 rows, streaming / these, us: 4096 x 17408 27.5 / 25.6, 4096 x 8192 15.3 / 14.6, 4096 x 4096 9.1 / 9.6, 2048 x 8704 9.9
-        # / 10.3; 24 rows 27.5 / 26.8, 18.1 / 15.8, 11.5 / 10.6, 12.7 / 12.0, with half the slabs at 4096 columns
-        if not self.f32 and (16 < M <= 32 or 12 < M <= 16 and n16 >= 256 and self.segs[0].w.K >= 8192):
-            return (True, 12), -(-256 // self._tiles(64, 32, M))
+        # 64 x 32 tiles, up to one to a CU (a few more take a second round: 24 x 2560 x 4096 8.9 us in six splits, 12.9 in seven). 16 rows, streaming /
+        # these, us: 4096 x 17408 27.5 / 25.6, 4096 x 8192 15.3 / 14.6, 4096 x 4096 9.1 / 9.6, 2048 x 8704 9.9 / 10.3; 24 rows 28.6 / 25.5, 19.3 / 15.5, 13.5 / 10.6,
+        # 12.1 / 10.8; 5120 x 4096 15.6 / 11.8, 2560 x 4096 9.7 / 8.9, 640 x 6144 7.9 / 7.8. Short launches end before the ring's first stages are in:
+        # 24 x 2048 x 2048 6.2 / 7.0, 1024 x 4096 6.8 / 7.2, 3072 x 2048 7.2 / 7.7. 14 x 7 layers x 17, 24 and 32 rows: 0.914 of streaming's time on average.
+        Kd, n32 = self.segs[0].w.K, self._tiles(64, 32, M)
+        if not self.f32 and (16 < M <= 32 and (Kd >= 6144 or n32 >= 64 or n32 * Kd >= 48 * 3072) or 12 < M <= 16 and n16 >= 256 and Kd >= 8192):
+            return (True, 12), max(1, 256 // n32)
         if M <= 16:
             rt = 1 if M <= 8 else 2
             return (False, 1, 8, rt), -(-512 * rt // (2 * n16)) if M > 8 else -(-512 // n16)

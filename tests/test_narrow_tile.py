@@ -47,3 +47,13 @@ def test_edges(M):
             K._check(K.lib().nls_lin_gemm(ctypes.byref(a), 0, 12, torch.cuda.current_stream().cuda_stream), "gemm")
             got = y[:2 * M].view(2, M, N)[:ks].sum(0).cpu().double()
             assert ((got - want).abs() <= bound + 2.0 ** -23 * want.abs()).all() and (y[-1] == 9).all(), (steps, ks)
+
+
+def test_splits_stay_in_one_round():
+    """Splits of the tile give each CU one workgroup at most, at widths that 256 is no multiple of too; short launches stream."""
+    for N in (640, 2560, 3072, 4096, 5120, 6144, 10240, 17000):
+        for M in (16, 17, 32):
+            c, ks = launch(N, 8192, 8).choice(M)
+            assert c[0] == (M > 16 or N >= 4096) and (not c[0] or ks == 1 or ks * -(-N // 64) <= 256)
+    for N, Kd in ((2048, 2048), (1024, 4096), (3072, 2048), (96, 4096)):
+        assert launch(N, Kd, 8).choice(24)[0][0] is False
