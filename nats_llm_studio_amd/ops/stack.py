@@ -656,15 +656,19 @@ def segments_us(kind: str, tokens: int, wgs: float, nseg: int) -> float:
 @lru_cache(maxsize=1024)
 def segments(kind: str, T: int, tokens: int, wgs: int, most: int) -> int:
     """The fastest number of segments, up to `most`, of a scan over T rows whose runs have at most `tokens`; wgs: workgroups of
-    one run."""
+    one run. Short runs have one: the fit does not see what three launches cost them (100 tokens, us, one / two: gla 49.4 / 56.2, delta 79 / 112; 150
+    tokens, one / three: gla 69 / 59, delta 113 / 126)."""
+    if tokens < (129 if kind == "gla" else 192):
+        return 1
     return min(range(1, max(1, min(-(-tokens // 64), most)) + 1), key=lambda s: segments_us(kind, tokens, wgs * T / tokens, s))
 
 
 def gla_shape(T: int, nruns: int, H: int, V: int, D: int = 64, longest: Optional[int] = None):
     """(segments, groups of 64 value columns per workgroup) of a gla_scan launch; longest: tokens of the longest run, if known.
-    Up to 64 channels two workgroups per CU from segments of 64 tokens and more, unless whole runs already give one (2.7 % behind
-    the fastest count on average; there a CU holds several workgroups). With 65 to 128 channels that rule was 11 % behind, as it
-    does not see a last round that is nearly empty (32 heads of 128 x 128, bf16: 6 runs of 650 tokens 382 us with 3
+    Up to 64 channels two workgroups per CU, unless whole runs already give one: one segment up to 128 tokens (65 tokens, 32 heads of 64 x 128, us, one /
+    two 26.6 / 34.8, 128 tokens 32.2 / 35.7, 150 in one / three 42.0 / 36.2), then as many as there are chunks of 64, since a segment has whole ones (333
+    tokens cut for five 57, for six 42); 0.1 % behind the fastest count on average, no size slower than with T / 64 rounded down. There a CU holds
+    several workgroups. With 65 to 128 channels that rule was 11 % behind, as it does not see a last round that is nearly empty (32 heads of 128 x 128, bf16: 6 runs of 650 tokens 382 us with 3
     segments, 265 with 1; 1 run of 333 tokens 93 us with 5, 63 with 6): the count is the one that segments_us finds fastest."""
     nt = 1 if V <= 64 else 2
     wgs = H * -(-V // (64 * nt))
@@ -672,7 +676,7 @@ def gla_shape(T: int, nruns: int, H: int, V: int, D: int = 64, longest: Optional
     most = min(-(-512 // (wgs * nruns)), 16)             # (what bounds the scratch, too)
     if 64 < D <= 128 and nt == 2:
         return segments("gla", T, longest or -(-T // nruns), wgs, most), nt
-    return 1 if wgs * nruns >= 256 else max(1, min(most, -(-n // 64))), nt
+    return 1 if wgs * nruns >= 256 or n <= 128 else max(1, min(most, -(-n // 64))), nt
 
 
 def gla_scan(q, k, v, a, qscale: float, o, norm, gate, out, state, runs, nruns: int, H: int, D: int, V: int, eps: float, shape,
@@ -751,8 +755,9 @@ def delta_conv(z, w, y, fac, state, runs, tok_seq, T: int, nruns: int, H: int, G
 
 def delta_shape(T: int, nruns: int, H: int, D: int, V: int, longest: Optional[int] = None):
     """(segments, groups of 64 value columns per workgroup) of a delta_scan launch, as gla_shape. Segments cost a second pass over
-    the tokens with D more columns: up to 64 channels they start where whole runs fill less than half the CUs, and stay longer
-    (at 16 heads of 128 x 128 that rule was 5.5 % behind the fastest count on average: 6 runs of 650 tokens 517 us with 3
+    the tokens with D more columns: up to 64 channels they start where whole runs fill less than half the CUs, up to one workgroup per CU (16 heads of
+    64 x 128, us: 128 tokens in one / two 69 / 70, 150 in one / three 93 / 72, 333 in one / two / six 183 / 157 / 109; 0.7 % behind the fastest count on
+    average). With 65 to 128 channels that rule was 5.5 % behind (16 heads of 128 x 128: 6 runs of 650 tokens 517 us with 3
     segments, 444 with the 1 that segments_us finds)."""
     nt = 1 if V <= 64 else 2
     wgs = H * -(-V // (64 * nt))
@@ -760,7 +765,7 @@ def delta_shape(T: int, nruns: int, H: int, D: int, V: int, longest: Optional[in
     most = min(-(-256 // (wgs * nruns)), 16)             # (what bounds the scratch, too)
     if 64 < D <= 128 and nt == 2:
         return segments("delta", T, longest or -(-T // nruns), wgs, most), nt
-    return 1 if wgs * nruns >= 128 else max(1, min(most, n // 128)), nt
+    return 1 if wgs * nruns >= 128 or n <= 128 else max(1, min(most, -(-n // 64))), nt
 
 
 def delta_scan(q, k, v, fac, beta, a, o, norm, gate, out, state, runs, nruns: int, H: int, G: int, D: int, V: int, eps: float,

@@ -23,3 +23,14 @@ def test_counts(kind, D, V, T, n, longest, H):
         one = H * -(-V // 128) * T / tokens
         us = [K.segments_us(kind, tokens, one, s) for s in range(1, nseg + 1)]
         assert us[-1] == min(us)
+
+
+@pytest.mark.parametrize("H, D, V", [(32, 64, 128), (16, 64, 64), (8, 32, 64), (16, 128, 128), (32, 128, 128), (16, 96, 256), (8, 256, 128)])
+def test_short_runs_are_not_cut(H, D, V):
+    """Segments cost three launches: none up to 128 tokens, however few runs; from 256 on one run of few heads has as many as chunks, or as
+    the model of whole rounds says."""
+    for n in (64, 65, 100, 128):
+        for runs in (1, 2):
+            assert K.gla_shape(n * runs, runs, H, V, D, n)[0] == K.delta_shape(n * runs, runs, H, D, V, n)[0] == 1
+    assert K.gla_shape(256, 1, H, V, D, 256)[0] == (4 if D <= 64 or D > 128 else K.segments("gla", 256, 256, H * -(-V // 128), 16))
+    assert K.gla_shape(256, 1, H, V, D, 256)[0] >= 3
