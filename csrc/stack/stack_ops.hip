@@ -473,7 +473,9 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(AttnRows p) {
 // of 4, 8, 16 .. 256 columns): no norm of the whole rows, but an RMS norm without weights of each rotated head on its own, whose
 // columns are lanes beside each other. Weights, angles and the first values are asked for with the row, ahead of the sums: behind them (and
 // behind the stores, which they might be written by for all that is known) each group of columns waited for its own: 3900 rows of
-// 32 + 8 heads of 128 60.6 -> 47.5 us with weights, 56.2 -> 36.5 without, 61.0 -> 30.6 with normed heads, 400 rows 8.6 -> 7.8, 16 rows 4.4 -> 4.2.
+// 32 + 8 heads of 128 60.8 -> 32.4 us with weights, 55.9 -> 30.7 without, 61.0 -> 30.7 with normed heads (32 bits 56.1 -> 37.1, 51.4 -> 34.8, 55.1 -> 39.4),
+// 400 rows 8.9 -> 7.2, 16 rows 4.4 -> 4.2. Loads for groups past the row, clamped to its last, cost as much as others: with them 3900 rows of 16 + 4
+// heads in 32 bits took 31.1, behind each other 26.5, without 20.4.
 template <typename T, int NV, int NTH, bool HN>
 __global__ __launch_bounds__(NTH) void attn_rows4_kernel(AttnRows p) {
   __shared__ float sh[2][NTH / 64];
@@ -492,6 +494,8 @@ __global__ __launch_bounds__(NTH) void attn_rows4_kernel(AttnRows p) {
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int e = threadIdx.x + j * NTH;
+    x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (j * NTH >= n) continue;                       // (uniform: no loads for groups that no thread has)
     const int ec = min(e, n - 1), i = ec < nq ? ec : ec - nq, c = 4 * (i - head(i) * D4);
     x[j] = *reinterpret_cast<const f32x4*>(ec < nq ? q + 4 * ec : k + 4 * i);
     if (AHEAD && weights) w[j] = *reinterpret_cast<const f32x4*>((ec < nq ? wq : wk) + 4 * i);
