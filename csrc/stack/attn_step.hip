@@ -3,9 +3,10 @@
 // Neither reads what the other writes. The recurrence streams its states (64 tokens of 32 heads of 64 x 128: 134 MB read and written),
 // the attention of few hundred keys is one chain of dependent loads, so each leaves idle what the other needs. Graph launches, bf16, 32
 // heads of 128 over 8 beside 32 states of 64 x 128, us, one behind the other / together: 1 token behind 90 keys 12.1 / 7.1,
-// behind 1500 16.4 / 11.0; 16 tokens 17.5 / 11.5, 47.0 / 39.6; 64 tokens 40.0 / 35.1, 127 / 111 (behind 20 keys 31.6 / 32.9, the only
-// loss of 90 sizes). The attention takes four waves and gives up the prefetch of the next keys: that leaves registers for
-// three workgroups on a CU, of which two would not keep the states' loads in flight.
+// behind 1500 16.4 / 11.0; with cold states and keys 16 tokens behind 90 and 1000 20 / 14 and 37 / 32, 64 tokens 43 / 37 and 101 / 86, 300 tokens 159 / 149 and
+// 424 / 369. Of 375 sizes of 1 to 300 tokens behind 20 to 3000 keys 0.80 of the time on average; slower are 128 tokens and more behind 20 keys (62 /
+// 64 to 142 / 146: three of four waves have no keys) and two sizes behind 3000 (2 %). The attention takes four waves and gives up the prefetch of
+// the next keys: that leaves registers for three workgroups on a CU, of which two would not keep the states' loads in flight.
 // In 32 bits the plain attention keeps all its registers, a CU holds one workgroup: that pays up to two rounds of states (3 tokens behind 330
 // keys 24.9 / 20.1, 16 tokens 30.6 / 23.4; 32 tokens, 1024 states, 45.1 / 49.4).
 #include "../kernels/attn_decode.h"
@@ -92,19 +93,19 @@ int plain(nls_plain::PA a, int T, int H, const Scan& p, const StepOut& y, hipStr
 
 extern "C" {
 
-// nls_gqa_attn (no window) and nls_gla_step of the same T rows, each a run of one token, in one launch.
+// nls_gqa_attn (no window) and nls_gla_step (with a norm) of the same T rows, each a run of one token, in one launch.
 // Dp 64 or 128 (32-bit: up to 256, ns and its scratch unused); at most 16 rows of a state per thread (step_rpt).
 int nls_attn_step(const void* aq, long ldaq, const void* ak, const void* av, const int* bt, int bts, int bs, const int* tok_seq,
                   const int* ctx_len, int T, int AH, int AG, int Dp, float scale, const float* agate, long ldag, void* aout,
                   long ldaout, int sink, int ns, float* part_o, float* part_ml, int* cnt, const void* q, const void* k, const void* v, long ld, const float* a, long lda,
                   const void* low, const void* a2, const float* a2b, int rank, float ia, float qscale, float* state, long sstride,
-                  const int* runs, const float* norm, const void* gate, long ldg, void* out, long ldout, float* o, long ldo, int H,
+                  const int* runs, const float* norm, const void* gate, long ldg, void* out, long ldout, int H,
                   int D, int V, float eps, int f32, void* stream) {
   using namespace nls_both;
-  if (T < 1 || AG < 1 || AH < 1 || AH % AG || bs < 1 || Dp < 1 || (norm ? !gate || !out : !o)) return -1;
+  if (T < 1 || AG < 1 || AH < 1 || AH % AG || bs < 1 || Dp < 1 || !norm || !gate || !out) return -1;
   if (H < 1 || D < 1 || D > 256 || V < 4 || V > 1024 || (V & 3) || (sstride & 3)) return -1;
   if (!a && (!low || !a2 || !a2b || rank < 1 || ((uintptr_t)low & 15) || ((uintptr_t)a2 & 15) || (ld & 7))) return -1;
-  const Scan p{q, k, v, a, nullptr, o, state, nullptr, nullptr, runs, ld, lda, ldo, sstride, 0, 0, H, D, V, 0, qscale,
+  const Scan p{q, k, v, a, nullptr, nullptr, state, nullptr, nullptr, runs, ld, lda, 0, sstride, 0, 0, H, D, V, 0, qscale,
                low, a2, a2b, rank, ia};
   const StepOut y{norm, gate, ldg, out, ldout, eps};
   if (f32)

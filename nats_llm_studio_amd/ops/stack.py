@@ -55,7 +55,7 @@ _SIGS = {
     "nls_gla_scan": [P, P, P, L, P, L, F, P, L, P, P, L, P, L, F, P, L, P, I, I, I, I, I, P, P, I, I, P],
     "nls_gla_step": [P, P, P, L, P, L, P, P, P, I, F, F, P, L, P, I, P, P, L, P, L, P, L, I, I, I, F, I, P],
     "nls_attn_step": [P, L, P, P, P, I, I, P, P, I, I, I, I, F, P, L, P, L, I, I, P, P, P, P, P, P, L, P, L, P, P, P, I, F, F, P, L, P, P, P, L, P,
-                      L, P, L, I, I, I, F, I, P],
+                      L, I, I, I, F, I, P],
     "nls_latent_rows": [P, L, I, P, P, L, P, L, I, I, I, P, P, P, P, P, L, I, F, I, P],
     "nls_stack_argmax": [P, L, I, P, I, P],
     "nls_moe_plan": [P, L, I, I, I, I, I, I, I, F, P, P, I, P, P, P, I, P, P],
@@ -713,8 +713,8 @@ def gla_step(q, k, v, a, gate_in, qscale: float, state, runs, nruns: int, norm, 
 
 def attn_step_fits(AH: int, AG: int, Dp: int, mfma: bool, window: int, H: int, D: int, V: int, f32: bool) -> int:
     """The most tokens whose attention and recurrence attn_step takes in one launch where that is the faster way (0: none): any
-    number in bf16, with one exception of 90 sizes 4 to 50 % less than one behind the other; in 32 bits (a workgroup per CU) up to
-    512 states (20 % less; 1024: 5 to 35 % more)."""
+    number in bf16 (1 to 300 tokens behind 20 to 3000 keys 45 % less to 4 % more than one behind the other, 20 % less on average); in 32 bits (a
+    workgroup per CU) up to 512 states (4 % more to 40 % less; 768 14 % less to 20 % more, 1024 up to 33 % more)."""
     if window or V % 4 or V > 1024 or -(-D // (256 // (V // 4))) > 16:
         return 0
     if f32:
@@ -737,7 +737,7 @@ def attn_step(aq, kc, vc, agate, aout, part, ns: int, block_tables, block_size: 
                                q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), _p(a), a.stride(0) if a is not None else 0,
                                _p(lo), _p(a2), _p(b), a2.shape[1] if a2 is not None else 0, ia, qscale, state.data_ptr(),
                                state.stride(0), runs.data_ptr(), norm.data_ptr(), gate.data_ptr(), gate.stride(0), out.data_ptr(),
-                               out.stride(0), None, 0, H, D, V, eps, int(q.dtype == torch.float32), st), "nls_attn_step")
+                               out.stride(0), H, D, V, eps, int(q.dtype == torch.float32), st), "nls_attn_step")
 
 
 # ---------------------------------------------------------------------------

@@ -61,3 +61,38 @@ def test_attn_step(dtype, AH, AG, Dp, H, D, V, ctx):
         sc = (norm.double() * gate[t].double()).view(H, V) / (o * o).mean(1, keepdim=True).add(1e-5).sqrt()
         err = (out[t, :H * V].double().view(H, V) - o * sc).abs()
         assert (err <= e * (m * sc.abs() + (o * sc).abs() * (m * m).mean(1, keepdim=True).sqrt() / (o * o).mean(1, keepdim=True).sqrt())).all(), t
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T", [1, 5])
+def test_given_decays(dtype, T):
+    """Decays per token and channel instead of the low-rank gate input: states and outputs of gla_step, attention of gqa_attention's width."""
+    from nats_llm_studio_amd.ops import stack as K
+    AH, AG, Dp, H, D, V, BS = 8, 2, 128, 6, 64, 128, 16
+    f32 = dtype == torch.float32
+    assert T <= K.attn_step_fits(AH, AG, Dp, not f32, 0, H, D, V, f32)
+    g = torch.Generator().manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).cuda()
+    kc, vc, aq, z = rnd(T * 48, AG * Dp), rnd(T * 48, AG * Dp), rnd(T, AH * Dp), rnd(T, H * (2 * D + V))
+    bt, ts = torch.arange(T * 3).int().view(T, 3).cuda(), torch.arange(T).int().cuda()
+    cl, runs = torch.tensor([40 - i for i in range(T)]).int().cuda(), torch.tensor([[i, 1, i, i] for i in range(T)]).int().cuda()
+    a, norm, gate = torch.rand(T, H * D, generator=g).cuda(), torch.rand(H * V, generator=g).cuda(), rnd(T, H * V)
+    S0 = torch.randn(T, H * D * V, generator=g).cuda()
+    part = (torch.zeros(T * AH * Dp).cuda(), torch.zeros(T * AH * 2).cuda(), torch.zeros(T * 2).int().cuda())
+    st = torch.cuda.current_stream().cuda_stream
+    q, k, v = z, z[:, H * D:], z[:, 2 * H * D:]
+    S, S1, aout, out, aref, ref = S0.clone(), S0.clone(), *(torch.zeros(T, n, dtype=dtype, device="cuda") for n in (AH * Dp, H * V) * 2)
+    K.attn_step(aq, kc, vc, None, aout, part, 1, bt, BS, ts, cl, T, AH, AG, Dp, 0.09, False, q, k, v, a, None, 0.5, S, runs, norm, gate, out, H, D, V,
+                1e-5, st)
+    K.gla_step(q, k, v, a, None, 0.5, S1, runs, T, norm, gate, ref, H, D, V, 1e-5, st)
+    K.gqa_attention(aq, kc, vc, None, aref, part, bt, BS, ts, cl, T, AH, AG, Dp, not f32, 1, 0.09, st)
+    assert torch.equal(S, S1) and (f32 or torch.equal(out, ref))
+    o = S1.double().view(T, H, D, V) * q[:, :H * D].double().view(T, H, D, 1) * 0.5
+    o, m = o.sum(2), o.abs().sum(2)
+    sc = norm.double().view(H, V) * gate.double().view(T, H, V) / (o * o).mean(2, keepdim=True).add(1e-5).sqrt()
+    bound = m * sc.abs() + (o * sc).abs() * ((m * m).mean(2, keepdim=True) / (o * o).mean(2, keepdim=True)).sqrt()
+    # (32 bits: eight waves to a state here, four there, so sums of 64 products, and squares of them, in another order)
+    assert ((out.double() - ref.double()).abs().view(T, H, V) <= 128 * 2.0 ** -22 * bound).all()
+    # another number of waves adds up to 40 keys: a rounding of 2^-22 a key, then the output's
+    e = 2.0 ** -7 if not f32 else 40 * 2.0 ** -22
+    assert ((aout.double() - aref.double()).abs() <= e * vc.double().abs().max()).all()
