@@ -254,6 +254,10 @@ class LinLaunch:
             if bm == 256:                 # (refused in 32 bits, whose tiles have up to 128 rows)
                 return True, 7
             if self.f32:
+                # (one list to an expert, each weight from memory once: two workgroups to a CU are not enough for parts either; eight experts of
+                # 4096 x 3072, 8 to 38 rows each 125 us, on the f32 MFMA 114)
+                if bm == 64 and M * self.plan.top <= 64 * self.plan.experts and self._tiles(64, 64, M) <= 512:
+                    return True, 5
                 return True, min((5, 0, 1) if bm == 64 else (2,), key=lambda c: self.split_us(c, M))
             if bm == 64:
                 # short products are over before the deeper tiles' stages pay: 64 x 64 / chosen by rounds, us: 64 experts of 30 rows, 512 x 2048 28 / 41

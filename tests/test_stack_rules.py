@@ -76,4 +76,9 @@ def test_tiles_of_32_bits():
     for N, Kd, M in ((4096, 12288, 257), (16384, 4096, 65), (35888, 4096, 33), (2048, 64, 200), (2048, 128, 200)):
         assert launch(N, Kd, True).config(M)[1] in (0, 1, 2)
     assert launch(2048, 8704, True, 4096, 8, 512).choice(64) == ((True, 5), 8)
+    for N, Kd, T, want in ((4096, 3072, 150, (5,)), (2048, 4096, 32, (5,)), (8192, 2048, 150, (0, 1)), (4096, 3072, 300, (0, 1))):
+        L = launch(N, Kd, True)
+        L.plan, L.segs[0].s.rows = S.MoePlan(T, 8, 2, 1, 1, 1.0, "cpu"), 1
+        L.segs[0].w.groups = 8
+        assert L.plan.bm(T) == 64 and L.config(T)[1] in want, (N, Kd, T)
     assert launch(2048, 8704, True, 8192, 8, 512).choice(900)[0][1] in (0, 1, 2)
