@@ -266,9 +266,10 @@ DEVI float sum8_32(const float (&o)[8], int lane) {
 
 // The scan of few runs, up to two workgroups for each CU. A wave takes a token's time to issue and to close its sums (240 cycles of the form above,
 // however many waves share the CU), so here a column's keys lie over 32 lanes, two columns to a wave, the sums of eight tokens are closed together,
-// and the next chunk is staged in a second buffer while one is summed, with a barrier for each. 3500 tokens, 32 heads of 64: 349 -> 261 us, 64 heads
-// 373 -> 362; 2000 tokens, 16 and 32 heads of 128: 301 -> 199 and 308 -> 271; with four workgroups to a CU it would be slower (4 x 900, 32 heads of 64:
-// 121 above, 173).
+// and the next chunk is staged in a second buffer while one is summed, with a barrier for each. 3500 tokens, 32 heads of 64: 348 -> 244 us, 64 heads
+// 351 -> 327, 16 and 32 heads of 128 533 -> 339 and 535 -> 450; 100 tokens 15.2 -> 12.4, 15.9 -> 17.1, 21.1 -> 15.1 and 22.9 -> 21.5. At two workgroups to a CU runs of up
+// to 100 tokens of heads of 64 lose up to 1.2 us; the rule does not ask for their length, since the bits of a prompt must not depend on how it is cut. With
+// four workgroups to a CU it would be slower (4 x 900, 32 heads of 64: 121 above, 173).
 template <typename T, int DP, bool VEC>
 __global__ __launch_bounds__(256) void wkv_few_kernel(Scan p) {
   constexpr int WC = 8, CH = 2048 / DP, R = DP / 32, LR = DP + 4, RQ = R < 4 ? 2 : 4, PF = 3, RB = PF + 1;

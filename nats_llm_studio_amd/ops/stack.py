@@ -203,8 +203,8 @@ GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 
 # together; 0 to 2 in bf16 parts (lin_split.hip), 5 on the f32 MFMA (1.3 us more a launch). One workgroup to a CU splits and multiplies in turn, and
 # the f32 MFMA is the faster one: 64 x 64, parts / f32, us: 65 x 4096 x 12288 356 / 226, 64 x 16384 x 4096 130 / 88, 256 x 2048 x 8704 249 / 162, in eight
 # splits 64 x 2048 x 8704 41 / 28.6; with two it loses (128 x 10240 x 4096 138 / 147), with four it takes 1.4 times as long. Up to 128 inputs
-# parts win (64 x 2048 x 128 6.9 / 7.6). 22 shapes x 16 row counts x 4 tiles x 1 to 8 splits lie 6 % around it, the tile it picks is 0.1 % behind the
-# fastest on average, tile and splits 1.2 %. 64 x 64 / 128 x 64 / 128 x 128 in parts, us: 900 x 20096 x 2048 467 / 432 / 394 (f32 658), 1500 x 35888 x 4096
+# parts win (64 x 2048 x 128 6.9 / 7.6). 22 shapes x 16 row counts x 4 tiles x 1 to 8 splits lie 7 % around it, the tile it picks is 0.6 % behind the
+# fastest on average, tile and splits 1.5 %. 64 x 64 / 128 x 64 / 128 x 128 in parts, us: 900 x 20096 x 2048 467 / 432 / 394 (f32 658), 1500 x 35888 x 4096
 # 2621 / 2223 / 2020 (3440).
 SPLIT_US = {0: (0.78, 0.30, 6), 1: (1.09, 0.49, 4), 2: (1.66, 0.87, 3), 5: (0.57, 0.57, 3)}
 
