@@ -676,11 +676,12 @@ def gla_shape(T: int, nruns: int, H: int, V: int, D: int = 64, longest: Optional
     segments, 265 with 1; 1 run of 333 tokens 93 us with 5, 63 with 6): the count is the one that segments_us finds fastest."""
     nt = 1 if V <= 64 else 2
     wgs = H * -(-V // (64 * nt))
-    n = T - nruns + 1 if longest is None else longest
     most = min(-(-512 // (wgs * nruns)), 16)             # (what bounds the scratch, too)
     if 64 < D <= 128 and nt == 2:
         return segments("gla", T, longest or -(-T // nruns), wgs, most), nt
-    return 1 if wgs * nruns >= 256 or n <= 128 else max(1, min(most, -(-n // 64))), nt
+    if longest is None:                                  # (no run can have more tokens than this)
+        return 1 if wgs * nruns >= 256 else max(1, min(most, (T - nruns + 1) // 64)), nt
+    return 1 if wgs * nruns >= 256 or longest <= 128 else min(most, -(-longest // 64)), nt
 
 
 def gla_scan(q, k, v, a, qscale: float, o, norm, gate, out, state, runs, nruns: int, H: int, D: int, V: int, eps: float, shape,
@@ -765,11 +766,12 @@ def delta_shape(T: int, nruns: int, H: int, D: int, V: int, longest: Optional[in
     segments, 444 with the 1 that segments_us finds)."""
     nt = 1 if V <= 64 else 2
     wgs = H * -(-V // (64 * nt))
-    n = T - nruns + 1 if longest is None else longest
     most = min(-(-256 // (wgs * nruns)), 16)             # (what bounds the scratch, too)
     if 64 < D <= 128 and nt == 2:
         return segments("delta", T, longest or -(-T // nruns), wgs, most), nt
-    return 1 if wgs * nruns >= 128 or n <= 128 else max(1, min(most, -(-n // 64))), nt
+    if longest is None:
+        return 1 if wgs * nruns >= 128 else max(1, min(most, (T - nruns + 1) // 128)), nt
+    return 1 if wgs * nruns >= 128 or longest <= 128 else min(most, -(-longest // 64)), nt
 
 
 def delta_scan(q, k, v, fac, beta, a, o, norm, gate, out, state, runs, nruns: int, H: int, G: int, D: int, V: int, eps: float,
