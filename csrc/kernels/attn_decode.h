@@ -1,6 +1,7 @@
 // Decode attention over a paged bf16 / fp8 K/V cache on MFMA (gfx950), shared by the GGUF families (attention.hip) and the
 // config-driven stacks (csrc/stack/attn.hip).
 #pragma once
+#include <type_traits>
 #include "common.h"
 
 namespace nls_attn {
@@ -115,21 +116,30 @@ constexpr int attn_decode_lds() {
   return VB > MB ? (VB > CB ? VB : CB) : (MB > CB ? MB : CB);
 }
 
-// by of gy: workgroup of token t's heads; Vsm: attn_decode_lds() bytes. AHEAD: the next keys' loads are in flight under a group's
-// arithmetic (at D = 128 220 registers, without it 168).
-template <typename KV, int WAVES, int D, typename OUT, bool WIN, bool AHEAD = true>
-DEVI void attn_decode_body(
-    uint8_t* Vsm, int t, int by, int gy, int split,
+// AHEAD: the next keys' loads are in flight under a group's arithmetic (at D = 128 220 registers, without it 168). Beside: other work of the
+// launch, asked first, which answers whether the workgroup is its own or sets the place (token t, `by` of gy, split) that it takes here; its `lds`
+// bytes lie in the same space, `waves` of a workgroup's fit a SIMD. (A body called from two kernels took this one past 128 registers at D = 64 with
+// a window: 200 tokens behind 300 keys 19.9 -> 23.1 us.)
+struct Alone {
+  static constexpr int lds = 0, waves = 1;
+};
+template <typename KV, int WAVES, int D, typename OUT = act_t, bool WIN = false, bool AHEAD = true, class Beside = Alone>
+__global__ __launch_bounds__(64 * WAVES, Beside::waves) void attn_decode_mfma_kernel(
     const __bf16* __restrict__ q, long ldq, const KV* __restrict__ kc, const KV* __restrict__ vc,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
     const int* __restrict__ ctx_len, int Hkv, int Gq, int bs, float scale, int chunk, int n_split,
     OUT* __restrict__ out, long ldo, float* __restrict__ part_o, float* __restrict__ part_ml,
-    int* __restrict__ cnt, const float* __restrict__ gate, long ldg, AttnMask mask) {
+    int* __restrict__ cnt, const float* __restrict__ gate, long ldg, AttnMask mask, Beside beside) {
   static_assert(D == 32 || D == 64 || D == 128 || (D == 256 && WAVES <= 2), "head dimension");
   constexpr int NKK = D / 32, NDT = D / 16, KG = 32;
   constexpr int NCH = D / 8, LPR = NCH, RPI = 64 / LPR, NVL = KG / RPI;   // V: chunks per row, lanes per row,
                                                                           // rows per load, loads per 32 keys
   typedef KVRaw<KV> R;
+  constexpr int LDS = attn_decode_lds<WAVES, D>();
+  __shared__ __attribute__((aligned(16))) uint8_t Vsm[LDS > Beside::lds ? LDS : Beside::lds];
+  int t = blockIdx.x, by = blockIdx.y, gy = gridDim.y, split = blockIdx.z;
+  if constexpr (!std::is_same<Beside, Alone>::value)
+    if (beside(Vsm, t, by, gy, split)) return;
   const int nhb = (Gq + 15) >> 4, kh = nhb == 1 ? by : by / nhb;
   const int hofs = nhb == 1 ? 0 : (by - kh * nhb) * 16;
   const int G = min(Gq - hofs, 16), h0 = kh * Gq + hofs;       // this workgroup's query heads: h0 .. h0 + G - 1
@@ -389,19 +399,6 @@ DEVI void attn_decode_body(
   if (!last) return;
   merge_splits<WAVES, D>(part_o, part_ml, t, h0, G, Hq, n_split, na, out, ldo, gate, ldg,
                          reinterpret_cast<float*>(Vsm));
-}
-
-template <typename KV, int WAVES, int D, typename OUT = act_t, bool WIN = false>
-__global__ __launch_bounds__(64 * WAVES) void attn_decode_mfma_kernel(
-    const __bf16* __restrict__ q, long ldq, const KV* __restrict__ kc, const KV* __restrict__ vc,
-    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tok_seq,
-    const int* __restrict__ ctx_len, int Hkv, int Gq, int bs, float scale, int chunk, int n_split,
-    OUT* __restrict__ out, long ldo, float* __restrict__ part_o, float* __restrict__ part_ml,
-    int* __restrict__ cnt, const float* __restrict__ gate, long ldg, AttnMask mask) {
-  __shared__ __attribute__((aligned(16))) uint8_t Vsm[attn_decode_lds<WAVES, D>()];
-  attn_decode_body<KV, WAVES, D, OUT, WIN>(Vsm, blockIdx.x, blockIdx.y, gridDim.y, blockIdx.z, q, ldq, kc, vc, block_tables,
-                                           bt_stride, tok_seq, ctx_len, Hkv, Gq, bs, scale, chunk, n_split, out, ldo, part_o,
-                                           part_ml, cnt, gate, ldg, mask);
 }
 
 }  // namespace nls_attn

@@ -25,7 +25,7 @@ int decode_w(const GA& a, hipStream_t st) {
   const int gq = a.H / a.G;
   hipLaunchKernelGGL((attn_decode_mfma_kernel<__bf16, W, D, __bf16, WIN>), dim3(a.T, a.G * ((gq + 15) / 16), a.ns), dim3(64 * W), 0,
                      st, (const __bf16*)a.q, a.ldq, (const __bf16*)a.k, (const __bf16*)a.v, a.bt, a.bts, a.tok_seq, a.ctx_len,
-                     a.G, gq, a.bs, a.scale, 0, a.ns, (__bf16*)a.out, a.ldo, a.part_o, a.part_ml, a.cnt, a.gate, a.ldg, a.mask);
+                     a.G, gq, a.bs, a.scale, 0, a.ns, (__bf16*)a.out, a.ldo, a.part_o, a.part_ml, a.cnt, a.gate, a.ldg, a.mask, Alone{});
   return (int)hipGetLastError();
 }
 

@@ -18,6 +18,7 @@
 // small grids. Three prompts of 300 tokens, 16 heads of 128 over 4: 823 us (one workgroup per row and head, a serial walk) -> 43 us;
 // four decoded tokens behind 300 keys: 136 -> 16 us.
 #pragma once
+#include <type_traits>
 #include "../kernels/common.h"
 
 namespace nls_plain {
@@ -88,9 +89,16 @@ DEVI void redo_row(const PA& p, int t, int h, int row, int bz, const float* mls,
     if ((int)threadIdx.x + NT * j < dv) y[threadIdx.x + NT * j] = (T)(acc[j] * f);
 }
 
-// NQ: 64-column blocks of the values; NW: waves. (bx, by, bz) of gx: workgroup; sm: plain_lds() bytes. PA is the kernel's first argument.
-template <typename T, int NQ, int NW>
-DEVI void attn_plain_body(float* sm, const PA& p, int bx, int by, int bz, int gx) {
+// NQ: 64-column blocks of the values; NW: waves. Beside: other work of the launch, asked first, which answers whether the workgroup is its own or
+// sets the place (bx, by, bz of gx) that it takes here. (A body called from two kernels compiled to other copies of the keys' registers in
+// this one: 8 to 25 % slower at 128 columns in 32 bits.)
+struct Alone {};
+template <typename T, int NQ, int NW, class Beside>
+__global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p, Beside beside) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z, gx = gridDim.x;
+  if constexpr (!std::is_same<Beside, Alone>::value)
+    if (beside(sm, bx, by, bz, gx)) return;
   constexpr int KC = NQ > 2 ? 4 : 8;               // 16-column steps of a key chunk
   constexpr int ML = NW * 32 + 16;                 // floats of the waves' maxima and sums, rows that are not finite
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -98,7 +106,7 @@ DEVI void attn_plain_body(float* sm, const PA& p, int bx, int by, int bz, int gx
   const int nks = (p.Dk + 15) >> 4, nc = (nks + KC - 1) / KC, ldl = nc * KC * 16 + 4;
   float *mls = sm, *ob = sm + ML, *qs = ob;        // (the merge takes the queries' place)
   int* bad = reinterpret_cast<int*>(sm + NW * 32);
-  const int kh = by / p.sub, h0 = (by % p.sub) * 16;          // key head, first of its query heads
+  const int kh = (uint32_t)by / p.sub, h0 = ((uint32_t)by % p.sub) * 16;          // key head, first of its query heads
   const int gr = min(p.gs - h0, 16);                                          // query heads of this workgroup
   const int t0 = (gx - 1 - bx) * p.tb, tn = min(p.tb, p.T - t0);      // (later tokens see more keys)
   const int nrow = tn * gr;
@@ -283,12 +291,6 @@ DEVI void attn_plain_body(float* sm, const PA& p, int bx, int by, int bz, int gx
   }
 }
 
-template <typename T, int NQ, int NW>
-__global__ __launch_bounds__(64 * NW) void attn_plain_kernel(PA p) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  attn_plain_body<T, NQ, NW>(sm, p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x);
-}
-
 inline size_t plain_lds(int Dk, int NQ, int NW) {
   const int KC = NQ > 2 ? 4 : 8, nc = ((Dk + 15) / 16 + KC - 1) / KC;
   return sizeof(float) * (NW * 32 + 16 + max(16 * (nc * KC * 16 + 4), NW * 16 * 68));
@@ -299,12 +301,12 @@ int launch_w(const PA& p, dim3 grid, hipStream_t st) {
   const size_t lds = plain_lds(p.Dk, NQ, NW);
   if (lds > 64 * 1024) {
     static bool attr = false;
-    if (!attr && hipFuncSetAttribute((const void*)attn_plain_kernel<T, NQ, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    if (!attr && hipFuncSetAttribute((const void*)attn_plain_kernel<T, NQ, NW, Alone>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      160 * 1024) != hipSuccess)
       return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((attn_plain_kernel<T, NQ, NW>), grid, dim3(64 * NW), lds, st, p);
+  hipLaunchKernelGGL((attn_plain_kernel<T, NQ, NW, Alone>), grid, dim3(64 * NW), lds, st, p, Alone{});
   return (int)hipGetLastError();
 }
 

@@ -4,8 +4,8 @@
 // the attention of few hundred keys is one chain of dependent loads, so each leaves idle what the other needs. Graph launches, bf16, 32
 // heads of 128 over 8 beside 32 states of 64 x 128, us, one behind the other / together: 1 token behind 90 keys 12.1 / 7.1,
 // behind 1500 16.4 / 11.0; with cold states and keys 16 tokens behind 90 and 1000 20 / 14 and 37 / 32, 64 tokens 43 / 37 and 101 / 86, 300 tokens 159 / 149 and
-// 424 / 369. Of 375 sizes of 1 to 300 tokens behind 20 to 3000 keys 0.80 of the time on average; slower are 128 tokens and more behind 20 keys (62 /
-// 64 to 142 / 146: three of four waves have no keys) and two sizes behind 3000 (2 %). The attention takes four waves and gives up the prefetch of
+// 424 / 369. Of 375 sizes of 1 to 300 tokens behind 20 to 3000 keys 0.80 of the time on average; slower are 128 tokens and more behind 20 keys (61 /
+// 65 to 138 / 141: three of four waves have no keys) and three sizes behind 3000 (1 to 6 %). The attention takes four waves and gives up the prefetch of
 // the next keys: that leaves registers for three workgroups on a CU, of which two would not keep the states' loads in flight.
 // In 32 bits the plain attention keeps all its registers, a CU holds one workgroup: that pays up to two rounds of states (3 tokens behind 330
 // keys 24.9 / 20.1, 16 tokens 30.6 / 23.4; 32 tokens, 1024 states, 45.1 / 49.4).
@@ -30,57 +30,76 @@ struct AT {
   AttnMask mask;
 };
 
-// Workgroups 0 .. T * gy * ns - 1: attention of a token's heads, a share of its keys; then a state of a token each.
-template <int D, int RPT>
-__global__ __launch_bounds__(256, 3) void attn_step_kernel(AT a, Scan p, StepOut y) {
-  constexpr int LDS = attn_decode_lds<4, D>() > step_lds(256) ? attn_decode_lds<4, D>() : step_lds(256);
-  __shared__ __attribute__((aligned(16))) uint8_t sm[LDS];
-  const int n = a.T * a.gy * a.ns, b = blockIdx.x;
-  if (b < n) {
-    const int u = b / a.T, split = u / a.gy;
-    attn_decode_body<__bf16, 4, D, __bf16, false, false>(sm, b - u * a.T, u - split * a.gy, a.gy, split, a.q, a.ldq, a.k, a.v, a.bt,
-                                                         a.bts, a.tok_seq, a.ctx_len, a.G, a.gq, a.bs, a.scale, 0, a.ns, a.out,
-                                                         a.ldo, a.part_o, a.part_ml, a.cnt, a.gate, a.ldg, a.mask);
-  } else {
+// The states of the launch: workgroups from T * gy * ns on, one each; those before are the attention of a token's heads, a share of its keys.
+template <int RPT>
+struct TokenStates {
+  static constexpr int lds = step_lds(256), waves = 3;
+  int T, gy, ns;
+  Scan p;
+  StepOut y;
+  DEVI bool operator()(uint8_t* sm, int& t, int& by, int& ngy, int& split) const {
+    const int n = T * gy * ns, b = t;
+    if (b < n) {
+      const int u = b / T;
+      split = u / gy;
+      t = b - u * T;
+      by = u - split * gy;
+      ngy = gy;
+      return false;
+    }
     const int row = (b - n) / p.H;
     step_body<__bf16, GLA, 256, RPT>(reinterpret_cast<float*>(sm), p, y, b - n - row * p.H, p.H, row);
+    return true;
   }
+};
+
+template <int D, int RPT>
+int launch_rpt(const AT& a, const Scan& p, const StepOut& y, hipStream_t st) {
+  hipLaunchKernelGGL((attn_decode_mfma_kernel<__bf16, 4, D, __bf16, false, false, TokenStates<RPT>>), dim3(a.T * (a.gy * a.ns + p.H)), dim3(256), 0,
+                     st, a.q, a.ldq, a.k, a.v, a.bt, a.bts, a.tok_seq, a.ctx_len, a.G, a.gq, a.bs, a.scale, 0, a.ns, a.out, a.ldo, a.part_o, a.part_ml, a.cnt,
+                     a.gate, a.ldg, a.mask, TokenStates<RPT>{a.T, a.gy, a.ns, p, y});
+  return (int)hipGetLastError();
 }
 
 template <int D>
 int launch(const AT& a, const Scan& p, const StepOut& y, hipStream_t st) {
   const int rpt = step_rpt(p.D, p.V, 256);
-  const dim3 grid(a.T * (a.gy * a.ns + p.H));
-  if (rpt <= 4) hipLaunchKernelGGL((attn_step_kernel<D, 4>), grid, dim3(256), 0, st, a, p, y);
-  else if (rpt <= 8) hipLaunchKernelGGL((attn_step_kernel<D, 8>), grid, dim3(256), 0, st, a, p, y);
-  else if (rpt <= 16) hipLaunchKernelGGL((attn_step_kernel<D, 16>), grid, dim3(256), 0, st, a, p, y);
-  else return -1;
-  return (int)hipGetLastError();
+  return rpt <= 4 ? launch_rpt<D, 4>(a, p, y, st) : rpt <= 8 ? launch_rpt<D, 8>(a, p, y, st) : rpt <= 16 ? launch_rpt<D, 16>(a, p, y, st) : -1;
 }
 
 // 32-bit models: the same with the plain attention's grid of gx x gy
-template <int NQ, int NW, int RPT>
-__global__ __launch_bounds__(64 * NW) void plain_step_kernel(nls_plain::PA a, int gx, int gy, Scan p, StepOut y) {
-  extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int n = gx * gy, b = blockIdx.x;
-  if (b < n) {
-    const int by = b / gx;
-    nls_plain::attn_plain_body<float, NQ, NW>(sm, a, b - by * gx, by, 0, gx);
-  } else {
+template <int NT, int RPT>
+struct States {
+  int gx, gy;
+  Scan p;
+  StepOut y;
+  DEVI bool operator()(float* sm, int& bx, int& by, int& bz, int& ngx) const {
+    const int n = gx * gy, b = bx;
+    if (b < n) {
+      by = b / gx;
+      bx = b - by * gx;
+      bz = 0;
+      ngx = gx;
+      return false;
+    }
     const int row = (b - n) / p.H;
-    step_body<float, GLA, 64 * NW, RPT>(sm, p, y, b - n - row * p.H, p.H, row);
+    step_body<float, GLA, NT, RPT>(sm, p, y, b - n - row * p.H, p.H, row);
+    return true;
   }
+};
+
+template <int NQ, int RPT>
+int plain_rpt(const nls_plain::PA& a, dim3 g, const Scan& p, const StepOut& y, hipStream_t st) {
+  const size_t lds = max(nls_plain::plain_lds(a.Dk, NQ, 8), (size_t)step_lds(512));
+  hipLaunchKernelGGL((nls_plain::attn_plain_kernel<float, NQ, 8, States<512, RPT>>), dim3(g.x * g.y + a.T * p.H), dim3(512), lds, st, a,
+                     States<512, RPT>{(int)g.x, (int)g.y, p, y});
+  return (int)hipGetLastError();
 }
 
 template <int NQ>
 int plain_launch(const nls_plain::PA& a, dim3 g, const Scan& p, const StepOut& y, hipStream_t st) {
   const int rpt = step_rpt(p.D, p.V, 512);
-  const size_t lds = max(nls_plain::plain_lds(a.Dk, NQ, 8), (size_t)step_lds(512));
-  const dim3 grid(g.x * g.y + a.T * p.H);
-  if (rpt <= 4) hipLaunchKernelGGL((plain_step_kernel<NQ, 8, 4>), grid, dim3(512), lds, st, a, g.x, g.y, p, y);
-  else if (rpt <= 8) hipLaunchKernelGGL((plain_step_kernel<NQ, 8, 8>), grid, dim3(512), lds, st, a, g.x, g.y, p, y);
-  else return -1;
-  return (int)hipGetLastError();
+  return rpt <= 4 ? plain_rpt<NQ, 4>(a, g, p, y, st) : rpt <= 8 ? plain_rpt<NQ, 8>(a, g, p, y, st) : -1;
 }
 
 int plain(nls_plain::PA a, int T, int H, const Scan& p, const StepOut& y, hipStream_t st) {

@@ -718,7 +718,7 @@ def gla_step(q, k, v, a, gate_in, qscale: float, state, runs, nruns: int, norm, 
 
 def attn_step_fits(AH: int, AG: int, Dp: int, mfma: bool, window: int, H: int, D: int, V: int, f32: bool) -> int:
     """The most tokens whose attention and recurrence attn_step takes in one launch where that is the faster way (0: none): any
-    number in bf16 (1 to 300 tokens behind 20 to 3000 keys 45 % less to 4 % more than one behind the other, 20 % less on average); in 32 bits (a
+    number in bf16 (1 to 300 tokens behind 20 to 3000 keys 47 % less to 7 % more than one behind the other, 20 % less on average); in 32 bits (a
     workgroup per CU) up to 512 states (4 % more to 40 % less; 768 14 % less to 20 % more, 1024 up to 33 % more)."""
     if window or V % 4 or V > 1024 or -(-D // (256 // (V // 4))) > 16:
         return 0
