@@ -213,13 +213,13 @@ int step_rows(const Scan& p, int nruns, const float* norm, const void* gate, lon
               hipStream_t st) {
   if (nruns < 1 || p.H < 1 || p.D < 1 || p.D > 256 || p.V < 4 || p.V > 1024 || (p.V & 3) || (p.sstride & 3)) return -1;
   const StepOut y{norm, gate, ldg, out, ldout, eps};
-  // The state's loads go out ahead where few workgroups leave memory idle meanwhile. Up to two to a CU, states cold, a graph's launches, behind the inputs /
+  // The state's loads go out ahead where few workgroups leave memory idle meanwhile. Below two to a CU, states cold, a graph's launches, behind the inputs /
   // ahead, us: 32 heads of 64 x 128 4 tokens 6.7 / 6.0, 12 tokens 11.0 / 10.0, 16 of 128 x 128 4 tokens 9.0 / 6.9, wkv of 128 x 128 12 tokens 14.6 / 11.8. With
-  // more, loads all at once and stores all at once are the slower way: 32 heads of 64 x 128, 96 tokens 43.1 / 46.5, 300 tokens 123 / 130; nothing to gain either with
+  // more, loads all at once and stores all at once are the slower way: 32 heads of 64 x 128, 16 tokens 11.7 / 11.9 (128 x 128 20.1 / 18.4), 96 tokens 43.1 / 46.5, 300 tokens 123 / 130; nothing to gain either with
   // one or two rows per thread (32 x 64 4.0 / 4.1), or where wkv's inputs, more of them, are the wait (one token of 16 heads of 64 4.3 / 4.4).
   const long n = (long)p.H * nruns;
   const int rpt = step_rpt(p.D, p.V, 256);
-  const bool ahead = n <= 512 && (KIND == WKV ? n > 32 : rpt > 2);
+  const bool ahead = n <= (rpt > 8 ? 512 : 448) && (KIND == WKV ? n > 32 : rpt > 2);
 #define NLS_STEP(N) \
   if (N == 0 || (ahead && rpt <= N)) { \
     hipLaunchKernelGGL((step_kernel<T, KIND, N>), dim3(p.H, nruns), dim3(256), 0, st, p, y); \
