@@ -68,6 +68,11 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
   static const NlsFuse none{};
   if (!fz) fz = &none;
   const float* xf = fz->xf;
+  if (mode == 3 && waves == 4 && (ldx % 8 || (uintptr_t)x % 16)) {      // its DMA moves 16 aligned bytes: mode 2 loads any rows
+    mode = 2;
+    waves = 8;
+    rt = rt > 8 ? 4 : 2;
+  }
   if (xf && (M > 16 || !fz->nw || (mode != 0 && !(mode == 1 && fz->ssq_in)))) return -1;
   if (fz->ssq_in && (!xf || fz->nss_in < 1 || fz->nss_in > fz->ldss)) return -1;
   if (fz->ssq_out) {      // producer of a split RMSNorm: path A residual add, whole tiles of tokens

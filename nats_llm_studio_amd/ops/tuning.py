@@ -51,9 +51,77 @@ def table():
     return _TABLE
 
 
+# Microseconds of a launch of quantised rows on shapes without a tuned entry, fitted to 39000 launches of 30 shapes (1536 to 128256 rows, K 1536 to 28672,
+# Q4_K, Q5_K, Q6_K and Q8_0, the launch behind it included, weights streamed). (mode, waves, rt): workgroups that share a CU, and what a last round of at
+# most one to a CU takes of a whole one; then of the launch: fixed, a round, a round's K (times bytes a weight up to 8 rows) / 4096, the same for each
+# 16 rows, a second launch (RoPE, SwiGLU of split sums, norm), a million slab values, a MB of weights.
+_FEW_US = (((0, 4, 1), 1, 1.0, (4.07, 0.97, 1.84, 0.0, 2.60, 0.0, 0.114)), ((0, 4, 2), 2, 0.6, (4.30, 3.00, 5.27, 0.0, 2.36, 0.0, 0.086)),
+           ((1, 4, 1), 2, 0.6, (3.37, 2.95, 15.3, 0.0, 2.95, 8.58, 0.058)), ((1, 8, 1), 1, 1.0, (2.13, 3.30, 13.7, 0.0, 3.44, 10.2, 0.065)))
+_SOME_US = (((0, 4, 1), 1, 1.0, (4.26, 0.90, 0.0, 3.37, 2.37, 0.0, 0.094)), ((0, 4, 2), 2, 0.6, (2.96, 4.73, 0.0, 6.48, 2.47, 0.0, 0.076)),
+            ((1, 4, 1), 2, 0.7, (2.39, 4.79, 5.20, 4.62, 3.43, 2.29, 0.068)), ((1, 8, 1), 3, 0.5, (0.22, 10.4, 16.4, 5.76, 3.80, 2.97, 0.073)))
+# ... above 64 rows, by (mode, rt): a round, its K / 4096, the same for the share of the block's rows in use, the second launch, a million slab values
+_MID_US = {(2, 1): (2, 0.5, (9.03, 0.0, 54.3, 5.37, 1.39)), (2, 2): (1, 1.0, (5.49, 28.1, 7.31, 5.62, 1.81)), (2, 4): (1, 1.0, (7.70, 25.9, 25.6, 4.51, 1.62)),
+           (3, 4): (2, 0.65, (5.94, 0.0, 40.2, 7.27, 0.74)), (3, 6): (2, 0.65, (8.91, 50.2, 0.0, 5.75, 1.20))}
+_WEIGHT_BYTES = {8: 1.0625, 12: 0.5625, 13: 0.6875, 14: 0.8203}
+_QUANT = frozenset(_WEIGHT_BYTES)
+
+
+def _rounds(n: int, share: int, last: float) -> float:
+    """Rounds of n workgroups, `share` of them to a CU; `last`: what a last round of at most one to a CU takes."""
+    full, part = divmod(n, 256 * share)
+    return full + (0.0 if not part else last if part <= 256 else 1.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _few_rule(rows, K: int, types, M: int, role: str):
+    """The cheapest of paths A (up to 32 rows) and B for 2 to 64 rows of a shape without a tuned entry. us of all projections of a layer of a 2048-wide
+    model at 2 / 4 / 16 / 32 / 48 rows, with the head, before and after (a rule that knew path B with 8 waves only from 9 rows on): Q4_K 164 -> 152,
+    172 -> 155, 170 -> 170, 204 -> 203, 258 -> 241; Q5_K 181 -> 166, 186 -> 170, 226 -> 181, 247 -> 213, 265 -> 244; Q8_0 181 -> 175, 189 -> 180,
+    237 -> 188, 262 -> 218, 271 -> 247."""
+    nb, mt, total = K // 256, -(-M // 16), sum(rows)
+    mb = sum(-(-n // 16) * 16 * K * _WEIGHT_BYTES[t] for n, t in zip(rows, types)) * 1e-6
+    width = max(_WEIGHT_BYTES[t] for t in types) if M <= 8 else 1.0
+
+    def us(fam, ks):
+        (mode, waves, rt), share, last, c = fam
+        tile = 16 * rt * (waves if mode else 1)
+        k = _rounds(sum(-(-n // tile) for n in rows) * ks, share, last)
+        kk = k * K / ks / 4096
+        more = mode != 0 if role == "qkv" else ks > 1 if role in ("gateup", "lm_head") else True
+        return (c[0] + c[1] * k + c[2] * kk * width + c[3] * kk * mt + c[4] * more + (c[5] * ks * M * total * 1e-6 if ks > 1 else 0.0) + c[6] * mb)
+    (cfg, *_), ks = min(((f, ks) for f in (_FEW_US if M <= 8 else _SOME_US) for ks in (1, 2, 3, 4, 6, 8)
+                         if (ks == 1 or f[0][0] == 1 and ks * 2 <= nb) and (f[0][0] == 1 or M <= 32)), key=lambda c: us(*c))
+    return (*cfg, ks)
+
+
+@functools.lru_cache(maxsize=4096)
+def _mid_rule(rows, K: int, types, M: int, role: str):
+    """65 to 255 rows: the cheapest of the LDS-dequant GEMM in blocks of 64 and 128 rows and (K-quants) the LDS-DMA GEMM in blocks of 64 and 96, 2.5 %
+    behind the fastest of 90 configs on average. us of all projections of a layer of a 2048 / 4096-wide model with the head, 96 rows, before and
+    after: Q4_K 377 -> 310, 555 -> 515; Q5_K 387 -> 325, 603 -> 530; Q8_0 (128-row tiles of path B, one launch on 16 of 256 CUs) 1042 -> 330, 1541 -> 550."""
+    nb, total = K // 256, sum(rows)
+    dma = 8 not in types                      # (raw Q8_0 tiles do not fit that kernel's LDS)
+
+    def us(fam, ks):
+        mode, rt = fam
+        share, last, c = _MID_US[fam]
+        bm = 64 * rt if mode == 2 else 16 * rt
+        k = _rounds(sum(-(-n // 128) for n in rows) * -(-M // bm) * ks, share, last)
+        kk = k * K / ks / 4096
+        more = role != "gateup" or ks > 1
+        return c[0] * k + c[1] * kk + c[2] * kk * min(M, bm) / bm + c[3] * more + (c[4] * ks * M * total * 1e-6 if ks > 1 else 0.0)
+    (mode, rt), ks = min(((f, ks) for f in _MID_US for ks in (1, 2, 3, 4, 6, 8) if (ks == 1 or ks * 2 <= nb) and (dma or f[0] == 2)), key=lambda c: us(*c))
+    return (mode, 8 if mode == 2 else 4, rt, ks)
+
+
 def heuristic(segs, M: int):
     rows = sum(s.w.rows for s in segs)
     K = segs[0].w.K
+    quant = all(int(s.w.type) in _QUANT for s in segs)
+    # (up to 64 rows below 64 M weights: the others' bytes are most of their time, what the rule chooses there is 4 % faster, here 17 at 16 to 48 rows)
+    if quant and 1 < M < 256 and (M > 64 or rows * K < 64 << 20):
+        rule = _few_rule if M <= 64 else _mid_rule
+        return rule(tuple(s.w.rows for s in segs), K, tuple(int(s.w.type) for s in segs), M, _role(segs))
     if M <= 8:
         # the batch-1 winners of every measured family (Llama-3-8B / -70B, Qwen2.5-7B, Mixtral; r03 sweeps,
         # profiles/b1_latency_r03.txt, profiles/b1_models_r03.txt): 4-wave workgroups; wide matrices (gate|up,
@@ -63,8 +131,8 @@ def heuristic(segs, M: int):
             return (1, 4, 2, 2) if rows >= 16 * K and K >= 1024 else (1, 4, 2, 1)
         return (0, 4, 2, 1) if len(segs) > 1 else (0, 4, 1, 1)
     if M > 64:
-        if all(int(s.w.type) in (12, 13, 14) for s in segs):
-            if M >= 256 and (rows >= 4 * K or K >= 2 * rows):
+        if quant:
+            if rows >= 4 * K or K >= 2 * rows:
                 # wide (gate|up, LM head) and down-projection shapes: the quantised GEMM on the raw tile-blocks
                 # (mode 9, 256 weight rows x 256 activation rows) won every measured one at M >= 256 -- Llama-3-8B
                 # gate|up / LM head, Llama-3-70B gate|up / down / LM head by 10-20 % over mode 2
@@ -74,13 +142,13 @@ def heuristic(segs, M: int):
                 while tiles * ks < 256 and ks * 2 <= min(8, max(1, nb // 4)):    # (ks <= 8: the tuned range)
                     ks *= 2
                 return (9, 8, 2, ks)
-            # LDS-dequant GEMM (mode 2): 128 weight rows x 256 (or 128) activation rows per workgroup;
+            # LDS-dequant GEMM (mode 2): 128 weight rows x 256 activation rows per workgroup;
             # split K until the grid covers the 256 CUs (the measured winners on the 8B shapes)
             tiles = sum((s.w.rows + 127) // 128 for s in segs) * ((M + 255) // 256)
             ks, nb = 1, K // 256
             while tiles * ks < 256 and ks * 2 <= max(1, nb // 4):
                 ks *= 2
-            return (2, 8, 4 if M >= 192 else 2, ks)
+            return (2, 8, 4, ks)
         return (1, 8, 1, 1)      # MFMA GEMM: 128 weight rows x 128 activation rows per workgroup
     waves, rt = 8, 1
     tiles = sum((s.w.rows + waves * rt * 16 - 1) // (waves * rt * 16) for s in segs)
@@ -144,10 +212,12 @@ def argmax_config(cfg, segs, M: int):
     """Config of a launch with an arg-max: path B unsplit ends in an atomic for every 16 weight rows and token, all on M neighbouring
     keys (32000 Q6_K rows, K = 4096, (1, 8, 1, 1): 62 us at 2 tokens, 108 at 8, 166 at 24, 248 at 64). Split in two, the reduce
     takes the maximum with few atomics: 26, 28, 34, 47; at K = 2048 2 / 8 / 24 / 64 tokens 58 / 105 / 150 / 217 -> 18 / 20 /
-    25 / 34, one token 36 -> 19; on 16-row tiles, (1, 8, 1, 2), 24 / 26 / 30 / 36."""
+    25 / 34, one token 36 -> 19; on 16-row tiles, (1, 8, 1, 2), 24 / 26 / 30 / 36. Path A ends so as well (29 us at 2 tokens), where it was not measured
+    with the arg-max."""
     if _FORCED and key(segs, M) in _FORCED:
         return cfg
-    if cfg[0] == 1 and 1 in cfg[2:] and M <= 64 and sum(s.w.rows for s in segs) >= 8192 and segs[0].w.K >= 1024:
+    if (M <= 64 and sum(s.w.rows for s in segs) >= 8192 and segs[0].w.K >= 1024
+            and (cfg[0] == 1 and 1 in cfg[2:] or cfg[0] == 0 and M > 1 and _tuned(segs, M) is None)):
         return (1, 4 if M == 1 else 8, 2, 2)
     return cfg
 
@@ -252,8 +322,13 @@ def _role_entry(segs, M: int):
     return table().get(f"{ref}:{_mb(M)}")
 
 
-def select(segs, M: int):
+def _tuned(segs, M: int):
     hit = table().get(key(segs, M))
     if hit is None and M <= 64 and os.environ.get("NLS_TUNING_ROLE", "1") == "1":
         hit = _role_entry(segs, M)
+    return hit
+
+
+def select(segs, M: int):
+    hit = _tuned(segs, M)
     return hit if hit is not None else heuristic(segs, M)
