@@ -707,13 +707,21 @@ inline bool valid(const TalkArgs& a) {
 extern "C" {
 using namespace nls_talk;
 
-// any shape, f32 arithmetic: talk f32 [H][H]
-int nls_talk_plain(const void* q, long ldq, const void* k, const void* v, const int* bt, int bts, int bs, const int* tok_seq,
-                   const int* ctx_len, int T, int H, int G, int Dp, int V, float scale, int window, const float* talk,
-                   const void* gate, long ldg, void* out, long ldo, int f32, void* stream) {
+// rows t0 .. t0 + rows - 1, any head count, f32 arithmetic: talk f32 [H][H], Dp a multiple of 4. sc [rows][H][ks], ks a multiple of 16 that
+// holds 16 * (first visible / 16) .. the last key; st [rows][ns1][H][2]; ns > 1 (one token to a workgroup of the mix): part [rows][H][ns][Dp],
+// cnt [rows][workgroups] zeros (left zero). tb1, tb: tokens of a workgroup of the scores and of the mix; kt: keys of its block; nw: its waves, 4 or 8
+int nls_talk_rows(const void* q, long ldq, const void* k, const void* v, const int* bt, int bts, int bs, const int* tok_seq,
+                  const int* ctx_len, int t0, int rows, int H, int G, int Dp, int V, float scale, int window, const float* talk,
+                  const void* gate, long ldg, void* out, long ldo, float* sc, long ks, float* st, float* part, int* cnt, int tb1, int ns1, int tb,
+                  int ns, int kt, int nw, int f32, void* stream) {
   const TalkArgs a{q, k, v, out, gate, talk, bt, tok_seq, ctx_len, ldq, ldo, ldg, bts, bs, H, G, Dp, V, scale, window};
-  if (T < 1 || bs < 1 || !valid(a)) return -1;
-  return f32 ? plain::launch<float>(a, T, (hipStream_t)stream) : plain::launch<__bf16>(a, T, (hipStream_t)stream);
+  if (rows < 1 || t0 < 0 || bs < 1 || !valid(a) || (Dp & 3) || !sc || !st || ks < 16 || (ks & 15) || ns1 < 1 || ns < 1 || ns1 > 65535 ||
+      ns > 65535 || (ns > 1 && (tb > 1 || !part || !cnt)) || kt < 16 || kt > plain::KT || (kt & 15) || (nw != 4 && nw != 8))
+    return -1;
+  const int most = H / G >= 16 ? 1 : 16 / (H / G), sub = (H / G + 15) / 16;
+  if (tb1 < 1 || tb1 > most || tb < 1 || tb > most || (long)G * sub > 65535) return -1;
+  const plain::Rows p{a, sc, st, part, cnt, ks, t0, rows, sub, tb1, ns1, tb, ns, kt};
+  return f32 ? plain::launch<float>(p, nw, (hipStream_t)stream) : plain::launch<__bf16>(p, nw, (hipStream_t)stream);
 }
 
 // rows t0 .. t0 + rows - 1, bf16; bs a power of two, Dp 32, 64, 128 or 256, H <= 128. talk: bf16 [32 kk][32 kk]. sc [rows][ks][hs], ks

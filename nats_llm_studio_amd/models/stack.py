@@ -417,11 +417,10 @@ class AttentionPart(_SharedPart):
                  inputs=[K.Seg(self.qkv, x, qkv)] + ([K.Seg(self.g, x, gate, "sigmoid", alpha=self.scale)]
                                                      if self.g is not None else []))
         if self.talk is not None:
-            if self.talk_plan.mfma:
-                sizes = self.talk_plan.scratch(P)
-                names = ("talk.sc", "talk.st", "talk.po", "talk.cnt")
-                e["part"] = [self.scratch(b, n, 1, s, f if n != "talk.cnt" else torch.int32) for n, s in zip(names, sizes)]
-                e["part"] = [t.view(-1) for t in e["part"]]
+            sizes = self.talk_plan.scratch(P)
+            names = ("talk.sc", "talk.st", "talk.po", "talk.cnt")
+            e["part"] = [self.scratch(b, n, 1, s, f if n != "talk.cnt" else torch.int32) for n, s in zip(names, sizes)]
+            e["part"] = [t.view(-1) for t in e["part"]]
             return e
         n = _SPLIT_WG // self.groups + 1                  # rows x splits
         e["part"] = (self.scratch(b, "attn.po", 1, n * H * self.Dp, f), self.scratch(b, "attn.pm", 1, n * H * 2, f),

@@ -44,7 +44,7 @@ _SIGS = {
     "nls_row_norm": [P, L, P, P, P, P, P, L, P, L, I, I, F, I, I, I, P],
     "nls_poly_norm": [P, L, P, P, L, I, I, F, I, P],
     "nls_attn_rows": [P, P, P, L, P, P, P, P, P, P, L, P, P, L, I, I, I, I, I, I, I, I, I, F, I, P],
-    "nls_talk_plain": [P, L, P, P, P, I, I, P, P, I, I, I, I, I, F, I, P, P, L, P, L, I, P],
+    "nls_talk_rows": [P, L, P, P, P, I, I, P, P, I, I, I, I, I, I, F, I, P, P, L, P, L, P, L, P, P, P, I, I, I, I, I, I, I, P],
     "nls_talk_decode": [P, L, P, P, P, I, I, P, P, I, I, I, I, I, I, F, I, P, P, L, P, L, P, L, P, P, P, I, I, I, P],
     "nls_talk_prefill": [P, L, P, P, P, I, I, P, I, I, I, I, I, I, F, I, P, P, L, P, L, P],
     "nls_gqa_attn": [P, L, P, P, P, I, I, P, P, I, I, I, I, I, F, P, L, P, L, P, P, P, I, I, I, I, I, P],
@@ -909,9 +909,32 @@ class TalkPlan:
             return ns1, max(1, min(16, 1024 // n)), 1
         return ns1, max(1, min(16, 256 // n)), 4
 
+    def plain_form(self, T: int):
+        """(tokens of a workgroup of the scores, shares of the keys, tokens of a workgroup of the mix, shares, keys of a block, waves) of the
+        plain kernels at T rows. Tokens share a workgroup, and so a tile of MFMA rows and their keys, once there are enough of them for the
+        chip; fewer have their keys shared out instead. us of both launches with 1 / 2 / 4 tokens to a workgroup of the mix, at 400, 700 and 1203
+        tokens of a prompt: 32 heads 125 / 94 / 127, 291 / 231 / 217, 726 / 545 / 491, 16 heads 61 / 66 / 81, 116 / 112 / 140, 267 / 199 / 231;
+        one token and 1203 keys, 16 heads, in 1 / 4 / 16 shares 78 / 39 / 31."""
+        most = max(1, 16 // (self.H // self.G))
+        jobs = self.groups * -(-self.Dp // 64)
+        tb1 = 1 if T <= 64 else min(most, -(-T * self.groups // 256))
+        tb = 1
+        while 2 * tb <= most and T * -(-jobs // 8) >= 340 * 2 * tb and 2 * tb * self.H * 36 <= 16384:
+            tb *= 2
+        kt = max(16, min(64, (16384 // (tb * self.H) - 4) // 16 * 16))
+        nw = 4 if tb == 1 else 8
+        ns1 = max(1, min(64, 1024 // (-(-T // tb1) * self.groups), -(-self.ks // 64)))
+        ns = 1 if tb > 1 else max(1, min(16, 256 // (T * -(-jobs // nw)), -(-self.ks // kt)))
+        return tb1, ns1, tb, ns, kt, nw
+
     def scratch(self, cap: int):
         """Element counts of (scores, score statistics, partial outputs, counters)."""
         R = self.rows(cap)
+        if not self.mfma:
+            forms = [(T, *self.plain_form(T)) for T in range(1, R + 1)]
+            part = max((T * ns for T, _, _, _, ns, _, _ in forms if ns > 1), default=0)
+            return (R * self.ks * self.hs, max(T * ns1 for T, _, ns1, *_ in forms) * self.hs * 2, part * self.H * self.Dp,
+                    min(R, 256) * -(-self.groups * -(-self.Dp // 64) // 4))
         part = max(T * self.splits(T)[1] for T in range(1, R + 1)) if R < 4096 else 16 * R
         return (R * self.ks * self.hs, max(T * self.splits(T)[0] for T in range(1, R + 1)) * self.hs * 2, part * self.H * self.Dp,
                 R * self.groups)
@@ -925,10 +948,20 @@ def talk_attention(plan: TalkPlan, q, kc, vc, talk, gate, out, scratch, block_ta
     if gate is not None and gate.dtype != out.dtype:
         raise ValueError("talk_attention: a gate of the outputs' type")
     if not p.mfma:
-        _check(lib().nls_talk_plain(q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), block_tables.data_ptr(),
-                                    block_tables.stride(0), block_size, tok_seq.data_ptr(), ctx_len.data_ptr(), T, p.H, p.G, p.Dp, V,
-                                    scale, p.window, talk.data_ptr(), _p(gate), ldg, out.data_ptr(), out.stride(0),
-                                    int(q.dtype == torch.float32), st), "nls_talk_plain")
+        if not scratch:
+            scratch = [torch.empty(n, device=q.device) for n in p.scratch(T)[:3]] + [torch.zeros(p.scratch(T)[3], dtype=torch.int32, device=q.device)]
+        sc, ss, po, cnt = scratch
+        R = min(p.rows(T), sc.numel() // (p.ks * p.H))
+        for t0 in range(0, T, R):
+            n = min(R, T - t0)
+            tb1, ns1, tb, ns, kt, nw = p.plain_form(n)
+            if (ss.numel() < n * ns1 * p.H * 2 or (ns > 1 and (po.numel() < n * ns * p.H * p.Dp or cnt.numel() < n * -(-p.groups * -(-p.Dp // 64) // nw)))):
+                raise ValueError("talk_attention: workspace too small")
+            _check(lib().nls_talk_rows(q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), block_tables.data_ptr(),
+                                       block_tables.stride(0), block_size, tok_seq.data_ptr(), ctx_len.data_ptr(), t0, n, p.H, p.G, p.Dp, V,
+                                       scale, p.window, talk.data_ptr(), _p(gate), ldg, out.data_ptr(), out.stride(0), sc.data_ptr(), p.ks,
+                                       ss.data_ptr(), po.data_ptr(), cnt.data_ptr(), tb1, ns1, tb, ns, kt, nw,
+                                       int(q.dtype == torch.float32), st), "nls_talk_rows")
         return
     sc, ss, po, cnt = scratch
     R = min(p.rows(T), sc.numel() // (p.ks * p.hs))

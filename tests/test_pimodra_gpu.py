@@ -202,6 +202,51 @@ def test_attention_far_pages(K, dt):
                 assert relerr(out[t].view(H, D), want[t]) < TOL[dt], (window, t)
 
 
+@pytest.mark.parametrize("dt,H,G,D,V", [("f32", 6, 2, 20, 36), ("f32", 18, 18, 32, 32), ("f32", 3, 3, 64, 130), ("bf16", 8, 2, 300, 10), ("f32", 70, 35, 8, 8)])
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("most", [None, 301])
+def test_rows_that_share_keys(K, dt, H, G, D, V, window, most):
+    """Prompts of several sequences row by row: tiles of tokens that see different keys, in one launch and in several, then with values that are
+    not finite at a key that the first rows of its tile do not see, and one that the last do not: those rows keep their results."""
+    d, bs = DT[dt], 16
+    Dp, _ = K.head_pad(max(D, V))
+    runs = [(0, 430), (9, 3), (100, 267)]                        # first position, rows
+    ctxs, scale, T = [p + n for p, n in runs], 0.7 / math.sqrt(D), 700
+    q, talk, gate = talk_inputs(d, T, H, D, V, Dp)
+    kc, vc, bt, rows = paged(d, ctxs, G, D, V, Dp, 30, bs, [[] for _ in runs])
+    seq = [i for i, (_, n) in enumerate(runs) for _ in range(n)]
+    pos = [p + j for p, n in runs for j in range(n)]
+    plan = K.TalkPlan(H, G, Dp, window, 480, dt == "f32", "cuda")
+    assert not plan.mfma and (H > 18 or G == H == 3 or plan.plain_form(T)[0] > 1)
+    plan.rows = lambda cap: min(cap, most or cap)
+    at = {0: (201, 0, 1), 2: (303, G - 1, V - 1)}                # sequence: key, key head, column that are made infinite
+    mask = {"size": window} if window else None
+    check = sorted({t for t in range(T) if seq[t] in at and abs(pos[t] - at[seq[t]][0]) in (0, 1, 2, 3, 4, 15, 16, 36, 37, 38)} | {0, 1, 429, 430, 432, 433, 699})
+    for wild in (False, True):
+        if wild:
+            for i, (k, h, c) in at.items():
+                rows[i][1][k, h, c] = math.inf
+                vc.view(-1, G, Dp)[int(bt[i, k // bs]) * bs + k % bs, h, c] = math.inf
+        out = torch.full((T + 1, H * Dp), 7.0, dtype=d, device="cuda")
+        K.talk_attention(plan, q.view(T, -1).cuda(), kc, vc, plan.matrix(talk), gate.cuda(), out, None, bt, bs, i32(seq), i32([p + 1 for p in pos]), T,
+                         V, scale, st())
+        o = out[:T].view(T, H, Dp).cpu()
+        assert (out[T] == 7).all() and (o[..., V:] == 7).all()
+        for t in check:
+            k, v = (x[:pos[t] + 1] for x in rows[seq[t]])
+            want = O.attend(q[t:t + 1, :, :D].double(), k, v, torch.tensor([pos[t]]), scale, mask, talk.double())[0] * gate[t].double().view(H, V)
+            if wild and seq[t] in at:                            # (0 * inf beside the window is the reference's own)
+                kk, h, c = at[seq[t]]
+                sees = kk <= pos[t] and (not window or pos[t] - kk < window)
+                hit = torch.zeros(H, V, dtype=torch.bool)
+                hit[h * (H // G):(h + 1) * (H // G), c] = True
+                assert torch.isfinite(o[t, :, :V])[~hit].all() and torch.isfinite(o[t, :, :V])[hit].all() == (not sees), (t, sees)
+                rest = torch.where(hit, 0.0, want)
+                assert relerr(torch.where(hit, 0.0, o[t, :, :V].double()), rest) < TOL[dt], t
+            else:
+                assert relerr(o[t, :, :V], want) < TOL[dt], t
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,D,V", [(1, 1, 8, 4), (6, 2, 20, 36), (5, 5, 33, 21), (4, 2, 64, 128), (2, 1, 128, 7), (3, 1, 256, 256),
                                      (2, 2, 300, 16), (40, 8, 128, 128)])
