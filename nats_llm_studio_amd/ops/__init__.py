@@ -294,7 +294,7 @@ def gemv_config(segs: Sequence[Seg], M: int):
     return tuning.select(segs, M)
 
 
-DENSE_MODES = (4, 5, 6, 10)
+DENSE_MODES = (4, 5, 6, 10, 11)
 
 
 def _merge_dense(segs: Sequence[Seg]):
@@ -416,7 +416,7 @@ def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: 
             if argmax is not None and not mapped:
                 from . import tuning
                 mode, waves, rt, ks = tuning.argmax_config((mode, waves, rt, ks), segs, M)
-            if mode == 10 and (x.stride(0) % 8 or y.stride(0) % 4):
+            if mode >= 10 and (x.stride(0) % 8 or y.stride(0) % 4):
                 from . import tuning
                 mode, waves, rt, ks = tuning.dense_heuristic(segs, M, aligned=False)
         if M > 64 and mode == 0:
@@ -729,7 +729,7 @@ def qkv_rope_kv(segs: Sequence[Seg], h: torch.Tensor, qkv: torch.Tensor, pos: to
         mode, waves, rt, ks = cfg or gemv_config(segs, T)
         ncol = sum(s.w.rows for s in segs)
         contiguous = all(s.ycol == sum(x.w.rows for x in segs[:i]) for i, s in enumerate(segs))
-        if (mode in (4, 5, 10) and ks == 1 and contiguous and ncol == (Hq + 2 * Hkv) * D
+        if (mode in (4, 5, 10, 11) and ks == 1 and contiguous and ncol == (Hq + 2 * Hkv) * D
                 and not neox and fuse_rope and kc.dtype == torch.bfloat16):
             # large-M GEMM on the dense f16 copies with RoPE + KV append in its epilogue (no f32 qkv round trip,
             # no RoPE launch)

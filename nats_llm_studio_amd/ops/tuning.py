@@ -11,6 +11,8 @@ import json
 import math
 import os
 
+import numpy as np
+
 _TABLE = None
 _FORCED = set()        # keys of NLS_TUNING_EXTRA's entries: no rule below changes those launches
 _PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gemv_tuning.json")
@@ -271,6 +273,84 @@ def _dense_rule(rows, K: int, M: int, aligned: bool):
     return (mode, 8 if mode == 10 or M < 128 else 16, rt, ks)
 
 
+# What mode 11's forms are weighed against a launch of the other modes by, in microseconds: rounds of workgroups (of one XCD: it has every eighth weight
+# tile, and 32 CUs; P is what a part of a round takes at least) times what a round takes, fixed and for 4096 of K; a MB of weights, which come from
+# memory; a split's second launch (where there is none anyway), a million slab values, and those past 16 million, which leave the caches. By (mode, rt,
+# activation rows of a block), fitted to 2000 launches of 27 shapes, 2048 to 57344 rows, K 2048 to 28672, at 128 to 4096 rows; 5 to 15 % each.
+_DENSE_US = {(10, 1, 256): (0.5, 11.3, 94.7, 0.056, 14.9, 0.0, 1.27), (10, 1, 192): (0.7, 10.6, 76.5, 0.035, 7.3, 0.49, 0.57),
+             (10, 2, 256): (0.6, 9.1, 59.9, 0.021, 7.7, 0.22, 0.87), (10, 2, 192): (0.78, 5.2, 47.8, 0.016, 6.9, 0.73, 0.52),
+             (10, 2, 320): (0.5, 12.5, 70.3, 0.034, 7.3, 0.24, 0.63), (4, 2, 128): (0.85, 6.6, 30.8, 0.085, 6.0, 0.0, 0.59)}
+# Mode 11's tiles are 32 nt weight rows x 32 mt activations, 3 <= nt <= 8, 3 <= mt <= 5 (the forms that are built); 9000 launches of the same shapes, 11 %
+_NT11, _MT11 = (v.ravel() for v in np.meshgrid(np.arange(3, 9), np.arange(3, 6), indexing="ij"))
+
+
+def _dense_us(rows, K: int, M: int, added: bool, mode: int, rt: int, ks: int) -> float:
+    """Predicted time of a launch of mode 10 or 4 (those of mode 5 and other wave counts are taken for mode 4's)."""
+    if mode != 10:
+        mode, rt = 4, 2
+    bn = 256 if (mode, rt) == (10, 1) else 128
+    tiles = sum((n + bn - 1) // bn for n in rows)
+    bm = _rows10(rt, tiles, M, ks) if mode == 10 else 128
+    P, fixed, per, mb, second, slab, far = _DENSE_US[mode, rt, bm]
+    full, part = divmod(-(-tiles // 8) * -(-M // bm) * ks, 32)
+    n, slabs = full + (P + (1 - P) * part / 32 if part else 0.0), ks * M * sum(rows)
+    return (n * (fixed + per * K / ks / 4096) + mb * sum(rows) * K * 2e-6
+            + ((0.0 if added else second) + slab * slabs * 1e-6 + far * max(0, slabs - (16 << 20)) * 1e-6 if ks > 1 else 0.0))
+
+
+def _best11(rows, K: int, M: int, added: bool):
+    """(time, config) of mode 11's fastest form. All forms at once (0.1 ms a product; a prompt's length is new each time)."""
+    ks = np.arange(1, 1 + max(1, min(8, K // 64 // 6)))[:, None]
+    nt, mt = _NT11, _MT11
+    tiles = sum(-(-n // (32 * nt)) for n in rows)
+    full, part = np.divmod(-(-tiles // 8) * -(-M // (32 * mt)) * ks, 32)
+    n = full + np.where(part > 0, 0.85 + 0.15 * part / 32, 0.0)
+    slabs = np.where(ks > 1, ks * (M * sum(rows) * 1e-6), 0.0)
+    t = (n * (2.16 + 0.201 * nt * mt + (0.39 + 0.252 * nt * mt + 3.41 * (nt + mt)) * K / ks / 4096) + 0.058 * sum(rows) * K * 2e-6
+         + np.where(ks > 1, 0.0 if added else 5.6, 0.0) + 0.86 * slabs + 0.49 * np.maximum(0.0, slabs - 16.8))
+    i = int(t.argmin())
+    k, j = divmod(i, len(nt))
+    return float(t.flat[i]), (11, 8, 512 + 16 * int(mt[j]) + int(nt[j]), k + 1)
+
+
+def _launch_rows(segs):
+    """Rows of a launch's segments, those whose f16 copies lie behind each other as one (ops._merge_dense)."""
+    rows, end = [], None
+    for s in segs:
+        w = s.w
+        at = w.d16.data_ptr() if len(segs) > 1 and getattr(w, "d16", None) is not None else None
+        if at is not None and at == end:
+            rows[-1] += w.rows
+        else:
+            rows.append(w.rows)
+        end = None if at is None else at + 2 * w.rows * w.K
+    return tuple(rows)
+
+
+MODE11_MAX_M = 2560          # (above, 256 x 256 tiles are as fast: 28672 x 4096 at 3000 rows 603 us, 633 on the best of mode 11, 2048 x 2048 45 and 45)
+
+
+def _or_mode11(cfg, segs, M: int):
+    """cfg, or mode 11's fastest form where that should be 5 % faster (times are known to 5 to 15 %: 1 % slower at worst on 138 measured products of 27 shapes,
+    4.4 % faster on average). us before and after: 2048 x 2048 at 192 / 1500 rows 19 / 35 -> 14 / 29, 3072 x 2048 at 128 / 640 17 / 31 -> 15 / 19,
+    16384 x 2048 at 128 / 512 30 / 45 -> 22 / 38, 6144 x 4096 at 320 / 640 39 / 53 -> 32 / 44, 5120 x 5120 at 128 / 1024 30 / 83 -> 25 / 71, 28672 x 4096 at 900
+    210 -> 197. (Operands whose strides suit modes 10 and 11 only: stores are 4 columns wide. Unsplit blocks of 320 rows stay: faster in mode 11 where
+    nothing but such launches runs, 85 -> 79 for 28672 x 4096 at 320 rows, but 80 either way in a step, between launches that draw less power.)"""
+    if M > MODE11_MAX_M or any(s.w.rows % 4 or s.ycol % 4 for s in segs):
+        return cfg
+    return _mode11_or(tuple(cfg), _launch_rows(segs), segs[0].w.K, M, _role(segs) in ("o", "down"))
+
+
+@functools.lru_cache(maxsize=4096)         # (a prompt's launches ask once for each layer and projection)
+def _mode11_or(cfg, rows, K: int, M: int, added: bool):
+    if len(rows) > 1:                      # (what was measured are whole products; a loaded model has Q, K and V copies behind each other)
+        return cfg
+    if cfg[0] == 10 and cfg[2:] == (2, 1) and _rows10(2, sum(-(-n // 128) for n in rows), M, 1) == 320:
+        return cfg
+    t, best = _best11(rows, K, M, added)
+    return best if t < 0.95 * _dense_us(rows, K, M, added, cfg[0], cfg[2], cfg[3]) else cfg
+
+
 def select_dense(segs, M: int):
     """Dense config, or None where the tuner measured the quantised GEMM faster (entry [-1])."""
     hit = table().get(dense_key(segs, M))
@@ -285,7 +365,8 @@ def select_dense(segs, M: int):
             hit = table().get(f"d:{sum(s.w.rows for s in segs)}:{segs[0].w.K}:{320 if M <= 320 else 640}")
         elif M > MBUCKETS[-1]:
             hit = None
-    return hit if hit is not None else dense_heuristic(segs, M)
+    cfg = hit if hit is not None else dense_heuristic(segs, M)
+    return cfg if dense_key(segs, M) in _FORCED else _or_mode11(cfg, segs, M)
 
 
 # Llama-3-8B Q4_K_M shapes per projection role: the tuned entries an untuned shape of the same role borrows at

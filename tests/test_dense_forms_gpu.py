@@ -1,0 +1,90 @@
+"""The dense f16 GEMM whose wave groups take alternate k-steps (mode 11): every form, at the edges of its tiles and of its ring of K-tiles."""
+import pytest
+import torch
+
+from nats_llm_studio_amd import ops
+from nats_llm_studio_amd.ops import tuning
+from test_dense_gemm_gpu import acts, relerr, weight
+
+FORMS = [512 + 16 * mt + nt for mt in (3, 4, 5) for nt in (3, 4, 5, 6, 7, 8)]
+
+
+class _W:
+    d16 = None
+
+    def __init__(self, rows, K):
+        self.type, self.rows, self.K = 12, rows, K
+
+
+def test_rule_gives_built_forms():
+    """The forms that the rule can choose are those that are built, with at least six K-tiles to a part; none for rows that its stores do not take."""
+    for rows in (256, 2048, 4100, 6144, 16384, 28672):
+        for K in (256, 512, 2048, 14336):
+            for M in (128, 190, 257, 640, 1000, 2560, 2561):
+                t, (mode, waves, rt, ks) = tuning._best11((rows,), K, M, False)
+                assert t > 0 and mode == 11 and waves == 8 and rt in FORMS and (ks == 1 or K // 64 // ks >= 6)
+                cfg = tuning.select_dense([ops.Seg(_W(rows, K))], M)
+                assert cfg[0] != 11 or M <= 2560
+            assert tuning.select_dense([ops.Seg(_W(rows + 1, K))], 300)[0] != 11
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rt", FORMS)
+@pytest.mark.parametrize("rows,K", [(772, 256), (64, 512), (1020, 1536)])
+def test_forms(gpu, rt, rows, K):
+    """Rows short of a weight tile and of a row block; fewer K-tiles than the ring holds, splits with parts of one K-tile more than others."""
+    w = weight(rows, K)
+    for M in (1, 95, 96, 161, 320, 333):
+        x = acts(M, K)
+        z = x[:M].double() @ w.d16.double().T
+        for epi, dt, ks in (("f32", torch.float32, 1), ("add", torch.float32, 1), ("act", torch.float16, 1), ("f32", torch.float32, 3)):
+            y = torch.full((M + 1, rows + 4), 7.0, device="cuda", dtype=dt)
+            ops.qgemv([ops.Seg(w, 4)], x, y, M, epi=epi, mode=11, waves=8, rt=rt, ks=ks)
+            # f32 sums of K products; f16 outputs round to 2^-11
+            assert relerr(y[:M, 4:] - (7 if epi == "add" else 0), z) < (5e-4 if epi == "act" else 4e-6), (M, ks, epi)
+            assert (y[M] == 7).all() and (y[:, :4] == 7).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rt", [563, 583, 599, 600])
+@pytest.mark.parametrize("M", [130, 300])
+def test_gate_and_head(gpu, rt, M):
+    """SwiGLU over a row count that no tile divides, a head's arg-max with its logits."""
+    rows, K = 2000, 512
+    w, x = weight(rows, K), acts(M, K)
+    z = x[:M].double() @ w.d16.double().T
+    v = z.view(M, rows // 16, 2, 8)
+    want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, rows // 2)
+    y = torch.full((M + 1, rows // 2), 7.0, device="cuda", dtype=torch.float16)
+    ops.qgemv([ops.Seg(w)], x, y, M, epi="swiglu", mode=11, waves=8, rt=rt, ks=1)
+    assert relerr(y[:M], want) < 5e-4 and (y[M:] == 7).all()                       # f16 outputs round to 2^-11
+    logits = torch.full((M + 1, rows), 7.0, device="cuda")
+    keys, ids = torch.zeros(M + 1, dtype=torch.int64, device="cuda"), torch.full((M + 1,), -1, dtype=torch.int32, device="cuda")
+    ops.qgemv([ops.Seg(w)], x, logits, M, epi="f32", argmax=keys, mode=11, waves=8, rt=rt, ks=1)
+    ops.argmax_unpack(keys, M, ids)
+    assert (ids[:M].long() == logits[:M].argmax(1)).all() and int(keys[M]) == 0 and relerr(logits[:M], z) < 4e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rt", [563, 599])
+@pytest.mark.parametrize("D,bias", [(128, True), (34, True), (64, False)])
+def test_rope(gpu, rt, D, bias):
+    """Three segments with RoPE and the cache rows, against mode 10."""
+    Hq, Hkv, K, M = 16, 8, 64 * 4, 200
+    ws = [weight(h * D, K, s) for s, h in enumerate((Hq, Hkv, Hkv))]
+    segs = [ops.Seg(ws[0], 0), ops.Seg(ws[1], Hq * D), ops.Seg(ws[2], (Hq + Hkv) * D)]
+    x, n = acts(M, K), (Hq + 2 * Hkv) * D
+    pad = x.shape[0]
+    cs = ops.rope_table(400, D, 10000.0, torch.device("cuda"))
+    pos = (torch.arange(pad, dtype=torch.int32, device="cuda") * 7) % 400
+    slot = torch.randperm(pad, generator=torch.Generator().manual_seed(2)).int().cuda()
+    slot[[0, 17, M - 1]] = -1
+    b = torch.randn(n, generator=torch.Generator().manual_seed(3)).cuda() if bias else None
+    outs = []
+    for cfg in ((11, 8, rt, 1), (10, 8, 2, 1)):
+        q = torch.full((pad, Hq * D), 776.0, dtype=torch.bfloat16, device="cuda")
+        kc, vc = (torch.full((pad, Hkv, D), 776.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        ops.qkv_rope_kv(segs, x, torch.zeros(pad, n, device="cuda"), pos, slot, cs, q, kc, vc, M, Hq, Hkv, D, cfg=cfg, bias=b)
+        outs.append((q, kc, vc))
+    for a, b in zip(*outs):      # one bf16 rounding apart at most, and the same places written
+        assert relerr(a, b) < 2e-3 and ((a == 776) == (b == 776)).all()
