@@ -28,6 +28,7 @@ using nls_dma::wait_vm_lgkm0;
 int lin_phased(LinArgs& a, hipStream_t st);      // lin_phased.hip
 int lin_split(LinArgs& a, int cfg, hipStream_t st);      // lin_split.hip
 int lin_thin(LinArgs& a, hipStream_t st);        // lin_thin.hip
+int lin_pair(LinArgs& a, int nt, int mt, hipStream_t st);      // lin_pair.hip
 
 template <int BN, int BM, int WN, int WM, int NST>
 struct LG {
@@ -182,6 +183,7 @@ int gemm_t(LinArgs& a, hipStream_t st) {
 }
 
 int lin_gemm(LinArgs& a, int cfg, hipStream_t st) {
+  if (cfg >= 256) return lin_pair(a, cfg >> 4 & 15, cfg & 15, st);
   switch (cfg) {
     case 0: return gemm_t<__bf16, 64, 64, 2, 2, 3>(a, st);
     case 1: return gemm_t<__bf16, 128, 64, 4, 1, 3>(a, st);
@@ -208,9 +210,10 @@ extern "C" {
 // cfg: tile of the launch (BN x BM): 0 = 64 x 64, 1 = 128 x 64, 2 = 128 x 128, 3 = 256 x 128, 4 = 256 x 256 in two stages (a launch's
 // own choice never is this one), 5 = 64 x 64 with 8 stages in flight (launches of at most one workgroup per CU),
 // 6 = 192 x 128, 7 = 256 x 256 in phases, 8 = 96 x 64, 9 = 160 x 64, 10 = 128 x 64 with four stages, 11 = 96 x 128, 12 = 64 x 32 with 8 stages,
-// 13 = 64 x 128 straight from memory (K up to 128, no routed rows).
+// 13 = 64 x 128 straight from memory (K up to 128, no routed rows), 256 + 16 nt + mt = 32 nt x 32 mt, two wave groups on alternate k-steps (no row
+// lists and maps).
 // f32: 5 = 64 x 64 on the f32 MFMA in three stages, 0, 1 and 2 in bf16 parts; the others run on one of these, but for 7 and 13 and for routed
-// rows on 4, which are refused.
+// rows on 4 and from 256 on, which are refused.
 int nls_lin_gemm(const void* args, int f32, int cfg, void* stream) {
   nls_lin::LinArgs a = *reinterpret_cast<const nls_lin::LinArgs*>(args);
   using namespace nls_lin;

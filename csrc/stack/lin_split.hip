@@ -214,7 +214,8 @@ int split_t(LinArgs& a, hipStream_t st) {
 }
 
 int lin_split(LinArgs& a, int cfg, hipStream_t st) {
-  if (cfg == 4)                                      // (lists in tiles of 256 rows do not fit the 128 of the tile it runs on)
+  if (cfg >= 256) cfg = 4;
+  if (cfg == 4)                                      // (lists in tiles of more rows do not fit the 128 of the tile it runs on)
     for (int i = 0; i < a.nseg; ++i)
       if (a.s[i].rows) return -1;
   switch (cfg) {

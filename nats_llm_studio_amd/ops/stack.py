@@ -187,18 +187,18 @@ class Seg:
         self.keep = (bias, gate, routed, rope, xmap)
 
 
+def PAIR(nt: int, mt: int) -> int:
+    """lin_gemm's config of lin_pair.hip's tile of 32 nt weight rows x 32 mt rows."""
+    return 256 + 16 * nt + mt
+
+
 # (weight rows, rows) of lin_gemm's configs
 GEMM_TILES = {0: (64, 64), 1: (128, 64), 2: (128, 128), 3: (256, 128), 4: (256, 256), 5: (64, 64), 6: (192, 128), 7: (256, 256),
-              8: (96, 64), 9: (160, 64), 10: (128, 64), 11: (96, 128), 12: (64, 32)}
+              8: (96, 64), 9: (160, 64), 10: (128, 64), 11: (96, 128), 12: (64, 32),
+              **{PAIR(n, m): (32 * n, 32 * m) for n, m in ((4, 4), (4, 5), (5, 4), (6, 4), (6, 5), (8, 4), (8, 5))}}
 THIN = 13                # config of products of up to 128 inputs straight from memory, 64 weight rows x 128 rows
 
 
-# Relative multiply rates of the tiles: (up to so many workgroups, below, above); the small tiles run two or more to a CU. 7, the
-# phased 256 x 256 tile: a round of 256 workgroups took 88 us at K = 4096 (1.24 PFLOP/s, 1.36 over many rounds), one of 3 (256 x 128)
-# 70 us, one of 6 (192 x 128) 54 us, so it wins where rounds fill: 2000 x 35888 490 us against 743 (3) and 652 (6), 512 x 24576 92
-# against 141 and 109, but 512 x 12288 83 against 72 and 57, 2000 x 4096 x 17408 297 against 269 (3).
-GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 0.47, 0.72),
-             1: (512, 0.5, 0.63), 0: (1024, 0.45, 0.55)}
 # 32-bit operands: microseconds of 32 input columns on a CU that runs one workgroup of a tile, more for each further one, and how many run
 # together; 0 to 2 in bf16 parts (lin_split.hip), 5 on the f32 MFMA (1.3 us more a launch). One workgroup to a CU splits and multiplies in turn, and
 # the f32 MFMA is the faster one: 64 x 64, parts / f32, us: 65 x 4096 x 12288 356 / 226, 64 x 16384 x 4096 130 / 88, 256 x 2048 x 8704 249 / 162, in eight
@@ -208,15 +208,16 @@ GEMM_RATE = {7: (0, 1.57, 1.57), 3: (0, 1.0, 1.0), 6: (0, 0.97, 0.97), 2: (256, 
 # 2621 / 2223 / 2020 (3440).
 SPLIT_US = {0: (0.78, 0.30, 6), 1: (1.09, 0.49, 4), 2: (1.66, 0.87, 3), 5: (0.57, 0.57, 3)}
 
-# Launches of 129 to 512 rows that do not fill the chip with 256 x 128 tiles (weight rows x rows of a round by its time): 300 x 4096 x 4096 28 us
-# on 96 x 64, 34 on 64 x 64, 46 on 192 x 128; 200 x 6144 x 4096 27, 32, 49; 160 x 10240 x 4096 45, 37, 47; 400 x 6144 x 2048 27, 29, 29, 28 on 96 x 128.
-GEMM_RATE_MID = {8: (0, 0.47, 0.47), 0: (0, 0.51, 0.51), 11: (0, 0.655, 0.655), 6: (0, 1.1, 1.1)}
-
-
-# Microseconds of a round of 256 workgroups of a tile: fixed + per input column (from rounds at K = 512 .. 17408). With the sum of the slabs
-# behind it, 5 / 10 (64 x 64, 128 x 64): 65 x 640 x 4096 in eight splits 12.2 / 14.5 us, 128 x 1030 x 2090 in four 15.2 / 17.6, 65 x 2048 x 5632 in
-# four / eight 16.5 / 18.6.
-ROUND_US = {7: (8.0, 0.0215), 3: (8.0, 0.0151), 6: (8.0, 0.0112), 10: (5.0, 0.0075), 5: (5.0, 0.0042)}
+# bf16 launches of more than 64 rows, microseconds: fixed, then for a round of 256 workgroups of a tile, 1000 input columns of it, the same for the share of
+# the CUs that a round uses, a MB of weights. Fitted to 13500 launches of 23 shapes (640 to 35888 outputs, 1024 to 17408 inputs, 65 to 3000 rows, 1 to 8
+# splits of K) that lie 3 to 6 % around it. The tile it picks is 0.8 % behind the fastest of these on average; weighing rounds by a tile's multiply rate was
+# 4 to 8 % behind (300 x 4096 x 9216 57 / 34 us, 200 x 14336 x 2048 31 / 25, 300 x 24576 x 4096 89 / 65, 800 x 10240 x 4096 83 / 68), the tiles without PAIR
+# (lin_pair.hip) 5 % (300 x 10240 x 4096 47 / 38 us). Above 128 rows PAIR and the phased 256 x 256 tile leave nothing to 3 and 6.
+TILE_US = {5: (2.71, 2.74, 2.72, 0.71, 0.063), 8: (5.54, 0.23, 3.61, 0.69, 0.063), 10: (2.74, 3.17, 4.79, 0.88, 0.054), 11: (3.11, 3.76, 5.69, 1.14, 0.036),
+           7: (2.85, 11.5, 14.1, 6.61, 0.0), 3: (1.65, 7.86, 9.78, 2.78, 0.057), 6: (2.86, 5.35, 7.53, 2.44, 0.056),
+           PAIR(4, 4): (2.35, 5.38, 5.41, 1.75, 0.069), PAIR(4, 5): (2.60, 6.49, 6.51, 2.00, 0.048), PAIR(5, 4): (2.89, 6.35, 6.73, 1.61, 0.056),
+           PAIR(6, 4): (2.70, 6.68, 6.49, 2.69, 0.074), PAIR(6, 5): (2.78, 8.07, 7.72, 2.91, 0.055), PAIR(8, 4): (1.20, 9.64, 8.21, 3.02, 0.079),
+           PAIR(8, 5): (1.68, 11.3, 9.65, 3.38, 0.054)}
 
 
 class LinLaunch:
@@ -292,29 +293,21 @@ class LinLaunch:
             return False, 1, 16, 1
         if self.f32:
             return True, min(SPLIT_US, key=lambda c: self.split_us(c, M))
-        if M <= 128:
-            if 160 <= self._tiles(96, 128, M) <= 256:        # 128 x 24576 x 4096: 52 us, 61 on 192 x 128, 65 on 64 x 64
-                return True, 11
-            if n64 > 256 and self._tiles(96, 64, M) <= 256:  # 96 x 10240 x 4096: 34 us, 37 on 64 x 64, 53 on 192 x 128
-                return True, 8
-        rate = GEMM_RATE
-        if M > 512:
-            cand = list(rate)
-        elif self._tiles(256, 128, M) >= 120:
-            cand = [3, 6, 7]
-        elif n64 <= 256:
-            return True, 5
-        else:
-            rate = GEMM_RATE_MID
-            cand = list(rate)
-        if 7 in cand and min(s.w.nsub for s in self.segs) < 6:      # (its DMA runs two steps ahead)
-            cand.remove(7)
+        return True, min(self.tiles(M), key=lambda c: self.tile_us(c, M))
 
-        # rounds of 256 workgroups times a tile's cost
-        def cost(c):
-            n, (few, lo, hi) = self._tiles(*GEMM_TILES[c], M), rate[c]
-            return -(-n // 256) * GEMM_TILES[c][0] * GEMM_TILES[c][1] / (lo if n <= few else hi)
-        return True, min(cand, key=cost)
+    def tiles(self, M: int):
+        """The tiles that a bf16 launch of more than 64 rows chooses from."""
+        cand = [5, 8, 10, 11] + ([7] if min(s.w.nsub for s in self.segs) >= 6 else [])       # (7: its DMA runs two steps ahead)
+        if M <= 128 or any(s.s.xmap or s.s.ldx >> 22 or s.w.nsub >> 16 for s in self.segs):      # (what lin_pair.hip does not take)
+            return cand + [3, 6]
+        return cand + [c for c in TILE_US if c >= 256]
+
+    def tile_us(self, c: int, M: int, ks: int = 1) -> float:
+        """About the microseconds of a bf16 launch on tile c in ks splits of K."""
+        fixed, per_round, per_k, busy, mb = TILE_US[c]
+        n = self._tiles(*GEMM_TILES[c], M) * ks
+        k = max(s.w.nsub for s in self.segs) * 0.032 / ks
+        return fixed + -(-n // 256) * (per_round + per_k * k) + n / 256 * busy * k + mb * 1.024e-3 * sum(s.w.groups * -(-s.w.N // 16) * s.w.nsub for s in self.segs)
 
     def balanced(self, M: int) -> int:
         """The GEMM config of launches with up to 64 rows to a tile, which read each weight once: the tile whose rounds of 256 workgroups
@@ -349,8 +342,7 @@ class LinLaunch:
         return max(s.w.nsub for s in self.segs) / (2 * ks) * step + (1.3 if c == 5 else 0)
 
     def split_config(self, M: int):
-        """(config, K splits) of a launch of up to slab_rows rows that may split K (200 x 4096 x 6144: 32 us in 8 splits of 256 x 128, 26 in the
-        five of 192 x 128 that are chosen, 25.5 in two of 128 x 64; 41, 34 and 32 with the launch that adds the slabs)."""
+        """(config, K splits) of a launch of up to slab_rows rows that may split K."""
         n16 = self._tiles(16, 16, M)
         # 64 x 32 tiles, up to one to a CU (a few more take a second round: 24 x 2560 x 4096 8.9 us in six splits, 12.9 in seven). 16 rows, streaming /
         # these, us: 4096 x 17408 27.5 / 25.6, 4096 x 8192 15.3 / 14.6, 4096 x 4096 9.1 / 9.6, 2048 x 8704 9.9 / 10.3; 24 rows 28.6 / 25.5, 19.3 / 15.5, 13.5 / 10.6,
@@ -364,14 +356,9 @@ class LinLaunch:
             return (False, 1, 8, rt), -(-512 * rt // (2 * n16)) if M > 8 else -(-512 // n16)
         if M <= 32:
             return (False, 2, 4, 4 if n16 >= 256 else 2), 8
-        big, small = self._tiles(256, 128, M), self._tiles(64, 64, M)
-        if self.f32:
-            c, ks = self.cheapest(M, self.segs[0].slabs)
-            return (True, c), ks
-        if small > 256:
-            return ((True, 3), -(-256 // big)) if M > 128 and big * 8 >= 256 else ((True, 0), -(-512 // small))
-        if M <= 64:                       # one workgroup to a CU, 8 stages in flight: 64 x 4096 x 17408 34 us in 8 splits of 64 x 64 with
-            return (True, 5), 256 // small                                      # three, 31 in 4 (and half the slabs), 40 x 4096 x 9216 19, 18
+        if not self.f32 and M <= 64:      # one workgroup to a CU, 8 stages in flight: 64 x 4096 x 17408 34 us in 8 splits of 64 x 64 with
+            small = self._tiles(64, 64, M)                                      # three, 31 in 4 (and half the slabs), 40 x 4096 x 9216 19, 18
+            return ((True, 0), -(-512 // small)) if small > 256 else ((True, 5), 256 // small)
         c, ks = self.cheapest(M, self.segs[0].slabs)
         return (True, c), ks
 
@@ -383,10 +370,8 @@ class LinLaunch:
         def us(c, ks):
             if self.f32:
                 return self.split_us(c, M, ks) + (ks - 1) * M * s.w.N * 2e-6
-            fixed, per = ROUND_US[c]
-            rounds = -(-self._tiles(*GEMM_TILES[c], M) * ks // 256)
-            return rounds * (fixed + per * s.w.K / ks) + (ks - 1) * M * s.w.N * 2e-6
-        return min(((c, ks) for c in (SPLIT_US if self.f32 else ROUND_US) for ks in range(1, max(1, min(most, s.w.nsub // 16)) + 1)), key=lambda v: us(*v))
+            return self.tile_us(c, M, ks) + (ks - 1) * M * s.w.N * 2e-6
+        return min(((c, ks) for c in (SPLIT_US if self.f32 else self.tiles(M)) for ks in range(1, max(1, min(most, s.w.nsub // 16)) + 1)), key=lambda v: us(*v))
 
     def tall_split(self, M: int):
         """(config, K splits) of more rows than slab_rows: as many slabs of M rows as y holds. A narrow product has fewer tiles than

@@ -129,6 +129,44 @@ def test_balanced_tiles(K, cfg, M, N, Kd):
     assert relerr(y[:M], x.double() @ w.double().T) < 2e-6 and (y[M] == 7).all()
 
 
+@pytest.mark.parametrize("nt,mt", [(4, 4), (4, 5), (5, 4), (6, 4), (6, 5), (8, 4), (8, 5)])
+def test_paired_wave_groups(K, nt, mt):
+    """lin_pair.hip: one K-tile to more than the ring holds, whole and in splits, rows and outputs at and past a tile's edges, products per head, two
+    segments with an epilogue. The products are summed in 32 bits: |error| <= 2^-24 K sum |x| |w|."""
+    bf, c = torch.bfloat16, K.PAIR(nt, mt)
+    assert K.GEMM_TILES[c] == (32 * nt, 32 * mt)
+    for Kd, ks in ((61, 1), (64, 1), (130, 2), (256, 1), (257, 1), (320, 1), (700, 3), (1030, 8)):
+        for M, N in ((1, 4), (32 * mt, 32 * nt), (32 * mt + 1, 32 * nt + 4), (48 * mt + 7, 40 * nt + 13)):
+            x, w = rnd(M, Kd, seed=1).to(bf), rnd(N, Kd, seed=2).to(bf)
+            y = torch.full((ks * M + 1, N), 7.0, device="cuda")
+            L = K.LinLaunch([K.Seg(K.PackedLinear(w, False, "cuda"), act(x, K.act_ld(Kd)), y, slabs=ks, slab_rows=M)])
+            L._cfg[M] = (True, c), ks
+            assert L.run(M, st()) == ks and (y[ks * L.slab_rows:] == 7).all()
+            if ks > 1 and L.slab_rows != M:
+                continue
+            got, want = y[:ks * M].view(ks, M, N).sum(0).cpu().double(), x.double() @ w.double().T
+            bound = 2.0 ** -24 * (Kd + 8 + ks) * (x.double().abs() @ w.double().abs().T)
+            assert ((got - want).abs() <= bound + 2.0 ** -23 * want.abs()).all(), (Kd, ks, M, N)
+    M, Kd, G, N = 32 * mt + 5, 200, 3, 148
+    x, wg, ws = rnd(M, G * 256, seed=3).to(bf), rnd(G, N, Kd, seed=4).to(bf), (rnd(2 * N, Kd, seed=5) * Kd ** -0.5).to(bf)
+    x.view(M, G, 256)[:, :, Kd:] = 0
+    yg, ys = torch.full((M + 1, G * (N + 8)), 7.0, device="cuda"), torch.full((M + 1, N), 7.0, dtype=bf, device="cuda")
+    X = x.cuda()
+    L = K.LinLaunch([K.Seg(K.PackedLinear(ws, False, "cuda"), X, ys[:M], "siluglu"), K.Seg(K.PackedLinear(wg, False, "cuda"), X, yg[:M], xgs=256, ygs=N + 8)])
+    L._cfg[M] = (True, c), 1
+    L.run(M, st())
+    z = x[:, :Kd].double() @ ws.double().T
+    assert relerr(ys[:M], torch.nn.functional.silu(z[:, 0::2]) * z[:, 1::2]) < 3e-3 and (ys[M] == 7).all()      # (bf16 outputs round to 2^-9)
+    o = yg.view(M + 1, G, N + 8)
+    for i in range(G):
+        assert relerr(o[:M, i, :N], x[:, i * 256:i * 256 + Kd].double() @ wg[i].double().T) < 2e-6
+    assert (o[:, :, N:] == 7).all() and (o[M] == 7).all()
+    m = K.LinLaunch([K.Seg(K.PackedLinear(ws, False, "cuda"), X, ys[:M], "siluglu", xmap=torch.zeros(M, dtype=torch.int32, device="cuda"))])
+    m._cfg[M] = (True, c), 1
+    with pytest.raises(RuntimeError):
+        m.run(M, st())                               # (row maps go to other tiles)
+
+
 @pytest.mark.parametrize("T", [7, 32, 33, 200])
 def test_padding_rows_are_not_routed(K, T):
     """Rows without keys get no entries, in both forms of the plan; none at all when every row is padding."""

@@ -53,6 +53,18 @@ def test_splits_of_a_launch(N, Kd, pad, f32):
             assert c in (1, 2, 4) and more[0] in (4, 8, 16) and more[1] in (1, 2, 4)
 
 
+def test_tiles_of_some_hundred_rows():
+    """The tiles of lin_pair.hip: above 128 rows, where their workgroups fill the chip and whole rounds of the phased tile do not; never for row maps."""
+    pair = lambda L, M: L.config(M)[1] >= 256
+    for N, Kd, M in ((10240, 4096, 300), (14336, 2048, 200), (24576, 4096, 300), (10240, 2048, 800), (17944, 2048, 400), (6144, 4096, 640)):
+        L = launch(N, Kd)
+        assert pair(L, M) and not pair(L, 128)
+        L.segs[0].s.xmap = 1
+        assert not pair(L, M)
+    for N, Kd, M in ((2048, 2048, 200), (3072, 2048, 512), (1024, 4096, 1024), (24576, 4096, 512), (35888, 4096, 3000)):
+        assert not pair(launch(N, Kd), M)
+
+
 def test_equal_rounds():
     """Wide launches of few rows whose rounds sum up to the same weight rows on two tiles: 64 rows to a tile up to 40 rows, then 128."""
     for N in (26880, 32000, 32768):
