@@ -314,16 +314,19 @@ def _best11(rows, K: int, M: int, added: bool):
 
 
 def _launch_rows(segs):
-    """Rows of a launch's segments, those whose f16 copies lie behind each other as one (ops._merge_dense)."""
+    """Rows of a launch's segments, those whose f16 copies lie behind each other in one buffer (QWeight.expand_dense_group) as one. (Copies of
+    their own may lie behind each other too, as the allocator deals them: the choice does not hang on that.)"""
+    if len(segs) == 1:
+        return (segs[0].w.rows,)
     rows, end = [], None
     for s in segs:
-        w = s.w
-        at = w.d16.data_ptr() if len(segs) > 1 and getattr(w, "d16", None) is not None else None
+        d = getattr(s.w, "d16", None)
+        at = (d.untyped_storage().data_ptr(), d.data_ptr()) if d is not None else None
         if at is not None and at == end:
-            rows[-1] += w.rows
+            rows[-1] += s.w.rows
         else:
-            rows.append(w.rows)
-        end = None if at is None else at + 2 * w.rows * w.K
+            rows.append(s.w.rows)
+        end = None if at is None else (at[0], at[1] + 2 * s.w.rows * s.w.K)
     return tuple(rows)
 
 

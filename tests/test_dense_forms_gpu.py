@@ -16,6 +16,17 @@ class _W:
         self.type, self.rows, self.K = 12, rows, K
 
 
+def test_one_product_is_one_buffer():
+    """Copies count as one product's rows where they are neighbours in one buffer, not where the allocator has put two behind each other."""
+    from types import SimpleNamespace as NS
+
+    def seg(rows, at, buf):
+        return NS(w=NS(rows=rows, K=64, d16=NS(data_ptr=lambda: at, untyped_storage=lambda: NS(data_ptr=lambda: buf))))
+    assert tuning._launch_rows([seg(96, 0, 0), seg(32, 96 * 128, 0), seg(32, 128 * 128, 0)]) == (160,)
+    assert tuning._launch_rows([seg(96, 0, 0), seg(32, 96 * 128, 96 * 128), seg(32, 128 * 128, 96 * 128)]) == (96, 64)
+    assert tuning._launch_rows([seg(96, 0, 0), seg(32, 97 * 128, 0)]) == (96, 32)
+
+
 def test_rule_gives_built_forms():
     """The forms that the rule can choose are those that are built, with at least six K-tiles to a part; none for rows that its stores do not take."""
     for rows in (256, 2048, 4100, 6144, 16384, 28672):
