@@ -699,6 +699,16 @@ __global__ __launch_bounds__(256) void swiglu16_kernel(const act_t* __restrict__
 // in the memory-side Infinity Cache (MALL, 256 MB) / L2 instead of HBM -- the batch-1 decode experiment: stream
 // the NEXT projection's weights while a latency-bound kernel (attention, a GEMV's tail) leaves HBM idle. The
 // loaded words feed a sum that is stored only if it equals a value it never takes (keeps the loads alive).
+// Rows of 16-bit values that the head reads, up to a multiple of 16 with zeros: one launch where index_select, its index's conversion, the fill and
+// cat were four of 4 to 5 us. A workgroup to a row, 16 bytes a thread.
+__global__ __launch_bounds__(256) void gather_rows_kernel(const uint16_t* __restrict__ x, long ldx, int nx, const int* __restrict__ rows, int n, int D,
+                                                          uint16_t* __restrict__ out) {
+  const int r = blockIdx.x < n ? rows[blockIdx.x] : -1;
+  const bool in = r >= 0 && r < nx;
+  for (int c = threadIdx.x * 8; c < D; c += 2048)
+    *reinterpret_cast<uint4*>(out + (size_t)blockIdx.x * D + c) = in ? *reinterpret_cast<const uint4*>(x + (size_t)r * ldx + c) : uint4{0, 0, 0, 0};
+}
+
 __global__ __launch_bounds__(256) void prefetch_kernel(const uint4* __restrict__ p, long n16, uint32_t never,
                                                        uint32_t* __restrict__ sink) {
   uint32_t acc = 0;
@@ -720,6 +730,14 @@ __global__ __launch_bounds__(256) void prefetch_kernel(const uint4* __restrict__
 // ===========================================================================
 
 extern "C" {
+
+// out[i] = x[rows[i]] (x: nx rows of D 16-bit values, D and ldx multiples of 8), zeros from row n to npad and for indexes outside x
+int nls_gather_rows(const void* x, long ldx, int nx, const void* rows, int n, int npad, int D, void* out, void* stream) {
+  if (n < 1 || npad < n || nx < 1 || D < 8 || D % 8 || ldx % 8 || (((uintptr_t)x | (uintptr_t)out) & 15)) return -1;
+  hipLaunchKernelGGL(gather_rows_kernel, dim3(npad), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x, ldx, nx, (const int*)rows, n, D, (uint16_t*)out);
+  return (int)hipGetLastError();
+}
+
 
 int nls_prefetch(const void* p, long bytes, int blocks, void* stream) {
   if (bytes <= 0) return 0;

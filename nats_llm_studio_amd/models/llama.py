@@ -157,6 +157,7 @@ class StepBuffers:
     cnt: Optional[torch.Tensor] = None         # int32 tickets of the last-workgroup residual+RMSNorm GEMVs
     ssq: Optional[torch.Tensor] = None         # f32 [pad, ldss] split-RMSNorm partial sums of squares
     ldss: int = 0
+    hsel: Optional[torch.Tensor] = None        # [rows of logits, d] the normed rows that the head reads
 
 
 class LlamaModel:
@@ -425,6 +426,7 @@ class LlamaModel:
         )
         b.meta = meta
         b.pad = pad
+        b.hsel = torch.zeros((b.logits.shape[0] + 15) // 16 * 16, cfg.d_model, **act)     # the rows that the head reads
         # keys hold the reset value (argmax_unpack(rearm=True) leaves them so): the next step skips the reset.
         # Device keys start zeroed; a CPU buffer starts at zero too, which is not its reset value.
         b.keys_clean = dev.type == "cuda"
@@ -447,6 +449,11 @@ class LlamaModel:
                 sel=torch.zeros(pad * k, dtype=torch.int32, device=dev),
                 yexp=torch.zeros(pad * k, cfg.d_model, dtype=torch.float32, device=dev),
             )
+            # each expert's rows and count, of all layers (views: 3 us each to make, 24 a layer of eight experts)
+            m = b.moe
+            m["xe"], m["ye"] = ([m[n][e * pad:] for e in range(E)] for n in ("xrows", "yrows"))
+            m["ce"] = [m["counts"][e:e + 1] for e in range(E)]
+            m["layer"] = [(c, [c[e:e + 1] for e in range(E)]) for c in m["lcounts"]]
         return b
 
     def n_splits(self, T: int) -> int:
@@ -513,9 +520,9 @@ class LlamaModel:
                               block_size, cfg.attn_softmax_scale, chunk=-_MIN_CHUNK, n_split=n_split, workspace=b.attn_ws,
                               counters=b.attn_cnt)
             moe_norm = fused and lw.router16 is not None and T <= _MOE_NORM_ROUTE_T
-            moe_routed, counts = False, None
+            moe_routed, counts, each = False, None, None
             if route:
-                m, counts = b.moe, b.moe["lcounts"][L]
+                m, (counts, each) = b.moe, b.moe["layer"][L]
                 moe_routed = ops.qgemv_add_rmsnorm_route(
                     Seg(lw.wo), b.ao, x, lw.ffn_norm, b.h, T, cfg.residual_scale, cfg.eps, lw.router16, m["rlogits"],
                     cfg.n_expert_used, m["topw"], counts, m["xrows"], m["yrows"], x.shape[0], sel=m["sel"])
@@ -544,7 +551,7 @@ class LlamaModel:
             if cfg.n_expert:
                 fused_prev = self._moe(lw, b, T, nxt if (fused or self.ep_exchange) else None,
                                        lw.ffn_norm if moe_norm and not moe_routed else None, routed=moe_routed,
-                                       counts=counts if moe_routed else None)
+                                       counts=(counts, each) if moe_routed and each is not None else None)
             else:
                 ops.qgemv([Seg(lw.gateup)], b.h, b.act, T, epi="swiglu")
                 if fused:
@@ -562,8 +569,7 @@ class LlamaModel:
         n = T
         if logit_rows is not None:
             n = int(n_logits)
-            h = b.h.index_select(0, logit_rows[:n].long())
-            h = torch.cat([h, h.new_zeros((-n) % 16, h.shape[1])]) if n % 16 else h
+            h = ops.gather_rows(b.h, logit_rows, n, b.hsel)
         if not b.keys_clean:
             ops.argmax_reset(b.keys)
         # greedy-only steps keep just the fused arg-max keys (no [n, V] logits written)
@@ -606,8 +612,7 @@ class LlamaModel:
         if logit_rows is not None:             # (prefill-style row pick: normalise, then gather)
             ops.rmsnorm(x, self.out_norm, b.h, T, cfg.eps)
             n = int(n_logits)
-            h = b.h.index_select(0, logit_rows[:n].long())
-            h = torch.cat([h, h.new_zeros((-n) % 16, h.shape[1])]) if n % 16 else h
+            h = ops.gather_rows(b.h, logit_rows, n, b.hsel)
             if not b.keys_clean:
                 ops.argmax_reset(b.keys)
             ops.qgemv([Seg(self.lm_head, 0)], h, b.logits, n, alpha=1.0 / cfg.logit_scale, argmax=b.keys,
@@ -748,7 +753,7 @@ class LlamaModel:
 
     def _moe(self, lw: LayerWeights, b: StepBuffers, T: int, next_norm: Optional[torch.Tensor] = None,
              in_norm: Optional[torch.Tensor] = None, routed: bool = False,
-             counts: Optional[torch.Tensor] = None) -> bool:
+             counts=None) -> bool:
         """Top-k routed experts: router GEMV -> route kernel (per-expert row lists on device)
         -> grouped expert GEMVs (tiles of experts with no routed rows exit before reading
         weights) -> deterministic weighted combine into the residual. `in_norm` (<= 4 tokens): b.h is
@@ -760,7 +765,7 @@ class LlamaModel:
         m = b.moe
         k, E = cfg.n_expert_used, cfg.n_expert
         cap = b.x.shape[0]
-        counts = m["counts"] if counts is None else counts
+        counts, each = (m["counts"], m["ce"]) if counts is None else counts       # (one tensor, and each expert's)
         # routed: the o projection already normalised b.h and routed the tokens (ops.qgemv_add_norm_route, .._rmsnorm_route)
         if in_norm is not None and not routed:
             use_sel = self.device.type == "cuda" and T * k < len(self.experts)
@@ -805,7 +810,7 @@ class LlamaModel:
                 ops.moe_route(m["rlogits"][c0:], n, k, m["topw"], counts, m["xrows"], m["yrows"], cap,
                               sel=m["sel"] if (use_sel or exch) else None, counts_zeroed=zeroed and c0 == 0)
             loc = list(zip(self.experts, lw.exp_gateup, lw.exp_down))
-            segs = [Seg(gu, 0, m["xrows"][e * cap:], m["yrows"][e * cap:], counts[e:e + 1]) for e, gu, _ in loc]
+            segs = [Seg(gu, 0, m["xe"][e], m["ye"][e], each[e]) for e, gu, _ in loc]
 
             def sel(s0):
                 return (m["sel"], n * k, self.experts[0] + s0) if use_sel else None
@@ -813,7 +818,7 @@ class LlamaModel:
                 ops.qgemv(segs[s0:s0 + 8], b.h[c0:], b.act, n, epi="swiglu", sel=sel(s0), routed=n * k, **gu)
             if self.ep and not exch:           # rows routed to other ranks' experts stay zero
                 m["yexp"][:n * k].zero_()
-            segs = [Seg(dn, 0, m["yrows"][e * cap:], m["yrows"][e * cap:], counts[e:e + 1]) for e, _, dn in loc]
+            segs = [Seg(dn, 0, m["ye"][e], m["ye"][e], each[e]) for e, _, dn in loc]
             for s0 in range(0, len(segs), 8):
                 ops.qgemv(segs[s0:s0 + 8], b.act, m["yexp"], dn_rows if dn.get("ks", 1) > 1 else n, epi="f32",
                           sel=sel(s0), routed=n * k, **dn)

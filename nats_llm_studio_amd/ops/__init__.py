@@ -42,7 +42,7 @@ ACT_DTYPE = torch.float16   # activation dtype of every GEMM/GEMV input and SwiG
 
 
 def _stream_ptr(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())      # (an eager prompt asks some 30 times: 0.3 us, 4 through torch.cuda)
 
 
 def _p(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -287,11 +287,22 @@ def gemv_config(segs: Sequence[Seg], M: int):
     mode 4/5 = large-M dense f16 GEMM on the weights' f16 copies, 128/256 weight rows per workgroup
     (rt as mode 2)."""
     from . import tuning
-    if dense_ok(segs, M):
-        cfg = tuning.select_dense(segs, M)
-        if cfg is not None:
-            return cfg
-    return tuning.select(segs, M)
+    # by what the rules look at (a prompt's launches ask once for each layer and projection, 10 us each to work out)
+    key = [M, DENSE_MIN_M, _os.environ.get("NLS_TUNING_ROLE") if M <= 64 else None]
+    for s in segs:
+        w = s.w
+        key += (w.rows, w.K, w.type, s.ycol & 3, w.d16 is None, s.xmap is None, s.ymap is None)
+    memo = tuning.memo()
+    if len(segs) > 1 and M >= DENSE_MIN_M:
+        key += tuning._launch_rows(segs)
+    key = tuple(key)
+    cfg = memo.get(key)
+    if cfg is None:
+        cfg = tuning.select_dense(segs, M) if dense_ok(segs, M) else None
+        if cfg is None:
+            cfg = tuning.select(segs, M)
+        memo[key] = cfg
+    return cfg
 
 
 DENSE_MODES = (4, 5, 6, 10, 11)
@@ -627,6 +638,18 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, M: int, eps: fl
     return out
 
 
+def gather_rows(h: torch.Tensor, rows: torch.Tensor, n: int, out: torch.Tensor) -> torch.Tensor:
+    """h[rows[:n]], up to a multiple of 16 rows with zeros: in `out`, one launch, where it holds them, else a tensor of its own."""
+    np_ = (n + 15) // 16 * 16
+    if (h.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and n <= rows.numel() and np_ <= out.shape[0] and h.dtype == out.dtype
+            and h.shape[1] == out.shape[1] and h.element_size() == 2 and h.shape[1] % 8 == 0 and h.stride(0) % 8 == 0 and out.is_contiguous()):
+        _lib.check(_lib.lib().nls_gather_rows(h.data_ptr(), h.stride(0), h.shape[0], rows.data_ptr(), n, np_, h.shape[1], out.data_ptr(),
+                                              _stream_ptr(h)), "nls_gather_rows")
+        return out[:np_]
+    g = h.index_select(0, rows[:n].long())
+    return torch.cat([g, g.new_zeros(np_ - n, g.shape[1])]) if n % 16 else g
+
+
 def rope_inv_freq(head_dim: int, base: float, freq_factors=None) -> np.ndarray:
     """theta_i = base^(-2i/D), divided by GGUF `rope_freqs.weight` when present (Llama-3.1+ long-context
     frequency scaling, llama.cpp `rope_freq_factors`)."""
@@ -706,8 +729,10 @@ def qkv_rope_kv(segs: Sequence[Seg], h: torch.Tensor, qkv: torch.Tensor, pos: to
     summed inside the RoPE kernel (no separate reduce pass, no fp32 qkv round trip)."""
     if h.is_cuda and all(s.xmap is None for s in segs):
         mode, waves, rt, ks = cfg or gemv_config(segs, T)
-        ncol = sum(s.w.rows for s in segs)
-        contiguous = all(s.ycol == sum(x.w.rows for x in segs[:i]) for i, s in enumerate(segs))
+        ncol, contiguous = 0, True
+        for s in segs:
+            contiguous = contiguous and s.ycol == ncol
+            ncol += s.w.rows
         if (mode == 0 and T <= 64 and not neox and contiguous and ncol == (Hq + 2 * Hkv) * D and fuse_rope
                 and kc.dtype == torch.bfloat16):
             # path A: RoPE + KV append in the GEMV epilogue (no qkv round trip, no RoPE launch)
@@ -726,9 +751,6 @@ def qkv_rope_kv(segs: Sequence[Seg], h: torch.Tensor, qkv: torch.Tensor, pos: to
                                                _stream_ptr(h), ctypes.byref(fz)), "nls_qgemv_ex(rope)")
             return
     if h.is_cuda and all(s.xmap is None for s in segs) and norm is None:
-        mode, waves, rt, ks = cfg or gemv_config(segs, T)
-        ncol = sum(s.w.rows for s in segs)
-        contiguous = all(s.ycol == sum(x.w.rows for x in segs[:i]) for i, s in enumerate(segs))
         if (mode in (4, 5, 10, 11) and ks == 1 and contiguous and ncol == (Hq + 2 * Hkv) * D
                 and not neox and fuse_rope and kc.dtype == torch.bfloat16):
             # large-M GEMM on the dense f16 copies with RoPE + KV append in its epilogue (no f32 qkv round trip,

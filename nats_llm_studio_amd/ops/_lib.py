@@ -48,6 +48,7 @@ _SIGS = {
     "nls_qgemv_norm": [ctypes.POINTER(NlsSeg), c_int, c_void_p, c_long, c_void_p, c_float, c_void_p, c_long, c_int,
                        c_float, c_int, c_void_p, c_int, c_int, c_void_p],
     "nls_prefetch": [c_void_p, c_long, c_int, c_void_p],
+    "nls_gather_rows": [c_void_p, c_long, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p],
     "nls_graph_kernel_names": [c_void_p, c_void_p, c_long],
     "nls_epx_bytes": [c_int, c_int],
     "nls_epx_wgs": [],

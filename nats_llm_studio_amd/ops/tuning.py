@@ -53,6 +53,18 @@ def table():
     return _TABLE
 
 
+_MEMO, _MEMO_OF = {}, None
+
+
+def memo() -> dict:
+    """Configs worked out so far (ops.gemv_config), for the table as it is loaded."""
+    global _MEMO, _MEMO_OF
+    t = table()
+    if _MEMO_OF is not t or len(_MEMO) > 8192:
+        _MEMO, _MEMO_OF = {}, t
+    return _MEMO
+
+
 # Microseconds of a launch of quantised rows on shapes without a tuned entry, fitted to 39000 launches of 30 shapes (1536 to 128256 rows, K 1536 to 28672,
 # Q4_K, Q5_K, Q6_K and Q8_0, the launch behind it included, weights streamed). (mode, waves, rt): workgroups that share a CU, and what a last round of at
 # most one to a CU takes of a whole one; then of the launch: fixed, a round, a round's K (times bytes a weight up to 8 rows) / 4096, the same for each
