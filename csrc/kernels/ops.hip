@@ -330,6 +330,67 @@ __global__ __launch_bounds__(256) void embed_kernel(int* __restrict__ ids, WDesc
   }
 }
 
+// The gather and the first layer's RMSNorm in one launch (rmsnorm_kernel's sums, one workgroup to a token), and `zero`, nz words that the step's
+// launches count in: at 32 rows of 2048 each of the three took 4 to 4.7 us, which is what a launch with one round trip to memory takes.
+template <int TYPE>
+DEVI void embed_norm_row(const WDesc& W, int id, float* __restrict__ o, float scale, const float* __restrict__ w, act_t* __restrict__ h, float eps) {
+  __shared__ float sh[8];
+  const int D = W.K;
+  float4 v[4], wv[4];
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = (threadIdx.x + j * 512) * 4;
+    v[j] = wv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i < D) {
+      wv[j] = *reinterpret_cast<const float4*>(w + i);
+      v[j] = make_float4(scale * dequant_elem(W, TYPE, id, i), scale * dequant_elem(W, TYPE, id, i + 1), scale * dequant_elem(W, TYPE, id, i + 2),
+                         scale * dequant_elem(W, TYPE, id, i + 3));
+      *reinterpret_cast<float4*>(o + i) = v[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+  ss = block_sum<512>(ss, sh);
+  const float inv = rsqrtf(ss / (float)D + eps);
+  typedef act_t act4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int i = (threadIdx.x + j * 512) * 4;
+    if (i < D)
+      *reinterpret_cast<act4*>(h + i) = act4{(act_t)(v[j].x * inv * wv[j].x), (act_t)(v[j].y * inv * wv[j].y), (act_t)(v[j].z * inv * wv[j].z),
+                                             (act_t)(v[j].w * inv * wv[j].w)};
+  }
+}
+
+__global__ __launch_bounds__(512) void embed_norm_kernel(int* __restrict__ ids, WDesc W, int type, float* __restrict__ out, long ldo, float scale,
+                                                         const int* __restrict__ next_ids, const int* __restrict__ use_prev,
+                                                         const float* __restrict__ w, act_t* __restrict__ h, long ldh, float eps,
+                                                         int* __restrict__ zero, int nz) {
+  const int t = blockIdx.x;
+  if (t == 0)
+    for (int i = threadIdx.x; i < nz; i += 512) zero[i] = 0;
+  int id = ids[t];
+  if (next_ids) {
+    if (use_prev[t]) id = next_ids[t];
+    __syncthreads();                         // every thread has read ids[t] before it is rewritten
+    if (threadIdx.x == 0) ids[t] = id;
+  }
+  id = min(max(id, 0), W.rows - 1);          // (as embed_kernel)
+  float* o = out + (size_t)t * ldo;
+  h += (size_t)t * ldh;
+  switch (type) {
+    case QT_F32: embed_norm_row<QT_F32>(W, id, o, scale, w, h, eps); break;
+    case QT_F16: embed_norm_row<QT_F16>(W, id, o, scale, w, h, eps); break;
+    case QT_BF16: embed_norm_row<QT_BF16>(W, id, o, scale, w, h, eps); break;
+    case QT_Q8_0: embed_norm_row<QT_Q8_0>(W, id, o, scale, w, h, eps); break;
+    case QT_Q4_K: embed_norm_row<QT_Q4_K>(W, id, o, scale, w, h, eps); break;
+    case QT_Q5_K: embed_norm_row<QT_Q5_K>(W, id, o, scale, w, h, eps); break;
+    case QT_Q6_K: embed_norm_row<QT_Q6_K>(W, id, o, scale, w, h, eps); break;
+    default: break;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Whole-tensor dequant to f16 (tests / debugging). One wave = 16 rows
 // x one 256 super-block, using the same register dequant as the GEMV.
@@ -825,6 +886,17 @@ int nls_embed_prev(int* ids, const int* next_ids, const int* use_prev, int T, co
   WDesc W{(const uint8_t*)w, rows, K};
   hipLaunchKernelGGL(embed_kernel, dim3(T, (K + 255) / 256), dim3(256), 0, (hipStream_t)stream, ids, W, type, out,
                      ldo, scale, next_ids, use_prev);
+  return (int)hipGetLastError();
+}
+
+// nls_embed_prev (next_ids null: nls_embed), then h[t] = f16(rmsnorm(out[t]) * nw); zero: nz words (null: none). -1: rows it does not take
+int nls_embed_norm(int* ids, const int* next_ids, const int* use_prev, int T, const void* w, int type, int rows, int K, float* out, long ldo,
+                   float scale, const float* nw, void* h, long ldh, float eps, int* zero, int nz, void* stream) {
+  if (T < 1 || K % 4 || K > 8192 || ldo % 4 || ldh % 4 || (((uintptr_t)out | (uintptr_t)nw) & 15) || ((uintptr_t)h & 7)) return -1;
+  if (type != QT_F32 && type != QT_F16 && type != QT_BF16 && type != QT_Q8_0 && type != QT_Q4_K && type != QT_Q5_K && type != QT_Q6_K) return -1;
+  WDesc W{(const uint8_t*)w, rows, K};
+  hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(512), 0, (hipStream_t)stream, ids, W, type, out, ldo, scale, next_ids, use_prev, nw, (act_t*)h,
+                     ldh, eps, zero, zero ? nz : 0);
   return (int)hipGetLastError();
 }
 

@@ -800,6 +800,23 @@ def embed(ids: torch.Tensor, w: QWeight, out: torch.Tensor, T: int, scale: float
     return out
 
 
+def embed_norm(ids: torch.Tensor, w: QWeight, out: torch.Tensor, T: int, nw: torch.Tensor, h: torch.Tensor, eps: float, scale: float = 1.0,
+               prev=None, zero: Optional[torch.Tensor] = None):
+    """embed, then rmsnorm(out, nw, h), and `zero` (int32) cleared: one launch on the GPU where the rows allow it."""
+    if ids.is_cuda and h.dtype == ACT_DTYPE and out.shape[1] == w.K and (zero is None or (zero.dtype == torch.int32 and zero.is_contiguous())):
+        nxt, use = prev if prev is not None else (None, None)
+        rc = _lib.lib().nls_embed_norm(ids.data_ptr(), _p(nxt), _p(use), T, w.data.data_ptr(), w.type, w.rows, w.K, out.data_ptr(), out.stride(0),
+                                       float(scale), nw.data_ptr(), h.data_ptr(), h.stride(0), float(eps), _p(zero),
+                                       0 if zero is None else zero.numel(), _stream_ptr(ids))
+        if rc != -1:
+            _lib.check(rc, "nls_embed_norm")
+            return
+    embed(ids, w, out, T, scale, prev=prev)
+    rmsnorm(out, nw, h, T, eps)
+    if zero is not None:
+        zero.zero_()
+
+
 def attention(q: torch.Tensor, kc: torch.Tensor, vc: torch.Tensor, block_tables: torch.Tensor,
               tok_seq: torch.Tensor, ctx_len: torch.Tensor, out: torch.Tensor, T: int, Hq: int, Hkv: int, D: int,
               block_size: int, scale: float, chunk: int = 256, n_split: int = 1,

@@ -70,6 +70,8 @@ _SIGS = {
     "nls_embed": [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_float, c_void_p],
     "nls_embed_prev": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_float,
                        c_void_p],
+    "nls_embed_norm": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_float, c_void_p, c_void_p, c_long,
+                       c_float, c_void_p, c_int, c_void_p],
     "nls_dequant": [c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_void_p],
     "nls_swiglu16": [c_void_p, c_long, c_int, c_int, c_float, c_void_p, c_long, c_void_p],
     "nls_argmax": [c_void_p, c_long, c_int, c_int, c_void_p, c_void_p],
