@@ -298,8 +298,8 @@ class LinLaunch:
     def tiles(self, M: int):
         """The tiles that a bf16 launch of more than 64 rows chooses from."""
         cand = [5, 8, 10, 11] + ([7] if min(s.w.nsub for s in self.segs) >= 6 else [])       # (7: its DMA runs two steps ahead)
-        if M <= 128 or any(s.s.xmap or s.s.ldx >> 22 or s.w.nsub >> 16 for s in self.segs):      # (what lin_pair.hip does not take)
-            return cand + [3, 6]
+        if M <= 128 or any(getattr(s.s, "xmap", None) or getattr(s.s, "ldx", 0) >> 22 or s.w.nsub >> 16 for s in self.segs):
+            return cand + [3, 6]                # (lin_pair.hip takes no row maps, and offsets of 32 bits)
         return cand + [c for c in TILE_US if c >= 256]
 
     def tile_us(self, c: int, M: int, ks: int = 1) -> float:
