@@ -563,7 +563,7 @@ class LightningPart(_SharedPart):
         if T == n and V % 4 == 0 and V <= 1024:
             K.gla_step(e["q"], e["k"], e["v"], self.a, None, 1.0, S, b.runs, T, None, None, None, H, D, V, eps, st, o=e["o"])
         else:
-            shape = K.gla_shape(T, n, H, V, D, step.longest)
+            shape = K.narrow_shape("gla", K.gla_shape(T, n, H, V, D, step.longest), T, n, H, V, D, step.longest, e["q"].dtype == torch.float32)
             seg = None
             if shape[0] > 1:
                 seg = (self.m.grown(b, "gla.seg", n * shape[0], H * D * V, torch.float32),
@@ -621,7 +621,7 @@ class DeltaPart(_SharedPart):
         z, y = self.scratch(b, "delta.z", P, self.ld), self.scratch(b, "delta.y", P, K.pad_to(self.nch, 8))
         fac, beta = self.scratch(b, "delta.fac", P, 2 * c.kv_heads, f), self.scratch(b, "delta.beta", P, c.heads, f)
         a, g = self.scratch(b, "delta.a", P, HD, f), self.scratch(b, "delta.g", P, K.pad_to(HV, 8))
-        o = self.scratch(b, "delta.o", P, HV, f) if c.vdim > 128 else None
+        o = self.scratch(b, "delta.o", P, HV, f) if c.vdim > (64 if 64 < c.dim <= 128 else 128) else None
         return dict(z=z, q=y, k=y[:, GD:], v=y[:, 2 * GD:], fac=fac, beta=beta, a=a, g=g, o=o, out=out,
                     low=z[:, self.low:], lowg=z[:, self.lowg:],
                     inputs=[K.Seg(self.zw, x, z), K.Seg(self.b, x, beta, "sigmoid")],
@@ -642,7 +642,7 @@ class DeltaPart(_SharedPart):
             K.delta_step(*qkv, None if own else e["a"], (e["low"], self.a2r, self.dt, self.rate), None if own else e["g"],
                          (e["lowg"], self.g2r), self.ld, S, b.runs, T, self.norm, e["out"], H, G, D, V, eps, st)
             return
-        shape = K.delta_shape(T, n, H, D, V, step.longest)
+        shape = K.narrow_shape("delta", K.delta_shape(T, n, H, D, V, step.longest), T, n, H, V, D, step.longest, e["q"].dtype == torch.float32)
         seg = None
         if shape[0] > 1:
             seg = (self.m.grown(b, "delta.seg", n * shape[0], H * D * V, torch.float32),

@@ -629,7 +629,9 @@ def scan_out(o, norm, gate, out, H: int, D: int, T: int, eps: float, st: int):
 # that finds what the segments end with, what segments add, the chain of their states: per segment in all, per segment of a run,
 # workgroups of that pass per one of the last.) Fitted to 400 launches of 1 to 64 runs of 60 to 3500 tokens, 16 and 32 heads of
 # 128 x 128, 1 to 16 segments: the count it picks is 0.6 % (gla) and 0.2 % (delta) behind the fastest on average.
-SEGMENT_US = {"gla": (32.4, 0.3424, 0.1862, -10.0, 0.05, 0.0, 1), "delta": (52.5, 0.59, 0.35, -36.0, 0.2215, 9.0, 2)}
+SEGMENT_US = {"gla": (32.4, 0.3424, 0.1862, -10.0, 0.05, 0.0, 1), "delta": (52.5, 0.59, 0.35, -36.0, 0.2215, 9.0, 2),
+              # the same on 64 value columns (narrow_shape), delta with the norm's launch behind it; 160 launches of 1 to 214 runs, 15 %
+              "gla1": (9.17, 0.311, 0.0593, 3.97, 0.0404, 1.3, 1), "delta1": (12.9, 0.483, 0.182, 0.0, 0.0818, 12.4, 2)}
 
 
 def segments_us(kind: str, tokens: int, wgs: float, nseg: int) -> float:
@@ -667,6 +669,27 @@ def gla_shape(T: int, nruns: int, H: int, V: int, D: int = 64, longest: Optional
     if longest is None:                                  # (no run can have more tokens than this)
         return 1 if wgs * nruns >= 256 else max(1, min(most, (T - nruns + 1) // 64)), nt
     return 1 if wgs * nruns >= 256 or longest <= 128 else min(most, -(-longest // 64)), nt
+
+
+def narrow_shape(kind: str, shape, T: int, nruns: int, H: int, V: int, D: int, longest: Optional[int], f32: bool):
+    """The shape of a launch over 65 to 128 channels and more than 64 value columns, or that of workgroups of 64 columns: half of the products to each,
+    and (delta) LDS for four chunks, which the four waves prepare side by side; with 128 columns two of them do and two wait. They are the faster ones
+    where whole rounds of CUs are not lost: twice as many, all at once (delta in 32 bits: always). The head's norm is then a launch of its own.
+    us with 128 / 64 columns, 128 x 128, bf16: delta, 16 heads, 6 runs of 650 tokens 451 / 301, 7 of 86 79 / 63, 1 of 40 40 / 31, 1 of 700 228 / 198; 32
+    heads, 1 of 330 189 / 152, 3 of 700 468 / 318, but 8 of 300 253 / 296; 32 bits 6 x 650 565 / 336, 214 of 16 519 / 474; plain, 16 heads, 1 of 330
+    59 / 49, 6 of 650 209 / 196. What it picks is 1 % behind the fastest on average, 128 columns were 16 (32 bits: 30) and 6 (8) %."""
+    nseg, nt = shape
+    if nt != 2 or not 64 < D <= 128:
+        return shape
+    tokens = longest or -(-T // nruns)
+    wide, narrow = H * -(-V // 128), H * -(-V // 64)
+    most = min(-(-(256 if kind == "delta" else 512) // (wide * nruns)), 16, max(1, -(-tokens // 64)))     # (as much scratch as the shape's)
+    fit = [s for s in range(1, most + 1) if narrow * nruns * s <= 256 or (s == 1 and f32 and kind == "delta")]
+    us = lambda s: segments_us(kind + "1", tokens, narrow * T / tokens, s)
+    best = min(fit, key=us, default=None)
+    if best is None or not (f32 and kind == "delta") and us(best) >= segments_us(kind, tokens, wide * T / tokens, nseg):
+        return shape
+    return best, 1
 
 
 def gla_scan(q, k, v, a, qscale: float, o, norm, gate, out, state, runs, nruns: int, H: int, D: int, V: int, eps: float, shape,

@@ -34,3 +34,23 @@ def test_short_runs_are_not_cut(H, D, V):
             assert K.gla_shape(n * runs, runs, H, V, D, n)[0] == K.delta_shape(n * runs, runs, H, D, V, n)[0] == 1
     assert K.gla_shape(256, 1, H, V, D, 256)[0] == (4 if D <= 64 or D > 128 else K.segments("gla", 256, 256, H * -(-V // 128), 16))
     assert K.gla_shape(256, 1, H, V, D, 256)[0] >= 3
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("kind", ["gla", "delta"])
+def test_narrow_workgroups(kind, f32):
+    """64 value columns to a workgroup where they are all under way at once, in no more segments than whole chunks and no more scratch; never for other
+    widths than the kernels that gain."""
+    shape = lambda T, n, H, V, D, l: K.gla_shape(T, n, H, V, D, l) if kind == "gla" else K.delta_shape(T, n, H, D, V, l)
+    for H, n, tokens in ((16, 1, 40), (16, 6, 650), (16, 7, 86), (32, 1, 330), (32, 3, 700), (16, 8, 300), (16, 1, 2000), (1, 64, 60), (32, 214, 16)):
+        T, old = n * tokens, shape(n * tokens, n, H, 128, 128, tokens)
+        nseg, nt = K.narrow_shape(kind, old, T, n, H, 128, 128, tokens, f32)
+        if nt == 2:
+            assert (nseg, nt) == old
+        else:
+            assert 1 <= nseg <= max(1, -(-tokens // 64)) and (nseg - 1) * H * n < (512 if kind == "gla" else 256)
+            assert 2 * H * n * nseg <= 256 or (f32 and kind == "delta" and nseg == 1)
+        assert not (kind == "delta" and 2 * H * n <= 256 and tokens < 1000) or nt == 1
+        for V, D in ((64, 128), (128, 64), (128, 129)):
+            old = shape(T, n, H, V, D, tokens)
+            assert K.narrow_shape(kind, old, T, n, H, V, D, tokens, f32) == old
