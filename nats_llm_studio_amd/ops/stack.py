@@ -212,7 +212,7 @@ SPLIT_US = {0: (0.78, 0.30, 6), 1: (1.09, 0.49, 4), 2: (1.66, 0.87, 3), 5: (0.57
 # the CUs that a round uses, a MB of weights. Fitted to 13500 launches of 23 shapes (640 to 35888 outputs, 1024 to 17408 inputs, 65 to 3000 rows, 1 to 8
 # splits of K) that lie 3 to 6 % around it. The tile it picks is 0.8 % behind the fastest of these on average; weighing rounds by a tile's multiply rate was
 # 4 to 8 % behind (300 x 4096 x 9216 57 / 34 us, 200 x 14336 x 2048 31 / 25, 300 x 24576 x 4096 89 / 65, 800 x 10240 x 4096 83 / 68), the tiles without PAIR
-# (lin_pair.hip) 5 % (300 x 10240 x 4096 47 / 38 us). Above 128 rows PAIR and the phased 256 x 256 tile leave nothing to 3 and 6.
+# (lin_pair.hip) 5 % (300 x 10240 x 4096 47 / 38 us).
 TILE_US = {5: (2.71, 2.74, 2.72, 0.71, 0.063), 8: (5.54, 0.23, 3.61, 0.69, 0.063), 10: (2.74, 3.17, 4.79, 0.88, 0.054), 11: (3.11, 3.76, 5.69, 1.14, 0.036),
            7: (2.85, 11.5, 14.1, 6.61, 0.0), 3: (1.65, 7.86, 9.78, 2.78, 0.057), 6: (2.86, 5.35, 7.53, 2.44, 0.056),
            PAIR(4, 4): (2.35, 5.38, 5.41, 1.75, 0.069), PAIR(4, 5): (2.60, 6.49, 6.51, 2.00, 0.048), PAIR(5, 4): (2.89, 6.35, 6.73, 1.61, 0.056),
@@ -300,12 +300,16 @@ class LinLaunch:
         cand = [5, 8, 10, 11] + ([7] if min(s.w.nsub for s in self.segs) >= 6 else [])       # (7: its DMA runs two steps ahead)
         if M <= 128 or any(getattr(s.s, "xmap", None) or getattr(s.s, "ldx", 0) >> 22 or s.w.nsub >> 16 for s in self.segs):
             return cand + [3, 6]                # (lin_pair.hip takes no row maps, and offsets of 32 bits)
-        return cand + [c for c in TILE_US if c >= 256]
+        return cand + [c for c in TILE_US if c >= 256] + [3, 6]
 
     def tile_us(self, c: int, M: int, ks: int = 1) -> float:
         """About the microseconds of a bf16 launch on tile c in ks splits of K."""
         fixed, per_round, per_k, busy, mb = TILE_US[c]
         n = self._tiles(*GEMM_TILES[c], M) * ks
+        # (long prompts: from the third round on the phased tile, whose workgroups stay, is faster in a running step, 2994 x 12288 x 4096 249 us, 269 on
+        # PAIR(8, 5). Fewer rows fill its tiles badly: a pass of 600 on four products of 35888 x 4096 1.61 ms, 1.53 on PAIR(6, 5))
+        if c >= 256 and n > 512 and M > 1024:
+            return float("inf")
         k = max(s.w.nsub for s in self.segs) * 0.032 / ks
         return fixed + -(-n // 256) * (per_round + per_k * k) + n / 256 * busy * k + mb * 1.024e-3 * sum(s.w.groups * -(-s.w.N // 16) * s.w.nsub for s in self.segs)
 
