@@ -115,6 +115,9 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
       (waves != 4 && waves != 8 && !(waves == 16 && mode >= 4) && !(waves == 7 && mode == 1 && rt == 1 && M == 1)))
     return -1;
   if (mode < 0 || mode > 11 || mode == 7 || mode == 8 || (mode == 6 && (waves != 8 || rt != 2))) return -1;
+  if (mode >= 9 && (epi != EPI_ARGMAX || ks > 1))       // (their stores are 4 columns wide, in slabs too)
+    for (int i = 0; i < nseg; ++i)
+      if (segs[i].rows % 4) return -1;
   if (mode >= 10) {            // mode 10: rt 1: 256-row weight tiles, rt 2: 128-row
     if (waves != 8 || (mode == 10 ? rt != 1 && rt != 2 : (rt >> 8) != 2 && (rt >> 8) != 4) || fz->xf || fz->onw || ldx % 8 ||
         ((epi == EPI_F32 || epi == EPI_ADD_F32 || epi == EPI_ACT) && ldy % 4))

@@ -308,6 +308,20 @@ def gemv_config(segs: Sequence[Seg], M: int):
 DENSE_MODES = (4, 5, 6, 10, 11)
 
 
+def fitting_config(cfg, segs: Sequence[Seg], M: int, x: torch.Tensor, y: Optional[torch.Tensor], epi: str):
+    """cfg, as gemv_config chose it by sizes alone, or the launch of the same products that takes x and y wherever their rows lie: modes 3 and
+    up copy 16 aligned bytes of x's rows to LDS, modes 9 to 11 store 4 columns at a time, in slabs too (y None: another launch writes it). A product
+    of 8195 rows in two splits put three columns of one slab row over the next one's first."""
+    from . import tuning
+    mode, ks = cfg[0], cfg[3]
+    if mode >= 3 and (x.stride(0) % 8 or x.data_ptr() % 16):
+        return tuning.any_rows(segs, M)
+    if mode >= 9 and (epi != "argmax" or ks > 1) and (any((s.ycol | s.w.rows) % 4 for s in segs)
+                                                      or (y is not None and epi in ("f32", "add", "act") and y.stride(0) % 4)):
+        return tuning.any_rows(segs, M) if mode == 9 else tuning.dense_heuristic(segs, M, aligned=False)
+    return cfg
+
+
 def _merge_dense(segs: Sequence[Seg]):
     """[d16 pointer, rows, K, ycol, seg] per launch segment: adjacent unmapped segments whose f16 copies are consecutive
     rows of one buffer (QWeight.expand_dense_group) and whose output columns are adjacent merge into one."""
@@ -427,9 +441,8 @@ def qgemv(segs: Sequence[Seg], x: torch.Tensor, y: torch.Tensor, M: int, alpha: 
             if argmax is not None and not mapped:
                 from . import tuning
                 mode, waves, rt, ks = tuning.argmax_config((mode, waves, rt, ks), segs, M)
-            if mode >= 10 and (x.stride(0) % 8 or y.stride(0) % 4):
-                from . import tuning
-                mode, waves, rt, ks = tuning.dense_heuristic(segs, M, aligned=False)
+            if not mapped:
+                mode, waves, rt, ks = fitting_config((mode, waves, rt, ks), segs, M, x, y, epi)
         if M > 64 and mode == 0:
             # mapped (MoE) rows / path A: chunks of 64 rows
             for m0 in range(0, M, 64):

@@ -128,6 +128,19 @@ def _mid_rule(rows, K: int, types, M: int, role: str):
     return (mode, 8 if mode == 2 else 4, rt, ks)
 
 
+def any_rows(segs, M: int):
+    """More than 64 rows: the launch that takes rows of x and y at any place, through registers on both sides."""
+    if not all(int(s.w.type) in _QUANT for s in segs):
+        return (1, 8, 1, 1)      # MFMA GEMM: 128 weight rows x 128 activation rows per workgroup
+    # LDS-dequant GEMM (mode 2): 128 weight rows x 256 (or 128) activation rows per workgroup;
+    # split K until the grid covers the 256 CUs (the measured winners on the 8B shapes)
+    tiles = sum((s.w.rows + 127) // 128 for s in segs) * ((M + 255) // 256)
+    ks, nb = 1, segs[0].w.K // 256
+    while tiles * ks < 256 and ks * 2 <= max(1, nb // 4):
+        ks *= 2
+    return (2, 8, 4 if M >= 192 else 2, ks)
+
+
 def heuristic(segs, M: int):
     rows = sum(s.w.rows for s in segs)
     K = segs[0].w.K
@@ -145,25 +158,19 @@ def heuristic(segs, M: int):
             return (1, 4, 2, 2) if rows >= 16 * K and K >= 1024 else (1, 4, 2, 1)
         return (0, 4, 2, 1) if len(segs) > 1 else (0, 4, 1, 1)
     if M > 64:
-        if quant:
-            if rows >= 4 * K or K >= 2 * rows:
-                # wide (gate|up, LM head) and down-projection shapes: the quantised GEMM on the raw tile-blocks
-                # (mode 9, 256 weight rows x 256 activation rows) won every measured one at M >= 256 -- Llama-3-8B
-                # gate|up / LM head, Llama-3-70B gate|up / down / LM head by 10-20 % over mode 2
-                # (profiles/tune_quant_70b_r05.txt); split K until the grid covers the 256 CUs
-                tiles = sum((s.w.rows + 255) // 256 for s in segs) * ((M + 255) // 256)
-                ks, nb = 1, K // 256
-                while tiles * ks < 256 and ks * 2 <= min(8, max(1, nb // 4)):    # (ks <= 8: the tuned range)
-                    ks *= 2
-                return (9, 8, 2, ks)
-            # LDS-dequant GEMM (mode 2): 128 weight rows x 256 activation rows per workgroup;
-            # split K until the grid covers the 256 CUs (the measured winners on the 8B shapes)
-            tiles = sum((s.w.rows + 127) // 128 for s in segs) * ((M + 255) // 256)
+        if quant and (rows >= 4 * K or K >= 2 * rows):
+            # wide (gate|up, LM head) and down-projection shapes: the quantised GEMM on the raw tile-blocks
+            # (mode 9, 256 weight rows x 256 activation rows) won every measured one at M >= 256 -- Llama-3-8B
+            # gate|up / LM head, Llama-3-70B gate|up / down / LM head by 10-20 % over mode 2
+            # (profiles/tune_quant_70b_r05.txt); split K until the grid covers the 256 CUs.
+            # Q8_0 too, path B / this (mode 2 where rows are not wide), us: 28672 x 4096 at 256 / 1000 / 3000 rows 120 / 113, 355 / 232, 1128 / 732,
+            # 2048 x 8192 86 / 43, 85 / 59, 178 / 148, 6144 x 4096 51 / 36, 97 / 91, 250 / 223, but 16384 x 2048 at 256 37 / 49, 6144 x 4096 at 512 51 / 62
+            tiles = sum((s.w.rows + 255) // 256 for s in segs) * ((M + 255) // 256)
             ks, nb = 1, K // 256
-            while tiles * ks < 256 and ks * 2 <= max(1, nb // 4):
+            while tiles * ks < 256 and ks * 2 <= min(8, max(1, nb // 4)):    # (ks <= 8: the tuned range)
                 ks *= 2
-            return (2, 8, 4, ks)
-        return (1, 8, 1, 1)      # MFMA GEMM: 128 weight rows x 128 activation rows per workgroup
+            return (9, 8, 2, ks)
+        return any_rows(segs, M)
     waves, rt = 8, 1
     tiles = sum((s.w.rows + waves * rt * 16 - 1) // (waves * rt * 16) for s in segs)
     ks = 1
