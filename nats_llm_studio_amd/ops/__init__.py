@@ -534,7 +534,7 @@ def qgemv_add_rmsnorm(seg: Seg, xin: torch.Tensor, x: torch.Tensor, norm_w: torc
     path-A launch (M <= ADDNORM_MAX_M, `counter`: a zeroed int32 device word) normalises in its last
     workgroup, so the norm costs no launch at all."""
     if x.is_cuda and seg.xmap is None:
-        mode, waves, rt, ks = cfg or gemv_config([seg], M)
+        mode, waves, rt, ks = cfg or fitting_config(gemv_config([seg], M), [seg], M, xin, None, "slabs")
         if (mode == 0 and counter is not None and M <= ADDNORM_MAX_M and seg.ycol == 0
                 and seg.w.rows == x.shape[1]):
             fz = _lib.NlsFuse(hout=h.data_ptr(), ldh=h.stride(0), onw=norm_w.data_ptr(), cnt=counter.data_ptr(),
@@ -575,7 +575,7 @@ def qgemv_add_rmsnorm_route(seg: Seg, xin: torch.Tensor, x: torch.Tensor, nw: to
     if (not x.is_cuda or seg.xmap is not None or seg.ycol or seg.w.rows != x.shape[1] or D != x.shape[1] or E not in (2, 4, 8)
             or k > E or D % 8 or D > 8192 or wr.dtype != ACT_DTYPE or not wr.is_contiguous() or logits.stride(0) != E or cap < M):
         return False
-    mode, waves, rt, ks = gemv_config([seg], M)
+    mode, waves, rt, ks = fitting_config(gemv_config([seg], M), [seg], M, xin, None, "slabs")
     st, L, ws = _stream_ptr(x), _lib.lib(), None
     if mode == 0 or ks < 2:
         ks = 0
@@ -741,7 +741,7 @@ def qkv_rope_kv(segs: Sequence[Seg], h: torch.Tensor, qkv: torch.Tensor, pos: to
     and writes q / K / V directly (one launch); with a split-K launch config the partial slabs are
     summed inside the RoPE kernel (no separate reduce pass, no fp32 qkv round trip)."""
     if h.is_cuda and all(s.xmap is None for s in segs):
-        mode, waves, rt, ks = cfg or gemv_config(segs, T)
+        mode, waves, rt, ks = cfg or fitting_config(gemv_config(segs, T), segs, T, h, None, "rope")
         ncol, contiguous = 0, True
         for s in segs:
             contiguous = contiguous and s.ycol == ncol

@@ -99,3 +99,50 @@ def test_rope(gpu, rt, D, bias):
         outs.append((q, kc, vc))
     for a, b in zip(*outs):      # one bf16 rounding apart at most, and the same places written
         assert relerr(a, b) < 2e-3 and ((a == 776) == (b == 776)).all()
+
+
+def ragged(x, how):
+    """x's rows as they are, 8 bytes off a multiple of 16, or from there on."""
+    M, K = x.shape
+    if how == "regular":
+        return x
+    wide = torch.zeros(M, K + 8, dtype=x.dtype, device=x.device)
+    v = wide.view(-1)[:M * (K + 4)].view(M, K + 4)[:, :K] if how == "stride" else wide[:, 4:4 + K]
+    return v.copy_(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", ["regular", "stride", "start"])
+@pytest.mark.parametrize("copies", [True, False])
+@pytest.mark.parametrize("M", [128, 192, 300])
+def test_fused_launches_take_any_rows(gpu, how, copies, M):
+    """Q, K and V with RoPE, and projections with residual, norm and route, as chosen by size, for rows that the copies to LDS do not take; with f16 copies
+    and without. Against the launches of irregular rows done on regular ones: the same products of f16 values, summed in 32 bits."""
+    D, Hq, Hkv, K = 128, 16, 8, 2048
+    ws = [weight(h * D, K, s) for s, h in enumerate((Hq, Hkv, Hkv))]
+    o = weight(K, K, 5)
+    if not copies:
+        for w in (*ws, o):
+            w.d16 = None
+    segs = [ops.Seg(ws[0], 0), ops.Seg(ws[1], Hq * D), ops.Seg(ws[2], (Hq + Hkv) * D)]
+    x, n = acts(M, K), (Hq + 2 * Hkv) * D
+    pad = x.shape[0]
+    cs = ops.rope_table(400, D, 10000.0, torch.device("cuda"))
+    pos, slot = (torch.arange(pad, dtype=torch.int32, device="cuda") * 7) % 400, torch.arange(pad, dtype=torch.int32, device="cuda")
+    nw, wr = torch.randn(K, device="cuda"), (torch.randn(4, K, device="cuda") * 0.05).half()
+    res = torch.randn(pad, K, device="cuda")
+
+    def run(x):
+        q = torch.zeros(pad, Hq * D, dtype=torch.bfloat16, device="cuda")
+        kc, vc = (torch.zeros(pad, Hkv, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        ops.qkv_rope_kv(segs, x, torch.zeros(pad, n, device="cuda"), pos, slot, cs, q, kc, vc, M, Hq, Hkv, D)
+        a, h = res.clone(), torch.zeros(pad, K, dtype=torch.float16, device="cuda")
+        ops.qgemv_add_rmsnorm(ops.Seg(o), x, a, nw, h, M, 0.5, 1e-5)
+        b, h2, lg = res.clone(), torch.zeros_like(h), torch.zeros(pad, 4, device="cuda")
+        ints = [torch.zeros(m, dtype=torch.int32, device="cuda") for m in (4, 4 * pad, 4 * pad)]
+        assert ops.qgemv_add_rmsnorm_route(ops.Seg(o), x, b, nw, h2, M, 0.5, 1e-5, wr, lg, 2, torch.zeros(pad * 2, device="cuda"), *ints, pad)
+        return q[:M], kc[:M], vc[:M], a[:M], h[:M], b[:M], h2[:M], lg[:M]
+    for got, want, tol in zip(run(ragged(x, how)), run(x), (2e-3, 2e-3, 2e-3, 4e-6, 5e-4, 4e-6, 5e-4, 2e-3)):
+        assert relerr(got, want) < tol
+    z = x[:M].double() @ torch.cat([w.dense().double().to("cuda") for w in ws]).T
+    assert relerr(run(x)[2].view(M, -1), z[:, (Hq + Hkv) * D:]) < 4e-3              # (bf16 rows: 2^-9; f16 copies round once more)
