@@ -1,14 +1,15 @@
-// Dense f16 GEMM, "mode 11" of the qgemv dispatcher (gfx950): tiles in steps of 16 weight rows and 32 activations that fill one round of the chip, the
+// Dense f16 GEMM, "mode 11" of the qgemv dispatcher (gfx950): tiles in steps of 32 weight rows and 32 activations that fill one round of the chip, the
 // two wave groups on alternate k-steps.
 //
 //   y[m, n] (epilogue) alpha * sum_k x[m, k] * W[n, k]      x f16 [M, K], W f16 [N, K] row-major
 //
-// 8 waves = 2 groups x 4; the four waves of a group are WM x 4 / WM, each with 16 MT activation rows x 16 NT weight rows of the tile. Group g takes
+// 8 waves = 2 groups x 4; the four waves of a group are 2 x 2, each with 16 MT activation rows x 16 NT weight rows of the tile. Group g takes
 // the k-steps (32 of K) of its parity, and the two halves meet in LDS at the end. A k-step is two sections a barrier apart: [read] NT + MT fragments,
 // half of the DMA of a later K-tile, lgkmcnt(0); [multiply] NT MT MFMAs from registers. Group 1 runs one section behind, so that on each SIMD one
 // wave multiplies while the other reads.
 // What bounds a product of a few hundred rows is how fast a CU takes in operands: 57 GB/s with one K-tile of 64 in flight and copies of 16 rows x 64
-// bytes, 80 with two and 8 rows x 128 bytes (96 and 128 x 320, 224 CUs; 16 x 64 bytes whose other half follows later: 48; with weights from memory 40 to
+// bytes, 80 with two and 8 rows x 128 bytes (tiles of 96 and 128 weight
+// rows x 320 activations of a trial, 224 CUs; 16 x 64 bytes whose other half follows later: 48; with weights from memory 40 to
 // 55). So LDS is a ring of R = 3 or 4
 // K-tiles (mode 10: two), copies are whole lines, and tiles are nearer to squares: 160 x 224 makes 256 workgroups of 320 x 28672 and takes in 384 rows
 // where 320 x 128 takes 448.
@@ -24,9 +25,9 @@ using namespace nls_gemv;
 using nls_dma::glds16;
 using nls_dma::lds_addr;
 
-template <int WM, int NT, int MT>
+template <int NT, int MT>
 struct H11 {
-  static constexpr int WN = 4 / WM, BN = 16 * NT * WN, BM = 16 * MT * WM;
+  static constexpr int BN = 32 * NT, BM = 32 * MT;
   static constexpr int TB = (BN + BM) * 128;              // a K-tile of 64: weight rows, then activations
   static constexpr int R = 4 * TB <= 160 * 1024 ? 4 : 3;  // K-tiles of the ring
   static constexpr int RT = (BN + BM) / 16;               // row-tiles; a group stages one half (8 rows, 1 KiB) of each
@@ -41,13 +42,13 @@ DEVI void wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
 }
 
-template <int WM, int NT, int MT, bool ROPE>
+template <int NT, int MT, bool ROPE>
 DEVI void h11_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a, float* ws, uint8_t* lds) {
-  typedef H11<WM, NT, MT> C;
+  typedef H11<NT, MT> C;
   constexpr int R = C::R, NJ = C::Q + (C::X ? 1 : 0), NA = C::NA, NW = C::BN / 16;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kg = wave >> 2, wc = wave & 3, wm = wc % WM, wn = wc / WM;
+  const int kg = wave >> 2, wc = wave & 3, wm = wc & 1, wn = wc >> 1;
   const int nkt_all = S.K / 64;
   const int t0 = (nkt_all * kslice) / ks, t1 = (nkt_all * (kslice + 1)) / ks;
   const int nkt = t1 - t0;
@@ -147,10 +148,10 @@ DEVI void h11_tile(const Seg& S, int row0, int kslice, int ks, const GemvArgs& a
   nls_dense::dense_epilogue<NA, MT, ROPE>(out, S, n0 + 16 * NA * kg, min(S.rows, n0 + (kg ? 16 * NT : 16 * NA)), wm * 16 * MT, kslice, ks, a, ws);
 }
 
-template <int WM, int NT, int MT, bool ROPE>
+template <int NT, int MT, bool ROPE>
 __global__ __launch_bounds__(512, 1) void hgemm11_kernel(SegList segs, GemvArgs a, int ks, float* ws, int ntiles, int nmb) {
   extern __shared__ __attribute__((aligned(16))) uint8_t h11lds[];
-  constexpr int BM = H11<WM, NT, MT>::BM;
+  constexpr int BM = H11<NT, MT>::BM;
   const int i = blockIdx.x, xcd = i & 7, j = i >> 3;
   const int kslice = j % ks;
   const int mb = (j / ks) % nmb;
@@ -167,28 +168,27 @@ __global__ __launch_bounds__(512, 1) void hgemm11_kernel(SegList segs, GemvArgs 
   a.y = (char*)a.y + (size_t)m0 * a.ldy * esz;
   if (a.argmax) a.argmax += m0;
   a.M = min(BM, a.M - m0);
-  h11_tile<WM, NT, MT, ROPE>(S, (tile - S.tile_begin) * H11<WM, NT, MT>::BN, kslice, ks, a, ws, h11lds);
+  h11_tile<NT, MT, ROPE>(S, (tile - S.tile_begin) * H11<NT, MT>::BN, kslice, ks, a, ws, h11lds);
 }
 
-template <int WM, int NT, int MT, bool ROPE>
+template <int NT, int MT, bool ROPE>
 int launch_e(const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
-  typedef H11<WM, NT, MT> C;
+  typedef H11<NT, MT> C;
   const int nmb = (a.M + C::BM - 1) / C::BM;
   static bool attr = false;
   if (!attr) {   // > 64 KiB of dynamic LDS must be opted into
-    if (hipFuncSetAttribute((const void*)hgemm11_kernel<WM, NT, MT, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) != hipSuccess) return -1;
+    if (hipFuncSetAttribute((const void*)hgemm11_kernel<NT, MT, ROPE>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS) != hipSuccess) return -1;
     attr = true;
   }
-  hipLaunchKernelGGL((hgemm11_kernel<WM, NT, MT, ROPE>), dim3((ntiles + 7) / 8 * 8 * nmb * ks), dim3(512), C::LDS, st, sl, a, ks, ws, ntiles, nmb);
+  hipLaunchKernelGGL((hgemm11_kernel<NT, MT, ROPE>), dim3((ntiles + 7) / 8 * 8 * nmb * ks), dim3(512), C::LDS, st, sl, a, ks, ws, ntiles, nmb);
   return (int)hipGetLastError();
 }
 
-// wm waves of a group along the activations (2 or 4), each with 16 mt of them, 4 / wm along the weights, each with 16 nt rows
-int launch_dense11(int wm, int nt, int mt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
-#define NLS_H11(WM, NT, MT) \
-  if (wm == WM && nt == NT && mt == MT) \
-    return a.epi == EPI_ROPE ? launch_e<WM, NT, MT, true>(sl, ntiles, ks, ws, a, st) : launch_e<WM, NT, MT, false>(sl, ntiles, ks, ws, a, st);
-#define NLS_H11N(MT) NLS_H11(2, 3, MT) NLS_H11(2, 4, MT) NLS_H11(2, 5, MT) NLS_H11(2, 6, MT) NLS_H11(2, 7, MT) NLS_H11(2, 8, MT)
+// nt: weight rows of a tile / 32, mt: activation rows / 32
+int launch_dense11(int nt, int mt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st) {
+#define NLS_H11(NT, MT) \
+  if (nt == NT && mt == MT) return a.epi == EPI_ROPE ? launch_e<NT, MT, true>(sl, ntiles, ks, ws, a, st) : launch_e<NT, MT, false>(sl, ntiles, ks, ws, a, st);
+#define NLS_H11N(MT) NLS_H11(3, MT) NLS_H11(4, MT) NLS_H11(5, MT) NLS_H11(6, MT) NLS_H11(7, MT) NLS_H11(8, MT)
   NLS_H11N(3) NLS_H11N(4) NLS_H11N(5)
 #undef NLS_H11N
 #undef NLS_H11

@@ -14,7 +14,7 @@ int launch_dense10(int bn, const SegList& sl, int ntiles, int ks, float* ws, con
 }
 namespace nls_hg11 {
 using namespace nls_gemv;
-int launch_dense11(int wm, int nt, int mt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st);
+int launch_dense11(int nt, int mt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st);
 }
 namespace nls_q9 {
 int launch_q9(int kset, int waves, int rt, const SegList& sl, int ntiles, int ks, float* ws, const GemvArgs& a, hipStream_t st);
@@ -60,8 +60,8 @@ struct NlsFuse {
 // mode 6: mode 4 at 128-row activation blocks (rt 2) with 2-deep rings: two workgroups per CU.
 // mode 10: dense f16 GEMM, 256 x 256 tiles, 4 phases per 64-deep K-tile with the two wave groups staggered
 //         by one barrier (hgemm10.hip); the mode-8 operands and epilogues, optional split-K.
-// mode 11: dense f16 GEMM, the two wave groups on alternate k-steps (hgemm11.hip); rt = 256 wm + 16 mt + nt: row blocks of 16 mt wm, weight tiles of
-//         16 nt (4 / wm) rows; operands, epilogues and split-K as mode 10.
+// mode 11: dense f16 GEMM, the two wave groups on alternate k-steps (hgemm11.hip); rt = 512 + 16 mt + nt: row blocks of 32 mt, mt 3 to 5, weight tiles
+//         of 32 nt rows, nt 3 to 8; operands, epilogues and split-K as mode 10.
 // (Modes 11-13 of another kind -- mode 10 on raw K-quant tiles, mode 9 at 64-row blocks, stream-K -- lost every measured shape in
 //  round 5 and were removed from the build; profiles/streamk_r05.txt, profiles/qgemm11_r05.txt.)
 // mode 9: quantised GEMM on the raw tile-blocks (qgemm9.hip; Q4_K/Q5_K/Q6_K/Q8_0/Q51): 256-row activation
@@ -118,8 +118,9 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
   if (mode >= 9 && (epi != EPI_ARGMAX || ks > 1))       // (their stores are 4 columns wide, in slabs too)
     for (int i = 0; i < nseg; ++i)
       if (segs[i].rows % 4) return -1;
+  const int nt11 = rt & 15, mt11 = rt >> 4 & 15;
   if (mode >= 10) {            // mode 10: rt 1: 256-row weight tiles, rt 2: 128-row
-    if (waves != 8 || (mode == 10 ? rt != 1 && rt != 2 : (rt >> 8) != 2 && (rt >> 8) != 4) || fz->xf || fz->onw || ldx % 8 ||
+    if (waves != 8 || (mode == 10 ? rt != 1 && rt != 2 : rt >> 8 != 2 || nt11 < 3 || nt11 > 8 || mt11 < 3 || mt11 > 5) || fz->xf || fz->onw || ldx % 8 ||
         ((epi == EPI_F32 || epi == EPI_ADD_F32 || epi == EPI_ACT) && ldy % 4))
       return -1;
     for (int i = 0; i < nseg; ++i)
@@ -151,7 +152,7 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
     mks = segs[i].ymap && segs[i].ycol == 0 && segs[i].rows == segs[0].rows;
   SegList sl{};
   int tiles = 0, cols = 0;
-  const int tile_rows = mode == 11 ? 16 * (rt & 15) * (4 / (rt >> 8)) : mode == 10 ? 256 / rt : mode == 9 ? 16 * waves * rt : (mode == 5 ? 256 : (mode >= 2 ? 128 : (mode == 1 ? waves : 1) * rt * 16));
+  const int tile_rows = mode == 11 ? 32 * nt11 : mode == 10 ? 256 / rt : mode == 9 ? 16 * waves * rt : (mode == 5 ? 256 : (mode >= 2 ? 128 : (mode == 1 ? waves : 1) * rt * 16));
   for (int i = 0; i < nseg; ++i) {
     if (segs[i].K % 256 || segs[i].rows < 1) return -1;
     if (epi == EPI_SWIGLU && segs[i].rows % 16) return -1;
@@ -252,7 +253,7 @@ static int qgemv_impl(const NlsSeg* segs, int nseg, const void* x, long ldx, voi
     if (ks < 1) ks = 1;
     int rc;
     if (mode == 11)
-      rc = nls_hg11::launch_dense11(rt >> 8, rt & 15, (rt >> 4) & 15, sl, tiles, ks, (float*)ws, a, st);
+      rc = nls_hg11::launch_dense11(nt11, mt11, sl, tiles, ks, (float*)ws, a, st);
     else if (mode == 10)
       rc = nls_hg10::launch_dense10(256 / rt, sl, tiles, ks, (float*)ws, a, st);
     else if (mode == 9)

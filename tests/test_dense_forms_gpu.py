@@ -39,6 +39,14 @@ def test_rule_gives_built_forms():
             assert tuning.select_dense([ops.Seg(_W(rows + 1, K))], 300)[0] != 11
 
 
+@pytest.mark.parametrize("rt", [0, 512, 512 + 16 * 3 + 2, 512 + 16 * 3 + 9, 512 + 16 * 2 + 3, 512 + 16 * 6 + 3, 512 + 48, 256 + 51, 768 + 51, 1024 + 51, -1, 4096 + 563])
+def test_unbuilt_forms_are_refused(rt):
+    """The launcher refuses forms that are not built, those of no weight rows among them."""
+    from nats_llm_studio_amd.ops import _lib
+    arr = (_lib.NlsSeg * 1)(_lib.NlsSeg(4096, None, None, None, 1, 2048, 2048, 0))
+    assert _lib.lib().nls_qgemv(arr, 1, 4096, 2048, 4096, 2048, 300, 1.0, ops.EPI["f32"], None, 8, rt, 11, 1, None, None) == -1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rt", FORMS)
 @pytest.mark.parametrize("rows,K", [(772, 256), (64, 512), (1020, 1536)])
