@@ -4,6 +4,7 @@ GPU tensors only: there is no eager form of these ops, a missing library raises.
 f32 norms / routing / softmax / recurrences) or, for 32-bit models, f32 throughout (f32 MFMA, or f32 in three bf16 parts)."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from functools import lru_cache
@@ -939,6 +940,16 @@ class TalkPlan:
         ns = 1 if tb > 1 else max(1, min(16, 256 // (T * -(-jobs // nw)), -(-self.ks // kt)))
         return tb1, ns1, tb, ns, kt, nw
 
+    def plain_buffers(self, T: int, ks: int, device):
+        """What one call of the plain kernels over T rows needs, with ks keys to a row of scores: (scores, score statistics, partial outputs, counters)."""
+        R = self.rows(T)
+        forms = [(n, *self.plain_form(n)) for n in {R, T % R or R}]
+        stats = max(n * ns1 for n, _, ns1, *_ in forms)
+        part = max((n * ns for n, _, _, _, ns, _, _ in forms if ns > 1), default=0)
+        cnt = max(n * -(-self.groups * -(-self.Dp // 64) // nw) for n, *_, nw in forms)
+        f = [torch.empty(n, dtype=torch.float32, device=device) for n in (R * ks * self.H, stats * self.H * 2, part * self.H * self.Dp)]
+        return (*f, torch.zeros(cnt, dtype=torch.int32, device=device))
+
     def scratch(self, cap: int):
         """Element counts of (scores, score statistics, partial outputs, counters)."""
         R = self.rows(cap)
@@ -952,6 +963,13 @@ class TalkPlan:
                 R * self.groups)
 
 
+def _allocating(device, st: int):
+    """Allocations belong to stream st: memory of another stream could be handed out again while the kernels on st still use it."""
+    if torch.cuda.current_stream(device).cuda_stream == st:
+        return contextlib.nullcontext()
+    return torch.cuda.stream(torch.cuda.ExternalStream(st, device) if st else torch.cuda.default_stream(device))
+
+
 def talk_attention(plan: TalkPlan, q, kc, vc, talk, gate, out, scratch, block_tables, block_size: int, tok_seq, ctx_len, T: int,
                    V: int, scale: float, st: int):
     """Row-by-row attention with mixed heads (talk: TalkPlan.matrix); `gate`: a factor per output column, heads V columns apart."""
@@ -961,7 +979,8 @@ def talk_attention(plan: TalkPlan, q, kc, vc, talk, gate, out, scratch, block_ta
         raise ValueError("talk_attention: a gate of the outputs' type")
     if not p.mfma:
         if not scratch:
-            scratch = [torch.empty(n, device=q.device) for n in p.scratch(T)[:3]] + [torch.zeros(p.scratch(T)[3], dtype=torch.int32, device=q.device)]
+            with _allocating(q.device, st):
+                scratch = p.plain_buffers(T, p.ks, q.device)
         sc, ss, po, cnt = scratch
         R = min(p.rows(T), sc.numel() // (p.ks * p.H))
         for t0 in range(0, T, R):

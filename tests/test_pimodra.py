@@ -116,6 +116,31 @@ def test_launch_plans():
     assert m.shape == (32, 32) and float(m.sum()) == 25.0 and float(m[:5, :5].sum()) == 25.0
 
 
+@pytest.mark.parametrize("H,G,Dp,window,ctx", [(16, 4, 128, 0, 2000), (32, 8, 128, 1024, 8192), (6, 2, 36, 37, 480), (70, 35, 8, 0, 480), (1, 1, 4, 0, 16)])
+def test_plain_buffers(H, G, Dp, window, ctx):
+    """What a call without kept buffers allocates is enough for each of its launches, in 32 bits whatever torch's default type is; the kept ones are enough
+    for every number of rows up to theirs."""
+    from nats_llm_studio_amd.ops import stack as K
+    p = K.TalkPlan(H, G, Dp, window, ctx, True, "cpu")
+    p.rows = lambda cap: min(cap, 300)
+    jobs = G * -(-(H // G) // 16) * -(-Dp // 64)
+
+    def enough(n, ks, sc, ss, po, cnt):
+        _, ns1, _, ns, _, nw = p.plain_form(n)
+        return sc >= n * ks * H and ss >= n * ns1 * H * 2 and (ns == 1 or (po >= n * ns * H * Dp and cnt >= n * -(-jobs // nw)))
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        for T in (1, 2, 7, 64, 65, 299, 300, 301, 700):
+            for ks in (p.ks, p.ks + 160):
+                part = p.plain_buffers(T, ks, "cpu")
+                assert [x.dtype for x in part] == [torch.float32] * 3 + [torch.int32] and not part[3].any()
+                assert all(enough(n, ks, *(x.numel() for x in part)) for n in {min(T, 300), T % 300 or min(T, 300)})
+    finally:
+        torch.set_default_dtype(torch.float32)
+    for cap in (1, 5, 64, 300):
+        assert all(enough(n, p.ks, *p.scratch(cap)) for n in range(1, cap + 1))
+
+
 # ---- the plain implementation against itself
 
 @pytest.mark.parametrize("i", [0, 1, 3])

@@ -247,6 +247,40 @@ def test_rows_that_share_keys(K, dt, H, G, D, V, window, most):
                 assert relerr(o[t, :, :V], want) < TOL[dt], t
 
 
+def plain_case(K, dt, H, G, D, V, ctxs, window):
+    """A row per context at its end: what talk_attention takes, and the outputs it should give."""
+    d, bs, T = DT[dt], 16, len(ctxs)
+    Dp, _ = K.head_pad(max(D, V))
+    q, talk, gate = talk_inputs(d, T, H, D, V, Dp)
+    scale = 0.7 / math.sqrt(D)
+    kc, vc, bt, rows = paged(d, ctxs, G, D, V, Dp, -(-max(ctxs) // bs), bs, [[] for _ in ctxs])
+    mask = {"size": window} if window else None
+    want = torch.stack([O.attend(q[t:t + 1, :, :D].double(), *rows[t], torch.tensor([c - 1]), scale, mask, talk.double())[0]
+                        for t, c in enumerate(ctxs)]) * gate.double().view(T, H, V)
+    return q.view(T, -1).cuda(), kc, vc, talk, gate.cuda(), bt, scale, want, Dp
+
+
+def test_plain_on_another_stream(K):
+    """Launches on a stream that is not the current one own their buffers there: what the current stream allocates and fills meanwhile is other memory."""
+    dt, H, G, D, V = "f32", 16, 4, 128, 128
+    ctxs = [471, 300, 64]
+    q, kc, vc, talk, gate, bt, scale, want, Dp = plain_case(K, dt, H, G, D, V, ctxs, 0)
+    plan = K.TalkPlan(H, G, Dp, 0, 480, True, "cuda")
+    n, m, seq, ctx = len(ctxs), plan.matrix(talk), i32([0, 1, 2]), i32(ctxs)
+    out = torch.full((n, H * Dp), 7.0, device="cuda")
+    sizes = plan.scratch(n)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)                    # (about 10 ms: the launches below wait behind it)
+    K.talk_attention(plan, q, kc, vc, m, gate, out, None, bt, 16, seq, ctx, n, V, scale, side.cuda_stream)
+    filled = [torch.full((s,), -1, dtype=torch.int32, device="cuda") for s in sizes for _ in range(4)]
+    torch.cuda.current_stream().wait_stream(side)
+    assert all((f == -1).all() for f in filled)
+    for t in range(n):
+        assert relerr(out[t].view(H, Dp)[:, :V], want[t]) < TOL[dt], t
+
+
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("H,G,D,V", [(1, 1, 8, 4), (6, 2, 20, 36), (5, 5, 33, 21), (4, 2, 64, 128), (2, 1, 128, 7), (3, 1, 256, 256),
                                      (2, 2, 300, 16), (40, 8, 128, 128)])
