@@ -708,7 +708,7 @@ extern "C" {
 using namespace nls_talk;
 
 // rows t0 .. t0 + rows - 1, any head count, f32 arithmetic: talk f32 [H][H], Dp a multiple of 4. sc [rows][H][ks], ks a multiple of 16 that
-// holds 16 * (first visible / 16) .. the last key; st [rows][ns1][H][2]; ns > 1 (one token to a workgroup of the mix): part [rows][H][ns][Dp],
+// holds 16 * (first visible / 16) .. the last key (values of keys beyond it are left out); st [rows][ns1][H][2]; ns > 1 (one token to a workgroup of the mix): part [rows][H][ns][Dp],
 // cnt [rows][workgroups] zeros (left zero). tb1, tb: tokens of a workgroup of the scores and of the mix; kt: keys of its block; nw: its waves, 4 or 8
 int nls_talk_rows(const void* q, long ldq, const void* k, const void* v, const int* bt, int bts, int bs, const int* tok_seq,
                   const int* ctx_len, int t0, int rows, int H, int G, int Dp, int V, float scale, int window, const float* talk,

@@ -147,7 +147,7 @@ __global__ __launch_bounds__(NT) void talk_rows_score_kernel(Rows p) {
         s[j] = k >= rlow && k < rctx ? s[j] * a.scale : -INFINITY;
         mx = fmaxf(mx, s[j]);
       }
-      if (16 * t >= first && 16 * t < rctx) *reinterpret_cast<f32x4*>(dst + 16 * t - first + 4 * g) = s;
+      if (16 * t >= first && 16 * t < rctx && 16 * t - first < p.ks) *reinterpret_cast<f32x4*>(dst + 16 * t - first + 4 * g) = s;
       const float base = mx == -INFINITY ? 0.f : mx;
       l *= m == -INFINITY ? 0.f : expf(m - base);
 #pragma unroll
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(64 * NW) void talk_rows_mix_kernel(Rows p) {
         float* w = ws + (size_t)tk * H * ldw + 16 * sb + 4 * g;
         const bool in = tk >= xa && tk < run.y;
         const int ctx = in ? a.ctx_len[t0 + tk] : 0, low = low_of(a, ctx);
-        const bool see = k >= low && k < ctx;
+        const bool see = k >= low && k < ctx && k - (low & ~15) < p.ks;
         const float* s = p.sc + (size_t)(tr0 + tk) * H * p.ks + (see ? k - (low & ~15) : 0);
         const float* mt = ml + 2 * (size_t)tk * H;
         for (int c0 = 0; c0 < nhb; c0 += HB) {
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(64 * NW) void talk_rows_mix_kernel(Rows p) {
   for (int tk = 0; tk < tn; ++tk) {
     if (!bad[tk]) continue;
     const size_t t = t0 + tk;
-    const int ctx = a.ctx_len[t], low = low_of(a, ctx);
+    const int low = low_of(a, a.ctx_len[t]), ctx = (int)min((long)a.ctx_len[t], (low & ~15) + p.ks);
     const int* bt = a.bt + (size_t)a.tok_seq[t] * a.bts;
     const float *mt = ml + 2 * (size_t)tk * H, *s = p.sc + (size_t)(tr0 + tk) * H * p.ks - (low & ~15);
     const int d = 64 * vb + lane;

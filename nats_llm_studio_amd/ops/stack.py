@@ -978,11 +978,14 @@ def talk_attention(plan: TalkPlan, q, kc, vc, talk, gate, out, scratch, block_ta
     if gate is not None and gate.dtype != out.dtype:
         raise ValueError("talk_attention: a gate of the outputs' type")
     if not p.mfma:
-        if not scratch:
+        # (no plan of the contexts was needed before there were scores in memory: a table that holds more keys than the plan's rows gets longer rows)
+        most = block_tables.shape[1] * block_size
+        ks = max(p.ks, pad_to(min(p.window + 15, most) if p.window else most, 16))
+        if not scratch or scratch[0].numel() < ks * p.H:
             with _allocating(q.device, st):
-                scratch = p.plain_buffers(T, p.ks, q.device)
+                scratch = p.plain_buffers(T, ks, q.device)
         sc, ss, po, cnt = scratch
-        R = min(p.rows(T), sc.numel() // (p.ks * p.H))
+        R = min(p.rows(T), sc.numel() // (ks * p.H))
         for t0 in range(0, T, R):
             n = min(R, T - t0)
             tb1, ns1, tb, ns, kt, nw = p.plain_form(n)
@@ -990,7 +993,7 @@ def talk_attention(plan: TalkPlan, q, kc, vc, talk, gate, out, scratch, block_ta
                 raise ValueError("talk_attention: workspace too small")
             _check(lib().nls_talk_rows(q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), block_tables.data_ptr(),
                                        block_tables.stride(0), block_size, tok_seq.data_ptr(), ctx_len.data_ptr(), t0, n, p.H, p.G, p.Dp, V,
-                                       scale, p.window, talk.data_ptr(), _p(gate), ldg, out.data_ptr(), out.stride(0), sc.data_ptr(), p.ks,
+                                       scale, p.window, talk.data_ptr(), _p(gate), ldg, out.data_ptr(), out.stride(0), sc.data_ptr(), ks,
                                        ss.data_ptr(), po.data_ptr(), cnt.data_ptr(), tb1, ns1, tb, ns, kt, nw,
                                        int(q.dtype == torch.float32), st), "nls_talk_rows")
         return

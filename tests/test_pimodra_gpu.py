@@ -260,6 +260,22 @@ def plain_case(K, dt, H, G, D, V, ctxs, window):
     return q.view(T, -1).cuda(), kc, vc, talk, gate.cuda(), bt, scale, want, Dp
 
 
+@pytest.mark.parametrize("kept", [False, True])
+def test_plain_contexts_beyond_the_plan(K, kept):
+    """Rows of scores are as long as what the block table holds, where the plan's contexts are shorter; with the plan's buffers too, in several launches."""
+    dt, H, G, D, V = "f32", 6, 2, 20, 36
+    ctxs = [700, 3, 128, 161, 689, 420]
+    q, kc, vc, talk, gate, bt, scale, want, Dp = plain_case(K, dt, H, G, D, V, ctxs, 0)
+    plan = K.TalkPlan(H, G, Dp, 0, 128, True, "cuda")
+    n = len(ctxs)
+    part = [torch.full((s,), math.nan, device="cuda") for s in plan.scratch(n)[:3]] + [i32([0] * plan.scratch(n)[3])] if kept else None
+    out = torch.full((n + 1, H * Dp), 7.0, device="cuda")
+    K.talk_attention(plan, q, kc, vc, plan.matrix(talk), gate, out, part, bt, 16, i32(list(range(n))), i32(ctxs), n, V, scale, st())
+    assert not kept or (part[3] == 0).all()
+    for t in range(n):
+        assert relerr(out[t].view(H, Dp)[:, :V], want[t]) < TOL[dt], t
+
+
 def test_plain_on_another_stream(K):
     """Launches on a stream that is not the current one own their buffers there: what the current stream allocates and fills meanwhile is other memory."""
     dt, H, G, D, V = "f32", 16, 4, 128, 128
