@@ -260,6 +260,26 @@ def plain_case(K, dt, H, G, D, V, ctxs, window):
     return q.view(T, -1).cuda(), kc, vc, talk, gate.cuda(), bt, scale, want, Dp
 
 
+@pytest.mark.parametrize("dt,H,G,D,V", [("f32", 6, 2, 20, 36), ("f32", 16, 4, 128, 128), ("bf16", 8, 2, 300, 10)])
+@pytest.mark.parametrize("window", [0, 37])
+def test_plain_workspace_is_kept(K, dt, H, G, D, V, window):
+    """The plain kernels on the buffers that a program keeps for its largest step: steps of many rows and of few behind each other, twice, with whatever
+    the last one left in them; the tickets end at zero."""
+    ctxs = [1, 16, 17, 64, 130, 300, 471, 33, 5, 200, 471, 15]
+    q, kc, vc, talk, gate, bt, scale, want, Dp = plain_case(K, dt, H, G, D, V, ctxs, window)
+    plan = K.TalkPlan(H, G, Dp, window, 480, dt == "f32", "cuda")
+    assert not plan.mfma and max(plan.plain_form(n)[3] for n in (1, 2, 12)) > 1
+    sizes = plan.scratch(len(ctxs))
+    part = [torch.full((n,), math.nan, device="cuda") for n in sizes[:3]] + [torch.zeros(sizes[3], dtype=torch.int32, device="cuda")]
+    for n, t0 in ((12, 0), (1, 6), (2, 5), (12, 0), (1, 0), (5, 3), (1, 10)) * 2:
+        out = torch.full((n + 1, H * Dp), 7.0, dtype=DT[dt], device="cuda")
+        K.talk_attention(plan, q[t0:t0 + n], kc, vc, plan.matrix(talk), gate[t0:t0 + n], out, part, bt, 16, i32(list(range(t0, t0 + n))),
+                         i32(ctxs[t0:t0 + n]), n, V, scale, st())
+        assert (part[3] == 0).all() and (out[n] == 7).all()
+        for t in range(n):
+            assert relerr(out[t].view(H, Dp)[:, :V], want[t0 + t]) < TOL[dt], (n, t0, t)
+
+
 @pytest.mark.parametrize("kept", [False, True])
 def test_plain_contexts_beyond_the_plan(K, kept):
     """Rows of scores are as long as what the block table holds, where the plan's contexts are shorter; with the plan's buffers too, in several launches."""
