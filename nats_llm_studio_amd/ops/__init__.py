@@ -654,8 +654,9 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, M: int, eps: fl
 def gather_rows(h: torch.Tensor, rows: torch.Tensor, n: int, out: torch.Tensor) -> torch.Tensor:
     """h[rows[:n]], up to a multiple of 16 rows with zeros: in `out`, one launch, where it holds them, else a tensor of its own."""
     np_ = (n + 15) // 16 * 16
-    if (h.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and n <= rows.numel() and np_ <= out.shape[0] and h.dtype == out.dtype
-            and h.shape[1] == out.shape[1] and h.element_size() == 2 and h.shape[1] % 8 == 0 and h.stride(0) % 8 == 0 and out.is_contiguous()):
+    if (h.is_cuda and rows.dtype == torch.int32 and rows.is_contiguous() and 0 < n <= rows.numel() and np_ <= out.shape[0] and h.dtype == out.dtype
+            and h.shape[1] == out.shape[1] and h.element_size() == 2 and h.shape[1] % 8 == 0 and h.stride(0) % 8 == 0 and h.stride(1) == 1
+            and out.is_contiguous() and (h.data_ptr() | out.data_ptr()) % 16 == 0):
         _lib.check(_lib.lib().nls_gather_rows(h.data_ptr(), h.stride(0), h.shape[0], rows.data_ptr(), n, np_, h.shape[1], out.data_ptr(),
                                               _stream_ptr(h)), "nls_gather_rows")
         return out[:np_]

@@ -29,6 +29,19 @@ def test_rows(n, D):
     assert not check("cuda", n, D, (n + 15) // 16 * 16 - 1, D) and not check("cuda", n, D - 1 if D > 8 else 4, 64, D + 16)
 
 
+@pytest.mark.gpu
+def test_rows_that_lie_elsewhere():
+    """Rows and buffers that do not start at a multiple of 16 bytes, columns that are not neighbours, and no rows at all go the general way."""
+    wide, rows = torch.randn(50, 80, device="cuda").half(), torch.arange(49, -1, -1, dtype=torch.int32, device="cuda")
+    buf = torch.full((65 * 64,), 7.0, device="cuda").half()
+    for h in (wide[:, :64], wide[:, 4:68], wide[:, 1:65], wide[:, 8:72], torch.randn(128, 50, device="cuda").half().t()[:, :64]):
+        for at in (0, 4, 8):
+            out = buf[at:at + 64 * 64].view(64, 64)
+            for n in (0, 5, 16):
+                got = ops.gather_rows(h, rows, n, out)
+                assert got.shape == ((n + 15) // 16 * 16, 64) and torch.equal(got[:n], h[rows[:n].long()]) and (got[n:] == 0).all()
+
+
 def test_configs_are_kept_by_what_the_rules_see(monkeypatch):
     """The memo gives what the rules give, for layers alike and unlike, and forgets with the table."""
     from types import SimpleNamespace as NS
