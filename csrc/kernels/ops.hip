@@ -756,10 +756,6 @@ __global__ __launch_bounds__(256) void swiglu16_kernel(const act_t* __restrict__
   *reinterpret_cast<f16x8*>(out + (size_t)m * ldo + 8 * j) = o;
 }
 
-// Touch `bytes` of device memory (16-B loads, grid-stride over the whole grid) so that a later kernel finds them
-// in the memory-side Infinity Cache (MALL, 256 MB) / L2 instead of HBM -- the batch-1 decode experiment: stream
-// the NEXT projection's weights while a latency-bound kernel (attention, a GEMV's tail) leaves HBM idle. The
-// loaded words feed a sum that is stored only if it equals a value it never takes (keeps the loads alive).
 // Rows of 16-bit values that the head reads, up to a multiple of 16 with zeros: one launch where index_select, its index's conversion, the fill and
 // cat were four of 4 to 5 us. A workgroup to a row, 16 bytes a thread.
 __global__ __launch_bounds__(256) void gather_rows_kernel(const uint16_t* __restrict__ x, long ldx, int nx, const int* __restrict__ rows, int n, int D,
@@ -770,6 +766,10 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint16_t* __rest
     *reinterpret_cast<uint4*>(out + (size_t)blockIdx.x * D + c) = in ? *reinterpret_cast<const uint4*>(x + (size_t)r * ldx + c) : uint4{0, 0, 0, 0};
 }
 
+// Touch `bytes` of device memory (16-B loads, grid-stride over the whole grid) so that a later kernel finds them
+// in the memory-side Infinity Cache (MALL, 256 MB) / L2 instead of HBM -- the batch-1 decode experiment: stream
+// the NEXT projection's weights while a latency-bound kernel (attention, a GEMV's tail) leaves HBM idle. The
+// loaded words feed a sum that is stored only if it equals a value it never takes (keeps the loads alive).
 __global__ __launch_bounds__(256) void prefetch_kernel(const uint4* __restrict__ p, long n16, uint32_t never,
                                                        uint32_t* __restrict__ sink) {
   uint32_t acc = 0;
@@ -798,7 +798,6 @@ int nls_gather_rows(const void* x, long ldx, int nx, const void* rows, int n, in
   hipLaunchKernelGGL(gather_rows_kernel, dim3(npad), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x, ldx, nx, (const int*)rows, n, D, (uint16_t*)out);
   return (int)hipGetLastError();
 }
-
 
 int nls_prefetch(const void* p, long bytes, int blocks, void* stream) {
   if (bytes <= 0) return 0;
