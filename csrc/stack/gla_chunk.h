@@ -79,6 +79,14 @@ constexpr int gc_chunks() {
   return GC<T, DP, NT, DELTA, 2>::LDS <= 160 * 1024 ? 2 : 1;
 }
 
+// Between what some lanes of a wave leave in LDS and what others read of it, or put in its place. The hardware runs a wave's LDS accesses in order;
+// the compiler sees a lane's own addresses only, takes those of a read and of a later write for different ones and may turn them round.
+DEVI void lanes_meet() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename T> DEVI void ldt4(const T* p, float (&v)[4]) {
   typedef T t4 __attribute__((ext_vector_type(4)));
   const t4 x = *reinterpret_cast<const t4*>(p);
@@ -255,6 +263,7 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void gla_chunk_kernel(GA p) 
         if (!LOCAL) *reinterpret_cast<t4*>(rq + (16 * wave + ts + e) * C::LR + cg) = fq[e];
       }
       if (DELTA && lane < 16) bs[16 * wave + lane] = fb;
+      lanes_meet();
       if (!LOCAL || DELTA) {
         // A (and L): lane = (key token j, channels 16 m + 4 dg ..), down the rows i = j, j + 1, ..; rows past the chunk clear the
         // part above the diagonal
@@ -303,8 +312,7 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void gla_chunk_kernel(GA p) 
         float x[16];
         const int col = lane & 15;
         float* bw = bm + wave * 16 * C::LK;
-        __builtin_amdgcn_wave_barrier();
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        lanes_meet();
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           float acc = col == i ? bs[16 * wave + i] : 0.f;
@@ -317,8 +325,7 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void gla_chunk_kernel(GA p) 
           }
           x[i] = acc;
         }
-        __builtin_amdgcn_wave_barrier();
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        lanes_meet();
         if (lane < 16)
 #pragma unroll
           for (int i = 0; i < 16; ++i) bw[i * C::LK + col] = x[i];
@@ -329,6 +336,7 @@ __global__ __launch_bounds__(256, DP <= 64 ? 2 : 1) void gla_chunk_kernel(GA p) 
       for (int u = 0; u < NDP; ++u)
 #pragma unroll
         for (int t = 0; t < 16; ++t) kx[u][t] = kr[t * C::LKR + min(lane + 64 * u, DP - 1)];
+      lanes_meet();                                                 // (scaled keys take the place of the keys, decays' products that of the decays)
 #pragma unroll
       for (int u = 0; u < NDP; ++u) {
         const int d = lane + 64 * u;

@@ -40,6 +40,31 @@ def test_delta(dt, H, G, D, V, nseg):
 
 
 @pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("D,V", [(132, 40), (200, 128), (256, 192)])
+@pytest.mark.parametrize("nseg,nt", [(1, 1), (3, 1), (1, 2), (3, 2)])
+def test_wide(dt, D, V, nseg, nt):
+    """The kernels whose lanes hand each other most through LDS, in place, and whose registers spill: more than 128 channels, in both forms. Three times the
+    same, and what the plain implementation gives."""
+    d, n, eps, H = DT[dt], 150, 1e-3, 2
+    (q, k, v, fac, beta, a), plain = delta_data(d, H, H, D, V, n)
+    GD, HD = H * D, H * D
+    cat = lambda t: torch.cat([t[0], t[1]]).cuda()      # noqa: E731
+    z = torch.cat([cat(q), cat(k), cat(v)], 1)
+    runs = i32([[0, n, 3, 0], [n, n, 1, 0]])
+    seg = (torch.full((2 * nseg * HD * V,), 5.0, device="cuda"), torch.full((2 * nseg * HD * D,), 5.0, device="cuda"))
+    first = None
+    for _ in range(3):
+        S, o = torch.full((4, HD * V), 9.0, device="cuda"), torch.full((2 * n, H * V), 7.0, device="cuda")
+        K.delta_scan(z, z[:, GD:], z[:, 2 * GD:], cat(fac), cat(beta), cat(a), o, None, None, None, S, runs, 2, H, H, D, V, eps, (nseg, nt), seg, st())
+        first = first or (o.clone(), S.clone())
+        assert torch.equal(o, first[0]) and torch.equal(S, first[1])
+    for i, slot in ((0, 3), (1, 1)):
+        want, Sx = O.delta_scan(*(t[i] for t in plain))
+        assert relerr(o[i * n:(i + 1) * n].view(n, H, V), want) < 2e-5 and relerr(S[slot].view(H, D, V), Sx) < 2e-5
+    assert (S[0] == 9).all() and (S[2] == 9).all()
+
+
+@pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("nseg", [1, 3])
 def test_plain(dt, nseg):
     """Lightning's form against workgroups of 128 columns: the same sums in another split of the columns, bit for bit."""
