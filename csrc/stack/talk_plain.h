@@ -54,7 +54,7 @@ template <typename T> DEVI f32x4 ld4(const T* p) {
   return f32x4{(float)a[0], (float)a[1], (float)a[2], (float)a[3]};
 }
 DEVI f32x4 mma(float a, float b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-// the matrix pipe's last result, past the branch that ends its loop (the wait that the compiler counts within a block)
+// 16 states more behind the matrix pipe's last result, past the branch that ends its loop: a precaution, the compiler counts its wait across branches
 DEVI void settle(f32x4& c) { asm volatile("s_nop 15" : "+v"(c)); }
 DEVI int low_of(const TalkArgs& a, int ctx) { return a.window > 0 ? max(0, ctx - a.window) : 0; }
 
