@@ -129,14 +129,16 @@ def test_fused_launches_take_any_rows(gpu, how, copies, M):
     D, Hq, Hkv, K = 128, 16, 8, 2048
     ws = [weight(h * D, K, s) for s, h in enumerate((Hq, Hkv, Hkv))]
     o = weight(K, K, 5)
-    if not copies:
-        for w in (*ws, o):
-            w.d16 = None
+    for w in (*ws, o) if not copies else ws:
+        w.d16 = None
+    if copies:
+        ops.QWeight.expand_dense_group(ws)               # (one buffer, as a loaded model has them)
     segs = [ops.Seg(ws[0], 0), ops.Seg(ws[1], Hq * D), ops.Seg(ws[2], (Hq + Hkv) * D)]
     x, n = acts(M, K), (Hq + 2 * Hkv) * D
     pad = x.shape[0]
     cs = ops.rope_table(400, D, 10000.0, torch.device("cuda"))
     pos, slot = (torch.arange(pad, dtype=torch.int32, device="cuda") * 7) % 400, torch.arange(pad, dtype=torch.int32, device="cuda")
+    assert ops.gemv_config(segs, M)[0] == (11 if copies else 2) and (M > 192 or ops.gemv_config([ops.Seg(o)], M)[0] == (11 if copies else 2))
     nw, wr = torch.randn(K, device="cuda"), (torch.randn(4, K, device="cuda") * 0.05).half()
     res = torch.randn(pad, K, device="cuda")
 
