@@ -14,6 +14,8 @@
 // What bounds it: decoded tokens the chain of a share (block table, keys, scores; then scores, mix, values), prompts the matrix pipe and the
 // walk of a workgroup's keys (half of the time is the values' MFMAs). Before, one workgroup walked a token's keys on the vector units, twice: 16 heads
 // of 128 over 4, 1203 keys in a window of 1024: one token 3290 us -> 31 for both launches, 1203 tokens of a prompt 6576 -> 199.
+// Relative error against 64 bits, before and now, 16 heads of 128 over 4: one token and 53 keys 3.0e-7 -> 2.8e-7, 1203 keys 10.2e-7 -> 4.2e-7, 1203 tokens
+// of a prompt 4.6e-7 -> 4.1e-7; 18 heads of 32 8.1e-7 -> 2.8e-7 at 1203 keys.
 #pragma once
 #include "../kernels/common.h"
 
