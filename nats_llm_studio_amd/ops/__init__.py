@@ -316,8 +316,9 @@ def fitting_config(cfg, segs: Sequence[Seg], M: int, x: torch.Tensor, y: Optiona
     mode, ks = cfg[0], cfg[3]
     if mode >= 3 and (x.stride(0) % 8 or x.data_ptr() % 16):
         return tuning.any_rows(segs, M)
-    if mode >= 9 and (epi != "argmax" or ks > 1) and (any((s.ycol | s.w.rows) % 4 for s in segs)
-                                                      or (y is not None and epi in ("f32", "add", "act") and y.stride(0) % 4)):
+    stores = epi != "argmax" or ks > 1
+    if mode >= 9 and (any(s.ycol % 4 or (stores and s.w.rows % 4) for s in segs)
+                      or (y is not None and epi in ("f32", "add", "act") and y.stride(0) % 4)):
         return tuning.any_rows(segs, M) if mode == 9 else tuning.dense_heuristic(segs, M, aligned=False)
     return cfg
 

@@ -66,8 +66,8 @@ def test_launches_fit_their_rows():
                                 segs = [ops.Seg(_W(t, rows, K), ycol)]
                                 got = ops.fitting_config(cfg, segs, M, x, y, epi)
                                 regular = x.stride(0) % 8 == 0 and x.data_ptr() == 0
-                                stores = (ycol == 0 and rows % 4 == 0 and (y is None or y.stride(0) % 4 == 0 or epi in ("swiglu", "argmax"))
-                                          or epi == "argmax" and cfg[3] == 1)
+                                stores = ycol == 0 and (epi == "argmax" and cfg[3] == 1 or rows % 4 == 0
+                                                        and (y is None or y.stride(0) % 4 == 0 or epi in ("swiglu", "argmax")))
                                 assert got == (cfg if regular and (stores or cfg[0] < 9) or cfg[0] < 3 else tuning.any_rows(segs, M))
                                 assert got[0] in (1, 2) or (regular and (stores or got[0] < 9))
 
@@ -101,8 +101,14 @@ def test_many_rows_anywhere(gpu, M, qt, rows, K):
             ops.qgemv([ops.Seg(w, at)], x, y, M)
             assert ((y[:M, at:at + rows].cpu().double() - z).abs() <= bound).all(), (at, ld)
             assert (y[M:] == 3.0).all() and (y[:, :at] == 3.0).all() and (y[:, at + rows:] == 3.0).all()
-        logits, keys = torch.full((M, rows), 3.0, device=gpu), torch.zeros(M + 1, dtype=torch.int64, device=gpu)
-        ops.qgemv([ops.Seg(w)], x, logits, M, argmax=keys)
-        ids = torch.full((M,), -1, dtype=torch.int32, device=gpu)
-        ops.argmax_unpack(keys, M, ids)
-        assert ((logits.cpu().double() - z).abs() <= bound).all() and (ids.long() == logits.argmax(1)).all() and int(keys[M]) == 0
+        for at in (0, 3):
+            for epi in ("f32", "argmax"):
+                keys = torch.zeros(M + 1, dtype=torch.int64, device=gpu)
+                if epi == "f32":
+                    logits = torch.full((M, at + rows), 3.0, device=gpu)
+                ops.qgemv([ops.Seg(w, at)], x, logits, M, epi=epi, argmax=keys)
+                ids = torch.full((M,), -1, dtype=torch.int32, device=gpu)
+                ops.argmax_unpack(keys, M, ids)
+                assert ((logits[:, at:].cpu().double() - z).abs() <= bound).all() and int(keys[M]) == 0
+                top = z.gather(1, ids.cpu().long()[:, None] - at)[:, 0]
+                assert (top >= (z - 2 * bound).amax(1)).all() and (epi == "argmax" or (ids.long() - at == logits[:, at:].argmax(1)).all())
